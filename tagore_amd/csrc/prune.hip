@@ -37,8 +37,10 @@ constexpr int POOL_MAX = 1024;  // K + 480 <= 608, padded to a power of two
 // the table above the most members it can hold, so a probe always ends.
 // -------------------------------------------------------------------------------------
 constexpr int HSET = 512;  // k_cal_ep: up to 256 members
+// (the 24-bit product is a full-rate instruction, the 32-bit one a quarter; ids that share
+// their low 24 bits chain)
 __device__ __forceinline__ uint32_t hslot(uint32_t id, int bits) {
-  return (id * 0x9E3779B1u) >> (32 - bits);
+  return ((id & 0xFFFFFFu) * 0x9E3779u) >> (32 - bits);
 }
 __device__ void hset_clear(uint32_t* tab, int bits) {
   for (int i = threadIdx.x; i < (1 << bits); i += TG_WAVE) tab[i] = TG_INV;
@@ -707,56 +709,12 @@ __global__ __launch_bounds__(64) void k_reverse(PruneArgs a) {
 // -------------------------------------------------------------------------------------
 // One-hop rank (CAGRA: id membership; DPG: occlusion by distance), spec A.8 / A.9.
 // -------------------------------------------------------------------------------------
-template <int MC, class T, int DPG>
-__global__ __launch_bounds__(64) void k_rank_forward(PruneArgs a) {
-  __shared__ uint64_t srt[256];   // (id << 32 | pos) sorted, then (detour << 32 | id)
-  __shared__ uint32_t det[128];
-  __shared__ uint32_t nei[128];
-  const uint32_t u = row_of_block(a.perm, a.N);
-  if (u >= a.N) return;
-  const int lane = threadIdx.x, g = lane >> 4, t = lane & 15;
-  const int K = a.K, D = a.D, d = a.FD;
+// The d = FD entries of smallest (detour count, id) of node u and their reverse pushes.
+// det / nei: the counts and ids by list position; srt: 128 keys of scratch.
+__device__ __forceinline__ void rank_select(const PruneArgs& a, uint32_t u, const uint32_t* det,
+                                            const uint32_t* nei, uint64_t* srt) {
+  const int lane = threadIdx.x, K = a.K, d = a.FD;
   const int n = pow2_at_least(K);
-  for (int j = lane; j < 128; j += TG_WAVE) {
-    det[j] = 0;
-    nei[j] = j < K ? a.G[size_t(u) * K + j] : TG_INV;
-  }
-  __syncthreads();
-  if (!DPG) {
-    for (int j = lane; j < n; j += TG_WAVE)
-      srt[j] = j < K ? ((uint64_t(nei[j]) << 32) | uint32_t(j)) : TG_KEY_INF;
-    __syncthreads();
-    wave_sort<128>(srt, n);
-    for (int r = 0; r < K; ++r) {
-      const uint32_t v = nei[r];
-      for (int l = lane; l < K; l += TG_WAVE) {
-        const uint32_t y = a.G[size_t(v) * K + l];
-        int lo = 0, hi = K;
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (uint32_t(srt[mid] >> 32) < y) lo = mid + 1; else hi = mid;
-        }
-        if (lo < K && uint32_t(srt[lo] >> 32) == y) {
-          const int j = int(uint32_t(srt[lo]));
-          if (j > r) atomicAdd(&det[j], 1u);
-        }
-      }
-    }
-    count_add(a.counters, 3, K);
-  } else {
-    // pairs r < j, row by row; the four groups take every fourth j of a row
-    const int npairs = K * (K - 1) / 2;
-    for (int r = 0; r + 1 < K; ++r) {
-      const T* xr = reinterpret_cast<const T*>(a.rows) + size_t(nei[r]) * D;
-      for (int j = r + 1 + g; j < K; j += 4) {
-        const float dd =
-            dist16_mm<MC>(xr, reinterpret_cast<const T*>(a.rows) + size_t(nei[j]) * D, D, t);
-        if (t == 0 && dd < a.GD[size_t(u) * K + j]) atomicAdd(&det[j], 1u);
-      }
-    }
-    count_add(a.counters, 1, npairs);
-  }
-  __syncthreads();
   for (int j = lane; j < n; j += TG_WAVE)
     srt[j] = j < K ? ((uint64_t(det[j]) << 32) | nei[j]) : TG_KEY_INF;
   __syncthreads();
@@ -769,58 +727,222 @@ __global__ __launch_bounds__(64) void k_rank_forward(PruneArgs a) {
   if (lane == 0) a.fwd_deg[u] = d;
 }
 
-// filter_reverse_1hop (spec A.10): half forward, up to half reverse, forward fill.
+// CAGRA: neighbour j of u gets one detour per earlier neighbour r < j whose list holds j.
+// K rows of K ids are looked up per node, so the lookups' instructions set the time.  u's ids
+// sit in an LDS hash of 256 buckets of four 32-bit entries: an id is its bucket and the 24
+// bits id >> 8 (the bucket adds a function of those bits to the low byte, so the two give
+// the id back), and an entry packs these bits and the id's list position.  A lookup is one
+// 16-byte read and four subtract-and-compares, which test the id and j > r at once, with no
+// loop; ids that find their bucket full (0.01 per node at K = 96) are tested one by one.
+// VEC ids per lane and load (16 bytes where rows are 16-byte aligned, K % 4 == 0), the rows'
+// id groups dealt to the lanes as one flat sequence, two groups in flight per lane.
+// 500k x K = 96: 9.84 -> 2.91 ms (seven-step binary searches of the
+// sorted ids before; 75 % of VALU issue now, LDS reads busy 65 %).
+constexpr int CAGRA_BUCKETS = 256;
+__device__ __forceinline__ uint32_t cagra_bucket(uint32_t id) {
+  return (((id >> 8) * 0x9E3779u + (id << 16)) >> 16) & (CAGRA_BUCKETS - 1);
+}
+__device__ __forceinline__ uint32_t cagra_entry(uint32_t id, uint32_t pos) {
+  return (id >> 8) << 7 | pos;
+}
+template <int VEC>
+__global__ __launch_bounds__(64) void k_cagra_forward(PruneArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t tab[CAGRA_BUCKETS * 4];
+  __shared__ uint32_t ovid[128], ovpos[128];  // ids of full buckets
+  __shared__ uint32_t novf;
+  __shared__ uint64_t srt[128];  // row offsets of the neighbours, then the selection's keys
+  __shared__ uint32_t det[128];
+  __shared__ uint32_t nei[128];
+  const uint32_t u = row_of_block(a.perm, a.N);
+  if (u >= a.N) return;
+  const int lane = threadIdx.x, K = a.K;
+  for (int i = lane; i < CAGRA_BUCKETS * 4; i += TG_WAVE) tab[i] = TG_INV;
+  for (int j = lane; j < 128; j += TG_WAVE) {
+    det[j] = 0;
+    nei[j] = j < K ? a.G[size_t(u) * K + j] : TG_INV;
+    srt[j] = uint64_t(nei[j]) * uint32_t(K) * 4;
+  }
+  if (lane == 0) novf = 0;
+  __syncthreads();
+  for (int j = lane; j < K; j += TG_WAVE) {
+    uint32_t* b = tab + 4 * cagra_bucket(nei[j]);
+    const uint32_t e = cagra_entry(nei[j], uint32_t(j));
+    int q = 0;
+    while (q < 4 && atomicCAS(&b[q], TG_INV, e) != TG_INV) ++q;
+    if (q == 4) {
+      const uint32_t o = atomicAdd(&novf, 1u);
+      ovid[o] = nei[j];
+      ovpos[o] = uint32_t(j);
+    }
+  }
+  __syncthreads();
+  const int nov = int(novf);
+  // an id listed twice counts at its first position only (rows given by a caller may repeat
+  // one); a position 0 never counts, so a later copy in the overflow list takes that
+  for (int j0 = 0; j0 < K; j0 += TG_WAVE) {
+    const int j = j0 + lane;
+    bool dup = false;
+    if (j < K) {
+      const uint32_t id = nei[j], none = cagra_entry(id, 0u);
+      const uint4 v = *reinterpret_cast<const uint4*>(tab + 4 * cagra_bucket(id));
+      dup = v.x - none < uint32_t(j) || v.y - none < uint32_t(j) || v.z - none < uint32_t(j) ||
+            v.w - none < uint32_t(j);
+      for (int o = 0; o < nov; ++o) dup = dup || (ovid[o] == id && int(ovpos[o]) < j);
+    }
+    __syncthreads();
+    if (dup) {
+      uint32_t* b = tab + 4 * cagra_bucket(nei[j]);
+      for (int q = 0; q < 4; ++q)
+        if (b[q] == cagra_entry(nei[j], uint32_t(j))) b[q] = TG_INV;
+      for (int o = 0; o < nov; ++o)
+        if (ovid[o] == nei[j] && int(ovpos[o]) == j) ovpos[o] = 0;
+    }
+    __syncthreads();
+  }
+  // groups of VEC ids, row by row; the last row has no later neighbour
+  const int per = K / VEC, total = (K - 1) * per;
+  const int dr = TG_WAVE / per, dc = TG_WAVE - dr * per;  // TG_WAVE groups further on
+  int r = lane / per, c = lane - r * per;
+  const char* G = reinterpret_cast<const char*>(a.G);
+  auto row_group = [&](uint32_t (&y)[VEC]) {
+    const char* p = G + srt[r] + uint32_t(c) * (VEC * 4);
+    if constexpr (VEC == 4) {
+      const uint4 q = *reinterpret_cast<const uint4*>(p);
+      y[0] = q.x; y[1] = q.y; y[2] = q.z; y[3] = q.w;
+    } else {
+      y[0] = *reinterpret_cast<const uint32_t*>(p);
+    }
+  };
+  auto advance = [&]() {
+    r += dr;
+    c += dc;
+    if (c >= per) {
+      c -= per;
+      ++r;
+    }
+  };
+  auto look_up = [&](const uint32_t (&y)[VEC], uint32_t r1) {  // r1 = r + 1
+    uint4 v[VEC];
+#pragma unroll
+    for (int q = 0; q < VEC; ++q)
+      v[q] = *reinterpret_cast<const uint4*>(tab + 4 * cagra_bucket(y[q]));
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) {
+      // entry - base is pos - (r + 1) when the ids are equal, which is below 127 - r for
+      // r < pos <= 127; other ids differ by at least 128 - r - 1 from there (an empty entry
+      // too), so the smallest difference of the bucket decides, and gives the position
+      const uint32_t base = cagra_entry(y[q], 0u) + r1;
+      const uint32_t m = min(min(v[q].x - base, v[q].y - base), min(v[q].z - base, v[q].w - base));
+      if (m < 128u - r1) atomicAdd(&det[m + r1], 1u);
+    }
+    if (nov)
+      for (int o = 0; o < nov; ++o)
+#pragma unroll
+        for (int q = 0; q < VEC; ++q)
+          if (ovid[o] == y[q] && ovpos[o] >= r1) atomicAdd(&det[ovpos[o]], 1u);
+  };
+  for (int e = lane; e < total; e += 2 * TG_WAVE) {
+    uint32_t ya[VEC], yb[VEC];
+    const uint32_t ra = uint32_t(r) + 1;
+    row_group(ya);
+    advance();
+    const bool second = e + TG_WAVE < total;
+    const uint32_t rb = uint32_t(r) + 1;
+    if (second) row_group(yb);
+    advance();
+    look_up(ya, ra);
+    if (second) look_up(yb, rb);
+  }
+  count_add(a.counters, 3, K);
+  __syncthreads();
+  rank_select(a, u, det, nei, srt);
+}
+
+template <int MC, class T>
+__global__ __launch_bounds__(64) void k_dpg_forward(PruneArgs a) {
+  __shared__ uint64_t srt[128];
+  __shared__ uint32_t det[128];
+  __shared__ uint32_t nei[128];
+  const uint32_t u = row_of_block(a.perm, a.N);
+  if (u >= a.N) return;
+  const int lane = threadIdx.x, g = lane >> 4, t = lane & 15;
+  const int K = a.K, D = a.D;
+  for (int j = lane; j < 128; j += TG_WAVE) {
+    det[j] = 0;
+    nei[j] = j < K ? a.G[size_t(u) * K + j] : TG_INV;
+  }
+  __syncthreads();
+  // pairs r < j, row by row; the four groups take every fourth j of a row
+  const int npairs = K * (K - 1) / 2;
+  for (int r = 0; r + 1 < K; ++r) {
+    const T* xr = reinterpret_cast<const T*>(a.rows) + size_t(nei[r]) * D;
+    for (int j = r + 1 + g; j < K; j += 4) {
+      const float dd =
+          dist16_mm<MC>(xr, reinterpret_cast<const T*>(a.rows) + size_t(nei[j]) * D, D, t);
+      if (t == 0 && dd < a.GD[size_t(u) * K + j]) atomicAdd(&det[j], 1u);
+    }
+  }
+  count_add(a.counters, 1, npairs);
+  __syncthreads();
+  rank_select(a, u, det, nei, srt);
+}
+
+// filter_reverse_1hop (spec A.10): half forward, up to half reverse, forward fill.  The
+// reverse entries w that the first `lim` forward ids do not name follow the forward half, in
+// (detour, id) order.  One reverse entry per lane (two past 64), its membership a scan of the
+// forward ids broadcast from LDS; the whole pass was lane 0's serial insertion sorts and
+// scans before (500k x FD = 32: 7.37 -> 0.65 ms).
 __global__ __launch_bounds__(64) void k_rank_reverse(PruneArgs a) {
   __shared__ uint64_t buf[256];
-  __shared__ uint32_t A[128];
+  __shared__ uint32_t T[128];
   const uint32_t u = blockIdx.x;
   if (u >= a.N) return;
   const int lane = threadIdx.x;
   const int d = a.FD, h = d / 2;
+  for (int i = lane; i < 128; i += TG_WAVE)
+    T[i] = i < d ? a.fwd_ids[size_t(u) * d + i] : TG_INV;
   // R1[u]: the d smallest (detour, src) pushes, already sorted by (detour, id)
   const int r = pb_top(a.rev, u, d, false, [](uint64_t) { return true; }, buf);
-  const uint32_t* T = a.fwd_ids + size_t(u) * d;
   uint32_t* row = a.out_ids + size_t(u) * d;
-  // Rv sorted by (id, detour); later copies of an id get detour INV; then by (detour,id).
-  // Pushes carry distinct sources, so the relabelling never fires; it is kept for parity.
-  if (lane == 0) {
-    // insertion-sort by id on buf[128..128+r)
-    for (int i = 0; i < r; ++i) {
-      const uint64_t k = (uint64_t(uint32_t(buf[i])) << 32) | uint32_t(buf[i] >> 32);
-      int j = i;
-      while (j > 0 && buf[128 + j - 1] > k) {
-        buf[128 + j] = buf[128 + j - 1];
-        --j;
-      }
-      buf[128 + j] = k;
-    }
-    for (int i = r - 1; i >= 1; --i)
-      if (uint32_t(buf[128 + i] >> 32) == uint32_t(buf[128 + i - 1] >> 32))
-        buf[128 + i] = (buf[128 + i] & 0xFFFFFFFF00000000ull) | TG_INV;
-    // back to (detour << 32 | id) order
-    for (int i = 0; i < r; ++i) {
-      const uint64_t k = (uint64_t(uint32_t(buf[128 + i])) << 32) | uint32_t(buf[128 + i] >> 32);
-      int j = i;
-      while (j > 0 && buf[j - 1] > k) {
-        buf[j] = buf[j - 1];
-        --j;
-      }
-      buf[j] = k;
-    }
-    int na = 0;
-    const int lim = (r < h) ? (d - r) : h;
-    for (int i = 0; i < r; ++i) {
-      if (r >= h && na >= h) break;
-      const uint32_t w = uint32_t(buf[i]);
-      bool in = false;
-      for (int j = 0; j < lim; ++j) in = in || (T[j] == w);
-      if (!in) A[na++] = w;
-    }
-    for (int i = 0; i < h; ++i) row[i] = T[i];
-    for (int i = 0; i < na; ++i) row[h + i] = A[i];
-    for (int i = 0; h + na + i < d; ++i) row[h + na + i] = T[h + i];
-    a.out_deg[u] = d;
+  // Later copies of a source get detour INV and go last, by id.  Sources repeat only where a
+  // given kNN row lists an id twice.
+  bool any = false;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = q * TG_WAVE + lane;
+    const uint32_t id = uint32_t(buf[i]);
+    bool dup = false;
+    const int top = min(r, (q + 1) * TG_WAVE);
+    if (top > q * TG_WAVE)
+      for (int j = 0; j + 1 < top; ++j) dup = dup || (j < i && uint32_t(buf[j]) == id);
+    dup = dup && i < r;
+    any = any || ballot(dup) != 0;
+    if (dup) buf[128 + i] = (uint64_t(TG_INV) << 32) | id;
+    else if (i < r) buf[128 + i] = buf[i];
   }
+  __syncthreads();
+  if (any) {
+    const int n = pow2_at_least(r);
+    for (int i = lane; i < n; i += TG_WAVE) buf[i] = i < r ? buf[128 + i] : TG_KEY_INF;
+    __syncthreads();
+    wave_sort<128>(buf, n);
+  }
+  const int lim = (r < h) ? (d - r) : h;
+  int na = 0;
+  for (int base = 0; base < r; base += TG_WAVE) {
+    const int i = base + lane;
+    const uint32_t w = i < r ? uint32_t(buf[i]) : TG_INV;
+    bool add = i < r;
+    for (int j = 0; j < lim; ++j) add = add && T[j] != w;
+    const uint64_t m = ballot(add);
+    const int p = na + mask_rank(m);
+    if (add && (r < h || p < h)) row[h + p] = w;
+    na += int(__popcll(m));
+  }
+  if (r >= h) na = min(na, h);
+  for (int i = lane; i < h; i += TG_WAVE) row[i] = T[i];
+  for (int i = lane; h + na + i < d; i += TG_WAVE) row[h + na + i] = T[h + i];
+  if (lane == 0) a.out_deg[u] = d;
 }
 
 // -------------------------------------------------------------------------------------
@@ -900,9 +1022,7 @@ static void launch_prune_mc(const PruneArgs& a, int phase, const float* centroid
       k_forward<MC, T, 1, 1><<<grid, block, fwd_layout(a.K, a.TOPM, a.FD).bytes, s>>>(a);
       break;
     case PH_REV: k_reverse<MC, T><<<grid, block, 0, s>>>(a); break;
-    case PH_CAGRA: k_rank_forward<MC, T, 0><<<grid, block, 0, s>>>(a); break;
-    case PH_DPG: k_rank_forward<MC, T, 1><<<grid, block, 0, s>>>(a); break;
-    case PH_RANK_REV: k_rank_reverse<<<grid, block, 0, s>>>(a); break;
+    case PH_DPG: k_dpg_forward<MC, T><<<grid, block, 0, s>>>(a); break;
     default: break;
   }
 }
@@ -934,6 +1054,15 @@ static void launch_prune_u8_mc(const PruneArgs& a, int phase, hipStream_t s) {
 
 void launch_prune(const PruneArgs& a, int phase, const float* centroid, uint32_t* ep,
                   hipStream_t s, uint32_t nseg) {
+  if (phase == PH_CAGRA) {  // ids only
+    if (a.K % 4 == 0) k_cagra_forward<4><<<grid_rows(a.perm, a.N), 64, 0, s>>>(a);
+    else k_cagra_forward<1><<<grid_rows(a.perm, a.N), 64, 0, s>>>(a);
+    return;
+  }
+  if (phase == PH_RANK_REV) {
+    k_rank_reverse<<<a.N, 64, 0, s>>>(a);
+    return;
+  }
   // (rows up to 256 values: wider u8 batches would not stay in registers)
   if (a.rows8 && a.D <= 256 && (phase == PH_FWD_PATH || phase == PH_FWD_2HOP || phase == PH_REV)) {
     PruneArgs b = a;

@@ -429,3 +429,12 @@ def test_knn_bit_identical_u8_rows(D):
     bad = np.nonzero((G != Gr).any(1))[0]
     assert bad.size == 0, f"D={D}: {bad.size} rows differ, first {bad[:5]}"
     assert np.array_equal(GD, GDr)
+
+
+@pytest.mark.parametrize("K,FD", [(24, 24), (25, 9), (50, 33), (96, 32), (127, 128 - 1), (128, 128)])
+def test_cagra_lookup_edges(K, FD):
+    """CAGRA's detour lookups on rows that are and are not 16-byte aligned (K % 4), at odd and
+    full degrees, up to the longest lists: equal to the oracle."""
+    X = gmm_int(1500, 32, 6, K)
+    G, GD = oracle.knn_bruteforce(X, K)
+    _compare(X, G, GD, 2, 0, 2, FD, 64, 0.0)
