@@ -61,8 +61,9 @@ typedef struct {
   int32_t init;       /* TG_INIT_* */
   uint32_t sample;    /* learned init: sample size (0: min(N, 50000)) */
   uint32_t epochs;    /* learned init: training epochs (0: 2) */
-  uint32_t tile;      /* local-join MFMA staging depth: 0 = 256-byte rows per LDS round,
-                         1 = 64-byte rows (results are identical; see tg_autotune_knn) */
+  uint32_t tile;      /* local-join MFMA staging depth: 0 = the default bytes of a row per LDS
+                         round, 1 = the other depth (results are identical; see
+                         tg_autotune_knn) */
   uint32_t flags;     /* TG_FLAG_*: 0 for the defaults */
 } tg_knn_params;
 /* learned init: capture the encoder's training loop (about 2,200 small kernels) as a HIP

@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -20,6 +21,7 @@
 #include "errors.hpp"
 #include "kernels.hpp"
 #include "learn.hpp"
+#include "screen.hpp"
 
 using namespace tg;
 
@@ -125,9 +127,11 @@ struct tg_state {
   uint8_t* Xq8 = nullptr;  // FP8 e4m3 copy of X with per-vector scales (screen)
   float *sc8 = nullptr, *nq8 = nullptr, *ne8 = nullptr;
   bool prep8_valid = false;
-  uint16_t* Xb = nullptr;  // BF16 copy of X (screen)
-  float *nrm2 = nullptr, *nq = nullptr, *ne = nullptr;
-  uint32_t* cert_flags = nullptr;  // [5], see k_screen_prep
+  uint16_t* Xb = nullptr;  // 16-bit copy of X (screen): BF16 when exact, else scaled FP16
+  float* nrm2 = nullptr;
+  uint32_t* cert_flags = nullptr;  // [7], see k_screen_prep and k_screen_copy
+  bool copy16 = false;             // Xb can serve as the screen copy
+  float kap16 = 0.f, pscale16 = 2.f;  // its bound and product scale (KnnArgs)
   bool prep_valid = false;         // Xb / norms / certificates match the current X
   bool cert_bf16 = false;          // every value of X is exactly representable in BF16
   bool cert_int = false;           // integer data whose screen distances are exact
@@ -252,24 +256,52 @@ int ensure_knn_scratch(tg_state* s, uint32_t K) {
   return TG_OK;
 }
 
-// BF16 copy, norms and data-set certificates of the current vectors (computed once per data
-// set, like the reference's host-side FP16 copy, pybind.cu:58-61).
+// Norms, data-set certificates and the 16-bit copy of the current vectors (computed once per
+// data set, like the reference's host-side FP16 copy, pybind.cu:58-61).
 int ensure_prep(tg_state* s) {
   if (s->prep_valid) return TG_OK;
   const size_t N = s->N;
   if (!s->nrm2) {
-    if (dalloc(&s->nrm2, N) || dalloc(&s->nq, N) || dalloc(&s->ne, N) ||
-        dalloc(&s->cert_flags, 5) || dalloc(&s->Xb, N * s->D))
+    if (dalloc(&s->nrm2, N) || dalloc(&s->cert_flags, 7) || dalloc(&s->Xb, N * s->D))
       return TG_ERR_HIP;
   }
-  fill_u32(s->cert_flags, 0, 5, s->stream);
-  launch_screen_prep(s->X, s->N, s->D, s->Xb, s->nrm2, s->nq, s->ne, s->cert_flags, s->stream);
-  uint32_t f[5];
+  fill_u32(s->cert_flags, 0, 7, s->stream);
+  launch_screen_prep(s->X, s->N, s->D, s->nrm2, s->cert_flags, s->stream);
+  uint32_t f[7];
   HIPX(hipMemcpyAsync(f, s->cert_flags, sizeof(f), hipMemcpyDeviceToHost, s->stream));
   HIPX(hipStreamSynchronize(s->stream));
   s->cert_bf16 = f[0] == 0;
-  float qmax;
+  float qmax, vmax;
   std::memcpy(&qmax, &f[3], 4);
+  std::memcpy(&vmax, &f[5], 4);
+  // the 16-bit copy: exact BF16, or FP16 with the largest value scaled below 2^15.  A row
+  // error above 2^-9 (rows far smaller than the largest value) or values beyond the scales
+  // that keep the products in FP32's range: no 16-bit screen, the FP32 one serves
+  s->copy16 = true;
+  s->pscale16 = 2.f;
+  double rho = 0.0;
+  if (s->cert_bf16) {
+    launch_screen_copy(s->X, s->N, s->D, false, 1.f, s->Xb, s->cert_flags, s->stream);
+  } else {
+    int ex = 0;
+    s->copy16 = std::isfinite(vmax);
+    if (s->copy16) {
+      (void)std::frexp(vmax, &ex);  // vmax < 2^ex
+      s->copy16 = ex >= -30 && ex <= 55;
+    }
+    if (s->copy16) {
+      launch_screen_copy(s->X, s->N, s->D, true, std::ldexp(1.f, 15 - ex), s->Xb, s->cert_flags,
+                         s->stream);
+      HIPX(hipMemcpyAsync(f, s->cert_flags, sizeof(f), hipMemcpyDeviceToHost, s->stream));
+      HIPX(hipStreamSynchronize(s->stream));
+      float r;
+      std::memcpy(&r, &f[6], 4);
+      s->copy16 = r <= 0x1p-9f;
+      rho = r;
+      s->pscale16 = std::ldexp(2.f, 2 * (ex - 15));
+    }
+  }
+  s->kap16 = screen_kappa16(rho, s->D);
   // every MFMA partial sum, |a|^2+|b|^2 and |a-b|^2 stay integers below 2^24
   const double lim = 16777216.0;
   s->cert_int = f[1] == 0 && (f[2] == 0 ? 2.0 * qmax < lim : 4.0 * qmax < lim);
@@ -341,9 +373,7 @@ KnnArgs knn_args(tg_state* s, uint64_t seed) {
   a.counters = s->counters;
   a.Xb = s->Xb;
   a.nrm2 = s->nrm2;
-  a.nq = s->nq;
-  a.ne = s->ne;
-  // relative slack of the screen bound: accumulation (2 D ulps per term, doubled) plus the
+  // relative slack of the FP8 bound: accumulation (2 D ulps per term, doubled) plus the
   // canonical distance's own rounding, with margin
   a.eta = float((8.0 * s->D + 128.0) * 5.9604644775390625e-8);
   return a;
@@ -495,8 +525,6 @@ int tg_free(tg_state* s) {
   dfree(s->nq8);
   dfree(s->ne8);
   dfree(s->nrm2);
-  dfree(s->nq);
-  dfree(s->ne);
   dfree(s->cert_flags);
   dfree(s->X8);
   dfree(s->n2s);
@@ -1098,6 +1126,8 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
   fill_u32(reinterpret_cast<uint32_t*>(s->counters), 0, 2 * CNT_SLOTS * CNT_N, st);
   clear_errors(s, {&s->pn, &s->po, &s->pc, &s->pr});
   HIPX(hipEventRecord(w0, st));
+  // data that no 16-bit copy screens well takes the FP32 screen instead (same graph)
+  const int prec = p->precision == TG_PREC_BF16 && !s->copy16 ? int(TG_PREC_FP32) : p->precision;
   // precision-dependent parts of the argument block (re-applied after every swap)
   // integer data makes the FP32 / BF16 screens exact; FP8 rounds integers above 16
   const bool exact_screen =
@@ -1116,6 +1146,8 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       k.seg_key = s->seg_key;
     }
     k.exact_screen = exact_screen ? 1 : 0;
+    k.kap = prec == TG_PREC_BF16 ? s->kap16 : screen_kappa32(s->D);
+    k.pscale = prec == TG_PREC_BF16 ? s->pscale16 : 2.f;
     k.Xr16 = rows16;
     k.X8 = (p->precision != TG_PREC_EXACT && s->cert_u8 && s->D <= 256) ? s->X8 : nullptr;
     k.n2s = k.X8 ? s->n2s : nullptr;
@@ -1172,7 +1204,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(3)) return TG_ERR_HIP;
       pb_reset(a.pc, N, s->fill, st);
-      launch_knn_localjoin(a, p->precision, int(p->tile), st);
+      launch_knn_localjoin(a, prec, int(p->tile), st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(4)) return TG_ERR_HIP;
       pb_group_overflow(a.pc, N, s->fill, s->scan_tmp, st);
@@ -1191,7 +1223,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
     for (uint32_t it = 0; it < it2; ++it) {
       if (sc.start(6)) return TG_ERR_HIP;
       pb_reset(a.pr, N, s->fill, st);
-      launch_knn_phase2(a, p->precision, st);
+      launch_knn_phase2(a, prec, st);
       pb_group_overflow(a.pr, N, s->fill, s->scan_tmp, st);
       launch_knn_rupdate(a, st);
       if (sc.stop()) return TG_ERR_HIP;
@@ -1212,7 +1244,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       key.insert(key.end(), b, b + n);
     };
     put(&a, sizeof(a));
-    const uint64_t extra[] = {it1, it2, uint64_t(p->precision), p->tile,
+    const uint64_t extra[] = {it1, it2, uint64_t(prec), p->tile,
                               uint64_t(reinterpret_cast<uintptr_t>(s->fill)),
                               uint64_t(reinterpret_cast<uintptr_t>(s->scan_tmp)),
                               uint64_t(reinterpret_cast<uintptr_t>(s->rv_hist)),
@@ -1385,7 +1417,7 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   a.rows8 = s->cert_u8 ? s->X8 : nullptr;
   // DPG's pair distances on an MFMA Gram (K <= 64) with exact re-scores near the threshold
   const bool dpg_screen = p->kind == TG_KIND_DPG && K <= 64 &&
-                          ((p->precision == TG_PREC_BF16 && s->D % 8 == 0) ||
+                          ((p->precision == TG_PREC_BF16 && s->D % 8 == 0 && s->copy16) ||
                            (p->precision == TG_PREC_FP8 && s->D % 16 == 0));
   if (dpg_screen && p->precision == TG_PREC_FP8)
     if (int rc = ensure_prep8(s)) return rc;
@@ -1423,8 +1455,10 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
       if (dpg_screen) {
         DpgScreen q{};
         q.nrm2 = s->nrm2;
-        q.nq = p->precision == TG_PREC_FP8 ? s->nq8 : s->nq;
-        q.ne = p->precision == TG_PREC_FP8 ? s->ne8 : s->ne;
+        q.nq = s->nq8;
+        q.ne = s->ne8;
+        q.kap = s->kap16;
+        q.pscale = s->pscale16;
         q.sc8 = s->sc8;
         q.Xb = s->Xb;
         q.Xq8 = s->Xq8;

@@ -205,6 +205,13 @@ __device__ __forceinline__ float row_shl(float v) {
                                                     false));
 }
 
+// lane i of each 16-lane DPP row reads lane i-S of the same row (lanes below S read 0)
+template <int S>
+__device__ __forceinline__ float row_shr(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x110 + S, 0xF, 0xF,
+                                                    false));
+}
+
 // Reduction of the group's partials (lane t holds p[4t..4t+3]): first inside the lane,
 // q[t] = (p[4t] + p[4t+1]) + (p[4t+2] + p[4t+3]), then the tree q[t] += q[t+s] for
 // s = 8,4,2,1 as DPP row shifts across the group.  Six levels, like any balanced tree of

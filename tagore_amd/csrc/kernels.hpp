@@ -52,14 +52,15 @@ struct PruneArgs {
 // the BF16 or FP8 copy, and the bound's relative slack
 struct DpgScreen {
   const float* nrm2;
-  const float* nq;
+  const float* nq;      // FP8: |x'| and |x' - x|, rounded up
   const float* ne;
   const float* sc8;
-  const uint16_t* Xb;
+  const uint16_t* Xb;   // 16-bit copy (KnnArgs::Xb)
   const uint8_t* Xq8;
-  float eta;
+  float eta;            // FP8: relative slack of the bound
+  float kap, pscale;    // 16-bit rows (see KnnArgs)
 };
-// precision: KP_BF16 or KP_FP8; K <= 64
+// precision: KP_BF16 (the 16-bit copy) or KP_FP8; K <= 64
 void launch_dpg_screen(const PruneArgs& a, const DpgScreen& q, int precision, hipStream_t s);
 
 // PH_EP runs one workgroup per segment: segment c starts its beam at its first row and
@@ -92,12 +93,16 @@ struct KnnArgs {
   uint32_t* Rn1;    // [N]
   uint64_t seed;
   unsigned long long* counters;  // [8] or null
-  // screening (precision FP32 / BF16): a screen distance s = |a|^2 + |b|^2 - 2 a'.b' on the
-  // screen copies a', b' with a rigorous bound |s - dist(a,b)| <= E(a,b); only candidates
-  // whose bound interval can change a decision are re-scored with the canonical distance.
-  const uint16_t* Xb;  // [N*D] BF16 rows (precision BF16)
+  // screening (precision FP32 / BF16): a screen distance s = |a|^2 + |b|^2 - pscale a'.b' on
+  // the screen copies a', b' with the rigorous bound |s - dist(a,b)| <= kap (|a|^2 + |b|^2)
+  // (screen.hpp); only candidates whose bound interval can change a decision are re-scored
+  // with the canonical distance.
+  const uint16_t* Xb;  // [N*D] 16-bit rows: BF16 when exact (then Xr16), else scaled FP16
   const float* nrm2;   // [N] |x|^2 (FP64 sum rounded once)
-  const float* nq;     // [N] |x'| of the screen copy (rounded up)
+  float kap;
+  float pscale;        // 2 / scale^2 of the 16-bit copy (2 for BF16 and FP32 rows)
+  // FP8: s +- 2 (ea qb + qa eb + ea eb) + eta (|a|^2 + |b|^2 + 2 qa qb)
+  const float* nq;     // [N] |x'| of the FP8 copy (rounded up)
   const float* ne;     // [N] |x' - x| (rounded up)
   float eta;           // relative slack of the bound
   // Integer data set (values in [-256, 256], |x|^2 small enough that every partial sum is
@@ -108,7 +113,7 @@ struct KnnArgs {
   const uint16_t* Xr16;
   const uint8_t* X8;     // u8 copy of X (every value an integer in [0, 255], D <= 256) or null
   const float* n2s;      // [N] |x - 128|^2 of the u8 rows (exact), with X8
-  // FP8 e4m3 copy with a per-vector scale (FP8 screen: nq/ne then hold its norms)
+  // FP8 e4m3 copy with a per-vector scale
   const uint8_t* Xq8;
   const float* sc8;
   // segments (see PruneArgs): the initial lists draw ids inside the row's own segment, from a
@@ -126,17 +131,20 @@ void launch_screen_prep8(const float* X, uint32_t N, uint32_t D, uint8_t* Xq, fl
 void launch_make_u8(const float* X, size_t n, uint8_t* X8, hipStream_t s);
 // |x - 128|^2 of every u8 row (the norms of the rows shifted into int8)
 void launch_u8_shift_norms(const uint8_t* X8, uint32_t N, uint32_t D, float* n2s, hipStream_t s);
-// screen-mode preparation: BF16 copy (if Xb), norms, quantisation-error norms and the
-// data-set certificates in flags[5] (zeroed by the caller)
-void launch_screen_prep(const float* X, uint32_t N, uint32_t D, uint16_t* Xb, float* nrm2,
-                        float* nq, float* ne, uint32_t* flags, hipStream_t s);
+// screen-mode preparation: norms and the data-set certificates in flags[0..5], then the
+// 16-bit copy (half: scaled FP16, its largest relative row error in flags[6]; else BF16
+// bits); flags zeroed by the caller
+void launch_screen_prep(const float* X, uint32_t N, uint32_t D, float* nrm2, uint32_t* flags,
+                        hipStream_t s);
+void launch_screen_copy(const float* X, uint32_t N, uint32_t D, bool half, float scale,
+                        uint16_t* Xb, uint32_t* flags, hipStream_t s);
 
 void launch_knn_init(const KnnArgs& a, hipStream_t s);
 // canonical distances of the ids in G, rows sorted by (d, id), flags cleared
 void launch_knn_init_sort(const KnnArgs& a, hipStream_t s);
 void launch_knn_sample(const KnnArgs& a, hipStream_t s);
 void launch_knn_rsample(const KnnArgs& a, hipStream_t s);
-// tile: staging depth of the MFMA screen (0: 256-byte rows per round, 1: 64-byte rows)
+// tile: staging depth of the MFMA screen (0: the default, 1: the other one)
 void launch_knn_localjoin(const KnnArgs& a, int precision, int tile, hipStream_t s);
 void launch_knn_merge(const KnnArgs& a, hipStream_t s);
 // Reverse lists as exact runs per destination in a.pr (cnt, ov_off, ov_sorted; read them with

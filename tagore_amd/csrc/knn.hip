@@ -14,6 +14,7 @@
 // of the reference's atomic slot counters.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "screen.hpp"
 
 namespace tg {
 
@@ -576,27 +577,6 @@ __device__ __forceinline__ void load_rowbf(RowBf<MB>& r, const uint16_t* x, int 
   }
 }
 
-template <int MB>
-__device__ __forceinline__ float dot_bf16(const RowBf<MB>& a, const uint16_t* y, int D, int t) {
-  float s = 0.f;
-#pragma unroll
-  for (int m = 0; m < MB; ++m) {
-    const int i = 128 * m + 8 * t;
-    if (i < D) {
-      const uint4 q = *reinterpret_cast<const uint4*>(y + i);
-      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        s = __builtin_fmaf(a.v[m][2 * k], bfbits2f(w[k] & 0xFFFFu), s);
-        s = __builtin_fmaf(a.v[m][2 * k + 1], bfbits2f(w[k] >> 16), s);
-      }
-    }
-  }
-#pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 16);
-  return s;
-}
-
 // FP8 screen of one candidate: lane t of the 16-lane group holds u's dequantised elements
 // 256m + 16t..+15 (D % 16 == 0); the scales are applied by the caller.
 template <int MF>
@@ -625,33 +605,52 @@ __device__ __forceinline__ void load_rowf8(RowF8<MF>& r, const uint8_t* x, int D
   }
 }
 
-template <int MF>
-__device__ __forceinline__ float dot_f8(const RowF8<MF>& a, const uint8_t* y, int D, int t) {
-  float s = 0.f;
+// FP16 screen: lane t of the 16-lane group holds u' elements 128m + 8t..+7 as FP16 pairs
+// (two products per instruction).  Four candidates at a time, their loads issued before any
+// arithmetic (as in the BF16 and FP8 forms below).
+template <int MB>
+struct RowH {
+  uint4 v[MB];
+};
+template <int MB>
+__device__ __forceinline__ void load_rowh(RowH<MB>& r, const uint16_t* x, int D, int t) {
 #pragma unroll
-  for (int m = 0; m < MF; ++m) {
-    const int i = 256 * m + 16 * t;
-    if (i < D) {
-      const uint4 q = *reinterpret_cast<const uint4*>(y + i);
-      const int w[4] = {int(q.x), int(q.y), int(q.z), int(q.w)};
+  for (int m = 0; m < MB; ++m) {
+    const int i = 128 * m + 8 * t;
+    r.v[m] = i < D ? *reinterpret_cast<const uint4*>(x + i) : make_uint4(0, 0, 0, 0);
+  }
+}
+template <int MB>
+__device__ __forceinline__ void dot_f16x4(const RowH<MB>& a, const uint16_t* const (&y)[4], int D,
+                                          int t, float (&out)[4]) {
+  uint4 q[4][MB];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(w[k], false);
-        const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(w[k], true);
-        s = __builtin_fmaf(a.v[m][4 * k], lo.x, s);
-        s = __builtin_fmaf(a.v[m][4 * k + 1], lo.y, s);
-        s = __builtin_fmaf(a.v[m][4 * k + 2], hi.x, s);
-        s = __builtin_fmaf(a.v[m][4 * k + 3], hi.y, s);
-      }
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int i = 128 * m + 8 * t;
+      q[b][m] = i < D ? *reinterpret_cast<const uint4*>(y[b] + i) : make_uint4(0, 0, 0, 0);
     }
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    float s = 0.f;
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const uint32_t x[4] = {a.v[m].x, a.v[m].y, a.v[m].z, a.v[m].w};
+      const uint32_t w[4] = {q[b][m].x, q[b][m].y, q[b][m].z, q[b][m].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        s = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, x[k]), __builtin_bit_cast(f16x2, w[k]),
+                                   s, false);
+    }
+    out[b] = s;
   }
 #pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 16);
-  return s;
+  for (int o = 8; o >= 1; o >>= 1)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) out[b] += __shfl_xor(out[b], o, 16);
 }
 
-// Four candidates at a time (their loads issued before any arithmetic); each result is
-// the same operation sequence as dot_bf16 / dot_f8 of that candidate.
 template <int MB>
 __device__ __forceinline__ void dot_bf16x4(const RowBf<MB>& a, const uint16_t* const (&y)[4],
                                            int D, int t, float (&out)[4]) {
@@ -722,7 +721,7 @@ __device__ __forceinline__ void dot_f8x4(const RowF8<MF>& a, const uint8_t* cons
     for (int b = 0; b < 4; ++b) out[b] += __shfl_xor(out[b], o, 16);
 }
 
-__device__ __forceinline__ float screen_bound2(float na, float qa, float ea, float nb, float qb,
+__device__ __forceinline__ float screen_bound8(float na, float qa, float ea, float nb, float qb,
                                                float eb, float eta) {
   return 2.0f * (ea * qb + qa * eb + ea * eb) + eta * (na + nb + 2.0f * qa * qb);
 }
@@ -817,21 +816,24 @@ __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
   constexpr int MB = (MC + 1) / 2;
   constexpr int MF = (MC + 3) / 4;
   constexpr bool SCREEN = PREC == KP_BF16 || PREC == KP_FP8;
-  RowBf<PREC == KP_BF16 ? MB : 1> ub;
+  constexpr bool HALF = PREC == KP_BF16 && std::is_same<T, float>::value;  // FP16 copy
+  RowBf<PREC == KP_BF16 && !HALF ? MB : 1> ub;
+  RowH<HALF ? MB : 1> uh;
   RowF8<PREC == KP_FP8 ? MF : 1> uf;
   float nu = 0.f, qu = 0.f, eu = 0.f, su = 1.f;
-  if (PREC == KP_BF16) load_rowbf(ub, a.Xb + size_t(u) * D, D, t);
+  if constexpr (HALF) load_rowh(uh, a.Xb + size_t(u) * D, D, t);
+  else if (PREC == KP_BF16) load_rowbf(ub, a.Xb + size_t(u) * D, D, t);
   if (PREC == KP_FP8) {
     load_rowf8(uf, a.Xq8 + size_t(u) * D, D, t);
     su = a.sc8[u];
   }
-  if (SCREEN) {
-    nu = a.nrm2[u];
+  if (SCREEN) nu = a.nrm2[u];
+  if (PREC == KP_FP8) {
     qu = a.nq[u];
     eu = a.ne[u];
   }
   for (int q = lane; q < nk; q += TG_WAVE) kv[q] = TG_KEY_INF;
-  // BF16 screen: keep (in order) only the candidates whose bound interval reaches below the
+  // 16-bit / FP8 screen: keep (in order) only the candidates whose bound interval reaches below the
   // worst distance; everything kept is re-scored exactly.  The keep flags use kv's space
   // (the keys are cleared again after the compaction).
   int nre = cnt;
@@ -874,18 +876,22 @@ __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
         const uint16_t* rb[4];
 #pragma unroll
         for (int b = 0; b < 4; ++b) rb[b] = a.Xb + size_t(y[b]) * D;
-        dot_bf16x4(ub, rb, D, t, dp);
+        if constexpr (HALF) dot_f16x4(uh, rb, D, t, dp);
+        else dot_bf16x4(ub, rb, D, t, dp);
       }
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         const int q = q0 + g + 4 * b;
         if (q >= cnt) continue;
-        const float s = (nu + nb[b]) - 2.0f * dp[b];
+        const float nsum = nu + nb[b];
+        const float s = HALF ? __builtin_fmaf(-a.pscale, dp[b], nsum) : nsum - 2.0f * dp[b];
         if (a.exact_screen) {
           // integer data: s is the canonical distance itself
           if (t == 0 && s < worst) kv[q] = mk_key(s, y[b]);
         } else {
-          const float E = screen_bound2(nu, qu, eu, nb[b], a.nq[y[b]], a.ne[y[b]], a.eta);
+          const float E = PREC == KP_FP8
+                              ? screen_bound8(nu, qu, eu, nb[b], a.nq[y[b]], a.ne[y[b]], a.eta)
+                              : a.kap * nsum;
           if (t == 0) keep[q] = (s - E < worst) ? 1 : 0;
         }
       }

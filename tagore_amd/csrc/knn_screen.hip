@@ -4,65 +4,130 @@
 // sampled node list A = new'(u) (<= 64 rows) and B = old'(u) (<= 64 rows), the per-16-wide-
 // tile minimum of the pair distances A x B, B x A and A x A.  Here the Gram matrices A.B^T and
 // A.A^T are contracted on the matrix cores from LDS-staged, coalesced row loads:
-//   BF16: v_mfma_f32_16x16x32_bf16 on a BF16 copy of the vectors,
+//   16-bit: v_mfma_f32_16x16x32_bf16 / _f16 on a 16-bit copy of the vectors (screen.hpp),
 //   FP32: v_mfma_f32_16x16x4_f32 on the FP32 vectors,
-// and turned into screen distances s = |a|^2 + |b|^2 - 2 a'.b'.  A rigorous bound E(a,b) on
+// and turned into screen distances s = |a|^2 + |b|^2 - 2 a'.b'.  A rigorous bound on
 // |s - dist(a,b)| (quantisation + accumulation + canonical-distance rounding) selects, per
 // tile, the only candidates that can be the exact (distance, id) minimum and pass the
 // destination's worst distance; those are re-scored with the canonical FP32 distance.  The
 // pushes are therefore bit-identical to the exact kernel's: graph decisions stay FP32.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "screen.hpp"
 
 namespace tg {
 
-
-constexpr int LJ_TILE = 16;
 constexpr int HROW_S = 128;
 
 
-// Per-vector screen statistics (one wave per row, FP64 sums) and data-set certificates:
+// Maximum / union over the workgroup of one value per thread, in thread 0 (sh: 4 words).
+template <class Op>
+__device__ __forceinline__ uint32_t wg_reduce(uint32_t v, uint32_t* sh, Op op) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = op(v, uint32_t(__shfl_xor(int(v), o, TG_WAVE)));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const uint32_t r = op(op(sh[0], sh[1]), op(sh[2], sh[3]));
+  __syncthreads();
+  return r;
+}
+__device__ __forceinline__ uint32_t op_max(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t op_or(uint32_t a, uint32_t b) { return a | b; }
+
+// |x|^2 of every row (FP64 sums, rounded once) and the data-set certificates:
 // flags[0] |= some value is not exactly representable in BF16,
 // flags[1] |= some value is not an integer in [-256, 256], flags[2] |= some value is
 // negative, flags[3] = max |x|^2 (FP32 bits; exact for integer data below 2^24),
-// flags[4] |= some value is above 255.
-__global__ void k_screen_prep(const float* X, uint32_t N, uint32_t D, uint16_t* Xb, float* nrm2,
-                              float* nq, float* ne, uint32_t* flags) {
-  const uint32_t row = blockIdx.x;
-  if (row >= N) return;
-  const float* x = X + size_t(row) * D;
-  double s2 = 0.0, q2 = 0.0, e2 = 0.0;
-  uint32_t not_bf16 = 0, not_int = 0, neg = 0, big = 0;
-  for (uint32_t j = threadIdx.x; j < D; j += TG_WAVE) {
-    const float v = x[j];
-    const uint16_t b = f2bf(v);
-    if (Xb) Xb[size_t(row) * D + j] = b;
-    const float w = bf2f(b);
-    not_bf16 |= w != v;
-    not_int |= !(rintf(v) == v && fabsf(v) <= 256.f);
-    neg |= v < 0.f;
-    big |= v > 255.f;
-    s2 += double(v) * double(v);
-    q2 += double(w) * double(w);
-    e2 += (double(w) - double(v)) * (double(w) - double(v));
+// flags[4] |= some value is above 255, flags[5] = max |value| (FP32 bits).
+// A 16-lane group per row with 16-byte loads; the flags leave a workgroup once (an atomic per
+// row on one word took 11.3 ms for 1M x 128 rows, all of it the atomics).
+__global__ __launch_bounds__(256) void k_screen_prep(const float* X, uint32_t N, uint32_t D,
+                                                     float* nrm2, uint32_t* flags) {
+  __shared__ uint32_t sh[4];
+  const int t = threadIdx.x & 15;
+  uint32_t bits = 0, top = 0, big = 0;  // bits: 1 not BF16, 2 not integer, 4 negative, 8 above 255
+  for (size_t row = size_t(blockIdx.x) * 16 + (threadIdx.x >> 4); row < N;
+       row += size_t(gridDim.x) * 16) {
+    const float* x = X + row * D;
+    double s2 = 0.0;
+    for (uint32_t j = 4 * t; j < D; j += 64) {
+      const float4 q = load4(x + j);
+      const float v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        bits |= (bf2f(f2bf(v[b])) != v[b]) ? 1u : 0u;
+        bits |= !(rintf(v[b]) == v[b] && fabsf(v[b]) <= 256.f) ? 2u : 0u;
+        bits |= v[b] < 0.f ? 4u : 0u;
+        bits |= v[b] > 255.f ? 8u : 0u;
+        big = op_max(big, __float_as_uint(v[b]) & 0x7FFFFFFFu);
+        s2 += double(v[b]) * double(v[b]);
+      }
+    }
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) s2 += __shfl_xor(s2, o, 16);
+    top = op_max(top, __float_as_uint(float(s2)));
+    if (t == 0) nrm2[row] = float(s2);
   }
-  for (int o = 32; o >= 1; o >>= 1) {
-    s2 += __shfl_xor(s2, o, TG_WAVE);
-    q2 += __shfl_xor(q2, o, TG_WAVE);
-    e2 += __shfl_xor(e2, o, TG_WAVE);
-  }
-  const uint64_t fb = __ballot(not_bf16 != 0), fi = __ballot(not_int != 0), fn = __ballot(neg != 0),
-                 fg = __ballot(big != 0);
+  bits = wg_reduce(bits, sh, op_or);
+  top = wg_reduce(top, sh, op_max);
+  big = wg_reduce(big, sh, op_max);
   if (threadIdx.x == 0) {
-    nrm2[row] = float(s2);
-    // norms rounded up, so the bound stays an upper bound
-    nq[row] = float(sqrt(q2) * (1.0 + 1e-6));
-    ne[row] = float(sqrt(e2) * (1.0 + 1e-6));
-    if (fb) atomicOr(&flags[0], 1u);
-    if (fi) atomicOr(&flags[1], 1u);
-    if (fn) atomicOr(&flags[2], 1u);
-    atomicMax(&flags[3], __float_as_uint(float(s2)));
-    if (fg) atomicOr(&flags[4], 1u);
+    if (bits & 1u) atomicOr(&flags[0], 1u);
+    if (bits & 2u) atomicOr(&flags[1], 1u);
+    if (bits & 4u) atomicOr(&flags[2], 1u);
+    atomicMax(&flags[3], top);
+    if (bits & 8u) atomicOr(&flags[4], 1u);
+    atomicMax(&flags[5], big);
+  }
+}
+
+// 16-bit copy of the rows: BF16 bits (HALF false; every value exact), or FP16 of x * scale
+// (a power of two that puts the largest value below 2^15; results below the smallest normal
+// FP16 value become 0).  HALF: flags[6] = max over the rows of |x' / scale - x| / |x|, rounded
+// up (FP32 bits).
+template <bool HALF>
+__global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N, uint32_t D,
+                                                     float scale, uint16_t* Xb, uint32_t* flags) {
+  __shared__ uint32_t sh[4];
+  const int t = threadIdx.x & 15;
+  const double inv = 1.0 / double(scale);
+  uint32_t worst = 0;
+  for (size_t row = size_t(blockIdx.x) * 16 + (threadIdx.x >> 4); row < N;
+       row += size_t(gridDim.x) * 16) {
+    const float* x = X + row * D;
+    double s2 = 0.0, e2 = 0.0;
+    for (uint32_t j = 4 * t; j < D; j += 64) {
+      const float4 q = load4(x + j);
+      const float v[4] = {q.x, q.y, q.z, q.w};
+      uint32_t h[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (HALF) {
+          _Float16 f = _Float16(v[b] * scale);
+          if (fabsf(float(f)) < 0x1p-14f) f = _Float16(0.f);
+          h[b] = __builtin_bit_cast(uint16_t, f);
+          const double w = double(float(f)) * inv;
+          s2 += double(v[b]) * double(v[b]);
+          e2 += (w - double(v[b])) * (w - double(v[b]));
+        } else {
+          h[b] = __float_as_uint(v[b]) >> 16;
+        }
+      }
+      *reinterpret_cast<uint2*>(Xb + row * D + j) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+    }
+    if (HALF) {
+#pragma unroll
+      for (int o = 8; o >= 1; o >>= 1) {
+        s2 += __shfl_xor(s2, o, 16);
+        e2 += __shfl_xor(e2, o, 16);
+      }
+      const float r = e2 > 0.0 ? float(sqrt(e2 / s2) * (1.0 + 1e-6)) : 0.f;
+      worst = op_max(worst, __float_as_uint(r));
+    }
+  }
+  if (HALF) {
+    worst = wg_reduce(worst, sh, op_max);
+    if (threadIdx.x == 0) atomicMax(&flags[6], worst);
   }
 }
 
@@ -146,304 +211,15 @@ void launch_screen_prep8(const float* X, uint32_t N, uint32_t D, uint8_t* Xq, fl
   k_screen_prep8<<<N, TG_WAVE, 0, s>>>(X, N, D, Xq, sc, nq, ne);
 }
 
-void launch_screen_prep(const float* X, uint32_t N, uint32_t D, uint16_t* Xb, float* nrm2,
-                        float* nq, float* ne, uint32_t* flags, hipStream_t s) {
-  k_screen_prep<<<N, TG_WAVE, 0, s>>>(X, N, D, Xb, nrm2, nq, ne, flags);
+static uint32_t prep_grid(uint32_t N) { return std::min<uint32_t>((N + 15) / 16, 2048u); }
+void launch_screen_prep(const float* X, uint32_t N, uint32_t D, float* nrm2, uint32_t* flags,
+                        hipStream_t s) {
+  k_screen_prep<<<prep_grid(N), 256, 0, s>>>(X, N, D, nrm2, flags);
 }
-
-__device__ __forceinline__ float screen_bound(float na, float qa, float ea, float nb, float qb,
-                                              float eb, float eta) {
-  return 2.0f * (ea * qb + qa * eb + ea * eb) + eta * (na + nb + 2.0f * qa * qb);
-}
-
-// Products of the screen copies of the node's sample rows, staged through LDS DC elements
-// at a time: wave w gets accB[c] = A rows 16w.. x B rows 16c.. and accA[c] = A rows 16w.. x
-// A rows 16c.. (mfma layout: lane l, register r holds row 4(l/16)+r, column l%16 of the
-// 16x16 block).  Rows past nA / nB are zero.
-template <int PREC, int DC>
-__device__ __forceinline__ void screen_products(const KnnArgs& a, const uint32_t* A,
-                                                const uint32_t* B, int nA, int nB,
-                                                unsigned char* sA, unsigned char* sB,
-                                                f32x4 (&accB)[4], f32x4 (&accA)[4]) {
-  constexpr int ESZ = PREC == 3 ? 1 : (PREC == 2 ? 2 : 4);  // element bytes
-  constexpr int CPR = DC * ESZ / 16;                // 16-byte loads per staged row
-  constexpr int RS = DC * ESZ + 16;                 // padded row stride in bytes
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int D = a.D;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    accB[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    accA[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  const unsigned char* src = PREC == 3   ? reinterpret_cast<const unsigned char*>(a.Xq8)
-                             : PREC == 2 ? reinterpret_cast<const unsigned char*>(a.Xb)
-                                         : reinterpret_cast<const unsigned char*>(a.X);
-  for (int d0 = 0; d0 < D; d0 += DC) {
-    // stage rows [d0, d0+DC) of A and B: 16 B per thread-load, CPR loads per row
-    for (int e = tid; e < 2 * 64 * CPR; e += 256) {
-      const int op = e / (64 * CPR), r = (e / CPR) % 64, c16 = e % CPR;
-      const int n = op == 0 ? nA : nB;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      const int col = d0 + c16 * (16 / ESZ);
-      if (r < n && col < D) {
-        const uint32_t id = op == 0 ? A[r] : B[r];
-        v = *reinterpret_cast<const uint4*>(src + (size_t(id) * D + col) * ESZ);
-      }
-      *reinterpret_cast<uint4*>((op == 0 ? sA : sB) + r * RS + c16 * 16) = v;
-    }
-    __syncthreads();
-    if (PREC == 3) {
-#pragma unroll
-      for (int k0 = 0; k0 < DC; k0 += 32) {
-        const int kk = k0 + 8 * (l >> 4);
-        const long fa = *reinterpret_cast<const long*>(sA + (16 * w + (l & 15)) * RS + kk);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const long fb = *reinterpret_cast<const long*>(sB + (16 * c + (l & 15)) * RS + kk);
-          const long fc = *reinterpret_cast<const long*>(sA + (16 * c + (l & 15)) * RS + kk);
-          accB[c] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(fa, fb, accB[c], 0, 0, 0);
-          accA[c] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(fa, fc, accA[c], 0, 0, 0);
-        }
-      }
-    } else if (PREC == 2) {
-#pragma unroll
-      for (int k0 = 0; k0 < DC; k0 += 32) {
-        const int kk = k0 + 8 * (l >> 4);
-        const bf16x8 fa = *reinterpret_cast<const bf16x8*>(sA + (16 * w + (l & 15)) * RS + kk * 2);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bf16x8 fb = *reinterpret_cast<const bf16x8*>(sB + (16 * c + (l & 15)) * RS + kk * 2);
-          const bf16x8 fc = *reinterpret_cast<const bf16x8*>(sA + (16 * c + (l & 15)) * RS + kk * 2);
-          accB[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, accB[c], 0, 0, 0);
-          accA[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fc, accA[c], 0, 0, 0);
-        }
-      }
-    } else {
-#pragma unroll 4
-      for (int k0 = 0; k0 < DC; k0 += 4) {
-        const int kk = k0 + (l >> 4);
-        const float fa = *reinterpret_cast<const float*>(sA + (16 * w + (l & 15)) * RS + kk * 4);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float fb = *reinterpret_cast<const float*>(sB + (16 * c + (l & 15)) * RS + kk * 4);
-          const float fc = *reinterpret_cast<const float*>(sA + (16 * c + (l & 15)) * RS + kk * 4);
-          accB[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa, fb, accB[c], 0, 0, 0);
-          accA[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa, fc, accA[c], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// -------------------------------------------------------------------------------------
-// Screened local join.  PREC 1: FP32 MFMA (16x16x4), PREC 2: BF16 MFMA (16x16x32),
-// PREC 3: FP8 e4m3 MFMA (16x16x32) with per-vector scales applied to the product.
-// 256 threads: wave w owns row block w (16 rows of A) against the 4 column blocks of B and
-// of A.  Staging chunk: DC elements per row (128 BF16 or 64 FP32 = 256 B).
-// -------------------------------------------------------------------------------------
-template <int PREC, int MC, class T, int DC>
-__global__ __launch_bounds__(256) void k_localjoin_screen(KnnArgs a) {
-  // DC: elements per staged chunk (the tile's k depth per LDS round)
-  constexpr int ESZ = PREC == 3 ? 1 : (PREC == 2 ? 2 : 4);  // element bytes
-  constexpr int CPR = DC * ESZ / 16;                // 16-byte loads per staged row
-  constexpr int RS = DC * ESZ + 16;                 // padded row stride in bytes
-  constexpr int STAGE = 64 * RS;                    // one operand
-  constexpr int MROW = 65;                          // padded distance-matrix row (floats)
-  constexpr int SMEM = 2 * STAGE > 2 * 64 * MROW * 4 ? 2 * STAGE : 2 * 64 * MROW * 4;
-  static_assert(DC % (PREC >= 2 ? 32 : 4) == 0 && CPR >= 1, "tile depth");
-  // the distance matrices alias the staging area once the products are done
-  __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
-  __shared__ uint32_t A[64], B[64];
-  __shared__ float naA[64], qA[64], eA[64], wA[64];
-  __shared__ float naB[64], qB[64], eB[64], wB[64];
-  __shared__ float scA[64], scB[64];
-  unsigned char* sA = smem;
-  unsigned char* sB = smem + STAGE;
-  float* MAB = reinterpret_cast<float*>(smem);
-  float* MAA = MAB + 64 * MROW;
-
-  const uint32_t u = row_of_block(a.perm, a.N);
-  if (u >= a.N) return;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int K = a.K, D = a.D;
-  const int nA = a.na[u], nB = a.nb[u];
-  if (tid < 64) {
-    if (tid < nA) {
-      const uint32_t v = a.H[size_t(u) * HROW_S + tid];
-      A[tid] = v;
-      naA[tid] = a.nrm2[v];
-      qA[tid] = a.nq[v];
-      eA[tid] = a.ne[v];
-      wA[tid] = a.GD[size_t(v) * K + K - 1];
-      if (PREC == 3) scA[tid] = a.sc8[v];
-    }
-  } else if (tid < 128) {
-    const int j = tid - 64;
-    if (j < nB) {
-      const uint32_t v = a.H[size_t(u) * HROW_S + 64 + j];
-      B[j] = v;
-      naB[j] = a.nrm2[v];
-      qB[j] = a.nq[v];
-      eB[j] = a.ne[v];
-      wB[j] = a.GD[size_t(v) * K + K - 1];
-      if (PREC == 3) scB[j] = a.sc8[v];
-    }
-  }
-  __syncthreads();
-
-  f32x4 accB[4], accA[4];
-  screen_products<PREC, DC>(a, A, B, nA, nB, sA, sB, accB, accA);
-  // screen distances into the (aliased) matrices: C[i][j], i = 4*(l/16)+r, j = l%16
-  const float INF = __uint_as_float(0x7F800000u);
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * w + 4 * (l >> 4) + r, j = 16 * c + (l & 15);
-      float sb = INF, sa = INF;
-      float pb = accB[c][r], pa = accA[c][r];
-      if (PREC == 3) {
-        // scale back: (s_i s_j) * sum q_i q_j
-        pb *= (i < nA && j < nB) ? scA[i] * scB[j] : 0.f;
-        pa *= (i < nA && j < nA) ? scA[i] * scA[j] : 0.f;
-      }
-      if (i < nA && j < nB && A[i] != B[j]) sb = (naA[i] + naB[j]) - 2.0f * pb;
-      if (i < nA && j < nA && i != j) sa = (naA[i] + naA[j]) - 2.0f * pa;
-      MAB[i * MROW + j] = sb;
-      MAA[i * MROW + j] = sa;
-    }
-  }
-  __syncthreads();
-
-  // per (row or column, tile): the exact (d, id) minimum among the candidates whose bound
-  // interval reaches below min(worst, min upper bound); pushed when d < worst
-  // Jobs = (destination row, 16-wide candidate tile) of the three kinds (A rows x B tiles,
-  // B columns x A tiles, A rows x A tiles), processed in chunks of QJ: one thread per job
-  // computes the band mask from the screen matrix, the band candidates are queued, the 16
-  // lane groups re-score the queue four pairs at a time, and each job keeps the exact
-  // (d, id) minimum.  Candidates already in the destination's list would be dropped by the
-  // merge and are not pushed.
-  constexpr int QJ = 64;
-  __shared__ uint32_t qent[QJ * LJ_TILE];  // (job in chunk << 8) | candidate column
-  __shared__ float qdist[QJ * LJ_TILE];
-  __shared__ int qoff[QJ + 1];
-  const int gg = tid >> 4, t = tid & 15;
-  const float eta = a.eta;
-  const int tB = (nB + LJ_TILE - 1) / LJ_TILE, tA = (nA + LJ_TILE - 1) / LJ_TILE;
-  // quotients by the tile counts (1..4) as multiply-shifts: exact for numerators < 21845
-  const uint32_t mB = (65536u + uint32_t(tB) - 1) / uint32_t(max(tB, 1));
-  const uint32_t mA = (65536u + uint32_t(tA) - 1) / uint32_t(max(tA, 1));
-  auto divB = [&](int x) { return int((uint32_t(x) * mB) >> 16); };
-  auto divA = [&](int x) { return int((uint32_t(x) * mA) >> 16); };
-  const int nj0 = nA * tB, nj1 = nB * tA, njobs = nj0 + nj1 + nA * tA;
-  uint32_t n_exact = 0;
-  // the band masks of QJ jobs at a time are formed by wave 0 (exact screens take
-  // k_localjoin_exact_screen)
-  for (int base = 0; base < njobs; base += QJ) {
-    int kind = 0, r = 0, lo = 0;
-    uint32_t mask = 0;
-    const int J = base + tid;
-    if (tid < QJ && J < njobs) {
-      if (J < nj0) {
-        kind = 0; r = divB(J); lo = (J - r * tB) * LJ_TILE;
-      } else if (J < nj0 + nj1) {
-        kind = 1; r = divA(J - nj0); lo = (J - nj0 - r * tA) * LJ_TILE;
-      } else {
-        kind = 2; r = divA(J - nj0 - nj1); lo = (J - nj0 - nj1 - r * tA) * LJ_TILE;
-      }
-      const bool col = kind == 1, cb = kind == 0;
-      const int nc = cb ? nB : nA, hi = min(nc, lo + LJ_TILE);
-      const float* M = kind == 2 ? MAA : MAB;
-      const float worst = col ? wB[r] : wA[r];
-      const float nd = col ? naB[r] : naA[r], qd = col ? qB[r] : qA[r];
-      const float ed = col ? eB[r] : eA[r];
-      float sv[LJ_TILE], ev[LJ_TILE];
-      float tau = worst;
-#pragma unroll
-      for (int q = 0; q < LJ_TILE; ++q) {
-        const int j = lo + q;
-        sv[q] = INF;
-        ev[q] = 0.f;
-        if (j < hi) {
-          sv[q] = col ? M[j * MROW + r] : M[r * MROW + j];
-          if (sv[q] < INF) {
-            ev[q] = screen_bound(nd, qd, ed, cb ? naB[j] : naA[j], cb ? qB[j] : qA[j],
-                                 cb ? eB[j] : eA[j], eta);
-            tau = fminf(tau, sv[q] + ev[q]);
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < LJ_TILE; ++q)
-        if (sv[q] < INF && !(sv[q] - ev[q] > tau)) mask |= 1u << q;
-    }
-    // ---- queue offsets (wave 0 scan)
-    if (tid < QJ) {
-      const int c = __popc(mask);
-      const int incl = wave_incl_scan(c);
-      qoff[tid + 1] = incl;
-      if (tid == 0) qoff[0] = 0;
-      int pos = incl - c;
-      uint32_t m = mask;
-      while (m) {
-        const int q = __ffs(m) - 1;
-        m &= m - 1;
-        qent[pos++] = (uint32_t(tid) << 8) | uint32_t(lo + q) | (uint32_t(kind) << 6);
-      }
-    }
-    __syncthreads();
-    const int nq = qoff[QJ];
-    // ---- exact re-scores, four pairs in flight per 16-lane group
-    for (int e0 = 0; e0 < nq; e0 += 64) {
-      const T* Xr = a.Xr16 ? reinterpret_cast<const T*>(a.Xr16) : reinterpret_cast<const T*>(a.X);
-      const T* ra[4];
-      const T* rb[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int e = e0 + gg + 16 * b;
-        ra[b] = rb[b] = Xr;  // unused slots read row 0
-        if (e < nq) {
-          const uint32_t q = qent[e];
-          const int jk = (q >> 6) & 3, jc = q & 63;
-          const int J2 = base + int(q >> 8);
-          const int rr = jk == 0 ? divB(J2) : (jk == 1 ? divA(J2 - nj0) : divA(J2 - nj0 - nj1));
-          const uint32_t dest = jk == 1 ? B[rr] : A[rr];
-          const uint32_t cid = jk == 0 ? B[jc] : A[jc];
-          ra[b] = Xr + size_t(dest) * D;
-          rb[b] = Xr + size_t(cid) * D;
-        }
-      }
-      float dd[4];
-      dist16_pairs<MC, 4>(ra, rb, D, t, dd);
-      if (t == 0) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int e = e0 + gg + 16 * b;
-          if (e < nq) qdist[e] = dd[b];
-        }
-      }
-    }
-    n_exact += nq;
-    __syncthreads();
-    // ---- per job: exact minimum of the band, push
-    if (tid < QJ && mask) {
-      const uint32_t dest = kind == 1 ? B[r] : A[r];
-      const float worst = kind == 1 ? wB[r] : wA[r];
-      uint64_t best = TG_KEY_INF;
-      for (int e = qoff[tid]; e < qoff[tid + 1]; ++e) {
-        const int jc = qent[e] & 63;
-        best = min(best, mk_key(qdist[e], kind == 0 ? B[jc] : A[jc]));
-      }
-      if (key_d(best) < worst && !row_has_key(a.G, a.GD, K, dest, best)) pb_push(a.pc, dest, best);
-    }
-    __syncthreads();
-  }
-  if (a.counters && tid == 0) {
-    // [0] pair evaluations (screen), [1] exact re-scores
-    atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
-    atomicAdd(&cnt_slot(a.counters)[1], (unsigned long long)n_exact);
-  }
+void launch_screen_copy(const float* X, uint32_t N, uint32_t D, bool half, float scale,
+                        uint16_t* Xb, uint32_t* flags, hipStream_t s) {
+  if (half) k_screen_copy<true><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags);
+  else k_screen_copy<false><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags);
 }
 
 // Local join when the screen distances are the canonical distances (integer data, FP32 or
@@ -643,20 +419,31 @@ __device__ __forceinline__ void lj_lists(const KnnArgs& a, uint32_t u, const flo
 template <int PREC, int DC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_localjoin_exact_screen(KnnArgs a) {
-  constexpr int ESZ = PREC == 2 ? 2 : 4;
-  constexpr int STAGE = 64 * (DC * ESZ + 16);
   static_assert(PREC == 1 || PREC == 2, "exact screens are FP32 or BF16 products");
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * STAGE];
-  __shared__ uint32_t A[64], B[64];
+  using St = ScreenStage<PREC, DC, 128>;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[St::BYTES];
+  __shared__ uint32_t ids[128];
   __shared__ float naA[64], wA[64], naB[64], wB[64];
   const uint32_t u = row_of_block(a.perm, a.N);
   if (u >= a.N) return;
+  uint32_t *A = ids, *B = ids + 64;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, t = l & 15;
   const int nA = a.na[u], nB = a.nb[u];
   lj_lists(a, u, a.nrm2, nA, nB, A, B, naA, wA, naB, wB);
   __syncthreads();
   f32x4 accB[4], accA[4];
-  screen_products<PREC, DC>(a, A, B, nA, nB, smem, smem + STAGE, accB, accA);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) accB[c] = accA[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  screen_chunks<PREC, DC, 128>(
+      PREC == 2 ? static_cast<const void*>(a.Xb) : a.X, ids, a.D,
+      [&](int r) { return r < 64 ? r < nA : r - 64 < nB; }, smem, [&]() {
+        const unsigned char* pa = smem + 16 * w * St::RS;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          screen_block<PREC, true, DC>(pa, smem + (64 + 16 * c) * St::RS, l, accB[c]);
+          screen_block<PREC, true, DC>(pa, smem + 16 * c * St::RS, l, accA[c]);
+        }
+      });
   uint64_t row_b = TG_KEY_INF, row_a = TG_KEY_INF, col_b = TG_KEY_INF;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -665,6 +452,307 @@ void k_localjoin_exact_screen(KnnArgs a) {
           reinterpret_cast<uint64_t*>(smem));
   if (a.counters && tid == 0)
     atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
+}
+
+// -------------------------------------------------------------------------------------
+// Screened local join of real-valued data.  PREC 1: FP32 MFMA, 2: 16-bit MFMA (FP16 copy, or
+// BF16 when T = uint16_t: rows that BF16 holds exactly), 3: FP8 MFMA.  The jobs are those of
+// k_localjoin_exact_screen: a row's minimum over a 16-wide tile, for rows of A over the tiles
+// of B and of A, and of B over the tiles of A.  Every 16 x 16 block of pairs holds whole jobs
+// of its rows and of its columns (A x A is symmetric: blocks on and above the diagonal only),
+// so the valid blocks, at most 26, are dealt to the four waves whatever the list lengths.  Per
+// job tau = min(worst, smallest s + E) straight from the accumulators; a pair with s - E <= tau
+// in its row's or its column's job is queued, once.  An exact minimum below the job's worst
+// distance is always among them, and one that a job did not want cannot be its minimum, so
+// every queued pair is offered to both jobs.  The queue is worked by all 16 lane groups:
+//   * rows up to 256 elements (MC <= 4): straight from global memory, where the block's rows
+//     have just been read (L2);
+//   * wider rows: 64 elements of every queued row at a time through LDS, 16 pairs per group
+//     with their partial sums in registers -- a row is read once more, not once per pair.
+// Two iterations of 500k x 96 (K = 64, learned lists, 150 re-scores per node): 48.5 -> 17.0 ms;
+// eight of 160k x 96 clusters from random lists 46 -> 15.4 ms; two of 100k x 960 (170 re-scores
+// per node) 48 -> 15.1 ms.  Before, one BF16 product left a bound eight times wider, one of the
+// four waves formed the masks, and each re-score read both rows from L2.  What is left: half
+// of the narrow kernel's cycles issue VALU work, the rest waits on the list, row and push
+// round trips; the wide one streams each sampled row twice.
+// -------------------------------------------------------------------------------------
+template <int PREC, int MC, class T, int DC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MC <= 4 ? 6 : 3)))
+void k_localjoin_screen(KnnArgs a) {
+  using St = ScreenStage<PREC, DC, 128>;
+  constexpr bool BF = std::is_same<T, uint16_t>::value;
+  constexpr int QCAP = 1024;  // pairs queued per pass (one pass, but for degenerate data)
+  constexpr int NBLK = 7;     // blocks per wave: (16 + 10) / 4, rounded up
+  constexpr bool WIDE = MC > 4;
+  constexpr int KEYS = 3 * 256 * 8, QBYTES = QCAP * 2;
+  constexpr int WRS = 64 * int(sizeof(T)) + 16;  // staged row of the wide re-scores
+  constexpr int WORK = KEYS + QBYTES + (WIDE ? 128 * WRS : 0);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[St::BYTES > WORK ? St::BYTES : WORK];
+  __shared__ __attribute__((aligned(16))) uint32_t ids[128];
+  __shared__ __attribute__((aligned(16))) float nn[128];
+  __shared__ __attribute__((aligned(16))) float wd[128];
+  __shared__ float qn[PREC == 3 ? 128 : 1], en[PREC == 3 ? 128 : 1], sc[PREC == 3 ? 128 : 1];
+  __shared__ uint32_t wsum[4];
+  const uint32_t u = row_of_block(a.perm, a.N);
+  if (u >= a.N) return;
+  const int tid = threadIdx.x, l = tid & 63, g = l >> 4, t = l & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int D = a.D;
+  const int nA = a.na[u], nB = a.nb[u];
+  uint32_t *A = ids, *B = ids + 64;
+  lj_lists(a, u, a.nrm2, nA, nB, A, B, nn, wd, nn + 64, wd + 64);
+  if (PREC == 3 && tid < 128) {
+    const bool in = tid < 64 ? tid < nA : tid - 64 < nB;
+    const uint32_t v = in ? a.H[size_t(u) * HROW_S + tid] : 0u;
+    qn[tid] = in ? a.nq[v] : 0.f;
+    en[tid] = in ? a.ne[v] : 0.f;
+    sc[tid] = in ? a.sc8[v] : 0.f;
+  }
+  __syncthreads();
+  // ---- this wave's blocks w, w + 4, ..: bi[b] = first row (of A), bj[b] = first candidate
+  // (index into ids: B tiles from 64 on), -1: none
+  const int RA = (nA + 15) >> 4, RB = (nB + 15) >> 4;
+  int bi[NBLK], bj[NBLK];
+#pragma unroll
+  for (int b = 0; b < NBLK; ++b) {
+    int x = w + 4 * b;
+    bi[b] = bj[b] = -1;
+    if (x < RA * RB) {
+      int rb = 0;
+      while (x >= RB) {
+        x -= RB;
+        ++rb;
+      }
+      bi[b] = 16 * rb;
+      bj[b] = 64 + 16 * x;
+    } else {
+      x -= RA * RB;
+      int rb = 0;
+      while (rb < RA && x >= RA - rb) {
+        x -= RA - rb;
+        ++rb;
+      }
+      if (rb < RA) {
+        bi[b] = 16 * rb;
+        bj[b] = 16 * (rb + x);
+      }
+    }
+  }
+  f32x4 acc[NBLK];
+#pragma unroll
+  for (int b = 0; b < NBLK; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const void* src = PREC == 3   ? static_cast<const void*>(a.Xq8)
+                    : PREC == 2 ? static_cast<const void*>(a.Xb)
+                                : static_cast<const void*>(a.X);
+  screen_chunks<PREC, DC, 128>(
+      src, ids, D, [&](int r) { return r < 64 ? r < nA : r - 64 < nB; }, smem, [&]() {
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b)
+          if (bi[b] >= 0)
+            screen_block<PREC, BF, DC>(smem + bi[b] * St::RS, smem + bj[b] * St::RS, l, acc[b]);
+      });
+  // the jobs' keys and the queue, in the staging area (free from here on)
+  uint64_t* kb = reinterpret_cast<uint64_t*>(smem);  // [64 rows of A][4 tiles of B]
+  uint64_t* ka = kb + 256;                           // [64 rows of A][4 tiles of A]
+  uint64_t* kc = ka + 256;                           // [4 tiles of A][64 rows of B]
+  uint16_t* queue = reinterpret_cast<uint16_t*>(kc + 256);  // row << 7 | candidate
+  kb[tid] = TG_KEY_INF;
+  ka[tid] = TG_KEY_INF;
+  kc[tid] = TG_KEY_INF;
+  // ---- which pairs to evaluate: bit 4b + r, element r of block b
+  const float INF = __uint_as_float(0x7F800000u);
+  const float kap = a.kap, ps = a.pscale;
+  uint32_t want = 0;
+#pragma unroll
+  for (int b = 0; b < NBLK; ++b) {
+    if (bi[b] < 0) continue;
+    const int i0 = bi[b] + 4 * g, jj = bj[b] + t;
+    const bool bt = bj[b] >= 64;
+    const bool jn = bt ? jj - 64 < nB : jj < nA;
+    const float4 ni = *reinterpret_cast<const float4*>(nn + i0);
+    const float4 wi = *reinterpret_cast<const float4*>(wd + i0);
+    const uint4 idi = *reinterpret_cast<const uint4*>(ids + i0);
+    const float nv[4] = {ni.x, ni.y, ni.z, ni.w}, wv[4] = {wi.x, wi.y, wi.z, wi.w};
+    const uint32_t iv[4] = {idi.x, idi.y, idi.z, idi.w};
+    const float nj = nn[jj], wj = wd[jj];
+    const uint32_t idj = ids[jj];
+    float lo[4];
+    uint32_t hi[4];
+    bool ok[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      ok[r] = i0 + r < nA && jn && (bt ? iv[r] != idj : i0 + r != jj);
+      const float nsum = nv[r] + nj;
+      float h;
+      if constexpr (PREC == 3) {
+        const int i = i0 + r;
+        const float s = nsum - 2.0f * ((sc[i] * sc[jj]) * acc[b][r]);
+        const float E = 2.0f * (en[i] * qn[jj] + qn[i] * en[jj] + en[i] * en[jj]) +
+                        a.eta * (nsum + 2.0f * qn[i] * qn[jj]);
+        lo[r] = s - E;
+        h = s + E;
+      } else {
+        const float s = __builtin_fmaf(-ps, acc[b][r], nsum);
+        lo[r] = __builtin_fmaf(-kap, nsum, s);
+        h = __builtin_fmaf(kap, nsum, s);
+      }
+      // non-negative bits order as unsigned integers; +inf where there is no bound
+      hi[r] = (ok[r] && h < INF) ? __float_as_uint(fmaxf(h, 0.f)) : 0x7F800000u;
+    }
+    uint32_t mc = min(min(hi[0], hi[1]), min(hi[2], hi[3]));
+    mc = min(mc, lane_xor32(mc, 16));
+    mc = min(mc, lane_xor32(mc, 32));
+    const float tc = fminf(wj, __uint_as_float(mc));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float tau = fmaxf(fminf(wv[r], __uint_as_float(row_min16(hi[r]))), tc);
+      // on the diagonal a pair appears twice: queued above it
+      if (ok[r] && !(lo[r] > tau) && (bi[b] != bj[b] || i0 + r < jj)) want |= 1u << (4 * b + r);
+    }
+  }
+  // ---- queue positions
+  const int own = __popc(want);
+  const int incl = wave_incl_scan(own);
+  if (l == 63) wsum[w] = uint32_t(incl);
+  __syncthreads();
+  int first = incl - own, total = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (q < w) first += int(wsum[q]);
+    total += int(wsum[q]);
+  }
+  const T* X = reinterpret_cast<const T*>(BF ? static_cast<const void*>(a.Xr16)
+                                             : static_cast<const void*>(a.X));
+  // offers pair (i, x)'s distance to its two jobs
+  auto offer = [&](uint32_t e, float d) {
+    const int i = int(e >> 7), x = int(e & 127u);
+    auto put = [](uint64_t* k, uint64_t v) {
+      atomicMin(reinterpret_cast<unsigned long long*>(k), (unsigned long long)v);
+    };
+    const uint64_t ki = mk_key(d, ids[x]), kx = mk_key(d, ids[i]);
+    if (x >= 64) {
+      put(&kb[4 * i + ((x - 64) >> 4)], ki);
+      put(&kc[64 * (i >> 4) + (x - 64)], kx);
+    } else {
+      put(&ka[4 * i + (x >> 4)], ki);
+      put(&ka[4 * x + (i >> 4)], kx);
+    }
+  };
+  for (int q0 = 0; q0 < total; q0 += QCAP) {
+    const int n = min(total - q0, QCAP);
+    uint32_t m = want;
+    int pos = first - q0;
+    while (m) {
+      const int p = __ffs(m) - 1;
+      m &= m - 1;
+      if (pos >= 0 && pos < QCAP) {
+        // block of element p: its first row and candidate
+        int x = w + (p >> 2) * 4, fi, fj;
+        if (x < RA * RB) {
+          fi = 0;
+          while (x >= RB) {
+            x -= RB;
+            ++fi;
+          }
+          fj = 64 + 16 * x;
+        } else {
+          x -= RA * RB;
+          fi = 0;
+          while (x >= RA - fi) {
+            x -= RA - fi;
+            ++fi;
+          }
+          fj = 16 * (fi + x);
+        }
+        queue[pos] = uint16_t((16 * fi + 4 * g + (p & 3)) << 7 | (fj + t));
+      }
+      ++pos;
+    }
+    __syncthreads();
+    const int gg = tid >> 4;
+    if constexpr (!WIDE) {
+      constexpr int NB = 2;  // pairs in flight per group: more would cost waves per SIMD
+      for (int e0 = 0; e0 < n; e0 += 16 * NB) {
+        uint32_t ent[NB];
+        const T *ra[NB], *rb[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int e = e0 + gg + 16 * b;
+          ent[b] = queue[e < n ? e : 0];
+          ra[b] = X + size_t(ids[ent[b] >> 7]) * D;
+          rb[b] = X + size_t(ids[ent[b] & 127u]) * D;
+        }
+        float dd[NB];
+        dist16_pairs<MC, NB>(ra, rb, D, t, dd);
+        // the group's lane b takes pair b (the distances are in lane 0)
+        const float d1 = row_shr<1>(dd[1]);
+        if (t < NB && e0 + gg + 16 * t < n) offer(t == 0 ? ent[0] : ent[1], t == 0 ? dd[0] : d1);
+      }
+    } else {
+      // 64 elements of every row at a time; pass p0 holds pairs p0 + gg + 16 k in group gg
+      constexpr int PK = 16;
+      constexpr int PPR = 64 * int(sizeof(T)) / 16, NP = 128 * PPR / 256;
+      unsigned char* stage = smem + KEYS + QBYTES;
+      for (int p0 = 0; p0 < n; p0 += 16 * PK) {
+        uint32_t ent[PK];
+        float p[PK][4];
+#pragma unroll
+        for (int k = 0; k < PK; ++k) {
+          const int e = p0 + gg + 16 * k;
+          ent[k] = queue[e < n ? e : p0];
+          p[k][0] = p[k][1] = p[k][2] = p[k][3] = 0.f;
+        }
+        const int nk = (min(n - p0, 16 * PK) + 15) >> 4;  // pairs per group in this pass
+        uint4 v[NP];
+        auto load = [&](int d0) {
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            const int e = tid + 256 * q, r = e / PPR, col = d0 + (e % PPR) * (16 / int(sizeof(T)));
+            v[q] = make_uint4(0u, 0u, 0u, 0u);
+            if ((r < 64 ? r < nA : r - 64 < nB) && col < D)
+              v[q] = *reinterpret_cast<const uint4*>(X + size_t(ids[r]) * D + col);
+          }
+        };
+        load(0);
+        for (int d0 = 0; d0 < D; d0 += 64) {
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            const int e = tid + 256 * q;
+            *reinterpret_cast<uint4*>(stage + (e / PPR) * WRS + (e % PPR) * 16) = v[q];
+          }
+          __syncthreads();
+          if (d0 + 64 < D) load(d0 + 64);
+          const bool in = d0 + 4 * t < D;
+#pragma unroll
+          for (int k = 0; k < PK; ++k) {
+            if (k < nk) {
+              const T* xa = reinterpret_cast<const T*>(stage + (ent[k] >> 7) * WRS) + 4 * t;
+              const T* xb = reinterpret_cast<const T*>(stage + (ent[k] & 127u) * WRS) + 4 * t;
+              const float4 xv = load4(xa), yv = load4(xb);
+              if (in) fold4(xv, yv, p[k]);
+            }
+          }
+          __syncthreads();
+        }
+#pragma unroll
+        for (int k = 0; k < PK; ++k) {
+          if (k < nk) {
+            const float d = tree16(p[k][0], p[k][1], p[k][2], p[k][3]);
+            if (t == 0 && p0 + gg + 16 * k < n) offer(ent[k], d);
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const int ir = 16 * w + 4 * g + (t & 3), tile = t >> 2;  // this lane's row jobs (lj_push)
+  const uint64_t row_b = kb[4 * ir + tile], row_a = ka[4 * ir + tile], col_b = kc[64 * w + l];
+  lj_push(a, A, B, wd, wd + 64, nA, nB, w, g, t, l, row_b, row_a, col_b, kc);
+  if (a.counters && tid == 0) {
+    // [0] pair evaluations (screen), [1] exact re-scores
+    atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
+    atomicAdd(&cnt_slot(a.counters)[1], (unsigned long long)total);
+  }
 }
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -739,9 +827,10 @@ __global__ __launch_bounds__(256) void k_localjoin_u8_screen(KnnArgs a) {
     atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
 }
 
-// tile 0: 256-byte staged rows (256 FP8 / 128 BF16 / 64 FP32 elements per round); tile 1:
-// 64-byte rows (64 / 32 / 16 elements per round): less zero padding at D not a multiple of
-// the depth, more LDS rounds
+// Staged bytes per row and round, tile 0 / 1: rows up to 256 elements 64 / 128 (little LDS and
+// few registers, so eight waves per SIMD, and D = 96 is whole rounds: 500k x 96, two
+// iterations, 17.0 / 17.9 ms), wider rows 128 / 64 (half the rounds and barriers; their
+// re-scores hold the LDS anyway: 100k x 960 15.1 / 18.9 ms; 256 bytes per round 17.0 ms).
 void launch_knn_localjoin_screen(const KnnArgs& a, int precision, int tile, hipStream_t s) {
   if (a.exact_screen && precision == KP_BF16 && a.X8 && a.n2s && a.D <= 256) {
     // u8 data: the BF16 screen's products on int8 MFMA (exact either way)
@@ -765,10 +854,11 @@ void launch_knn_localjoin_screen(const KnnArgs& a, int precision, int tile, hipS
   const int mc = (int(a.D) + 63) / 64;
 #define LJS(P, M, T, DC) \
   k_localjoin_screen<P, M, T, DC><<<grid_rows(a.perm, a.N), 256, 0, s>>>(a)
-#define LJS_DC(P, M, T)                                                    \
-  do {                                                                     \
-    if (tile == 1) LJS(P, M, T, (P == 3 ? 64 : P == 2 ? 32 : 16));        \
-    else LJS(P, M, T, (P == 3 ? 256 : P == 2 ? 128 : 64));                 \
+#define LJS_DC(P, M, T)                                                      \
+  do {                                                                       \
+    constexpr int near_ = (P == 3 ? 64 : P == 2 ? 32 : 16);                  \
+    if ((tile == 1) == (M > 4)) LJS(P, M, T, near_);                         \
+    else LJS(P, M, T, 2 * near_);                                            \
   } while (0)
 #define LJS_MC(P, T)                                                       \
   do {                                                                     \

@@ -4,7 +4,7 @@
 // the earlier neighbours r < j with d(G[u][r], G[u][j]) < D[u][j].  That is K(K-1)/2
 // canonical distances per node (2,016 at K=64), which at dimension 960 makes the plain kernel
 // read each pair's two rows: ~15 MB per node.  Here the K rows are staged through LDS once,
-// their Gram matrix runs on MFMA (BF16 16x16x32, or FP8 e4m3 16x16x32 with per-vector scales),
+// their Gram matrix runs on MFMA (16-bit 16x16x32, or FP8 e4m3 16x16x32 with per-vector scales),
 // and each screen distance s comes with the rigorous bound E of the local join's screen:
 //   s + E <  D[u][j]  -> occludes (d <= s + E);
 //   s - E >= D[u][j]  -> does not (d >= s - E);
@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "screen.hpp"
 
 namespace tg {
 
@@ -23,16 +24,19 @@ __device__ __forceinline__ float dpg_bound(float na, float qa, float ea, float n
   return 2.0f * (ea * qb + qa * eb + ea * eb) + eta * (na + nb + 2.0f * qa * qb);
 }
 
-// PREC 2: BF16 rows (a.Xb), PREC 3: FP8 rows (a.Xq8, scales a.sc8).  256 threads; wave w
-// owns rows 16w..16w+15 of the 64 x 64 Gram, against the 4 column blocks.
+// PREC 2: 16-bit rows (q.Xb; BF16 when T = uint16_t, else scaled FP16), PREC 3: FP8 rows
+// (q.Xq8, scales q.sc8).  256 threads; wave w owns rows 16w..16w+15 of the 64 x 64 Gram,
+// against the column blocks at or after its own (pairs r < j only).
+// 100k x 960, K = 64: 15.5 -> 5.5 ms (the FP16 copy leaves 55 of the 2,016 pairs undecided;
+// one BF16 product with its eight times wider bound left several times as many, and each reads
+// two 3.8 KB rows).
 template <int PREC, int MC, class T>
 __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
   constexpr int DC = PREC == 3 ? 256 : 128;  // elements staged per round (256 bytes per row)
-  constexpr int ESZ = PREC == 3 ? 1 : 2;
-  constexpr int CPR = DC * ESZ / 16;
-  constexpr int RS = DC * ESZ + 16;
+  constexpr bool BF = std::is_same<T, uint16_t>::value;
+  using St = ScreenStage<PREC, DC, 64>;
   constexpr int MROW = 65;
-  constexpr int SMEM = 64 * RS > 64 * MROW * 4 ? 64 * RS : 64 * MROW * 4;
+  constexpr int SMEM = St::BYTES > 64 * MROW * 4 ? St::BYTES : 64 * MROW * 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
   __shared__ uint32_t nei[64], det[64];
   __shared__ float nn[64], nq[64], ne[64], sc[64], thr[64];
@@ -51,9 +55,11 @@ __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
       const uint32_t v = a.G[size_t(u) * K + tid];
       nei[tid] = v;
       nn[tid] = q.nrm2[v];
-      nq[tid] = q.nq[v];
-      ne[tid] = q.ne[v];
-      sc[tid] = PREC == 3 ? q.sc8[v] : 1.f;
+      if (PREC == 3) {
+        nq[tid] = q.nq[v];
+        ne[tid] = q.ne[v];
+        sc[tid] = q.sc8[v];
+      }
       thr[tid] = a.GD[size_t(u) * K + tid];
     }
   }
@@ -62,39 +68,14 @@ __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
   f32x4 acc[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const unsigned char* src = PREC == 3 ? reinterpret_cast<const unsigned char*>(q.Xq8)
-                                       : reinterpret_cast<const unsigned char*>(q.Xb);
-  for (int d0 = 0; d0 < D; d0 += DC) {
-    for (int e = tid; e < 64 * CPR; e += 256) {
-      const int r = e / CPR, c16 = e % CPR;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      const int col = d0 + c16 * (16 / ESZ);
-      if (r < K && col < D)
-        v = *reinterpret_cast<const uint4*>(src + (size_t(nei[r]) * D + col) * ESZ);
-      *reinterpret_cast<uint4*>(smem + r * RS + c16 * 16) = v;
-    }
-    __syncthreads();
+  screen_chunks<PREC, DC, 64>(
+      PREC == 3 ? static_cast<const void*>(q.Xq8) : static_cast<const void*>(q.Xb), nei, D,
+      [&](int r) { return r < K; }, smem, [&]() {
 #pragma unroll
-    for (int k0 = 0; k0 < DC; k0 += 32) {
-      const int kk = k0 + 8 * (l >> 4);
-      if (PREC == 3) {
-        const long fa = *reinterpret_cast<const long*>(smem + (16 * w + (l & 15)) * RS + kk);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const long fc = *reinterpret_cast<const long*>(smem + (16 * c + (l & 15)) * RS + kk);
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(fa, fc, acc[c], 0, 0, 0);
-        }
-      } else {
-        const bf16x8 fa = *reinterpret_cast<const bf16x8*>(smem + (16 * w + (l & 15)) * RS + kk * 2);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bf16x8 fc = *reinterpret_cast<const bf16x8*>(smem + (16 * c + (l & 15)) * RS + kk * 2);
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fc, acc[c], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-  }
+        for (int c = 0; c < 4; ++c)
+          if (c >= w)
+            screen_block<PREC, BF, DC>(smem + 16 * w * St::RS, smem + 16 * c * St::RS, l, acc[c]);
+      });
   // screen distances (the matrix aliases the staging area, free after the last round)
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -102,8 +83,10 @@ __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * w + 4 * (l >> 4) + r, j = 16 * c + (l & 15);
       float s = 0.f;
-      if (i < K && j < K) s = (nn[i] + nn[j]) - 2.0f * ((sc[i] * sc[j]) * acc[c][r]);
-      M[i * MROW + j] = s;
+      if (i < K && j < K)
+        s = PREC == 3 ? (nn[i] + nn[j]) - 2.0f * ((sc[i] * sc[j]) * acc[c][r])
+                      : __builtin_fmaf(-q.pscale, acc[c][r], nn[i] + nn[j]);
+      M[i * MROW + j] = s;  // used where i < j
     }
   }
   __syncthreads();
@@ -116,7 +99,8 @@ __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
     while ((j + 1) * j / 2 <= p) ++j;
     const int r = p - j * (j - 1) / 2;
     const float s = M[r * MROW + j];
-    const float E = dpg_bound(nn[r], nq[r], ne[r], nn[j], nq[j], ne[j], q.eta);
+    const float E = PREC == 3 ? dpg_bound(nn[r], nq[r], ne[r], nn[j], nq[j], ne[j], q.eta)
+                              : q.kap * (nn[r] + nn[j]);
     const float tau = thr[j];
     if (s + E < tau) {
       atomicAdd(&det[j], 1u);

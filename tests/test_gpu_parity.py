@@ -438,3 +438,38 @@ def test_cagra_lookup_edges(K, FD):
     X = gmm_int(1500, 32, 6, K)
     G, GD = oracle.knn_bruteforce(X, K)
     _compare(X, G, GD, 2, 0, 2, FD, 64, 0.0)
+
+
+def _screen_data(name, N, D, seed):
+    rng = np.random.default_rng(seed)
+    C = rng.standard_normal((6, D))
+    X = C[rng.integers(0, 6, N)] + 0.5 * rng.standard_normal((N, D))
+    if name == "offset":      # |x|^2 far above the distances: the screens decide little, and a
+        X = X + 300.0         # node's queue of re-scores takes several passes
+    elif name == "scales":    # rows far below the largest value: no 16-bit copy, FP32 screen
+        X = X * np.where(np.arange(N) % 2, 1.0, 1e-7)[:, None]
+    elif name == "twins":     # zero distances and equal ids' neighbours
+        X[1::2] = X[::2][: X[1::2].shape[0]]
+    return X.astype(np.float32)
+
+
+@pytest.mark.parametrize("name", ["plain", "offset", "scales", "twins"])
+@pytest.mark.parametrize("D,K", [(8, 5), (36, 24), (96, 33), (136, 20), (256, 40), (264, 24),
+                                 (968, 32)])
+def test_screened_join_edges(name, D, K):
+    """The screened local join, phase 2 and DPG's Gram on real-valued rows: dimensions at and
+    around the chunk and register limits, list lengths that leave partial and empty tiles,
+    both staging depths.  Graphs equal to the oracle bit for bit."""
+    X = _screen_data(name, 900, D, D + K)
+    Gr, GDr, ev = oracle.gnn_descent(X, K, 4, 77)
+    for prec in (["fp32", "bf16"] if D % 8 == 0 else ["fp32"]):
+        for tile in (0, 1):
+            _say(f"screened join {name} D={D} K={K} {prec} tile {tile}")
+            with State(*X.shape) as s:
+                s.set_data(X)
+                s.knn_build(K, 4, 77, prec, tile=tile)
+                G, GD = s.get_knn()
+                assert s.stats()["knn_evals"] == ev
+            assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
+    if D % 8 == 0 and K >= 24:
+        _compare(X, Gr, GDr, 3, 0, 2, 16, 64, 0.0, "bf16")
