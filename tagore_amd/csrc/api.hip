@@ -1415,6 +1415,13 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
     a.rows_bf16 = 1;
   }
   a.rows8 = s->cert_u8 ? s->X8 : nullptr;
+  if (s->copy16 && s->D % 8 == 0) {
+    a.Xb = s->Xb;
+    a.nrm2 = s->nrm2;
+    a.kap = s->kap16;
+    a.pscale = s->pscale16;
+    a.h_bf16 = s->cert_bf16 ? 1 : 0;
+  }
   // DPG's pair distances on an MFMA Gram (K <= 64) with exact re-scores near the threshold
   const bool dpg_screen = p->kind == TG_KIND_DPG && K <= 64 &&
                           ((p->precision == TG_PREC_BF16 && s->D % 8 == 0 && s->copy16) ||

@@ -59,7 +59,7 @@ __device__ __forceinline__ unsigned long long* cnt_slot(unsigned long long* c) {
 template <int MC>
 struct Row16 {
   float4 v[MC];  // FP32 rows: elements m*64 + 4t .. +3; u8 rows: 16 bytes (quad layout below)
-  int n2;        // u8 rows only: |x|^2 of the row, exact, in every lane
+  int n2;        // u8 rows only: |x - 128|^2 of the row, exact, in every lane
 };
 
 // Four consecutive elements as FP32: rows are stored as FP32, or as BF16 bits when every
@@ -120,8 +120,10 @@ __device__ __forceinline__ float4 load4(const uint16_t* p) {
                      __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xFFFF0000u));
 }
 
-// u8 rows use a quad layout: the four lanes j = lane & 3 of every 4-lane quad share one row,
-// lane j holding bytes m*64 + 16j .. +15 of each 64-byte chunk m (zero past D).  A row is
+// u8 rows (integers in [0, 255]) are stored as the signed bytes x - 128, which int8 MFMA takes
+// as they are; distances do not change.  They use a quad layout: the four lanes j = lane & 3 of
+// every 4-lane quad share one row, lane j holding bytes m*64 + 16j .. +15 of each 64-byte
+// chunk m (zero past D).  A row is
 // then two 16-byte loads per lane at D = 128, and a dot product ends with two DPP steps
 // inside the quad.  All of it is integer arithmetic, so the lane layout does not change a
 // result.
@@ -140,12 +142,12 @@ __device__ __forceinline__ uint4 as_u4(const float4& v) {
   return make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z),
                     __float_as_uint(v.w));
 }
-// acc + the dot product of 16 bytes pairs (v_dot4_u32_u8)
-__device__ __forceinline__ uint32_t dot16_u8(const uint4& a, const uint4& b, uint32_t acc) {
-  acc = __builtin_amdgcn_udot4(a.x, b.x, acc, false);
-  acc = __builtin_amdgcn_udot4(a.y, b.y, acc, false);
-  acc = __builtin_amdgcn_udot4(a.z, b.z, acc, false);
-  return __builtin_amdgcn_udot4(a.w, b.w, acc, false);
+// acc + the dot product of 16 signed byte pairs (v_dot4_i32_i8)
+__device__ __forceinline__ int dot16_u8(const uint4& a, const uint4& b, int acc) {
+  acc = __builtin_amdgcn_sdot4(int(a.x), int(b.x), acc, false);
+  acc = __builtin_amdgcn_sdot4(int(a.y), int(b.y), acc, false);
+  acc = __builtin_amdgcn_sdot4(int(a.z), int(b.z), acc, false);
+  return __builtin_amdgcn_sdot4(int(a.w), int(b.w), acc, false);
 }
 // Sum of an integer over the 4 lanes of a quad, in every lane of it.
 __device__ __forceinline__ int quad_sum(int q) {
@@ -153,37 +155,21 @@ __device__ __forceinline__ int quad_sum(int q) {
   return q + __builtin_amdgcn_mov_dpp(q, 0x4E, 0xF, 0xF, false);  // lane ^ 2
 }
 
-// u8 rows, quad layout: v[m] holds the lane's 16 bytes of chunk m as bits.  The loads are
-// issued by row16_u8_load and |x|^2 (n2, in every lane) formed by row16_u8_norm, so that
-// other work can run while the loads are in flight.
-template <int MC>
-__device__ __forceinline__ void row16_u8_load(Row16<MC>& r, const uint8_t* __restrict__ x, int D) {
-  const int j = threadIdx.x & 3;
-#pragma unroll
-  for (int m = 0; m < MC; ++m) {
-    const uint4 w = m * 64 < D ? load_u8x16(x, m, D, j) : make_uint4(0u, 0u, 0u, 0u);
-    r.v[m] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
-                         __uint_as_float(w.w));
-  }
-}
-template <int MC>
-__device__ __forceinline__ void row16_u8_norm(Row16<MC>& r) {
-  uint32_t sq = 0;
-#pragma unroll
-  for (int m = 0; m < MC; ++m) {
-    const uint4 w = make_uint4(__float_as_uint(r.v[m].x), __float_as_uint(r.v[m].y),
-                               __float_as_uint(r.v[m].z), __float_as_uint(r.v[m].w));
-    sq = dot16_u8(w, w, sq);
-  }
-  r.n2 = quad_sum(int(sq));
-}
-
 template <int MC, class T>
 __device__ __forceinline__ void load_row16(Row16<MC>& r, const T* __restrict__ x, int D, int t) {
   if constexpr (std::is_same<T, uint8_t>::value) {
-    // u8 rows, quad layout (t is not used: the layout follows lane & 3)
-    row16_u8_load<MC>(r, x, D);
-    row16_u8_norm<MC>(r);
+    // u8 rows, quad layout (t is not used: the layout follows lane & 3): v[m] holds the lane's
+    // 16 bytes of chunk m as bits, n2 = |x|^2 of the signed bytes in every lane
+    const int j = threadIdx.x & 3;
+    int sq = 0;
+#pragma unroll
+    for (int m = 0; m < MC; ++m) {
+      const uint4 w = m * 64 < D ? load_u8x16(x, m, D, j) : make_uint4(0u, 0u, 0u, 0u);
+      r.v[m] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z),
+                           __uint_as_float(w.w));
+      sq = dot16_u8(w, w, sq);
+    }
+    r.n2 = quad_sum(sq);
   } else {
 #pragma unroll
     for (int m = 0; m < MC; ++m) {
@@ -288,20 +274,6 @@ __device__ __forceinline__ void dist16_batch(const Row16<MC>& a, const T* const 
   }
 #pragma unroll
   for (int k = 0; k < NB; ++k) out[k] = tree16(p[k][0], p[k][1], p[k][2], p[k][3]);
-}
-
-// Distance between two u8 rows held in registers (quad layout), in every lane: the integer
-// |a|^2 + |b|^2 - 2 a.b with v_dot4_u32_u8, exact.  The u8 rows are used only when every
-// value of the data set is an integer in [0, 255] and every squared distance is below 2^24:
-// then every partial sum of the canonical FP32 fold is an exact integer too, so both give
-// the same float.
-template <int MC>
-__device__ __forceinline__ float dist_rows_u8(const Row16<MC>& a, const Row16<MC>& b, int D) {
-  uint32_t ab = 0;
-#pragma unroll
-  for (int m = 0; m < MC; ++m)
-    if (m * 64 < D) ab = dot16_u8(as_u4(a.v[m]), as_u4(b.v[m]), ab);
-  return float(a.n2 + b.n2 - 2 * quad_sum(int(ab)));
 }
 
 // NB distances between the row pairs (a[k], b[k]), both read from memory; every pointer
@@ -832,65 +804,21 @@ __device__ __forceinline__ void load_quad_u8(uint4 (&y)[MC], const uint8_t* r, i
 #pragma unroll
   for (int m = 0; m < MC; ++m) y[m] = m * 64 < D ? load_u8x16(r, m, D, j) : make_uint4(0u, 0u, 0u, 0u);
 }
-// |a - y|^2 for the register row a and the loaded row y (quad layout), in every quad lane.
+// |a - y|^2 for the register row a and the loaded row y (quad layout), in every quad lane: the
+// integer |a|^2 + |y|^2 - 2 a.y with v_dot4, exact.  The u8 rows are used only when every value
+// of the data set is an integer in [0, 255] and every squared distance is below 2^24: then
+// every partial sum of the canonical FP32 fold is an exact integer too, so both give the same
+// float.
 template <int MC>
 __device__ __forceinline__ float quad_dist_u8(const Row16<MC>& a, const uint4 (&y)[MC], int D) {
-  uint32_t ab = 0, bb = 0;
+  int ab = 0, bb = 0;
 #pragma unroll
   for (int m = 0; m < MC; ++m) {
     if (m * 64 >= D) break;
     ab = dot16_u8(as_u4(a.v[m]), y[m], ab);
     bb = dot16_u8(y[m], y[m], bb);
   }
-  return float(a.n2 + quad_sum(int(bb) - 2 * int(ab)));
-}
-
-// d(ta, y) and d(tb, y) for the loaded row y (quad layout), in every quad lane.
-template <int MC>
-__device__ __forceinline__ void quad_dist2_u8(const Row16<MC>& ta, const Row16<MC>& tb,
-                                              const uint4 (&y)[MC], int D, float& da, float& db) {
-  uint32_t aa = 0, ab = 0, bb = 0;
-#pragma unroll
-  for (int m = 0; m < MC; ++m) {
-    if (m * 64 >= D) break;
-    aa = dot16_u8(as_u4(ta.v[m]), y[m], aa);
-    ab = dot16_u8(as_u4(tb.v[m]), y[m], ab);
-    bb = dot16_u8(y[m], y[m], bb);
-  }
-  da = float(ta.n2 + quad_sum(int(bb) - 2 * int(aa)));
-  db = float(tb.n2 + quad_sum(int(bb) - 2 * int(ab)));
-}
-
-// Two u8 targets at once: each candidate row is read once and gives d(ta, c) and d(tb, c).
-// One candidate per quad, 32 per step while more than 16 remain, then 16 (as eval_batch);
-// emit(q, da, db) runs in lanes 0..31 (0..15) for the items q0 + lane.
-template <int MC, class IdOf, class Emit>
-__device__ __forceinline__ void eval_batch2_u8(const uint8_t* X, int D, const Row16<MC>& ta,
-                                               const Row16<MC>& tb, int n, IdOf id_of,
-                                               Emit emit) {
-  const int lane = threadIdx.x, c = lane >> 2, src = (lane & 15) * 4;
-  int q0 = 0;
-  for (; q0 + 16 < n; q0 += 32) {
-    const int qb = q0 + 16 + c;
-    uint4 ya[MC], yb[MC];
-    load_quad_u8<MC>(ya, X + size_t(id_of(q0 + c)) * D, D);  // q0 + c < q0 + 16 < n
-    load_quad_u8<MC>(yb, qb < n ? X + size_t(id_of(qb)) * D : X, D);
-    float da0, db0, da1, db1;
-    quad_dist2_u8<MC>(ta, tb, ya, D, da0, db0);
-    quad_dist2_u8<MC>(ta, tb, yb, D, da1, db1);
-    const float xa0 = __shfl(da0, src, TG_WAVE), xb0 = __shfl(db0, src, TG_WAVE);
-    const float xa1 = __shfl(da1, src, TG_WAVE), xb1 = __shfl(db1, src, TG_WAVE);
-    if (lane < 32 && q0 + lane < n) emit(q0 + lane, lane < 16 ? xa0 : xa1, lane < 16 ? xb0 : xb1);
-  }
-  if (q0 < n) {
-    const int q = q0 + c;
-    uint4 y[MC];
-    load_quad_u8<MC>(y, q < n ? X + size_t(id_of(q)) * D : X, D);  // unused quads read row 0
-    float da, db;
-    quad_dist2_u8<MC>(ta, tb, y, D, da, db);
-    const float va = __shfl(da, src, TG_WAVE), vb = __shfl(db, src, TG_WAVE);
-    if (lane < 16 && q0 + lane < n) emit(q0 + lane, va, vb);
-  }
+  return float(a.n2 + quad_sum(bb - 2 * ab));
 }
 
 // Evaluates the targets id_of(0..n) against the register row `tgt`, emit(q, d) once per item.

@@ -39,8 +39,15 @@ struct PruneArgs {
   const void* rows;
   int rows_bf16;
   // u8 copy of X (or null) when every value is an integer in [0, 255] and every squared
-  // distance is below 2^24: the forward and reverse passes then take exact dot4 distances
+  // distance is below 2^24 (signed bytes x - 128): the forward and reverse passes then take
+  // exact dot4 and int8 MFMA distances
   const uint8_t* rows8;
+  // 16-bit copy (or null), its norms, bound and format, as in KnnArgs: the filter's screen of
+  // real-valued rows
+  const uint16_t* Xb;
+  const float* nrm2;
+  float kap, pscale;
+  int h_bf16;            // the copy is BF16 (every value exact), else scaled FP16
   // segments: rows [seg_lo[c], seg_lo[c+1]) form independent data sets (null: one segment)
   const uint32_t* seg_of;  // [N] segment of each row
   const uint32_t* seg_lo;  // [nseg + 1]
@@ -111,7 +118,7 @@ struct KnnArgs {
   int exact_screen;
   // rows used for canonical re-scores: BF16 copy when the data set is BF16-exact, else X
   const uint16_t* Xr16;
-  const uint8_t* X8;     // u8 copy of X (every value an integer in [0, 255], D <= 256) or null
+  const uint8_t* X8;     // u8 copy of X (integers in [0, 255] as x - 128, D <= 256) or null
   const float* n2s;      // [N] |x - 128|^2 of the u8 rows (exact), with X8
   // FP8 e4m3 copy with a per-vector scale
   const uint8_t* Xq8;
@@ -127,7 +134,7 @@ struct KnnArgs {
 // FP8 copy: q = e4m3(x / s), s = max|x| / 440, with |s q| and |x - s q| (rounded up)
 void launch_screen_prep8(const float* X, uint32_t N, uint32_t D, uint8_t* Xq, float* sc,
                          float* nq, float* ne, hipStream_t s);
-// u8 copy of the n values of X (n % 4 == 0; every value an integer in [0, 255])
+// u8 copy of the n values of X as x - 128 (n % 4 == 0; every value an integer in [0, 255])
 void launch_make_u8(const float* X, size_t n, uint8_t* X8, hipStream_t s);
 // |x - 128|^2 of every u8 row (the norms of the rows shifted into int8)
 void launch_u8_shift_norms(const uint8_t* X8, uint32_t N, uint32_t D, float* n2s, hipStream_t s);

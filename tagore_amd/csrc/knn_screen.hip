@@ -131,12 +131,14 @@ __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N,
   }
 }
 
-// u8 copy of X, four values per thread (every value an integer in [0, 255], D % 4 == 0)
+// u8 copy of X as signed bytes x - 128 (the byte XOR 0x80), four values per thread (every value
+// an integer in [0, 255], D % 4 == 0)
 __global__ void k_make_u8(const float4* X, size_t n4, uint32_t* X8) {
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n4;
        i += size_t(gridDim.x) * blockDim.x) {
     const float4 v = X[i];
-    X8[i] = uint32_t(v.x) | uint32_t(v.y) << 8 | uint32_t(v.z) << 16 | uint32_t(v.w) << 24;
+    X8[i] = (uint32_t(v.x) | uint32_t(v.y) << 8 | uint32_t(v.z) << 16 | uint32_t(v.w) << 24) ^
+            0x80808080u;
   }
 }
 
@@ -155,7 +157,7 @@ __global__ void k_u8_shift_norms(const uint8_t* X8, uint32_t N, uint32_t D, floa
   const uint8_t* x = X8 + size_t(row) * D;
   int acc = 0;
   for (uint32_t j = threadIdx.x; j < D; j += TG_WAVE) {
-    const int v = int(x[j]) - 128;
+    const int v = int(int8_t(x[j]));
     acc += v * v;
   }
 #pragma unroll
@@ -758,7 +760,7 @@ void k_localjoin_screen(KnnArgs a) {
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Exact screen on int8 MFMA for u8 data (every value an integer in [0, 255], D <= DC <= 256):
-// rows are staged whole as x - 128 (the byte XOR 0x80, a signed int8), and
+// rows (stored as x - 128, a signed int8) are staged whole, and
 // v_mfma_i32_16x16x64_i8 gives a'.b' exactly, so s = |a'|^2 + |b'|^2 - 2 a'.b' = |a - b|^2
 // exactly (|a'|^2 from n2s): the canonical distance of this data, as in the BF16 exact
 // screen.  Half the staged bytes and MFMA instructions of the BF16 rows; the column blocks
@@ -793,10 +795,6 @@ __global__ __launch_bounds__(256) void k_localjoin_u8_screen(KnnArgs a) {
         if (col + 8 < D) v.z = *reinterpret_cast<const uint32_t*>(src + 8);
         if (col + 12 < D) v.w = *reinterpret_cast<const uint32_t*>(src + 12);
       }
-      v.x ^= col < D ? 0x80808080u : 0u;
-      v.y ^= col + 4 < D ? 0x80808080u : 0u;
-      v.z ^= col + 8 < D ? 0x80808080u : 0u;
-      v.w ^= col + 12 < D ? 0x80808080u : 0u;
     }
     *reinterpret_cast<uint4*>((op == 0 ? sA : sB) + r * RS + col) = v;
   }

@@ -14,6 +14,7 @@
 // separate buffers, so one kNN build can feed several prunings.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "screen.hpp"
 
 namespace tg {
 
@@ -368,7 +369,8 @@ __device__ __forceinline__ int advance_cl(uint64_t* P, uint16_t* cl, int from, i
 // Incremental Filter over the sorted pool P[0..L) (spec A.4 in the oracle).  Writes the
 // kept entries to sel[] and returns their number.  cl holds the round's candidates: the pool
 // indices after the current selection p that are not invalidated and do not repeat p's id,
-// in pool order, so a round touches only the survivors of the previous round.
+// in pool order, so a round touches only the survivors of the previous round.  For rows that
+// filter_pool_mfma does not take: wider than 256 elements, or without an 8-, 16-bit copy.
 // -------------------------------------------------------------------------------------
 template <int MC, class T>
 __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int L, uint32_t u,
@@ -402,71 +404,7 @@ __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int 
     const int cnt = nl;  // this round's candidates cl[0..cnt)
     Row16<MC> prow;
     const long long e0 = pclock(a);
-    if constexpr (std::is_same<T, uint8_t>::value) {
-      // Two rounds in one pass: the first candidate c1 is the next selection exactly when
-      // this round keeps it, which d(p, c1) -- two rows in registers -- decides.  Then each
-      // candidate row is read once for d(p, c) and d(c1, c), and every candidate meets the
-      // two rounds' rules in their order: one invalidated by p is not an evaluation of the
-      // second round, an entry repeating c1's id is dropped uncounted (as at a round's
-      // start), the others count for the second round.
-      const uint8_t* X8 = reinterpret_cast<const uint8_t*>(a.rows);
-      Row16<MC> qrow;
-      const bool two = cnt > 1 && nsel + 1 < FD;
-      const int i1 = two ? int(cl[0]) : 0;
-      row16_u8_load<MC>(prow, X8 + size_t(pid) * D, D);
-      if (two) row16_u8_load<MC>(qrow, X8 + size_t(key_id(P[i1])) * D, D);
-      row16_u8_norm<MC>(prow);
-      if (two) {
-        row16_u8_norm<MC>(qrow);
-        const uint64_t k1 = P[i1];
-        const uint32_t id1 = key_id(k1);
-        const float cur1 = key_d(k1);
-        const float d1 = dist_rows_u8<MC>(prow, qrow, D);
-        if (!(rule_eval(rule, d1, cur1, cur, a.th) < 0.0f) && i1 + 1 < L) {
-          int n2 = 0;
-          eval_batch2_u8<MC>(X8, D, prow, qrow, cnt, [&](int q) { return key_id(P[cl[q]]); },
-                             [&](int q, float da, float db) {
-                               if (q == 0) return;  // c1: kept by this round
-                               const int i = cl[q];
-                               const uint64_t k = P[i];
-                               if (rule_eval(rule, da, key_d(k), cur, a.th) < 0.0f) {
-                                 P[i] = key_with_id(k, TG_INV);
-                               } else if (key_id(k) == id1) {
-                                 P[i] = key_with_id(k, TG_INV);
-                               } else {
-                                 ++n2;
-                                 if (rule_eval(rule, db, key_d(k), cur1, a.th) < 0.0f)
-                                   P[i] = key_with_id(k, TG_INV);
-                               }
-                             });
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) n2 += __shfl_xor(n2, o, TG_WAVE);
-          ph.ev += pclock(a) - e0;
-          n_eval += cnt + n2;
-          __syncthreads();
-          // the first round's selection is c1; the second's is its first survivor
-          if (lane == 0) sel[nsel] = k1;
-          ++nsel;
-          int pi;
-          nl = advance_cl(P, cl, 1, cnt - 1, pi);
-          if (pi >= 0) {
-            if (lane == 0) sel[nsel] = P[pi];
-            cur = key_d(P[pi]);
-            pid = key_id(P[pi]);
-            tix = pi;
-          } else {
-            tix = L;
-          }
-          ++nsel;
-          ++tix;
-          __syncthreads();
-          if (tix >= L) break;
-          continue;
-        }
-      }
-    } else {
-      load_row16<MC>(prow, reinterpret_cast<const T*>(a.rows) + size_t(pid) * D, D, t);
-    }
+    load_row16<MC>(prow, reinterpret_cast<const T*>(a.rows) + size_t(pid) * D, D, t);
     eval_batch<MC>(reinterpret_cast<const T*>(a.rows), D, prow, cnt, [&](int q) { return key_id(P[cl[q]]); },
                    [&](int q, float res) {
                      const int i = cl[q];
@@ -497,6 +435,302 @@ __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int 
   return nsel - 1;  // the last appended entry is never kept (Tagore_src.cu:1462-1477)
 }
 
+// -------------------------------------------------------------------------------------
+// The same Filter with the distances on the matrix cores, up to 16 rounds at a time: the next
+// 16 live candidates are the rows of 16 x 16 products against every live candidate's row,
+// which is read once for all of them (one round, or two, per read before: long live lists were
+// bound by the row reads).  Whether row i's rule kills column j does not depend on which rows
+// are selected, so each column gets a 16-bit mask of its killers; the selections among the 16
+// rows follow from their own masks in order, and a column survives when its mask holds no
+// selected row.  Rounds, selections and evaluation counts are those of one round at a time: a
+// column counts for every selection before it up to its first killer (a killer that repeats
+// its id is not an evaluation).
+//   u8 rows (int8 MFMA): the distances are exact.
+//   16-bit copy (a.Xb): s +- kap (|p|^2 + |c|^2) brackets the canonical distance and the rules
+//   are monotone in it, so equal verdicts at both ends are the verdict; other pairs of a
+//   selected row are queued and evaluated canonically from a.rows.
+// A lane loads 16 bytes of row t = lane & 15 per step of 64 bytes, straight into the operand
+// layout; KS steps.
+// k_forward / k_reverse, before and after: Vamana (alpha 1.2, 12.8 k evaluations per node) over
+// 400k x 128 u8 rows 51.1 -> 18.3 / 4.98 -> 1.36 ms, over 160k x 96 real-valued rows 22.5 -> 5.5 /
+// 3.16 -> 0.67 ms; NSG over 1M x 128 u8 rows 34.3 -> 31.9 / 3.29 -> 1.77 ms; two-hop with angles
+// over 300k x 96 13.8 -> 8.8 / 3.26 -> 1.06 ms.  Now bound by the chain of a block (its rows, its
+// own columns, the tiles' loads), not by the products.
+// LDS: cl and km [L + 16] (live pool indices, killer masks), queue [FQ_CAP] (16-bit copy).
+// -------------------------------------------------------------------------------------
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+constexpr int FQ_CAP = 512;
+
+// Verdict of the rule for a distance in [lo, hi]: 1 below zero, 0 not, 2 undecided.  rule 0 is
+// evaluated at both ends.  rule 1 (angle): th - ((dis + cur) - res) / 2 / sqrt(dis cur) < 0 where
+// res < T = dis + cur - 2 th sqrt(dis cur); its roundings and those of T here move the border by
+// less than (1 + |th|)(dis + cur) 2^-20, as long as dis cur is a normal number.
+__device__ __forceinline__ int rule_bracket(int rule, float lo, float hi, float dis, float cur,
+                                            float th) {
+  if (rule == 0) {
+    const float a = th * lo - dis, b = th * hi - dis;
+    return (a < 0.0f && b < 0.0f) ? 1 : (a >= 0.0f && b >= 0.0f) ? 0 : 2;
+  }
+  const float dc = dis * cur, sum = dis + cur;
+  if (!(dc > 1e-30f && dc < 1e37f)) return 2;
+  const float T = __builtin_fmaf(-2.0f * th, __builtin_amdgcn_sqrtf(dc), sum);
+  const float sl = (1.0f + fabsf(th)) * sum * 0x1p-20f;
+  return hi < T - sl ? 1 : lo > T + sl ? 0 : 2;
+}
+
+template <int MC, class T>
+__device__ __forceinline__ int filter_pool_mfma(const PruneArgs& a, const uint64_t* P, int L,
+                                                uint32_t u, int rule, uint64_t* sel,
+                                                uint16_t* cl, uint16_t* km, uint16_t* queue,
+                                                uint32_t& n_eval, PhaseAcc& ph) {
+  constexpr bool U8 = std::is_same<T, uint8_t>::value;
+  constexpr int KS = U8 ? MC : 2 * MC;  // 64-byte steps of a row
+  constexpr int ESZ = U8 ? 1 : 2;
+  using Acc = typename std::conditional<U8, i32x4, f32x4>::type;
+  const int lane = threadIdx.x, t = lane & 15, g = lane >> 4;
+  const int D = a.D;
+  const float th = a.th;
+  const unsigned char* X8 = U8 ? reinterpret_cast<const unsigned char*>(a.rows)
+                               : reinterpret_cast<const unsigned char*>(a.Xb);
+  const int tix = next_valid(P, 0, L, u);
+  if (tix >= L || a.FD < 2) return 0;
+  const int rounds = int(a.FD) - 1;  // the last appended entry is never kept
+  // the live list: the first selection and every valid entry after it
+  int cnt = 0;
+  for (int base = tix; base < L; base += TG_WAVE) {
+    const int i = base + lane;
+    const bool live = i < L && key_id(P[i]) != TG_INV;
+    const uint64_t m = ballot(live);
+    if (live) cl[cnt + mask_rank(m)] = uint16_t(i);
+    cnt += __popcll(m);
+  }
+  __syncthreads();
+
+  auto load_row = [&](uint4 (&f)[KS], uint32_t id) {
+    const unsigned char* x = X8 + size_t(id) * (D * ESZ);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      f[k] = make_uint4(0u, 0u, 0u, 0u);
+      if constexpr (U8) {
+        if (64 * k < D) f[k] = load_u8x16(x, k, D, g);
+      } else {
+        if (32 * k + 8 * g < D) f[k] = *reinterpret_cast<const uint4*>(x + 64 * k + 16 * g);
+      }
+    }
+  };
+  auto product = [&](const uint4 (&x)[KS], const uint4 (&y)[KS]) {
+    Acc c = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      if (k * 64 >= D * ESZ) break;
+      if constexpr (U8) {
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, x[k]),
+                                                  __builtin_bit_cast(i32x4, y[k]), c, 0, 0, 0);
+      } else if (a.h_bf16) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[k]),
+                                                    __builtin_bit_cast(bf16x8, y[k]), c, 0, 0, 0);
+      } else {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[k]),
+                                                   __builtin_bit_cast(f16x8, y[k]), c, 0, 0, 0);
+      }
+    }
+    return c;
+  };
+  // |x|^2 of the lane's row t (u8: of the signed bytes), in every lane of that row
+  auto norm_u8 = [&](const uint4 (&f)[KS]) {
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) s = dot16_u8(f[k], f[k], s);
+    s += int(lane_xor32(uint32_t(s), 16));
+    return s + int(lane_xor32(uint32_t(s), 32));
+  };
+  auto or_groups = [&](uint32_t m) {
+    m |= lane_xor32(m, 16);
+    return m | lane_xor32(m, 32);
+  };
+
+  int kept = 0;
+  while (kept < rounds && cnt > 0) {
+    const int nb = min(16, cnt);
+    const long long e0 = pclock(a);
+    // row t of the block in the lanes t + 16 g; rows past nb repeat row 0, their bits masked
+    const uint64_t krow = P[cl[t < nb ? t : 0]];
+    const uint32_t idt = key_id(krow);
+    uint4 fr[KS];
+    load_row(fr, idt);
+    float nf = 0.f;  // |x|^2 of row t
+    int ni = 0;
+    if constexpr (U8) ni = norm_u8(fr);
+    else nf = a.nrm2[idt];
+    // rows 4g + r, as the products hold them
+    uint32_t rid[4];
+    float rcur[4], rnf[4];
+    int rni[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      rid[r] = uint32_t(__shfl(int(idt), 4 * g + r, TG_WAVE));
+      rcur[r] = __shfl(key_d(krow), 4 * g + r, TG_WAVE);
+      if constexpr (U8) rni[r] = __shfl(ni, 4 * g + r, TG_WAVE);
+      else rnf[r] = __shfl(nf, 4 * g + r, TG_WAVE);
+    }
+    int qn = 0;  // queued pairs
+    // killer bits of column (key kc, norm) from its products; `rows`: the rows that matter;
+    // undecided pairs are queued under column number col
+    auto kill_bits = [&](const Acc& c, uint64_t kc, float cnf, int cni, uint32_t rows, int col) {
+      const float dis = key_d(kc);
+      const uint32_t cid = key_id(kc);
+      uint32_t nib = 0, und = 0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (U8) {
+          const float res = float(rni[r] + cni - 2 * c[r]);
+          if (rule == 0) {
+            nib |= (th * res - dis < 0.0f) ? 1u << r : 0u;
+          } else {
+            const int v = rule_bracket(1, res, res, dis, rcur[r], th);
+            nib |= v == 1 ? 1u << r : 0u;
+            und |= v == 2 ? 1u << r : 0u;
+          }
+        } else {
+          const float nsum = rnf[r] + cnf;
+          const float s = __builtin_fmaf(-a.pscale, c[r], nsum);
+          const int v = rule_bracket(rule, __builtin_fmaf(-a.kap, nsum, s),
+                                     __builtin_fmaf(a.kap, nsum, s), dis, rcur[r], th);
+          nib |= v == 1 ? 1u << r : 0u;
+          und |= v == 2 ? 1u << r : 0u;
+        }
+        if (rid[r] == cid) {  // a repeated id is dropped whatever its distance
+          nib |= 1u << r;
+          und &= ~(1u << r);
+        }
+      }
+      und &= rows >> (4 * g);
+      if (ballot((und & 15u) != 0) != 0) {
+        if constexpr (U8) {  // the distances are exact: the rule itself
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float res = float(rni[r] + cni - 2 * c[r]);
+            if (((und >> r) & 1u) && rule_eval(rule, res, dis, rcur[r], th) < 0.0f) nib |= 1u << r;
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const bool q = (und >> r) & 1u;
+            const uint64_t m = ballot(q);
+            if (q) queue[qn + mask_rank(m)] = uint16_t((4 * g + r) << 10 | col);
+            qn += __popcll(m);
+          }
+        }
+      }
+      return or_groups((nib & 15u) << (4 * g)) & rows;
+    };
+    // canonical distances of the queued pairs, one per 16-lane group (few, and a second pair's
+    // registers would cost a wave per SIMD)
+    auto flush = [&]() {
+      if constexpr (!U8) {
+        __syncthreads();
+        const T* X = reinterpret_cast<const T*>(a.rows);
+        for (int q0 = 0; q0 < qn; q0 += 4) {
+          const int q = q0 + g;
+          const uint32_t ent = queue[q < qn ? q : 0], i = ent >> 10, col = ent & 1023u;
+          const uint64_t ki = P[cl[i]], kcol = P[cl[col]];
+          const T* const ra[1] = {X + size_t(key_id(ki)) * D};
+          const T* const rb[1] = {X + size_t(key_id(kcol)) * D};
+          float dd[1];
+          dist16_pairs<MC, 1>(ra, rb, D, t, dd);
+          if (t == 0 && q < qn && rule_eval(rule, dd[0], key_d(kcol), key_d(ki), th) < 0.0f)
+            atomicOr(reinterpret_cast<uint32_t*>(km) + (col >> 1), (1u << i) << (16 * (col & 1)));
+        }
+        qn = 0;
+        __syncthreads();
+      }
+    };
+    // ---- the block's own columns: row j is selected when no selected row kills it
+    const uint32_t before = t < nb ? ((1u << t) - 1u) : 0u;
+    uint32_t own = kill_bits(product(fr, fr), krow, nf, ni, before, t);
+    if (qn) {
+      if (g == 0) km[t] = uint16_t(own);
+      flush();
+      own = km[t];
+    }
+    // a selection at the pool's last position ends the filter unkept, but for the first one
+    const bool at_end = int(cl[cnt - 1]) == L - 1;
+    uint32_t chosen = 0;
+    int n = kept;
+    bool done = false;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const uint32_t mj = uint32_t(__builtin_amdgcn_readlane(int(own), j));
+      if (j < nb && !done && (mj & chosen) == 0) {
+        if (n == rounds || (at_end && j == cnt - 1 && n > 0)) done = true;
+        else {
+          chosen |= 1u << j;
+          ++n;
+        }
+      }
+    }
+    if (g == 0) {
+      km[t] = uint16_t(own);
+      if ((chosen >> t) & 1u) sel[kept + __popc(chosen & before)] = krow;
+    }
+    kept = n;
+    // ---- the other columns; u8: two tiles' rows in flight (16-bit rows take the registers)
+    constexpr int TI = U8 ? 2 : 1;
+    for (int c0 = 16; c0 < cnt; c0 += 16 * TI) {
+      uint64_t kc[TI];
+      uint4 fc[TI][KS];
+      float nc[TI];
+#pragma unroll
+      for (int x = 0; x < TI; ++x) {
+        const int c = c0 + 16 * x + t;
+        kc[x] = P[cl[c < cnt ? c : 0]];
+        load_row(fc[x], key_id(kc[x]));
+        nc[x] = U8 ? 0.f : a.nrm2[key_id(kc[x])];
+      }
+      if (qn > FQ_CAP - 256) flush();
+#pragma unroll
+      for (int x = 0; x < TI; ++x) {
+        const int c = c0 + 16 * x + t;
+        const uint32_t m = kill_bits(product(fr, fc[x]), kc[x], nc[x], U8 ? norm_u8(fc[x]) : 0,
+                                     c < cnt ? chosen : 0u, c);
+        if (g == 0 && c < cnt) km[c] = uint16_t(m);
+      }
+    }
+    if (qn) flush();
+    else __syncthreads();
+    ph.ev += pclock(a) - e0;
+    // ---- evaluations and the survivors, in order (in place: a chunk is read before any of
+    // its entries is written, and writes land at or below it)
+    int live = 0;
+    uint32_t ev = 0;
+    for (int base = 0; base < cnt; base += TG_WAVE) {
+      const int c = base + lane;
+      const bool in = c < cnt;
+      const uint32_t idx = in ? cl[c] : 0u;
+      const uint32_t rows = c < 16 ? chosen & ((1u << c) - 1u) : chosen;
+      const uint32_t k = in ? km[c] & rows : 0u;
+      const int f = k ? __ffs(k) - 1 : 0;
+      const uint32_t fid = uint32_t(__shfl(int(idt), f, TG_WAVE));
+      if (in) {
+        ev += k ? __popc(rows & ((1u << f) - 1u)) + (fid != key_id(P[idx]) ? 1u : 0u)
+                : __popc(rows);
+      }
+      const bool alive = in && k == 0 && !(c < 16 && ((chosen >> c) & 1u));
+      const uint64_t m = ballot(alive);
+      __syncthreads();
+      if (alive) cl[live + mask_rank(m)] = uint16_t(idx);
+      live += __popcll(m);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ev += uint32_t(__shfl_xor(int(ev), o, TG_WAVE));
+    n_eval += ev;
+    cnt = live;
+    if (done) break;
+  }
+  return kept;
+}
+
 __device__ __forceinline__ void count_add(unsigned long long* c, int idx, uint32_t v) {
   if (c && threadIdx.x == 0 && v) atomicAdd(&cnt_slot(c)[idx], (unsigned long long)v);
 }
@@ -508,7 +742,7 @@ __device__ __forceinline__ void count_add(unsigned long long* c, int idx, uint32
 //   during the beam: the 480-slot ring (padded to 512 for its sort), then S | tab | beam
 //       compaction indices;
 //   afterwards: the pool (K + 480 keys, over the ring and the dead start of the beam's
-//       scratch), then the selected list and the filter's compaction indices (K + 480).
+//       scratch), then the selected list and the filter's lists.
 // The pool is the merge of the sorted own list and the sorted ring, formed in registers as
 // one bitonic merge of [own list ascending | +inf | ring descending] (1024 slots); it is
 // the sequence a sort of their union gives.
@@ -518,7 +752,8 @@ constexpr int RING_P = 512;
 struct FwdLayout {
   int W, NS, L, HB, offB, offF, bytes;
 };
-__host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD) {
+__host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD,
+                                                         bool mfma) {
   FwdLayout l;
   l.W = (K <= 64 && TOPM <= 64) ? 1 : 2;
   l.NS = 64 * l.W;
@@ -529,20 +764,26 @@ __host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD) {
   l.offB = RING_P * 8;
   l.offF = ((l.L > RING_P ? l.L : RING_P) * 8 + 15) / 16 * 16;
   const int beam = l.offB + l.NS * 8 + (4 << l.HB) + l.NS * 2;
-  const int filt = l.offF + (FD + 1) * 8 + l.L * 2;
+  // the filter's selection, live list, killer masks and re-score queue
+  const int filt = l.offF + (FD + 1) * 8 + (l.L + 17) * 4 + (mfma ? FQ_CAP * 2 : 0);
   l.bytes = ((beam > filt ? beam : filt) + 15) / 16 * 16;
   return l;
 }
 
-template <int MC, class T, int KIND, int W>
-// Six waves per SIMD: 80 VGPRs at most (the 64-candidate distance steps need 86 otherwise).
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_forward(PruneArgs a) {
+// mfma: filter_pool_mfma on the 16-bit copy (u8 rows always take it).
+template <int MC, class T, int KIND, int W, bool MF>
+// Waves per SIMD: six (80 VGPRs) for u8 rows up to 128 elements, fewer where the rows' registers
+// would spill.
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(MC == 2 ? (std::is_same<T, uint8_t>::value || !MF ? 6 : 5)
+                                           : (MC == 4 ? (std::is_same<T, uint8_t>::value ? 5 : 3) : 2))))
+void k_forward(PruneArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
   const uint32_t u = row_of_block(a.perm, a.N);
   if (u >= a.N) return;
   const int lane = threadIdx.x, t = lane & 15;
   const int K = a.K, D = a.D;
-  const FwdLayout ly = fwd_layout(K, int(a.TOPM), int(a.FD));
+  const FwdLayout ly = fwd_layout(K, int(a.TOPM), int(a.FD), MF && !std::is_same<T, uint8_t>::value);
   uint64_t* R = reinterpret_cast<uint64_t*>(dsm);
   uint64_t* P = R;  // after the pool is formed
   uint64_t* S = reinterpret_cast<uint64_t*>(dsm + ly.offB);
@@ -550,6 +791,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
   uint16_t* clb = reinterpret_cast<uint16_t*>(tab + (1 << ly.HB));
   uint64_t* sel = reinterpret_cast<uint64_t*>(dsm + ly.offF);  // after the beam
   uint16_t* cl = reinterpret_cast<uint16_t*>(sel + a.FD + 1);
+  uint16_t* km = cl + ((ly.L + 17) & ~1);
+  uint16_t* fq = km + ((ly.L + 17) & ~1);
   const int L = ly.L;
   Row16<MC> xu;
   load_row16<MC>(xu, reinterpret_cast<const T*>(a.rows) + size_t(u) * D, D, t);
@@ -620,7 +863,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
     if (dup[q]) P[q * TG_WAVE + lane] = key_with_id(P[q * TG_WAVE + lane], TG_INV);
   __syncthreads();
   const long long c2 = pclock(a);
-  const int deg = filter_pool<MC, T>(a, P, L, u, a.fwd_rule, sel, cl, n_flt, ph);
+  int deg;
+  if constexpr (MF) deg = filter_pool_mfma<MC, T>(a, P, L, u, a.fwd_rule, sel, cl, km, fq, n_flt, ph);
+  else deg = filter_pool<MC, T>(a, P, L, u, a.fwd_rule, sel, cl, n_flt, ph);
   __syncthreads();
   if (a.phase_clock && lane == 0 && a.counters) {
     const long long c3 = clock64();
@@ -647,11 +892,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
 // Reverse pass (filter_reverse, spec A.7): forward list plus the K best reverse pushes;
 // re-filtered with the reverse rule when more than FD, otherwise their union.
 // -------------------------------------------------------------------------------------
-template <int MC, class T>
+template <int MC, class T, bool MF>
 __global__ __launch_bounds__(64) void k_reverse(PruneArgs a) {
   __shared__ uint64_t buf[256];
   __shared__ uint64_t P[256];
-  __shared__ uint16_t cl[256];
+  __shared__ __attribute__((aligned(4))) uint16_t cl[272], km[MF ? 272 : 2];
+  __shared__ uint16_t fq[MF && !std::is_same<T, uint8_t>::value ? FQ_CAP : 1];
   __shared__ uint64_t sel[129];
   const uint32_t u = row_of_block(a.perm, a.N);
   if (u >= a.N) return;
@@ -669,7 +915,9 @@ __global__ __launch_bounds__(64) void k_reverse(PruneArgs a) {
     else merge_pool<4>(a, u, deg, buf, nr, P);
     mark_dups(P, n);
     PhaseAcc ph;  // not reported for the reverse pass
-    const int nd = filter_pool<MC, T>(a, P, L, u, a.rev_rule, sel, cl, n_flt, ph);
+    int nd;
+    if constexpr (MF) nd = filter_pool_mfma<MC, T>(a, P, L, u, a.rev_rule, sel, cl, km, fq, n_flt, ph);
+    else nd = filter_pool<MC, T>(a, P, L, u, a.rev_rule, sel, cl, n_flt, ph);
     __syncthreads();
     for (int k = lane; k < FD; k += TG_WAVE) row[k] = k < nd ? key_id(sel[k]) : TG_INV;
     if (lane == 0) a.out_deg[u] = nd;
@@ -1006,24 +1254,18 @@ __global__ void k_centroid_final(const double* part, uint32_t nch, uint32_t N, u
 }
 
 // ------------------------------------------------------------------------- launchers
-template <int MC, class T>
-static void launch_prune_mc(const PruneArgs& a, int phase, const float* centroid, uint32_t* ep,
-                            hipStream_t s, uint32_t nseg) {
+// The passes with a filter.
+template <int MC, class T, bool MF>
+static void launch_filter_mc(const PruneArgs& a, int phase, hipStream_t s) {
   const dim3 grid(grid_rows(a.perm, a.N)), block(64);
+  const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD, MF && !std::is_same<T, uint8_t>::value);
   switch (phase) {
-    case PH_EP: k_cal_ep<MC, T><<<nseg, 64, 0, s>>>(a, centroid, ep); break;
     case PH_FWD_PATH:
-      if (fwd_layout(a.K, a.TOPM, a.FD).W == 1)
-        k_forward<MC, T, 0, 1><<<grid, block, fwd_layout(a.K, a.TOPM, a.FD).bytes, s>>>(a);
-      else
-        k_forward<MC, T, 0, 2><<<grid, block, fwd_layout(a.K, a.TOPM, a.FD).bytes, s>>>(a);
+      if (f.W == 1) k_forward<MC, T, 0, 1, MF><<<grid, block, f.bytes, s>>>(a);
+      else k_forward<MC, T, 0, 2, MF><<<grid, block, f.bytes, s>>>(a);
       break;
-    case PH_FWD_2HOP:
-      k_forward<MC, T, 1, 1><<<grid, block, fwd_layout(a.K, a.TOPM, a.FD).bytes, s>>>(a);
-      break;
-    case PH_REV: k_reverse<MC, T><<<grid, block, 0, s>>>(a); break;
-    case PH_DPG: k_dpg_forward<MC, T><<<grid, block, 0, s>>>(a); break;
-    default: break;
+    case PH_FWD_2HOP: k_forward<MC, T, 1, 1, MF><<<grid, block, f.bytes, s>>>(a); break;
+    default: k_reverse<MC, T, MF><<<grid, block, 0, s>>>(a); break;
   }
 }
 
@@ -1031,25 +1273,25 @@ template <class T>
 static void launch_prune_t(const PruneArgs& a, int phase, const float* centroid, uint32_t* ep,
                            hipStream_t s, uint32_t nseg) {
   const int mc = (a.D + 63) / 64;
-  if (mc <= 2) launch_prune_mc<2, T>(a, phase, centroid, ep, s, nseg);
-  else if (mc <= 4) launch_prune_mc<4, T>(a, phase, centroid, ep, s, nseg);
-  else launch_prune_mc<16, T>(a, phase, centroid, ep, s, nseg);
-}
-
-// The passes whose targets are rows of X, on the u8 copy.
-template <int MC>
-static void launch_prune_u8_mc(const PruneArgs& a, int phase, hipStream_t s) {
-  const dim3 grid(grid_rows(a.perm, a.N)), block(64);
-  const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD);
-  switch (phase) {
-    case PH_FWD_PATH:
-      if (f.W == 1) k_forward<MC, uint8_t, 0, 1><<<grid, block, f.bytes, s>>>(a);
-      else k_forward<MC, uint8_t, 0, 2><<<grid, block, f.bytes, s>>>(a);
-      break;
-    case PH_FWD_2HOP: k_forward<MC, uint8_t, 1, 1><<<grid, block, f.bytes, s>>>(a); break;
-    case PH_REV: k_reverse<MC, uint8_t><<<grid, block, 0, s>>>(a); break;
-    default: break;
-  }
+#define PR_MC(CALL)                       \
+  do {                                    \
+    if (mc <= 2) CALL(2);                 \
+    else if (mc <= 4) CALL(4);            \
+    else CALL(16);                        \
+  } while (0)
+#define PR_EP(M) k_cal_ep<M, T><<<nseg, 64, 0, s>>>(a, centroid, ep)
+#define PR_DPG(M) k_dpg_forward<M, T><<<grid_rows(a.perm, a.N), 64, 0, s>>>(a)
+#define PR_FLT(M) launch_filter_mc<M, T, false>(a, phase, s)
+  if (phase == PH_EP) PR_MC(PR_EP);
+  else if (phase == PH_DPG) PR_MC(PR_DPG);
+  // the 16-bit copy, rows up to 256 elements (operands of wider rows do not stay in registers)
+  else if (a.Xb && mc <= 2) launch_filter_mc<2, T, true>(a, phase, s);
+  else if (a.Xb && mc <= 4) launch_filter_mc<4, T, true>(a, phase, s);
+  else PR_MC(PR_FLT);
+#undef PR_FLT
+#undef PR_DPG
+#undef PR_EP
+#undef PR_MC
 }
 
 void launch_prune(const PruneArgs& a, int phase, const float* centroid, uint32_t* ep,
@@ -1068,8 +1310,8 @@ void launch_prune(const PruneArgs& a, int phase, const float* centroid, uint32_t
     PruneArgs b = a;
     b.rows = a.rows8;
     b.rows_bf16 = 0;
-    if (a.D <= 128) launch_prune_u8_mc<2>(b, phase, s);
-    else launch_prune_u8_mc<4>(b, phase, s);
+    if (a.D <= 128) launch_filter_mc<2, uint8_t, true>(b, phase, s);
+    else launch_filter_mc<4, uint8_t, true>(b, phase, s);
     return;
   }
   if (a.rows_bf16) launch_prune_t<uint16_t>(a, phase, centroid, ep, s, nseg);

@@ -473,3 +473,30 @@ def test_screened_join_edges(name, D, K):
             assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
     if D % 8 == 0 and K >= 24:
         _compare(X, Gr, GDr, 3, 0, 2, 16, 64, 0.0, "bf16")
+
+
+@pytest.mark.parametrize("name", ["u8", "signed", "bf16", "real", "scales"])
+@pytest.mark.parametrize("D", [4, 64, 100, 128, 200, 256, 264])
+def test_block_filter_edges(name, D):
+    """The Filter's blocks of 16 selections: degrees 1, 2, one block and its neighbours, and the
+    largest; both rules and thresholds that keep much, little and everything; u8 rows, rows
+    with a BF16 or FP16 copy, and rows without one.  Rows and evaluation counts equal to the
+    oracle."""
+    rng = np.random.default_rng(D)
+    N = 600
+    if name in ("u8", "signed"):
+        lo = 0 if name == "u8" else -60
+        X = rng.integers(lo, lo + 120, (N, D)).astype(np.float32)
+        X[:200] = np.clip(X[0] + rng.integers(-5, 6, (200, D)), lo, lo + 119)
+    else:
+        X = (rng.standard_normal((5, D))[rng.integers(0, 5, N)]
+             + rng.standard_normal((N, D))).astype(np.float32)
+        if name == "bf16":
+            X = (X.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+        if name == "scales":
+            X = X * np.where(np.arange(N) % 2, 1.0, 1e-7)[:, None].astype(np.float32)
+    G, GD = oracle.knn_bruteforce(X, 40)
+    for kind, fr, rr, FD, th in [(0, 0, 0, 1, 1.0), (0, 0, 1, 2, 0.3), (0, 0, 0, 17, 1.2),
+                                 (1, 1, 1, 16, 0.5), (1, 0, 0, 33, 1.05), (0, 1, 0, 128, -0.2),
+                                 (0, 0, 0, 40, 3.0)]:
+        _compare(X, G, GD, kind, fr, rr, FD, 64, th)
