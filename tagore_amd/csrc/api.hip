@@ -1774,6 +1774,7 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
     fill_u32(reinterpret_cast<uint32_t*>(s->scnt), 0, 4, s->stream);
     SearchArgs a{};
     a.X = s->X;
+    a.X8 = s->prep_valid && s->cert_u8 && D <= 256 ? s->X8 : nullptr;
     a.N = N;
     a.D = D;
     a.deg = s->out_deg;
@@ -1892,6 +1893,7 @@ int tg_search_noalloc(tg_state* s, uint32_t nq, const float* queries_dev,
   fill_u32(bitmap, 0, size_t(grid) * words, st);
   SearchArgs a{};
   a.X = s->X;
+  a.X8 = s->prep_valid && s->cert_u8 && s->D <= 256 ? s->X8 : nullptr;
   a.N = N;
   a.D = s->D;
   a.deg = s->out_deg;

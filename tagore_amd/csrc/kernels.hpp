@@ -179,6 +179,7 @@ void fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 // workgroup.  counters: [0] distance evaluations, [1] expansions.
 struct SearchArgs {
   const float* X;
+  const uint8_t* X8;  // u8 copy (KnnArgs::X8) or null
   uint32_t N, D;
   const uint32_t* deg;
   const uint32_t* ids;
@@ -190,6 +191,7 @@ struct SearchArgs {
   uint32_t words;
   uint32_t* vlist;
   uint32_t vcap;
+  uint32_t hbits;     // set by launch_search
   uint32_t* out_ids;
   float* out_d;
   unsigned long long* counters;

@@ -176,3 +176,33 @@ def test_index_search_recall_regression(name, th):
         r = s.search_recall(Q, ids, 10)
     _say(f"{name}: search recall@10 {r:.4f}")
     assert r >= 0.95
+
+
+@pytest.mark.parametrize("D,FD,L", [(32, 8, 10), (100, 32, 64), (128, 64, 65), (256, 48, 128),
+                                    (260, 96, 200), (128, 128, 256)])
+def test_search_visited_set_and_rows(D, FD, L):
+    """Random graphs: nearly every neighbour is new, so searches outgrow the visited hash and go
+    on in the bitmap, queries after them on the same workgroups.  Integer data with integer
+    and fractional queries side by side (u8 and FP32 rows up to 256 elements), a graph that
+    was installed before any preparation of the data and after one."""
+    rng = np.random.default_rng(D + L)
+    N, nq = 20000, 40
+    X = rng.integers(0, 256, (N, D)).astype(np.float32)
+    Q = rng.integers(0, 256, (nq, D)).astype(np.float32)
+    Q[1::3] += 0.25
+    Q[2::7] -= 300
+    ids = rng.integers(0, N, (N, FD)).astype(np.uint32)
+    deg = rng.integers(FD // 2, FD + 1, N).astype(np.uint32)
+    ids[5, 1] = ids[5, 0]  # a repeated neighbour
+    oi, od, oc = oracle.search(X, deg, ids, 5, Q, L, 10, 0x77)
+    with State(N, D) as s:
+        s.set_data(X)
+        s.set_pruned(deg, ids, 5)
+        for step in range(2):
+            _say(f"search D={D} FD={FD} L={L} step {step}")
+            gi, gd, st = s.search(Q, k=10, L=L, seed=0x77)
+            assert np.array_equal(gi, oi) and np.array_equal(gd, od)
+            assert st["evals"] == oc["evals"] and st["expansions"] == oc["expansions"]
+            if step == 0 and D % 8 == 0:
+                s.knn_build(4, 2, 1, "bf16")  # prepares the data
+                s.set_pruned(deg, ids, 5)
