@@ -78,13 +78,18 @@ struct EventPair {
 struct PB {
   PushBuf d{};
   uint32_t N = 0;
+  // overflow entries for a request of ov_cap: whole areas, indexed with 32 bits
+  static uint32_t area(size_t ov_cap) {
+    return uint32_t(std::min<size_t>((ov_cap + OV_AREAS - 1) / OV_AREAS, 0xFFFFFFFFu / OV_AREAS));
+  }
   bool alloc(uint32_t n, uint32_t cap, size_t ov_cap) {
     N = n;
     d.cap = cap;
-    d.ov_cap = uint32_t(std::min<size_t>(ov_cap, 0xFFFFFFF0u));
+    d.ov_area = area(ov_cap);
+    d.ov_cap = OV_AREAS * d.ov_area;
     if (dalloc(&d.cnt, n) || dalloc(&d.slots, size_t(n) * cap) || dalloc(&d.ov_dest, d.ov_cap) ||
-        dalloc(&d.ov_key, d.ov_cap) || dalloc(&d.ov_used, 1) || dalloc(&d.ov_off, size_t(n) + 1) ||
-        dalloc(&d.ov_sorted, d.ov_cap) || dalloc(&d.err, 1))
+        dalloc(&d.ov_key, d.ov_cap) || dalloc(&d.ov_used, OV_AREAS * OV_STRIDE) ||
+        dalloc(&d.ov_off, size_t(n) + 1) || dalloc(&d.ov_sorted, d.ov_cap))
       return false;
     return true;
   }
@@ -96,7 +101,7 @@ struct PB {
     dfree(d.ov_used);
     dfree(d.ov_off);
     dfree(d.ov_sorted);
-    dfree(d.err);
+    d.err = nullptr;  // part of the handle's status words
   }
 };
 
@@ -140,7 +145,7 @@ struct tg_state {
   float* n2s = nullptr;            // [N] |x - 128|^2 of the u8 rows
   uint32_t* fill = nullptr;
   uint32_t* scan_tmp = nullptr;
-  unsigned long long* counters = nullptr;  // [CNT_SLOTS * CNT_N], summed over the slots
+  unsigned long long* counters = nullptr;  // [CNT_SLOTS * CNT_N] and the push buffers' errors
   // prune
   uint32_t FD_alloc = 0;
   uint32_t *fwd_deg = nullptr, *fwd_ids = nullptr, *out_deg = nullptr, *out_ids = nullptr;
@@ -193,34 +198,28 @@ int ensure_events(tg_state* s, size_t n) {
   return TG_OK;
 }
 
-int check_pb_err(tg_state* s, PB& pb, const char* what) {
-  uint32_t e = 0;
-  HIPX(hipMemcpyAsync(&e, pb.d.err, 4, hipMemcpyDeviceToHost, s->stream));
-  HIPX(hipStreamSynchronize(s->stream));
-  if (e)
-    return fail(TG_ERR_CAPACITY, std::string("push-buffer overflow area exhausted in ") + what);
+// The evaluation counters and the push buffers' error words lie together: one fill clears
+// them, one copy reads them.
+constexpr size_t STATUS_WORDS = 2 * size_t(CNT_SLOTS) * CNT_N;
+enum { ERR_PN = 0, ERR_PO, ERR_PC, ERR_PR, ERR_REV, ERR_N };
+
+int alloc_pb(tg_state* s, PB& pb, uint32_t cap, size_t ov_cap, int err) {
+  if (!(pb.d.cnt && pb.d.cap == cap && pb.d.ov_area >= PB::area(ov_cap) && pb.N == s->N)) {
+    pb.release();
+    if (!pb.alloc(s->N, cap, ov_cap)) return TG_ERR_HIP;
+  }
+  pb.d.err = reinterpret_cast<uint32_t*>(s->counters) + STATUS_WORDS + err;
   return TG_OK;
 }
 
-int alloc_pb(tg_state* s, PB& pb, uint32_t cap, size_t ov_cap) {
-  if (pb.d.cnt && pb.d.cap == cap && pb.d.ov_cap >= std::min<size_t>(ov_cap, 0xFFFFFFF0u) &&
-      pb.N == s->N)
-    return TG_OK;
-  pb.release();
-  if (!pb.alloc(s->N, cap, ov_cap)) return TG_ERR_HIP;
-  fill_u32(pb.d.err, 0, 1, s->stream);
-  return TG_OK;
-}
-
-void clear_errors(tg_state* s, std::initializer_list<PB*> pbs) {
-  for (PB* pb : pbs)
-    if (pb->d.err) fill_u32(pb->d.err, 0, 1, s->stream);
+void clear_status(tg_state* s) {
+  fill_u32(reinterpret_cast<uint32_t*>(s->counters), 0, STATUS_WORDS + ERR_N, s->stream);
 }
 
 int ensure_common_scratch(tg_state* s) {
   if (!s->fill) {
-    if (dalloc(&s->fill, s->N) || dalloc(&s->scan_tmp, scan_tmp_words(s->N) + 16) ||
-        dalloc(&s->counters, size_t(CNT_SLOTS) * CNT_N))
+    if (dalloc(&s->fill, 2 * size_t(s->N)) || dalloc(&s->scan_tmp, 2 * scan_tmp_words(s->N) + 16) ||
+        dalloc(&s->counters, size_t(CNT_SLOTS) * CNT_N + ERR_N))
       return TG_ERR_HIP;
   }
   return TG_OK;
@@ -250,8 +249,8 @@ int ensure_knn_scratch(tg_state* s, uint32_t K) {
       return TG_ERR_HIP;
   }
   if (ensure_common_scratch(s)) return TG_ERR_HIP;
-  if (alloc_pb(s, s->pn, 64, N * 32) || alloc_pb(s, s->po, 64, N * 32) ||
-      alloc_pb(s, s->pc, 256, N * 256) || alloc_pb(s, s->pr, 128, N * size_t(K)))
+  if (alloc_pb(s, s->pn, 64, N * 32, ERR_PN) || alloc_pb(s, s->po, 64, N * 32, ERR_PO) ||
+      alloc_pb(s, s->pc, 256, N * 256, ERR_PC) || alloc_pb(s, s->pr, 128, N * size_t(K), ERR_PR))
     return TG_ERR_HIP;
   return TG_OK;
 }
@@ -413,14 +412,24 @@ int check_launch(const char* what) {
   return TG_OK;
 }
 
-// the evaluation counters, summed over their slots
-int read_counters(tg_state* s, unsigned long long (&cnt)[CNT_N]) {
-  std::vector<unsigned long long> all(size_t(CNT_SLOTS) * CNT_N);
-  HIPX(hipMemcpy(all.data(), s->counters, all.size() * 8, hipMemcpyDeviceToHost));
+// the evaluation counters, summed over their slots, and the push buffers' error words
+int read_status(tg_state* s, unsigned long long (&cnt)[CNT_N]) {
+  static const char* const what[ERR_N] = {"reverse sampling", "reverse sampling", "local join",
+                                          "reverse lists", "reverse edges"};
+  std::vector<uint32_t> all(STATUS_WORDS + ERR_N);
+  HIPX(hipMemcpy(all.data(), s->counters, all.size() * 4, hipMemcpyDeviceToHost));
   for (int i = 0; i < CNT_N; ++i) {
     cnt[i] = 0;
-    for (int b = 0; b < CNT_SLOTS; ++b) cnt[i] += all[size_t(b) * CNT_N + i];
+    for (int b = 0; b < CNT_SLOTS; ++b) {
+      unsigned long long v;
+      std::memcpy(&v, &all[2 * (size_t(b) * CNT_N + i)], 8);
+      cnt[i] += v;
+    }
   }
+  for (int e = 0; e < ERR_N; ++e)
+    if (all[STATUS_WORDS + e])
+      return fail(TG_ERR_CAPACITY,
+                  std::string("push-buffer overflow area exhausted in ") + what[e]);
   return TG_OK;
 }
 
@@ -1123,8 +1132,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
   hipEvent_t w0 = win.e0, w1 = win.e1;
   Sections sec{s};
   sec.next = 0;
-  fill_u32(reinterpret_cast<uint32_t*>(s->counters), 0, 2 * CNT_SLOTS * CNT_N, st);
-  clear_errors(s, {&s->pn, &s->po, &s->pc, &s->pr});
+  clear_status(s);
   HIPX(hipEventRecord(w0, st));
   // data that no 16-bit copy screens well takes the FP32 screen instead (same graph)
   const int prec = p->precision == TG_PREC_BF16 && !s->copy16 ? int(TG_PREC_FP32) : p->precision;
@@ -1192,22 +1200,18 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
     } restore{s, prof};
     for (uint32_t it = 0; it < it1; ++it) {
       if (sc.start(1)) return TG_ERR_HIP;
-      pb_reset(a.pn, N, s->fill, st);
-      pb_reset(a.po, N, s->fill, st);
+      pb_reset({&a.pn, &a.po, &a.pc}, N, st);
       launch_knn_sample(a, st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(2)) return TG_ERR_HIP;
-      pb_group_overflow(a.pn, N, s->fill, s->scan_tmp, st);
-      fill_u32(s->fill, 0, N, st);
-      pb_group_overflow(a.po, N, s->fill, s->scan_tmp, st);
+      pb_group_overflow({&a.pn, &a.po}, N, s->fill, s->scan_tmp, st);
       launch_knn_rsample(a, st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(3)) return TG_ERR_HIP;
-      pb_reset(a.pc, N, s->fill, st);
       launch_knn_localjoin(a, prec, int(p->tile), st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(4)) return TG_ERR_HIP;
-      pb_group_overflow(a.pc, N, s->fill, s->scan_tmp, st);
+      pb_group_overflow({&a.pc}, N, s->fill, s->scan_tmp, st);
       launch_knn_merge(a, st);
       if (sc.stop()) return TG_ERR_HIP;
       if (int rc = check_launch("GNN-Descent phase 1")) return rc;
@@ -1222,9 +1226,9 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
     if (sc.stop()) return TG_ERR_HIP;
     for (uint32_t it = 0; it < it2; ++it) {
       if (sc.start(6)) return TG_ERR_HIP;
-      pb_reset(a.pr, N, s->fill, st);
+      pb_reset({&a.pr}, N, st);
       launch_knn_phase2(a, prec, st);
-      pb_group_overflow(a.pr, N, s->fill, s->scan_tmp, st);
+      pb_group_overflow({&a.pr}, N, s->fill, s->scan_tmp, st);
       launch_knn_rupdate(a, st);
       if (sc.stop()) return TG_ERR_HIP;
       swap_lists(s);
@@ -1291,12 +1295,11 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
   for (double& v : s->stats.knn_kernel_ms) v = 0.0;
   if (sec.collect(s->stats.knn_kernel_ms)) return TG_ERR_HIP;
   unsigned long long cnt[CNT_N];
-  if (int rc = read_counters(s, cnt)) return rc;
+  const int rs = read_status(s, cnt);
+  if (rs == TG_ERR_HIP) return rs;
   s->stats.knn_evals = cnt[0] + extra_evals;
   s->stats.knn_rescored = cnt[1];
-  if (check_pb_err(s, s->pn, "reverse sampling") || check_pb_err(s, s->po, "reverse sampling") ||
-      check_pb_err(s, s->pc, "local join") || check_pb_err(s, s->pr, "reverse lists"))
-    return TG_ERR_CAPACITY;
+  if (rs) return rs;
   s->has_knn = true;
   s->has_prune = false;
   s->order_valid = use_order;
@@ -1378,7 +1381,7 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   }
   if (!s->cpart && dalloc(&s->cpart, size_t((N + 1023) / 1024) * s->D)) return TG_ERR_HIP;
   if (ensure_common_scratch(s)) return TG_ERR_HIP;
-  if (alloc_pb(s, s->rev, 64, size_t(N) * FD)) return TG_ERR_HIP;
+  if (alloc_pb(s, s->rev, 64, size_t(N) * FD, ERR_REV)) return TG_ERR_HIP;
   hipStream_t st = s->stream;
   PruneArgs a{};
   a.X = s->X;
@@ -1433,11 +1436,10 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   HIPX(hipEventCreate(&win.e1));
   hipEvent_t w0 = win.e0, w1 = win.e1;
   Sections sec{s};
-  fill_u32(reinterpret_cast<uint32_t*>(s->counters), 0, 2 * CNT_SLOTS * CNT_N, st);
+  clear_status(s);
   fill_u32(s->ep_dev, 0, 1, st);
-  clear_errors(s, {&s->rev});
   HIPX(hipEventRecord(w0, st));
-  pb_reset(a.rev, N, s->fill, st);
+  pb_reset({&a.rev}, N, st);
   if (p->kind == TG_KIND_PATH) {
     if (sec.start(0)) return TG_ERR_HIP;
     if (s->nseg) {
@@ -1478,7 +1480,7 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   }
   if (sec.stop()) return TG_ERR_HIP;
   if (sec.start(3)) return TG_ERR_HIP;
-  pb_group_overflow(a.rev, N, s->fill, s->scan_tmp, st);
+  pb_group_overflow({&a.rev}, N, s->fill, s->scan_tmp, st);
   if (sec.stop()) return TG_ERR_HIP;
   if (sec.start(2)) return TG_ERR_HIP;
   launch_prune(a, rank ? PH_RANK_REV : PH_REV, nullptr, nullptr, st);
@@ -1492,7 +1494,8 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   for (double& v : s->stats.prune_kernel_ms) v = 0.0;
   if (sec.collect(s->stats.prune_kernel_ms)) return TG_ERR_HIP;
   unsigned long long cnt[CNT_N];
-  if (int rc = read_counters(s, cnt)) return rc;
+  const int rs = read_status(s, cnt);
+  if (rs == TG_ERR_HIP) return rs;
   for (int i = 0; i < 15; ++i) s->stats.prune_counters[i] = cnt[i];
   if (s->nseg) {
     s->seg_ep_host.resize(s->nseg);
@@ -1504,7 +1507,7 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
   } else {
     HIPX(hipMemcpy(&s->ep, s->ep_dev, 4, hipMemcpyDeviceToHost));
   }
-  if (check_pb_err(s, s->rev, "reverse edges")) return TG_ERR_CAPACITY;
+  if (rs) return rs;
   s->has_prune = true;
   s->last_prune = *p;
   return TG_OK;

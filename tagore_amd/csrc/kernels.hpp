@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 #include "common.hpp"
 
 namespace tg {
@@ -166,9 +168,12 @@ void launch_knn_final(const KnnArgs& a, hipStream_t s);
 
 // ------------------------------------------------------------------------------ utilities
 // push-buffer bookkeeping
-void pb_reset(const PushBuf& pb, uint32_t N, uint32_t* fill, hipStream_t s);
-void pb_group_overflow(const PushBuf& pb, uint32_t N, uint32_t* fill, uint32_t* scan_tmp,
-                       hipStream_t s);
+// (up to three) counters to zero, in one launch
+void pb_reset(std::initializer_list<const PushBuf*> pbs, uint32_t N, hipStream_t s);
+// overflow entries of one or two buffers grouped by destination; fill: 2 N words, scan_tmp:
+// 2 scan_tmp_words(N)
+void pb_group_overflow(std::initializer_list<const PushBuf*> pbs, uint32_t N, uint32_t* fill,
+                       uint32_t* scan_tmp, hipStream_t s);
 size_t scan_tmp_words(uint32_t N);
 // exclusive scan of v[0..n) in place, v[n] = total
 void excl_scan_u32(uint32_t* v, uint32_t n, uint32_t* tmp, hipStream_t s);

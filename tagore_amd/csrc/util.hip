@@ -30,7 +30,6 @@ void fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------------------ scans
-// Exclusive scan of c[v] = max(0, cnt[v] - cap) into off[0..N]; off[N] = total.
 constexpr int SCAN_BLOCK = 1024;  // elements per block (256 threads x 4)
 
 __device__ int block_excl_scan_256(int v, int* sh) {
@@ -49,42 +48,43 @@ __device__ int block_excl_scan_256(int v, int* sh) {
   return incl - v;
 }
 
-__global__ void k_scan1(const uint32_t* cnt, uint32_t cap, uint32_t N, uint32_t* off,
-                        uint32_t* bsum) {
+__global__ void k_scan1(uint32_t* x, uint32_t N, uint32_t* bsum) {
   __shared__ int sh[256];
   const size_t base = size_t(blockIdx.x) * SCAN_BLOCK + threadIdx.x * 4;
   int v[4], tot = 0;
   for (int q = 0; q < 4; ++q) {
     const size_t i = base + q;
-    const uint32_t c = i < N ? cnt[i] : 0;
-    v[q] = c > cap ? int(c - cap) : 0;
+    v[q] = i < N ? int(x[i]) : 0;
     tot += v[q];
   }
   int ex = block_excl_scan_256(tot, sh);
   for (int q = 0; q < 4; ++q) {
     const size_t i = base + q;
-    if (i < N) off[i] = ex;
+    if (i < N) x[i] = ex;
     ex += v[q];
   }
   if (threadIdx.x == 255) bsum[blockIdx.x] = ex;
 }
 
-__global__ void k_scan2(uint32_t* bsum, uint32_t nb, uint32_t* off, uint32_t N) {
+// exclusive scan of the nb block sums in place by one 256-thread workgroup; off[N] = total
+__device__ __forceinline__ void scan_sums(uint32_t* bsum, uint32_t nb, uint32_t* off, uint32_t N) {
   __shared__ int sh[256];
+  __shared__ int tot;
   int carry = 0;
   for (uint32_t base = 0; base < nb; base += 256) {
     const uint32_t i = base + threadIdx.x;
     const int v = i < nb ? int(bsum[i]) : 0;
     const int ex = block_excl_scan_256(v, sh);
     if (i < nb) bsum[i] = carry + ex;
-    // total of this chunk
-    __shared__ int tot;
-    if (threadIdx.x == 255) tot = ex + v;
+    if (threadIdx.x == 255) tot = ex + v;  // total of this chunk
     __syncthreads();
     carry += tot;
     __syncthreads();
   }
   if (threadIdx.x == 0) off[N] = carry;
+}
+__global__ void k_scan2(uint32_t* bsum, uint32_t nb, uint32_t* off, uint32_t N) {
+  scan_sums(bsum, nb, off, N);
 }
 
 __global__ void k_scan3(uint32_t* off, const uint32_t* bsum, uint32_t N) {
@@ -100,14 +100,117 @@ size_t scan_tmp_words(uint32_t N) { return (size_t(N) + SCAN_BLOCK - 1) / SCAN_B
 
 void excl_scan_u32(uint32_t* v, uint32_t n, uint32_t* tmp, hipStream_t s) {
   const uint32_t nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
-  k_scan1<<<nb, 256, 0, s>>>(v, 0, n, v, tmp);  // each thread reads its elements before writing
+  k_scan1<<<nb, 256, 0, s>>>(v, n, tmp);
   k_scan2<<<1, 256, 0, s>>>(tmp, nb, v, n);
   k_scan3<<<nb, 256, 0, s>>>(v, tmp, n);
 }
 
-__global__ void k_ov_scatter(PushBuf pb, uint32_t* fill) {
-  const uint32_t used = min(*pb.ov_used, pb.ov_cap);
-  for (uint32_t o = blockIdx.x * blockDim.x + threadIdx.x; o < used; o += gridDim.x * blockDim.x) {
+// ------------------------------------------------------------------- push-buffer grouping
+// One or two push buffers in the same launches (blockIdx.y).  fill: [N] words per buffer,
+// zeroed by the scan; tmp: block sums.
+struct GroupArgs {
+  PushBuf pb[2];
+  uint32_t* fill[2];
+  uint32_t* tmp[2];
+};
+
+// whether any overflow entry was taken (a wave-uniform answer, in every wave)
+__device__ __forceinline__ bool pb_overflowed(const PushBuf& pb) {
+  static_assert(OV_AREAS == TG_WAVE, "one counter per lane");
+  return __ballot(pb.ov_used[lane_id() * OV_STRIDE] != 0) != 0;
+}
+
+struct ResetArgs {
+  uint32_t* cnt[3];
+  uint32_t* used[3];
+};
+__global__ __launch_bounds__(256) void k_pb_reset(ResetArgs r, uint32_t n, uint32_t N) {
+  const uint32_t stride = gridDim.x * 256;
+  for (uint32_t b = 0; b < n; ++b) {
+    for (uint64_t i = blockIdx.x * 256 + threadIdx.x; i < N; i += stride) r.cnt[b][i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < OV_AREAS) r.used[b][threadIdx.x * OV_STRIDE] = 0;
+  }
+}
+void pb_reset(std::initializer_list<const PushBuf*> pbs, uint32_t N, hipStream_t s) {
+  ResetArgs r{};
+  uint32_t n = 0;
+  for (const PushBuf* pb : pbs) {
+    r.cnt[n] = pb->cnt;
+    r.used[n++] = pb->ov_used;
+  }
+  k_pb_reset<<<grid_for(N), 256, 0, s>>>(r, n, N);
+}
+
+// Small N: the offsets in one launch of one workgroup per buffer, each thread a run of counts.
+constexpr uint32_t GROUP_ONE_MAX = 32768;
+__global__ __launch_bounds__(1024) void k_group_one(GroupArgs g, uint32_t N) {
+  __shared__ uint32_t wsum[16];
+  const PushBuf& pb = g.pb[blockIdx.y];
+  if (!pb_overflowed(pb)) return;
+  uint32_t* fill = g.fill[blockIdx.y];
+  const uint32_t per = (N + 1023) / 1024, i0 = min(N, threadIdx.x * per), i1 = min(N, i0 + per);
+  uint32_t own = 0;
+  for (uint32_t i = i0; i < i1; ++i) {
+    const uint32_t c = pb.cnt[i];
+    own += c > pb.cap ? c - pb.cap : 0u;
+  }
+  const uint32_t incl = uint32_t(wave_incl_scan(int(own)));
+  const int w = threadIdx.x / TG_WAVE;
+  if (lane_id() == TG_WAVE - 1) wsum[w] = incl;
+  __syncthreads();
+  uint32_t run = incl - own;
+  for (int q = 0; q < w; ++q) run += wsum[q];
+  for (uint32_t i = i0; i < i1; ++i) {
+    const uint32_t c = pb.cnt[i];
+    pb.ov_off[i] = run;
+    fill[i] = 0;
+    run += c > pb.cap ? c - pb.cap : 0u;
+  }
+  if (threadIdx.x == 1023) pb.ov_off[N] = run;
+}
+
+__global__ __launch_bounds__(256) void k_group_scan1(GroupArgs g, uint32_t N) {
+  __shared__ int sh[256];
+  const PushBuf& pb = g.pb[blockIdx.y];
+  if (!pb_overflowed(pb)) return;
+  uint32_t* fill = g.fill[blockIdx.y];
+  const size_t base = size_t(blockIdx.x) * SCAN_BLOCK + threadIdx.x * 4;
+  int v[4], tot = 0;
+  for (int q = 0; q < 4; ++q) {
+    const size_t i = base + q;
+    const uint32_t c = i < N ? pb.cnt[i] : 0;
+    v[q] = c > pb.cap ? int(c - pb.cap) : 0;
+    tot += v[q];
+    if (i < N) fill[i] = 0;
+  }
+  int ex = block_excl_scan_256(tot, sh);
+  for (int q = 0; q < 4; ++q) {
+    const size_t i = base + q;
+    if (i < N) pb.ov_off[i] = ex;
+    ex += v[q];
+  }
+  if (threadIdx.x == 255) g.tmp[blockIdx.y][blockIdx.x] = ex;
+}
+__global__ __launch_bounds__(256) void k_group_scan2(GroupArgs g, uint32_t nb, uint32_t N) {
+  const PushBuf& pb = g.pb[blockIdx.y];
+  if (pb_overflowed(pb)) scan_sums(g.tmp[blockIdx.y], nb, pb.ov_off, N);
+}
+__global__ __launch_bounds__(256) void k_group_scan3(GroupArgs g, uint32_t N) {
+  const PushBuf& pb = g.pb[blockIdx.y];
+  if (!pb_overflowed(pb)) return;
+  const size_t base = size_t(blockIdx.x) * SCAN_BLOCK + threadIdx.x * 4;
+  const uint32_t add = g.tmp[blockIdx.y][blockIdx.x];
+  for (int q = 0; q < 4; ++q)
+    if (base + q < N) pb.ov_off[base + q] += add;
+}
+// area a's entries by the workgroups a, a + OV_AREAS, ..
+__global__ __launch_bounds__(256) void k_ov_scatter(GroupArgs g) {
+  const PushBuf& pb = g.pb[blockIdx.y];
+  uint32_t* fill = g.fill[blockIdx.y];
+  const uint32_t area = blockIdx.x % OV_AREAS, per = gridDim.x / OV_AREAS;
+  const uint32_t used = min(pb.ov_used[area * OV_STRIDE], pb.ov_area);
+  for (uint64_t i = (blockIdx.x / OV_AREAS) * 256 + threadIdx.x; i < used; i += per * 256) {
+    const size_t o = size_t(area) * pb.ov_area + i;
     const uint32_t v = pb.ov_dest[o];
     const uint32_t dst = pb.ov_off[v] + atomicAdd(&fill[v], 1u);
     // the grouped offsets count every overflowing push; when the overflow area itself was
@@ -116,26 +219,27 @@ __global__ void k_ov_scatter(PushBuf pb, uint32_t* fill) {
   }
 }
 
-__global__ void k_pb_reset_small(PushBuf pb) {
-  if (threadIdx.x == 0) {
-    *pb.ov_used = 0;
+void pb_group_overflow(std::initializer_list<const PushBuf*> pbs, uint32_t N, uint32_t* fill,
+                       uint32_t* scan_tmp, hipStream_t s) {
+  GroupArgs g{};
+  uint32_t n = 0;
+  for (const PushBuf* pb : pbs) {
+    g.pb[n] = *pb;
+    g.fill[n] = fill + size_t(n) * N;
+    g.tmp[n] = scan_tmp + n * scan_tmp_words(N);
+    ++n;
   }
-}
-
-void pb_reset(const PushBuf& pb, uint32_t N, uint32_t* fill, hipStream_t s) {
-  fill_u32(pb.cnt, 0, N, s);
-  fill_u32(fill, 0, N, s);
-  k_pb_reset_small<<<1, 64, 0, s>>>(pb);
-}
-
-void pb_group_overflow(const PushBuf& pb, uint32_t N, uint32_t* fill, uint32_t* scan_tmp,
-                       hipStream_t s) {
+  if (N <= GROUP_ONE_MAX) {
+    k_group_one<<<dim3(1, n), 1024, 0, s>>>(g, N);
+    k_ov_scatter<<<dim3(OV_AREAS, n), 256, 0, s>>>(g);
+    return;
+  }
   const uint32_t nb = (N + SCAN_BLOCK - 1) / SCAN_BLOCK;
-  k_scan1<<<nb, 256, 0, s>>>(pb.cnt, pb.cap, N, pb.ov_off, scan_tmp);
-  k_scan2<<<1, 256, 0, s>>>(scan_tmp, nb, pb.ov_off, N);
-  k_scan3<<<nb, 256, 0, s>>>(pb.ov_off, scan_tmp, N);
-  // a grid-stride loop of returning atomics: 8 workgroups per CU keep enough waves in flight
-  k_ov_scatter<<<2048, 256, 0, s>>>(pb, fill);
+  k_group_scan1<<<dim3(nb, n), 256, 0, s>>>(g, N);
+  k_group_scan2<<<dim3(1, n), 256, 0, s>>>(g, nb, N);
+  k_group_scan3<<<dim3(nb, n), 256, 0, s>>>(g, N);
+  // a strided loop of returning atomics: 8 workgroups per CU keep enough waves in flight
+  k_ov_scatter<<<dim3(2048, n), 256, 0, s>>>(g);
 }
 
 // ---------------------------------------------------------------------- synthetic data

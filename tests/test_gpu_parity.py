@@ -500,3 +500,24 @@ def test_block_filter_edges(name, D):
                                  (1, 1, 1, 16, 0.5), (1, 0, 0, 33, 1.05), (0, 1, 0, 128, -0.2),
                                  (0, 0, 0, 40, 3.0)]:
         _compare(X, G, GD, kind, fr, rr, FD, 64, th)
+
+
+@pytest.mark.parametrize("N,D,K", [(34, 32, 33), (48, 32, 40), (70, 64, 64), (130, 32, 100),
+                                   (32768, 32, 8), (32769, 32, 8), (50000, 32, 6)])
+def test_overflow_areas_and_grouping(N, D, K):
+    """Push lists beyond their slots: few nodes, whose workgroups fill their own overflow areas
+    and go on in others', and a hub in every list around the size where the grouping takes
+    one workgroup.  Graphs and the NSG prune equal to the oracle."""
+    rng = np.random.default_rng(N)
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    X[N // 2] = 0.01 * X[N // 2]  # nearest to everything
+    for prec in ("exact", "bf16"):
+        _say(f"overflow N={N} K={K} {prec}")
+        Gr, GDr, ev = oracle.gnn_descent(X, K, 6, 5)
+        with State(N, D) as s:
+            s.set_data(X)
+            s.knn_build(K, 6, 5, prec)
+            G, GD = s.get_knn()
+            assert s.stats()["knn_evals"] == ev
+        assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
+    _compare(X, Gr, GDr, 0, 0, 0, min(K, 24), 32, 1.2)
