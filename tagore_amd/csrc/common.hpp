@@ -785,14 +785,15 @@ __device__ __forceinline__ int lower_bound_lds(const T* a, int n, T x) {
 // canonical distances, so a listed id always appears under exactly this key.
 __device__ __forceinline__ bool row_has_key(const uint32_t* G, const float* GD, int K, uint32_t v,
                                             uint64_t key) {
-  const uint32_t* g = G + size_t(v) * K;
   const float* gd = GD + size_t(v) * K;
   int lo = 0, hi = K;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
-    if (mk_key(gd[mid], g[mid]) < key) lo = mid + 1; else hi = mid;
+    if (gd[mid] < key_d(key)) lo = mid + 1; else hi = mid;
   }
-  return lo < K && mk_key(gd[lo], g[lo]) == key;
+  for (; lo < K && gd[lo] == key_d(key); ++lo)
+    if (G[size_t(v) * K + lo] == key_id(key)) return true;
+  return false;
 }
 
 template <class T>

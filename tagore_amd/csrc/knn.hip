@@ -838,7 +838,7 @@ __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
   // (the keys are cleared again after the compaction).
   int nre = cnt;
   bool done = false;
-  if constexpr (PREC == KP_BF16 && MC <= 4) {
+  if constexpr ((PREC == KP_BF16 || PREC == KP_EXACT) && MC <= 4) {  // (X8: not in exact mode)
     if (a.exact_screen && a.X8) {
       // integer data in [0, 255] (D <= 256): exact distances from the u8 copy (quad layout,
       // 32 candidates per step), the canonical distances themselves

@@ -224,13 +224,13 @@ void launch_screen_copy(const float* X, uint32_t N, uint32_t D, bool half, float
   else k_screen_copy<false><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags);
 }
 
-// Local join when the screen distances are the canonical distances (integer data, FP32 or
-// BF16 products): each job's answer is the (s, id) minimum of its 16-wide tile, taken from
-// the accumulators by cross-lane minima instead of distance matrices in LDS, so the kernel
-// holds only the staging area (and runs more workgroups per CU).  Jobs, as in the screened
-// kernel: A rows x B tiles, B columns x A tiles, A rows x A tiles.  Lane t of group g owns
-// row job (row 16w + 4g + (t & 3), tile t >> 2) of both row kinds, and lane l owns column
-// job (column l, tile w).
+// Local join when the screen distances are the canonical distances (integer data): each job's
+// answer is the (s, id) minimum of its 16-wide tile, taken from the accumulators by cross-lane
+// minima, so the kernel holds only the staging area (and runs more workgroups per CU).  Jobs:
+// A rows x B tiles, B columns x A tiles, A rows x A tiles.  Only blocks that hold pairs are
+// formed (an iteration from fresh lists has no B), shared evenly by the waves.
+// 1M x 128 u8 rows, K = 96, one iteration: 8.7 -> 6.7 ms; 10k x 128, K = 32 with precision FP32
+// (u8 products are as exact): 264 -> 62 us per iteration.
 // (d, id) minimum over the lanes l ^ x for the masks x in [x0, x1) (powers of two): the
 // smallest d, then the smallest id among the lanes holding it.  The exact screen's distances
 // are integers >= 0 or +inf, whose FP32 bits order as unsigned integers, so both minima are
@@ -269,77 +269,120 @@ __device__ __forceinline__ uint64_t key_min_row16(float d, uint32_t id) {
 }
 
 // Membership of Q keys in kNN rows (rows sorted by (distance, id), canonical distances):
-// found[q] = key[q] is an entry of row v[q], for the searches with on[q].  The binary
-// searches run in lockstep, so the dependent loads of one step are in flight together.
+// found[q] = key[q] is an entry of row v[q], for the searches with on[q].  The binary searches
+// run on the distances alone -- one load per step; the ids are read where a distance is equal
+// -- and in lockstep, so the dependent loads of one step are in flight together.  (Every lane
+// searches a row of its own, so each load is an L2 request of its own: their number sets the
+// push phase's time.)
 template <int Q>
 __device__ __forceinline__ void rows_have_keys(const uint32_t* G, const float* GD, int K,
                                                const uint32_t (&v)[Q], const uint64_t (&key)[Q],
                                                const bool (&on)[Q], bool (&found)[Q]) {
   int lo[Q], hi[Q];
+  const float* row[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     lo[q] = 0;
     hi[q] = on[q] ? K : 0;
+    row[q] = GD + size_t(v[q]) * K;
+    found[q] = false;
   }
+  // lower bound of the distance
   for (;;) {
     bool any = false;
 #pragma unroll
     for (int q = 0; q < Q; ++q) any = any || lo[q] < hi[q];
     if (!any) break;
-    uint64_t kk[Q];
+    float x[Q];
     int mid[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       mid[q] = (lo[q] + hi[q]) >> 1;
-      kk[q] = lo[q] < hi[q] ? mk_key(GD[size_t(v[q]) * K + mid[q]], G[size_t(v[q]) * K + mid[q]])
-                            : 0ull;
+      x[q] = lo[q] < hi[q] ? row[q][mid[q]] : 0.f;
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       if (lo[q] < hi[q]) {
-        if (kk[q] < key[q]) lo[q] = mid[q] + 1;
+        if (x[q] < key_d(key[q])) lo[q] = mid[q] + 1;
         else hi[q] = mid[q];
       }
     }
   }
+  // the entries of that distance
 #pragma unroll
-  for (int q = 0; q < Q; ++q)
-    found[q] = on[q] && lo[q] < K &&
-               mk_key(GD[size_t(v[q]) * K + lo[q]], G[size_t(v[q]) * K + lo[q]]) == key[q];
+  for (int q = 0; q < Q; ++q) {
+    if (!on[q]) continue;
+    for (int p = lo[q]; p < K && row[q][p] == key_d(key[q]); ++p)
+      if (G[size_t(v[q]) * K + p] == key_id(key[q])) {
+        found[q] = true;
+        break;
+      }
+  }
 }
 
-// Column block c of an exact screen (wave w, lane l = 16g + t): accB holds A rows
-// 16w + 4g + r against B row 16c + t, accA the same A rows against A row 16c + t, as exact
-// products with s = (na[i] + na[j]) - 2 acc.  Folds the block into the row jobs' minima
-// (row_b / row_a: the lane t == 4c + r owns job (16w + 4g + r, c)) and into this lane's
-// column job of the block (col_b: the minimum over the wave's 16 A rows, held by g == c).
-__device__ __forceinline__ void lj_block_minima(int c, const f32x4& accB, const f32x4& accA,
-                                                const uint32_t* A, const uint32_t* B,
-                                                const float* naA, const float* naB, int nA,
-                                                int nB, int w, int g, int t, uint64_t& row_b,
-                                                uint64_t& row_a, uint64_t& col_b) {
+// The 16 x 16 blocks of a node's pairs, A x B and -- A x A being symmetric -- A x A on and above
+// the diagonal, dealt to the four waves: block b of wave w is number w + 4b (NBLK of 26 at
+// most).  Lane x holds block x's first candidate (an index into ids: B tiles from 64 on) and
+// first row << 8, LJ_NONE past the last one; a wave reads its blocks' lanes.  (Scalar loops
+// over the tiles for each block issued more instructions than everything else.)
+constexpr int NBLK = 7;
+constexpr int LJ_NONE = 0xFFFF;
+__device__ __forceinline__ int lj_blocks(int RA, int RB) {
+  const int x = lane_id();
+  if (x < RA * RB) {
+    const int rb = (x >= RB ? 1 : 0) + (x >= 2 * RB ? 1 : 0) + (x >= 3 * RB ? 1 : 0);
+    return (16 * rb) << 8 | (64 + 16 * (x - rb * RB));
+  }
+  const int y = x - RA * RB;
+  if (y >= RA * (RA + 1) / 2) return LJ_NONE;
+  // row tile rb starts at number rb RA - rb (rb - 1) / 2
+  const int rb = (y >= RA ? 1 : 0) + (y >= 2 * RA - 1 ? 1 : 0) + (RA > 1 && y >= 3 * RA - 3 ? 1 : 0);
+  return (16 * rb) << 8 | 16 * (rb + y - (rb * RA - rb * (rb - 1) / 2));
+}
+
+// The jobs of a block of exact distances (s = (n_i + n_j) - 2 acc): the (d, id) minimum of every
+// row over the 16 candidates, and of every candidate over the 16 rows.  kb: [64 rows of A][4
+// tiles of B], ka: [64 rows of A][4 tiles of A], kc: [4 tiles of A][64 rows of B]; every job is
+// one block's, so its key is stored, not merged.  Lane t of group g stores row 4g + t (t < 4),
+// group 0 the candidates.
+__device__ __forceinline__ void lj_block_minima(int bi, int bj, const f32x4& acc,
+                                                const uint32_t* ids, const float* nn, int nA,
+                                                int nB, uint64_t* kb, uint64_t* ka,
+                                                uint64_t* kc) {
+  const int l = threadIdx.x & 63, g = l >> 4, t = l & 15;
   const float INF = __uint_as_float(0x7F800000u);
-  const int j = 16 * c + t;
-  float cd = INF;  // column job: this lane's 4 rows, then across the groups
+  const int i0 = bi + 4 * g, jj = bj + t;
+  const bool bt = bj >= 64;
+  const bool jn = bt ? jj - 64 < nB : jj < nA;
+  const float nj = nn[jj];
+  const uint32_t idj = ids[jj];
+  const float4 ni = *reinterpret_cast<const float4*>(nn + i0);
+  const uint4 idi = *reinterpret_cast<const uint4*>(ids + i0);
+  const float nv[4] = {ni.x, ni.y, ni.z, ni.w};
+  const uint32_t iv[4] = {idi.x, idi.y, idi.z, idi.w};
+  float cd = INF;  // the candidate's minimum: this lane's 4 rows, then across the groups
   uint32_t cid = 0xFFFFFFFFu;
+  uint64_t mine = TG_KEY_INF;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int i = 16 * w + 4 * g + r;
-    const float sb = (i < nA && j < nB && A[i] != B[j]) ? (naA[i] + naB[j]) - 2.0f * accB[r] : INF;
-    const float sa = (i < nA && j < nA && i != j) ? (naA[i] + naA[j]) - 2.0f * accA[r] : INF;
-    const uint64_t kb = key_min_row16(sb, B[j]);
-    const uint64_t ka = key_min_row16(sa, A[j]);
-    if (t == 4 * c + r) {
-      row_b = kb;
-      row_a = ka;
-    }
-    if (sb < cd || (sb == cd && A[i] < cid)) {
-      cd = sb;
-      cid = A[i];
+    const bool ok = i0 + r < nA && jn && (bt ? iv[r] != idj : i0 + r != jj);
+    const float d = ok ? (nv[r] + nj) - 2.0f * acc[r] : INF;
+    const uint64_t k = key_min_row16(d, idj);
+    if (t == r) mine = k;
+    if (d < cd || (d == cd && iv[r] < cid)) {
+      cd = d;
+      cid = iv[r];
     }
   }
-  const uint64_t kc = key_min_lanes<16, 64>(cd, cid);
-  if (g == c) col_b = kc;
+  // a tile of invalid pairs keeps +inf distances, which no worst distance admits
+  if (t < 4) (bt ? kb : ka)[4 * (i0 + t) + ((bt ? bj - 64 : bj) >> 4)] = mine;
+  if (bi != bj) {
+    const uint64_t kj = key_min_lanes<16, 64>(cd, cid);
+    if (g == 0) {
+      if (bt) kc[64 * (bi >> 4) + (jj - 64)] = kj;
+      else ka[4 * jj + (bi >> 4)] = kj;
+    }
+  }
 }
 
 // The jobs' pushes: a job's minimum enters when it beats the destination's worst entry and
@@ -418,40 +461,100 @@ __device__ __forceinline__ void lj_lists(const KnnArgs& a, uint32_t u, const flo
   }
 }
 
+// Products of the exact kernels.  PREC 0: u8 data on int8 MFMA (every value an integer in
+// [0, 255], D <= DC <= 256): rows, stored as x - 128, are staged whole and
+// v_mfma_i32_16x16x64_i8 gives a'.b' exactly, so s = |a'|^2 + |b'|^2 - 2 a'.b' = |a - b|^2
+// exactly (|a'|^2 from n2s), the canonical distance of this data.  PREC 1 / 2: FP32 / BF16
+// MFMA, exact for integers too (values in [-256, 256]).
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 template <int PREC, int DC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PREC == 0 && DC == 128 ? 8 : 4)))
 void k_localjoin_exact_screen(KnnArgs a) {
-  static_assert(PREC == 1 || PREC == 2, "exact screens are FP32 or BF16 products");
-  using St = ScreenStage<PREC, DC, 128>;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[St::BYTES];
-  __shared__ uint32_t ids[128];
-  __shared__ float naA[64], wA[64], naB[64], wB[64];
+  static_assert(PREC <= 2, "u8, FP32 or BF16 products");
+  using St = ScreenStage<(PREC == 0 ? 3 : PREC), DC, 128>;
+  constexpr int RS = St::RS;
+  constexpr int KEYS = 3 * 256 * 8;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[St::BYTES > KEYS ? St::BYTES : KEYS];
+  __shared__ __attribute__((aligned(16))) uint32_t ids[128];
+  __shared__ __attribute__((aligned(16))) float nn[128];
+  __shared__ float wd[128];
   const uint32_t u = row_of_block(a.perm, a.N);
   if (u >= a.N) return;
-  uint32_t *A = ids, *B = ids + 64;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, t = l & 15;
+  const int tid = threadIdx.x, l = tid & 63, g = l >> 4, t = l & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int D = a.D;
   const int nA = a.na[u], nB = a.nb[u];
-  lj_lists(a, u, a.nrm2, nA, nB, A, B, naA, wA, naB, wB);
+  lj_lists(a, u, PREC == 0 ? a.n2s : a.nrm2, nA, nB, ids, ids + 64, nn, wd, nn + 64, wd + 64);
   __syncthreads();
-  f32x4 accB[4], accA[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) accB[c] = accA[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  screen_chunks<PREC, DC, 128>(
-      PREC == 2 ? static_cast<const void*>(a.Xb) : a.X, ids, a.D,
-      [&](int r) { return r < 64 ? r < nA : r - 64 < nB; }, smem, [&]() {
-        const unsigned char* pa = smem + 16 * w * St::RS;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          screen_block<PREC, true, DC>(pa, smem + (64 + 16 * c) * St::RS, l, accB[c]);
-          screen_block<PREC, true, DC>(pa, smem + 16 * c * St::RS, l, accA[c]);
+  const int blocks = lj_blocks((nA + 15) >> 4, (nB + 15) >> 4);
+  f32x4 acc[NBLK];
+  if constexpr (PREC == 0) {
+    // rows of both lists, up to whole tiles: bytes past D and rows past the list ends are 0
+    constexpr int CPR = DC / 16;
+    for (int e = tid; e < 2 * 64 * CPR; e += 256) {
+      const int r = e / CPR, col = (e % CPR) * 16;
+      const int n = r < 64 ? nA : nB, x = r & 63;
+      if (x >= ((n + 15) & ~15)) continue;
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (x < n && col < D) {
+        const uint8_t* src = a.X8 + size_t(ids[r]) * D + col;
+        if ((D & 15) == 0) {
+          v = *reinterpret_cast<const uint4*>(src);
+        } else {
+          v.x = *reinterpret_cast<const uint32_t*>(src);
+          if (col + 4 < D) v.y = *reinterpret_cast<const uint32_t*>(src + 4);
+          if (col + 8 < D) v.z = *reinterpret_cast<const uint32_t*>(src + 8);
+          if (col + 12 < D) v.w = *reinterpret_cast<const uint32_t*>(src + 12);
         }
-      });
-  uint64_t row_b = TG_KEY_INF, row_a = TG_KEY_INF, col_b = TG_KEY_INF;
+      }
+      *reinterpret_cast<uint4*>(smem + r * RS + col) = v;
+    }
+    __syncthreads();
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-    lj_block_minima(c, accB[c], accA[c], A, B, naA, naB, nA, nB, w, g, t, row_b, row_a, col_b);
-  lj_push(a, A, B, wA, wB, nA, nB, w, g, t, l, row_b, row_a, col_b,
-          reinterpret_cast<uint64_t*>(smem));
+    for (int b = 0; b < NBLK; ++b) {
+      const int d = __builtin_amdgcn_readlane(blocks, w + 4 * b);
+      if (d == LJ_NONE) continue;
+      const int bi = d >> 8, bj = d & 255;
+      i32x4 p = {0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < DC / 64; ++k)
+        p = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+            *reinterpret_cast<const i32x4*>(smem + (bi + t) * RS + 64 * k + 16 * g),
+            *reinterpret_cast<const i32x4*>(smem + (bj + t) * RS + 64 * k + 16 * g), p, 0, 0, 0);
+      acc[b] = f32x4{float(p[0]), float(p[1]), float(p[2]), float(p[3])};
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int b = 0; b < NBLK; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    screen_chunks<PREC, DC, 128>(
+        PREC == 2 ? static_cast<const void*>(a.Xb) : a.X, ids, D,
+        [&](int r) { return r < 64 ? r < nA : r - 64 < nB; }, smem, [&]() {
+#pragma unroll
+          for (int b = 0; b < NBLK; ++b) {
+            const int d = __builtin_amdgcn_readlane(blocks, w + 4 * b);
+            if (d != LJ_NONE)
+              screen_block<PREC, true, DC>(smem + (d >> 8) * RS, smem + (d & 255) * RS, l, acc[b]);
+          }
+        });
+  }
+  // the jobs' keys, in the staging area (free from here on)
+  uint64_t* kb = reinterpret_cast<uint64_t*>(smem);
+  uint64_t* ka = kb + 256;
+  uint64_t* kc = ka + 256;
+  kb[tid] = TG_KEY_INF;
+  ka[tid] = TG_KEY_INF;
+  kc[tid] = TG_KEY_INF;
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < NBLK; ++b) {
+    const int d = __builtin_amdgcn_readlane(blocks, w + 4 * b);
+    if (d != LJ_NONE) lj_block_minima(d >> 8, d & 255, acc[b], ids, nn, nA, nB, kb, ka, kc);
+  }
+  __syncthreads();
+  const int ir = 16 * w + 4 * g + (t & 3), tile = t >> 2;  // this lane's row jobs (lj_push)
+  const uint64_t row_b = kb[4 * ir + tile], row_a = ka[4 * ir + tile], col_b = kc[64 * w + l];
+  lj_push(a, ids, ids + 64, wd, wd + 64, nA, nB, w, g, t, l, row_b, row_a, col_b, kc);
   if (a.counters && tid == 0)
     atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
 }
@@ -471,9 +574,9 @@ void k_localjoin_exact_screen(KnnArgs a) {
 //     have just been read (L2);
 //   * wider rows: 64 elements of every queued row at a time through LDS, 16 pairs per group
 //     with their partial sums in registers -- a row is read once more, not once per pair.
-// Two iterations of 500k x 96 (K = 64, learned lists, 150 re-scores per node): 48.5 -> 17.0 ms;
-// eight of 160k x 96 clusters from random lists 46 -> 15.4 ms; two of 100k x 960 (170 re-scores
-// per node) 48 -> 15.1 ms.  Before, one BF16 product left a bound eight times wider, one of the
+// Two iterations of 500k x 96 (K = 64, learned lists, 150 re-scores per node): 48.5 -> 13.0 ms;
+// eight of 160k x 96 clusters from random lists 46 -> 12.8 ms; two of 100k x 960 (170 re-scores
+// per node) 48 -> 16.1 ms.  Before, one BF16 product left a bound eight times wider, one of the
 // four waves formed the masks, and each re-score read both rows from L2.  What is left: half
 // of the narrow kernel's cycles issue VALU work, the rest waits on the list, row and push
 // round trips; the wide one streams each sampled row twice.
@@ -484,7 +587,6 @@ void k_localjoin_screen(KnnArgs a) {
   using St = ScreenStage<PREC, DC, 128>;
   constexpr bool BF = std::is_same<T, uint16_t>::value;
   constexpr int QCAP = 1024;  // pairs queued per pass (one pass, but for degenerate data)
-  constexpr int NBLK = 7;     // blocks per wave: (16 + 10) / 4, rounded up
   constexpr bool WIDE = MC > 4;
   constexpr int KEYS = 3 * 256 * 8, QBYTES = QCAP * 2;
   constexpr int WRS = 64 * int(sizeof(T)) + 16;  // staged row of the wide re-scores
@@ -511,34 +613,14 @@ void k_localjoin_screen(KnnArgs a) {
     sc[tid] = in ? a.sc8[v] : 0.f;
   }
   __syncthreads();
-  // ---- this wave's blocks w, w + 4, ..: bi[b] = first row (of A), bj[b] = first candidate
-  // (index into ids: B tiles from 64 on), -1: none
-  const int RA = (nA + 15) >> 4, RB = (nB + 15) >> 4;
+  // ---- this wave's blocks
+  const int blocks = lj_blocks((nA + 15) >> 4, (nB + 15) >> 4);
   int bi[NBLK], bj[NBLK];
 #pragma unroll
   for (int b = 0; b < NBLK; ++b) {
-    int x = w + 4 * b;
-    bi[b] = bj[b] = -1;
-    if (x < RA * RB) {
-      int rb = 0;
-      while (x >= RB) {
-        x -= RB;
-        ++rb;
-      }
-      bi[b] = 16 * rb;
-      bj[b] = 64 + 16 * x;
-    } else {
-      x -= RA * RB;
-      int rb = 0;
-      while (rb < RA && x >= RA - rb) {
-        x -= RA - rb;
-        ++rb;
-      }
-      if (rb < RA) {
-        bi[b] = 16 * rb;
-        bj[b] = 16 * (rb + x);
-      }
-    }
+    const int d = __builtin_amdgcn_readlane(blocks, w + 4 * b);
+    bi[b] = d == LJ_NONE ? -1 : d >> 8;
+    bj[b] = d & 255;
   }
   f32x4 acc[NBLK];
 #pragma unroll
@@ -644,31 +726,13 @@ void k_localjoin_screen(KnnArgs a) {
     const int n = min(total - q0, QCAP);
     uint32_t m = want;
     int pos = first - q0;
-    while (m) {
-      const int p = __ffs(m) - 1;
+    while (ballot(m != 0) != 0) {
+      const int p = m ? __ffs(m) - 1 : 0;
+      const int d = __shfl(blocks, w + (p & ~3), TG_WAVE);  // block of element p
+      if (m && pos >= 0 && pos < QCAP)
+        queue[pos] = uint16_t(((d >> 8) + 4 * g + (p & 3)) << 7 | ((d & 255) + t));
+      pos += m ? 1 : 0;
       m &= m - 1;
-      if (pos >= 0 && pos < QCAP) {
-        // block of element p: its first row and candidate
-        int x = w + (p >> 2) * 4, fi, fj;
-        if (x < RA * RB) {
-          fi = 0;
-          while (x >= RB) {
-            x -= RB;
-            ++fi;
-          }
-          fj = 64 + 16 * x;
-        } else {
-          x -= RA * RB;
-          fi = 0;
-          while (x >= RA - fi) {
-            x -= RA - fi;
-            ++fi;
-          }
-          fj = 16 * (fi + x);
-        }
-        queue[pos] = uint16_t((16 * fi + 4 * g + (p & 3)) << 7 | (fj + t));
-      }
-      ++pos;
     }
     __syncthreads();
     const int gg = tid >> 4;
@@ -757,90 +821,19 @@ void k_localjoin_screen(KnnArgs a) {
   }
 }
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// Exact screen on int8 MFMA for u8 data (every value an integer in [0, 255], D <= DC <= 256):
-// rows (stored as x - 128, a signed int8) are staged whole, and
-// v_mfma_i32_16x16x64_i8 gives a'.b' exactly, so s = |a'|^2 + |b'|^2 - 2 a'.b' = |a - b|^2
-// exactly (|a'|^2 from n2s): the canonical distance of this data, as in the BF16 exact
-// screen.  Half the staged bytes and MFMA instructions of the BF16 rows; the column blocks
-// are formed and folded one at a time, so only two accumulators are live.
-template <int DC>
-__global__ __launch_bounds__(256) void k_localjoin_u8_screen(KnnArgs a) {
-  constexpr int RS = DC + 16;  // padded LDS row stride in bytes
-  constexpr int CPR = DC / 16;  // 16-byte pieces per staged row
-  constexpr int KQ = DC / 64;   // MFMA K-steps
-  __shared__ __attribute__((aligned(16))) unsigned char sA[64 * RS], sB[64 * RS];
-  __shared__ uint32_t A[64], B[64];
-  __shared__ float naA[64], wA[64], naB[64], wB[64];
-  const uint32_t u = row_of_block(a.perm, a.N);
-  if (u >= a.N) return;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, t = l & 15;
-  const int D = a.D;
-  const int nA = a.na[u], nB = a.nb[u];
-  lj_lists(a, u, a.n2s, nA, nB, A, B, naA, wA, naB, wB);
-  __syncthreads();
-  // stage both lists' rows: bytes past D and rows past the list ends are 0 (no product)
-  for (int e = tid; e < 2 * 64 * CPR; e += 256) {
-    const int op = e / (64 * CPR), r = (e / CPR) % 64, col = (e % CPR) * 16;
-    const int n = op == 0 ? nA : nB;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (r < n && col < D) {
-      const uint8_t* src = a.X8 + size_t(op == 0 ? A[r] : B[r]) * D + col;
-      if ((D & 15) == 0) {
-        v = *reinterpret_cast<const uint4*>(src);
-      } else {
-        v.x = *reinterpret_cast<const uint32_t*>(src);
-        if (col + 4 < D) v.y = *reinterpret_cast<const uint32_t*>(src + 4);
-        if (col + 8 < D) v.z = *reinterpret_cast<const uint32_t*>(src + 8);
-        if (col + 12 < D) v.w = *reinterpret_cast<const uint32_t*>(src + 12);
-      }
-    }
-    *reinterpret_cast<uint4*>((op == 0 ? sA : sB) + r * RS + col) = v;
-  }
-  __syncthreads();
-  // A-operand pieces of this wave's 16 rows, every K-step (lane group g: bytes 16g..16g+15)
-  i32x4 fa[KQ];
-#pragma unroll
-  for (int k = 0; k < KQ; ++k)
-    fa[k] = *reinterpret_cast<const i32x4*>(sA + (16 * w + t) * RS + 64 * k + 16 * g);
-  uint64_t row_b = TG_KEY_INF, row_a = TG_KEY_INF, col_b = TG_KEY_INF;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    i32x4 pB = {0, 0, 0, 0}, pA = {0, 0, 0, 0};
-#pragma unroll
-    for (int k = 0; k < KQ; ++k) {
-      const i32x4 fb = *reinterpret_cast<const i32x4*>(sB + (16 * c + t) * RS + 64 * k + 16 * g);
-      const i32x4 fc = *reinterpret_cast<const i32x4*>(sA + (16 * c + t) * RS + 64 * k + 16 * g);
-      pB = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[k], fb, pB, 0, 0, 0);
-      pA = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[k], fc, pA, 0, 0, 0);
-    }
-    const f32x4 accB = {float(pB[0]), float(pB[1]), float(pB[2]), float(pB[3])};
-    const f32x4 accA = {float(pA[0]), float(pA[1]), float(pA[2]), float(pA[3])};
-    lj_block_minima(c, accB, accA, A, B, naA, naB, nA, nB, w, g, t, row_b, row_a, col_b);
-  }
-  lj_push(a, A, B, wA, wB, nA, nB, w, g, t, l, row_b, row_a, col_b,
-          reinterpret_cast<uint64_t*>(sA));
-  if (a.counters && tid == 0)
-    atomicAdd(&cnt_slot(a.counters)[0], (unsigned long long)(nA * nB + nA * (nA - 1) / 2));
-}
-
 // Staged bytes per row and round, tile 0 / 1: rows up to 256 elements 64 / 128 (little LDS and
 // few registers, so eight waves per SIMD, and D = 96 is whole rounds: 500k x 96, two
-// iterations, 17.0 / 17.9 ms), wider rows 128 / 64 (half the rounds and barriers; their
+// iterations, 17.0 / 17.9 ms before the dealt blocks), wider rows 128 / 64 (half the rounds and barriers; their
 // re-scores hold the LDS anyway: 100k x 960 15.1 / 18.9 ms; 256 bytes per round 17.0 ms).
 void launch_knn_localjoin_screen(const KnnArgs& a, int precision, int tile, hipStream_t s) {
-  if (a.exact_screen && precision == KP_BF16 && a.X8 && a.n2s && a.D <= 256) {
-    // u8 data: the BF16 screen's products on int8 MFMA (exact either way)
-    const dim3 grid(grid_rows(a.perm, a.N));
-    if (a.D <= 128) k_localjoin_u8_screen<128><<<grid, 256, 0, s>>>(a);
-    else k_localjoin_u8_screen<256><<<grid, 256, 0, s>>>(a);
-    return;
-  }
   if (a.exact_screen && (precision == KP_BF16 || precision == KP_FP32)) {
-    // 256-byte staged rows (128 BF16 / 64 FP32 elements), 64-byte rows with tile 1
     const dim3 grid(grid_rows(a.perm, a.N));
-    if (precision == KP_BF16) {
+    if (a.X8 && a.n2s && a.D <= 256) {
+      // u8 data: the products on int8 MFMA, exact as the FP32 and BF16 ones are
+      if (a.D <= 128) k_localjoin_exact_screen<0, 128><<<grid, 256, 0, s>>>(a);
+      else k_localjoin_exact_screen<0, 256><<<grid, 256, 0, s>>>(a);
+    } else if (precision == KP_BF16) {
+      // 256-byte staged rows (128 BF16 / 64 FP32 elements), 64-byte rows with tile 1
       if (tile == 1) k_localjoin_exact_screen<2, 32><<<grid, 256, 0, s>>>(a);
       else k_localjoin_exact_screen<2, 128><<<grid, 256, 0, s>>>(a);
     } else {

@@ -521,3 +521,25 @@ def test_overflow_areas_and_grouping(N, D, K):
             assert s.stats()["knn_evals"] == ev
         assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
     _compare(X, Gr, GDr, 0, 0, 0, min(K, 24), 32, 1.2)
+
+
+@pytest.mark.parametrize("lo,hi", [(0, 255), (-200, 200)])
+@pytest.mark.parametrize("D,K", [(4, 3), (20, 17), (64, 16), (100, 33), (128, 64), (136, 40),
+                                 (256, 20), (264, 12)])
+def test_exact_join_edges(D, K, lo, hi):
+    """Exact screens on integer data: u8 rows (int8 products) in both screened precisions, with
+    signed values FP32 and BF16 products; lists that leave one to four tiles, partly filled,
+    dimensions around the staged row sizes.  Graphs equal to the oracle."""
+    rng = np.random.default_rng(D * K)
+    C = rng.integers(lo, hi + 1, (7, D))
+    X = np.clip(C[rng.integers(0, 7, 700)] + rng.integers(-9, 10, (700, D)), lo, hi).astype(np.float32)
+    Gr, GDr, ev = oracle.gnn_descent(X, K, 4, 21)
+    for prec in (["fp32", "bf16"] if D % 8 == 0 else ["fp32"]):
+        for tile in (0, 1):
+            _say(f"exact join D={D} K={K} [{lo}, {hi}] {prec} tile {tile}")
+            with State(*X.shape) as s:
+                s.set_data(X)
+                s.knn_build(K, 4, 21, prec, tile=tile)
+                G, GD = s.get_knn()
+                assert s.stats()["knn_evals"] == ev
+            assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
