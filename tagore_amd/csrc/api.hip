@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -15,6 +16,7 @@
 #include <initializer_list>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/tagore.h"
@@ -63,15 +65,39 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
-// The two window events of a build or a prune, destroyed on every return path.
-struct EventPair {
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  EventPair() = default;
-  EventPair(const EventPair&) = delete;
-  EventPair& operator=(const EventPair&) = delete;
-  ~EventPair() {
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
+// Pinned host memory of a handle for its copies to the caller's (pageable) arrays: COPY_LANES
+// threads with two chunks each, made by the first large copy (small results go through the
+// first chunk).
+constexpr int COPY_LANES = 4;
+constexpr size_t COPY_CHUNK = size_t(1) << 20;
+constexpr size_t COPY_DIRECT = size_t(4) << 20;  // below: one plain copy
+struct CopyOut {
+  unsigned char* pin = nullptr;
+  hipEvent_t ev[2 * COPY_LANES] = {};
+  void release() {
+    for (auto& e : ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+  }
+  bool ready() {
+    if (!pin) {
+      void* p = nullptr;
+      if (hipHostMalloc(&p, 2 * COPY_LANES * COPY_CHUNK, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      pin = static_cast<unsigned char*>(p);
+    }
+    for (auto& e : ev)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        e = nullptr;
+        return false;
+      }
+    return true;
   }
 };
 
@@ -160,7 +186,6 @@ struct tg_state {
   // search validator: per-workgroup visited bitmaps (all zero between calls) and id lists
   uint32_t* sbm = nullptr;
   uint32_t* svl = nullptr;
-  unsigned long long* scnt = nullptr;
   // segments (clusters stored back to back; nseg == 0: one data set)
   uint32_t nseg = 0;
   std::vector<uint32_t> seg_lo_host;
@@ -182,12 +207,78 @@ struct tg_state {
   int profiling = 0;  // 1: per-kernel events, 2: also prune phase clocks
   tg_stats stats{};
   std::vector<hipEvent_t> ev_pool;
+  hipEvent_t win[2] = {};      // window events of a build, prune or search
+  CopyOut out;
+  // search: queries on the device, and [counters | ids | dists] of the results, grown on demand
+  float* sq = nullptr;
+  size_t sq_cap = 0;
+  unsigned char* sres = nullptr;
+  size_t sres_cap = 0;
   // captured iteration sequences of tg_knn_build (TG_FLAG_GRAPH_ITERS), keyed by their
   // launch arguments; two entries cover the G / G1 alternation of odd expansion counts
   std::vector<std::pair<std::vector<unsigned char>, hipGraphExec_t>> iter_graphs;
 };
 
 namespace {
+
+int ensure_window(tg_state* s) {
+  for (auto& e : s->win)
+    if (!e) HIPX(hipEventCreate(&e));
+  return TG_OK;
+}
+
+// Copies n bytes of finished device work to the caller's memory.  Large copies go through
+// pinned chunks on several threads: the caller's array is often fresh, so its pages are
+// touched here for the first time, and one thread's page faults and memcpy held a copy to 10
+// of the link's 50 GB/s (132 MB of rows: 13 ms).
+int copy_out(tg_state* s, void* dst, const void* src, size_t n) {
+  if (n < COPY_DIRECT || !s->out.ready()) {
+    HIPX(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
+    return TG_OK;
+  }
+  const size_t nc = (n + COPY_CHUNK - 1) / COPY_CHUNK;
+  std::atomic<int> err{int(hipSuccess)};
+  // lane l: chunks l, l + COPY_LANES, ..; the next one is on its way (all on the handle's
+  // stream) while one is stored
+  auto lane = [&](int l) {
+    hipError_t e = hipSetDevice(s->device);
+    unsigned char* buf = s->out.pin + 2 * size_t(l) * COPY_CHUNK;
+    hipEvent_t* ev = s->out.ev + 2 * l;
+    auto fetch = [&](size_t c, int half) {
+      const size_t o = c * COPY_CHUNK;
+      const hipError_t f =
+          hipMemcpyAsync(buf + half * COPY_CHUNK, static_cast<const unsigned char*>(src) + o,
+                         std::min(COPY_CHUNK, n - o), hipMemcpyDeviceToHost, s->stream);
+      return f == hipSuccess ? hipEventRecord(ev[half], s->stream) : f;
+    };
+    int half = 0;
+    if (e == hipSuccess && size_t(l) < nc) e = fetch(l, 0);
+    for (size_t c = l; c < nc && e == hipSuccess; c += COPY_LANES, half ^= 1) {
+      e = hipEventSynchronize(ev[half]);
+      if (e == hipSuccess && c + COPY_LANES < nc) e = fetch(c + COPY_LANES, half ^ 1);
+      if (e == hipSuccess) {
+        const size_t o = c * COPY_CHUNK;
+        std::memcpy(static_cast<unsigned char*>(dst) + o, buf + half * COPY_CHUNK,
+                    std::min(COPY_CHUNK, n - o));
+      }
+    }
+    if (e != hipSuccess) err = int(e);
+  };
+  std::thread th[COPY_LANES];
+  int started = 1;
+  try {
+    for (; started < COPY_LANES; ++started) th[started] = std::thread(lane, started);
+  } catch (const std::exception&) {
+    // no more threads: the calling thread takes the remaining lanes too
+  }
+  lane(0);
+  for (int l = started; l < COPY_LANES; ++l) lane(l);
+  for (int l = 1; l < started; ++l) th[l].join();
+  if (err != int(hipSuccess)) (void)hipStreamSynchronize(s->stream);  // no copy left behind
+  if (err != int(hipSuccess))
+    return fail(TG_ERR_HIP, std::string("copy to the host: ") + hipGetErrorString(hipError_t(err.load())));
+  return TG_OK;
+}
 
 int ensure_events(tg_state* s, size_t n) {
   while (s->ev_pool.size() < n) {
@@ -542,7 +633,11 @@ int tg_free(tg_state* s) {
   dfree(s->counters);
   dfree(s->sbm);
   dfree(s->svl);
-  dfree(s->scnt);
+  dfree(s->sq);
+  dfree(s->sres);
+  s->out.release();
+  for (auto e : s->win)
+    if (e) (void)hipEventDestroy(e);
   dfree(s->fwd_deg);
   dfree(s->fwd_ids);
   dfree(s->fwd_d);
@@ -1126,10 +1221,8 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
   hipStream_t st = s->stream;
   if (ensure_events(s, 2)) return TG_ERR_HIP;
   // window events (separate from the per-section pool)
-  EventPair win;
-  HIPX(hipEventCreate(&win.e0));
-  HIPX(hipEventCreate(&win.e1));
-  hipEvent_t w0 = win.e0, w1 = win.e1;
+  if (ensure_window(s)) return TG_ERR_HIP;
+  hipEvent_t w0 = s->win[0], w1 = s->win[1];
   Sections sec{s};
   sec.next = 0;
   clear_status(s);
@@ -1341,8 +1434,10 @@ int tg_get_knn(tg_state* s, uint32_t* ids, float* dists) {
   if (!s) return fail(TG_ERR_ARG, "null handle");
   if (!s->has_knn) return fail(TG_ERR_STATE, "no kNN graph");
   HIPX(hipSetDevice(s->device));
-  if (ids) HIPX(hipMemcpy(ids, s->G, size_t(s->N) * s->K * 4, hipMemcpyDeviceToHost));
-  if (dists) HIPX(hipMemcpy(dists, s->GD, size_t(s->N) * s->K * 4, hipMemcpyDeviceToHost));
+  if (ids)
+    if (int rc = copy_out(s, ids, s->G, size_t(s->N) * s->K * 4)) return rc;
+  if (dists)
+    if (int rc = copy_out(s, dists, s->GD, size_t(s->N) * s->K * 4)) return rc;
   return TG_OK;
 }
 
@@ -1431,10 +1526,8 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
                            (p->precision == TG_PREC_FP8 && s->D % 16 == 0));
   if (dpg_screen && p->precision == TG_PREC_FP8)
     if (int rc = ensure_prep8(s)) return rc;
-  EventPair win;
-  HIPX(hipEventCreate(&win.e0));
-  HIPX(hipEventCreate(&win.e1));
-  hipEvent_t w0 = win.e0, w1 = win.e1;
+  if (ensure_window(s)) return TG_ERR_HIP;
+  hipEvent_t w0 = s->win[0], w1 = s->win[1];
   Sections sec{s};
   clear_status(s);
   fill_u32(s->ep_dev, 0, 1, st);
@@ -1521,8 +1614,10 @@ int tg_get_pruned(tg_state* s, uint32_t* deg, uint32_t* ids, uint32_t* ep) {
   if (!s->has_prune) return fail(TG_ERR_STATE, "no pruned graph");
   HIPX(hipSetDevice(s->device));
   const uint32_t FD = s->last_prune.FD;
-  if (deg) HIPX(hipMemcpy(deg, s->out_deg, size_t(s->N) * 4, hipMemcpyDeviceToHost));
-  if (ids) HIPX(hipMemcpy(ids, s->out_ids, size_t(s->N) * FD * 4, hipMemcpyDeviceToHost));
+  if (deg)
+    if (int rc = copy_out(s, deg, s->out_deg, size_t(s->N) * 4)) return rc;
+  if (ids)
+    if (int rc = copy_out(s, ids, s->out_ids, size_t(s->N) * FD * 4)) return rc;
   if (ep) *ep = s->ep;
   return TG_OK;
 }
@@ -1539,9 +1634,12 @@ int tg_get_forward(tg_state* s, uint32_t* deg, uint32_t* ids, float* dists) {
   if (!s->has_prune) return fail(TG_ERR_STATE, "no pruned graph");
   HIPX(hipSetDevice(s->device));
   const uint32_t FD = s->last_prune.FD;
-  if (deg) HIPX(hipMemcpy(deg, s->fwd_deg, size_t(s->N) * 4, hipMemcpyDeviceToHost));
-  if (ids) HIPX(hipMemcpy(ids, s->fwd_ids, size_t(s->N) * FD * 4, hipMemcpyDeviceToHost));
-  if (dists) HIPX(hipMemcpy(dists, s->fwd_d, size_t(s->N) * FD * 4, hipMemcpyDeviceToHost));
+  if (deg)
+    if (int rc = copy_out(s, deg, s->fwd_deg, size_t(s->N) * 4)) return rc;
+  if (ids)
+    if (int rc = copy_out(s, ids, s->fwd_ids, size_t(s->N) * FD * 4)) return rc;
+  if (dists)
+    if (int rc = copy_out(s, dists, s->fwd_d, size_t(s->N) * FD * 4)) return rc;
   return TG_OK;
 }
 
@@ -1738,6 +1836,7 @@ int tg_store_index(tg_state* s, const char* path, const char* index_type, uint64
 namespace {
 constexpr uint32_t SEARCH_GRID = 256 * 12;  // workgroups: 12 queries in flight per CU
 constexpr uint32_t SEARCH_VCAP = 8192;      // listed visited ids per query
+constexpr size_t SEARCH_HEAD = 64;          // bytes of the counters before the results
 }  // namespace
 
 int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_params* p,
@@ -1755,73 +1854,84 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
   const uint32_t words = (N + 31) / 32;
   if (!s->sbm) {
     if (dalloc(&s->sbm, size_t(SEARCH_GRID) * words) ||
-        dalloc(&s->svl, size_t(SEARCH_GRID) * SEARCH_VCAP) || dalloc(&s->scnt, 2))
+        dalloc(&s->svl, size_t(SEARCH_GRID) * SEARCH_VCAP))
       return TG_ERR_HIP;
     fill_u32(s->sbm, 0, size_t(SEARCH_GRID) * words, s->stream);
   }
-  float* Q = nullptr;
-  uint32_t* oi = nullptr;
-  float* od = nullptr;
-  if (dalloc(&Q, size_t(nq) * D) || dalloc(&oi, size_t(nq) * p->k) ||
-      dalloc(&od, size_t(nq) * p->k)) {
-    dfree(Q);
-    dfree(oi);
-    return TG_ERR_HIP;
+  // device buffers of the handle, grown to the largest call so far
+  const size_t nr = size_t(nq) * p->k * 4;          // bytes of the ids, and of the distances
+  const size_t need = SEARCH_HEAD + 2 * nr;
+  if (s->sq_cap < size_t(nq) * D) {
+    dfree(s->sq);
+    s->sq_cap = 0;
+    if (dalloc(&s->sq, size_t(nq) * D)) return TG_ERR_HIP;
+    s->sq_cap = size_t(nq) * D;
   }
-  int rc = TG_OK;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipError_t e = hipMemcpyAsync(Q, queries, size_t(nq) * D * 4, hipMemcpyHostToDevice, s->stream);
-  if (e == hipSuccess) e = hipEventCreate(&e0);
-  if (e == hipSuccess) e = hipEventCreate(&e1);
-  if (e == hipSuccess) {
-    fill_u32(reinterpret_cast<uint32_t*>(s->scnt), 0, 4, s->stream);
-    SearchArgs a{};
-    a.X = s->X;
-    a.X8 = s->prep_valid && s->cert_u8 && D <= 256 ? s->X8 : nullptr;
-    a.N = N;
-    a.D = D;
-    a.deg = s->out_deg;
-    a.ids = s->out_ids;
-    a.FD = s->last_prune.FD;
-    a.ep = ep;
-    a.Q = Q;
-    a.nq = nq;
-    a.L = p->L;
-    a.k = p->k;
-    a.seed = p->seed;
-    a.bitmap = s->sbm;
-    a.words = words;
-    a.vlist = s->svl;
-    a.vcap = SEARCH_VCAP;
-    a.out_ids = oi;
-    a.out_d = od;
-    a.counters = s->scnt;
-    e = hipEventRecord(e0, s->stream);
-    launch_search(a, std::min(nq, SEARCH_GRID), s->stream);
-    if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess) e = hipEventRecord(e1, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+  if (s->sres_cap < need) {
+    dfree(s->sres);
+    s->sres_cap = 0;
+    if (dalloc(&s->sres, need)) return TG_ERR_HIP;
+    s->sres_cap = need;
   }
+  if (ensure_window(s)) return TG_ERR_HIP;
+  hipStream_t st = s->stream;
+  // small calls go through the pinned chunk: no staging inside the runtime's copies
+  const bool pinned = size_t(nq) * D * 4 <= COPY_CHUNK && need <= COPY_CHUNK && s->out.ready();
+  unsigned char* pin = s->out.pin;
+  if (pinned) std::memcpy(pin, queries, size_t(nq) * D * 4);
+  HIPX(hipMemcpyAsync(s->sq, pinned ? static_cast<const void*>(pin) : queries, size_t(nq) * D * 4,
+                      hipMemcpyHostToDevice, st));
+  auto* scnt = reinterpret_cast<unsigned long long*>(s->sres);
+  fill_u32(reinterpret_cast<uint32_t*>(scnt), 0, 4, st);
+  SearchArgs a{};
+  a.X = s->X;
+  a.X8 = s->prep_valid && s->cert_u8 && D <= 256 ? s->X8 : nullptr;
+  a.N = N;
+  a.D = D;
+  a.deg = s->out_deg;
+  a.ids = s->out_ids;
+  a.FD = s->last_prune.FD;
+  a.ep = ep;
+  a.Q = s->sq;
+  a.nq = nq;
+  a.L = p->L;
+  a.k = p->k;
+  a.seed = p->seed;
+  a.bitmap = s->sbm;
+  a.words = words;
+  a.vlist = s->svl;
+  a.vcap = SEARCH_VCAP;
+  a.out_ids = reinterpret_cast<uint32_t*>(s->sres + SEARCH_HEAD);
+  a.out_d = reinterpret_cast<float*>(s->sres + SEARCH_HEAD + nr);
+  a.counters = scnt;
+  HIPX(hipEventRecord(s->win[0], st));
+  launch_search(a, std::min(nq, SEARCH_GRID), st);
+  HIPX(hipGetLastError());
+  HIPX(hipEventRecord(s->win[1], st));
   unsigned long long cnt[2] = {0, 0};
-  if (e == hipSuccess)
-    e = hipMemcpy(ids, oi, size_t(nq) * p->k * 4, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && dists)
-    e = hipMemcpy(dists, od, size_t(nq) * p->k * 4, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(cnt, s->scnt, sizeof(cnt), hipMemcpyDeviceToHost);
-  if (e == hipSuccess && out) {
+  if (pinned) {
+    // (the queries' copy is finished when the results' one runs: the same stream)
+    HIPX(hipMemcpyAsync(pin + COPY_CHUNK, s->sres, need, hipMemcpyDeviceToHost, st));
+    HIPX(hipStreamSynchronize(st));
+    const unsigned char* r = pin + COPY_CHUNK;
+    std::memcpy(cnt, r, sizeof(cnt));
+    std::memcpy(ids, r + SEARCH_HEAD, nr);
+    if (dists) std::memcpy(dists, r + SEARCH_HEAD + nr, nr);
+  } else {
+    HIPX(hipStreamSynchronize(st));
+    HIPX(hipMemcpy(cnt, scnt, sizeof(cnt), hipMemcpyDeviceToHost));
+    if (int rc = copy_out(s, ids, a.out_ids, nr)) return rc;
+    if (dists)
+      if (int rc = copy_out(s, dists, a.out_d, nr)) return rc;
+  }
+  if (out) {
     float ms = 0.f;
-    e = hipEventElapsedTime(&ms, e0, e1);
+    HIPX(hipEventElapsedTime(&ms, s->win[0], s->win[1]));
     out->ms = ms;
     out->evals = cnt[0];
     out->expansions = cnt[1];
   }
-  if (e != hipSuccess) rc = fail(TG_ERR_HIP, std::string("search: ") + hipGetErrorString(e));
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
-  dfree(Q);
-  dfree(oi);
-  dfree(od);
-  return rc;
+  return TG_OK;
 }
 
 // ------------------------------------------------------------ allocation-free search

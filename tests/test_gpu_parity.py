@@ -543,3 +543,19 @@ def test_exact_join_edges(D, K, lo, hi):
                 G, GD = s.get_knn()
                 assert s.stats()["knn_evals"] == ev
             assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
+
+
+@pytest.mark.parametrize("N,K", [(1 << 19, 2), ((1 << 19) + 1, 2), (262145, 5), (300007, 31),
+                                 (1048575, 4)])
+def test_large_copies_round_trip(N, K):
+    """Results above the size where copies to the host go through pinned chunks: whole chunks, a
+    few bytes more, fewer chunks than threads, and two calls in turn."""
+    rng = np.random.default_rng(N)
+    ids = rng.integers(0, N, (N, K)).astype(np.uint32)
+    d = np.sort(rng.random((N, K)).astype(np.float32), axis=1)
+    ids2, d2 = ids[::-1].copy(), d[::-1].copy()
+    with State(N, 4) as s:
+        for i, x in ((ids, d), (ids2, d2)):
+            s.set_knn(i, x)
+            G, GD = s.get_knn()
+            assert np.array_equal(G, i) and np.array_equal(GD, x)
