@@ -552,7 +552,8 @@ def test_large_copies_round_trip(N, K):
     few bytes more, fewer chunks than threads, and two calls in turn."""
     rng = np.random.default_rng(N)
     ids = rng.integers(0, N, (N, K)).astype(np.uint32)
-    d = np.sort(rng.random((N, K)).astype(np.float32), axis=1)
+    # strictly rising rows: equal distances would have to come in id order
+    d = (np.arange(K) + 0.5 * rng.random((N, K))).astype(np.float32)
     ids2, d2 = ids[::-1].copy(), d[::-1].copy()
     with State(N, 4) as s:
         for i, x in ((ids, d), (ids2, d2)):
