@@ -33,6 +33,12 @@ __device__ __forceinline__ bool key_finite(uint64_t k) { return uint32_t(k >> 32
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// lane l's value, in scalar registers (l uniform)
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
+  return uint64_t(uint32_t(__builtin_amdgcn_readlane(int(v >> 32), l))) << 32 |
+         uint32_t(__builtin_amdgcn_readlane(int(uint32_t(v)), l));
+}
+
 // wave-wide ballot (64-bit mask)
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 

@@ -20,52 +20,83 @@ namespace tg {
 
 constexpr int RING = 480;
 
-// shader clock when phase profiling is on (PruneArgs::phase_clock), else 0
-__device__ __forceinline__ long long pclock(const PruneArgs& a) {
-  return a.phase_clock ? clock64() : 0;
-}
-
-// phase-clock sums of one workgroup (profiling): distance batches, and the beam rounds'
-// candidate step, sort, merge and id-set rebuild.  Held in registers (no address taken).
-struct PhaseAcc {
+// phase-clock sums of one workgroup (profiling builds of the forward kernels): distance batches,
+// and the beam rounds' candidate step, sort, merge and id-set rebuild.  A type, not a flag:
+// the sums and the tests of a flag took scalar registers across the whole kernel (95 of them
+// spilled in the u8 path kernel).
+struct PhaseOff {
+  static constexpr bool on = false;
+  long long ev, sub[4];
+};
+struct PhaseOn {
+  static constexpr bool on = true;
   long long ev = 0;
   long long sub[4] = {0, 0, 0, 0};
 };
+template <class Ph>
+__device__ __forceinline__ long long pclock(const Ph&) {
+  return Ph::on ? clock64() : 0;
+}
+template <class Ph>
+__device__ __forceinline__ void padd(Ph&, long long& sum, long long dt) {
+  if (Ph::on) sum += dt;
+}
 constexpr int POOL_MAX = 1024;  // K + 480 <= 608, padded to a power of two
 
+// Id set in LDS: HS_BUCKETS buckets of four ids (INV: empty), each with a 16-bit count, in
+// HS_WORDS words.  An insert takes a place by adding to its bucket's count and moves on to the
+// next bucket when this one is full; a look-up reads one bucket and moves on only past a full
+// one.  The beam's set holds at most TOPM + K <= 256 members, half of the places, so both end
+// whatever the ids are.  Against open addressing over single slots there is no chain of
+// compare-and-swaps, as long as the longest of the wave's 64: the inserts of one round overlap.
+// (Path Collect over 1M x 128 u8 rows, K 96, TOPM 64, profiled cycles per node: look-ups and
+// compaction 106k with 256 single slots, 43k with 512, 36k with the buckets; inserts 62k / 58k
+// with 512 / the buckets.)
 // -------------------------------------------------------------------------------------
-// Id set in LDS: open addressing over 2^bits slots, INV marks an empty slot.  Callers size
-// the table above the most members it can hold, so a probe always ends.
-// -------------------------------------------------------------------------------------
-constexpr int HSET = 512;  // k_cal_ep: up to 256 members
+constexpr int HS_BUCKETS = 128, HS_WORDS = HS_BUCKETS * 4 + HS_BUCKETS / 2;
 // (the 24-bit product is a full-rate instruction, the 32-bit one a quarter; ids that share
-// their low 24 bits chain)
-__device__ __forceinline__ uint32_t hslot(uint32_t id, int bits) {
-  return ((id & 0xFFFFFFu) * 0x9E3779u) >> (32 - bits);
+// their low 24 bits share a bucket)
+__device__ __forceinline__ uint32_t hbucket(uint32_t id) {
+  return ((id & 0xFFFFFFu) * 0x9E3779u) >> (32 - 7);
 }
-__device__ void hset_clear(uint32_t* tab, int bits) {
-  for (int i = threadIdx.x; i < (1 << bits); i += TG_WAVE) tab[i] = TG_INV;
+__device__ __forceinline__ void hset_clear(uint32_t* tab) {  // tab 16-byte aligned
+  for (int i = 4 * threadIdx.x; i < HS_BUCKETS * 4; i += 4 * TG_WAVE)
+    *reinterpret_cast<uint4*>(tab + i) = make_uint4(TG_INV, TG_INV, TG_INV, TG_INV);
+  tab[HS_BUCKETS * 4 + threadIdx.x] = 0;
 }
-__device__ __forceinline__ void hset_insert(uint32_t* tab, uint32_t id, int bits) {
-  if (id == TG_INV) return;
-  const uint32_t mask = (1u << bits) - 1;
-  uint32_t h = hslot(id, bits);
-  for (;;) {
-    const uint32_t old = atomicCAS(&tab[h], TG_INV, id);
-    if (old == TG_INV || old == id) return;
-    h = (h + 1) & mask;
+// inserts one id per lane and list entry (INV: none)
+template <int C>
+__device__ __forceinline__ void hset_insert(uint32_t* tab, const uint32_t (&id)[C]) {
+  uint32_t h[C], old[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    h[c] = hbucket(id[c]);
+    old[c] = 0;
+    if (id[c] != TG_INV)
+      old[c] = atomicAdd(&tab[HS_BUCKETS * 4 + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (id[c] == TG_INV) continue;
+    uint32_t at = (old[c] >> ((h[c] & 1) * 16)) & 0xFFFFu;
+    while (at >= 4) {
+      h[c] = (h[c] + 1) & (HS_BUCKETS - 1);
+      const uint32_t o = atomicAdd(&tab[HS_BUCKETS * 4 + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
+      at = (o >> ((h[c] & 1) * 16)) & 0xFFFFu;
+    }
+    tab[h[c] * 4 + at] = id[c];
   }
 }
-__device__ __forceinline__ bool hset_has(const uint32_t* tab, uint32_t id, int bits) {
-  const uint32_t mask = (1u << bits) - 1;
-  uint32_t h = hslot(id, bits);
+__device__ __forceinline__ bool hset_has(const uint32_t* tab, uint32_t id) {
+  uint32_t h = hbucket(id);
   for (;;) {
-    const uint32_t v = tab[h];
-    if (v == id) return true;
-    if (v == TG_INV) return false;
-    h = (h + 1) & mask;
+    const uint4 v = *reinterpret_cast<const uint4*>(tab + h * 4);
+    if (v.x == id || v.y == id || v.z == id || v.w == id) return true;
+    if (v.w == TG_INV) return false;
+    h = (h + 1) & (HS_BUCKETS - 1);
   }
 }
+static_assert(HS_BUCKETS / 2 == TG_WAVE, "one lane clears one word of counts");
 
 // -------------------------------------------------------------------------------------
 // Beam search shared by cal_ep and path Collect (spec in the oracle's beam_search).
@@ -80,18 +111,26 @@ __device__ __forceinline__ bool hset_has(const uint32_t* tab, uint32_t id, int b
 // beam never holds two finite entries with one id, and an expanded node that falls out of
 // the beam can never re-enter it (the beam's TOPM-th key only decreases).  `out` (optional)
 // receives the final beam (TOPM keys).
+// With six waves per SIMD the rounds are bound by instruction issue, not by the loads: the
+// profiling sums as a type, the buckets and the next list's early load took the NSG forward
+// pass at that size from 31.9 to 29.3 ms.
 // -------------------------------------------------------------------------------------
-template <int MC, class T, int W>
+template <int MC, class T, int W, class Ph>
 __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>& tgt,
                                             uint32_t start,
-                            int max_exp, uint64_t* S, uint32_t* tab, int hbits,
-                            uint16_t* cl, uint64_t* ring, uint64_t* out, uint32_t& ring_c,
-                            uint32_t& n_eval, uint32_t& n_adj, PhaseAcc& ph) {
+                                            int max_exp, uint64_t* S, uint32_t* tab,
+                                            uint16_t* cl, uint64_t* ring, uint64_t* out, uint32_t& ring_c,
+                                            uint32_t& n_eval, uint32_t& n_adj, Ph& ph) {
   const int lane = threadIdx.x;
   const int K = a.K, TOPM = a.TOPM, D = a.D;
   constexpr int NS = 64 * W;
   const T* X = reinterpret_cast<const T*>(a.rows);
   const uint64_t INFKEY = mk_key(__uint_as_float(0x7F800000u), 0u);
+  auto load_adj = [&](uint32_t x, uint32_t (&y)[W]) {
+#pragma unroll
+    for (int q = 0; q < W; ++q)
+      y[q] = q * TG_WAVE + lane < K ? a.G[size_t(x) * K + q * TG_WAVE + lane] : TG_INV;
+  };
   // start list S = G[start] with distances (ring slots 0..K-1 in list order)
   for (int j = lane; j < NS; j += TG_WAVE)
     S[j] = j < K ? (INFKEY | a.G[size_t(start) * K + j]) : TG_KEY_INF;
@@ -105,13 +144,17 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
   n_eval += K;
   n_adj += 1;
   ring_c = K;
-  hset_clear(tab, hbits);
+  hset_clear(tab);
   __syncthreads();
   uint64_t v[W], bk[W];
+  {
+    uint32_t ids[W];  // the first dedup set is ids(S); padding ids are INV
 #pragma unroll
-  for (int r = 0; r < W; ++r) {
-    v[r] = S[r * 64 + lane];
-    hset_insert(tab, key_id(v[r]), hbits);  // the first dedup set is ids(S); padding ids are INV
+    for (int r = 0; r < W; ++r) {
+      v[r] = S[r * 64 + lane];
+      ids[r] = key_id(v[r]);
+    }
+    hset_insert(tab, ids);
   }
   reg_bitonic<W>(v);
 #pragma unroll
@@ -120,40 +163,38 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
   // the expanded ids in registers: lane e < nexpl holds the e-th (max_exp <= 64)
   uint32_t ex = TG_INV;
   int nexpl = 0;
-  for (int r = 0; r < max_exp; ++r) {
-    const long long s0 = pclock(a);
-    // first explorable beam entry (position order)
-    int first = -1;
-    uint32_t x = 0;
+  // key of the first explorable beam entry (position order), TG_KEY_INF when there is none
+  auto explorable = [&]() {
+    uint64_t k = TG_KEY_INF;
 #pragma unroll
     for (int b = 0; b < W; ++b) {
-      if (first >= 0) break;
+      if (k != TG_KEY_INF) break;
       const uint32_t id = key_id(bk[b]);
       bool ok = key_finite(bk[b]);
       for (int e = 0; e < nexpl; ++e)
         ok = ok & (id != uint32_t(__builtin_amdgcn_readlane(int(ex), e)));
       const uint64_t m = ballot(ok);
-      if (m) {
-        const int fl = __ffsll((unsigned long long)m) - 1;
-        first = b * 64 + fl;
-        x = uint32_t(__builtin_amdgcn_readlane(int(id), fl));
-      }
+      if (m) k = readlane64(bk[b], __ffsll((unsigned long long)m) - 1);
     }
-    if (first < 0) break;
-    __syncthreads();
-    if (lane == nexpl) ex = x;
+    return k;
+  };
+  uint64_t next = explorable();
+  uint32_t y[W];
+  if (next != TG_KEY_INF) load_adj(key_id(next), y);
+  for (int r = 0; r < max_exp && next != TG_KEY_INF; ++r) {
+    const long long s0 = pclock(ph);
+    if (lane == nexpl) ex = key_id(next);
     ++nexpl;
     n_adj += 1;
     // new candidates: duplicates of the dedup set get +inf; the rest compacted in j order
     int cnt = 0;
 #pragma unroll
-    for (int base = 0; base < NS; base += TG_WAVE) {
-      const int j = base + lane;
+    for (int q = 0; q < W; ++q) {
+      const int j = q * TG_WAVE + lane;
       bool fresh = false;
       if (j < K) {
-        const uint32_t y = a.G[size_t(x) * K + j];
-        fresh = !hset_has(tab, y, hbits);
-        S[j] = INFKEY | y;
+        fresh = !hset_has(tab, y[q]);
+        S[j] = INFKEY | y[q];
       } else {
         S[j] = TG_KEY_INF;
       }
@@ -163,8 +204,8 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
     }
     __syncthreads();
     const uint32_t c0 = ring_c;
-    const long long e0 = pclock(a);
-    ph.sub[0] += e0 - s0;
+    const long long e0 = pclock(ph);
+    padd(ph, ph.sub[0], e0 - s0);
     eval_batch<MC, T, true>(X, D, tgt, cnt, [&](int q) { return key_id(S[cl[q]]); },
                    [&](int q, float d) {
                      const int j = cl[q];
@@ -172,33 +213,29 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
                      S[j] = k;
                      if (ring) ring[(c0 + q) % RING] = k;
                    });
-    ph.ev += pclock(a) - e0;
+    padd(ph, ph.ev, pclock(ph) - e0);
     ring_c += cnt;
     n_eval += cnt;
     __syncthreads();
-    const long long s1 = pclock(a);
+    const long long s1 = pclock(ph);
 #pragma unroll
     for (int q = 0; q < W; ++q) v[q] = S[q * 64 + lane];
-    // next dedup set: ids of this round's beam and candidates
-    hset_clear(tab, hbits);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-      hset_insert(tab, key_id(bk[q]), hbits);
-      hset_insert(tab, key_id(v[q]), hbits);
-    }
-    const long long s2 = pclock(a);
     // Only candidates below the beam's TOPM-th key can enter it (a fresh id is in neither
-    // the beam nor the previous candidates, so no key ties one in the beam).  With two
-    // slots per lane and at most 64 such candidates (and TOPM <= 64), they are compacted
-    // and merged with one-slot sorts; none leaves the beam as it is.  Either way the beam
-    // becomes the TOPM smallest keys of beam and candidates.
+    // the beam nor the previous candidates, so no key ties one in the beam).  With TOPM <= 64
+    // and at most 64 such candidates, they are compacted and merged with one-slot sorts; none
+    // leaves the beam as it is.  (One slot per lane: only once the beam is full of finite keys;
+    // until then the merge also keeps keys without a distance, which count as seen.)  Either way the beam becomes the TOPM smallest keys of beam and
+    // candidates.
+    uint64_t worst = TG_KEY_INF;
+#pragma unroll
+    for (int b = 0; b < W; ++b)
+      if (b == (TOPM - 1) >> 6) worst = readlane64(bk[b], (TOPM - 1) & 63);
     int m = 64 * W;
     bool small = false;
-    if (W > 1 && TOPM <= 64) {
-      const uint64_t wk = bk[0];
-      const uint64_t worst = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(wk >> 32), TOPM - 1))) << 32) |
-                             uint32_t(__builtin_amdgcn_readlane(int(uint32_t(wk)), TOPM - 1));
+    uint64_t c[W];  // the candidates, sorted
+#pragma unroll
+    for (int q = 0; q < W; ++q) c[q] = v[q];
+    if (TOPM <= 64 && (W > 1 || key_finite(worst))) {
       uint64_t qm[W];
       m = 0;
 #pragma unroll
@@ -216,43 +253,60 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
         }
         if (lane >= m) S[lane] = TG_KEY_INF;
         __syncthreads();
-        v[0] = S[lane];
+        c[0] = S[lane];
+        // keys in lanes 0..m-1, +inf above: sorting blocks of the next power of two is enough
+        if (m <= 16) reg_bitonic_upto<16>(c[0]);
+        else if (m <= 32) reg_bitonic_upto<32>(c[0]);
+        else reg_bitonic_upto<64>(c[0]);
       }
     }
-    long long s3 = 0;
+    if (!small) reg_bitonic<W>(c);
+    const long long s2 = pclock(ph);
+    padd(ph, ph.sub[1], s2 - s1);
+    // The next expansion is known before the merge: the smaller of the first explorable entry
+    // and the smallest candidate that enters (an entry that the candidates push out of the beam
+    // has a smaller candidate before it; an expanded id never comes back as one).  Its list is
+    // on its way while the id set is rebuilt and the beam merged.
+    next = explorable();
+    if (m > 0) {
+      const uint64_t cmin = readlane64(c[0], 0);
+      if (cmin < worst && key_finite(cmin) && cmin < next) next = cmin;
+    }
+    if (next != TG_KEY_INF) load_adj(key_id(next), y);
+    // next dedup set: ids of this round's beam and candidates
+    hset_clear(tab);
+    __syncthreads();
+    {
+      uint32_t ids[2 * W];
+#pragma unroll
+      for (int q = 0; q < W; ++q) {
+        ids[2 * q] = key_id(bk[q]);
+        ids[2 * q + 1] = key_id(v[q]);
+      }
+      hset_insert(tab, ids);
+    }
+    const long long s3 = pclock(ph);
+    padd(ph, ph.sub[3], s3 - s2);
     if (small) {
       if (m > 0) {
-        // keys in lanes 0..m-1, +inf above: sorting blocks of the next power of two is enough
-        uint64_t w1 = v[0];
-        if (m <= 16) reg_bitonic_upto<16>(w1);
-        else if (m <= 32) reg_bitonic_upto<32>(w1);
-        else reg_bitonic_upto<64>(w1);
-        s3 = pclock(a);
-        const uint64_t rv = lane_xor64(w1, 63);
-        uint64_t c[1] = {bk[0] < rv ? bk[0] : rv};
-        reg_bitonic_merge<1>(c);
-        bk[0] = lane < TOPM ? c[0] : TG_KEY_INF;
-      } else {
-        s3 = pclock(a);
+        const uint64_t rv = lane_xor64(c[0], 63);
+        uint64_t w1[1] = {bk[0] < rv ? bk[0] : rv};
+        reg_bitonic_merge<1>(w1);
+        bk[0] = lane < TOPM ? w1[0] : TG_KEY_INF;
       }
     } else {
-      reg_bitonic<W>(v);
-      s3 = pclock(a);
-      uint64_t c[W];
+      uint64_t w[W];
 #pragma unroll
       for (int b = 0; b < W; ++b) {
-        const uint64_t rv = lane_xor64(v[W - 1 - b], 63);  // candidate 64W-1-p
-        c[b] = bk[b] < rv ? bk[b] : rv;
+        const uint64_t rv = lane_xor64(c[W - 1 - b], 63);  // candidate 64W-1-p
+        w[b] = bk[b] < rv ? bk[b] : rv;
       }
-      reg_bitonic_merge<W>(c);
+      reg_bitonic_merge<W>(w);
 #pragma unroll
-      for (int b = 0; b < W; ++b) bk[b] = b * 64 + lane < TOPM ? c[b] : TG_KEY_INF;
+      for (int b = 0; b < W; ++b) bk[b] = b * 64 + lane < TOPM ? w[b] : TG_KEY_INF;
     }
     __syncthreads();
-    const long long s4 = pclock(a);
-    ph.sub[1] += s3 - s2;
-    ph.sub[2] += s4 - s3;
-    ph.sub[3] += s2 - s1;
+    padd(ph, ph.sub[2], pclock(ph) - s3);
   }
   if (out) {
 #pragma unroll
@@ -372,10 +426,10 @@ __device__ __forceinline__ int advance_cl(uint64_t* P, uint16_t* cl, int from, i
 // in pool order, so a round touches only the survivors of the previous round.  For rows that
 // filter_pool_mfma does not take: wider than 256 elements, or without an 8-, 16-bit copy.
 // -------------------------------------------------------------------------------------
-template <int MC, class T>
+template <int MC, class T, class Ph>
 __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int L, uint32_t u,
                                            int rule, uint64_t* sel, uint16_t* cl,
-                                           uint32_t& n_eval, PhaseAcc& ph) {
+                                           uint32_t& n_eval, Ph& ph) {
   const int lane = threadIdx.x, t = lane & 15;
   const int D = a.D, FD = a.FD;
   int tix = next_valid(P, 0, L, u);
@@ -403,7 +457,7 @@ __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int 
   while (nsel < FD) {
     const int cnt = nl;  // this round's candidates cl[0..cnt)
     Row16<MC> prow;
-    const long long e0 = pclock(a);
+    const long long e0 = pclock(ph);
     load_row16<MC>(prow, reinterpret_cast<const T*>(a.rows) + size_t(pid) * D, D, t);
     eval_batch<MC>(reinterpret_cast<const T*>(a.rows), D, prow, cnt, [&](int q) { return key_id(P[cl[q]]); },
                    [&](int q, float res) {
@@ -412,7 +466,7 @@ __device__ __forceinline__ int filter_pool(const PruneArgs& a, uint64_t* P, int 
                      if (rule_eval(rule, res, key_d(k), cur, a.th) < 0.0f)
                        P[i] = key_with_id(k, TG_INV);
                    });
-    ph.ev += pclock(a) - e0;
+    padd(ph, ph.ev, pclock(ph) - e0);
     n_eval += cnt;
     __syncthreads();
     // the next selection is the first survivor; the survivors after it are the next round's
@@ -478,11 +532,11 @@ __device__ __forceinline__ int rule_bracket(int rule, float lo, float hi, float 
   return hi < T - sl ? 1 : lo > T + sl ? 0 : 2;
 }
 
-template <int MC, class T>
+template <int MC, class T, class Ph>
 __device__ __forceinline__ int filter_pool_mfma(const PruneArgs& a, const uint64_t* P, int L,
                                                 uint32_t u, int rule, uint64_t* sel,
                                                 uint16_t* cl, uint16_t* km, uint16_t* queue,
-                                                uint32_t& n_eval, PhaseAcc& ph) {
+                                                uint32_t& n_eval, Ph& ph) {
   constexpr bool U8 = std::is_same<T, uint8_t>::value;
   constexpr int KS = U8 ? MC : 2 * MC;  // 64-byte steps of a row
   constexpr int ESZ = U8 ? 1 : 2;
@@ -552,7 +606,7 @@ __device__ __forceinline__ int filter_pool_mfma(const PruneArgs& a, const uint64
   int kept = 0;
   while (kept < rounds && cnt > 0) {
     const int nb = min(16, cnt);
-    const long long e0 = pclock(a);
+    const long long e0 = pclock(ph);
     // row t of the block in the lanes t + 16 g; rows past nb repeat row 0, their bits masked
     const uint64_t krow = P[cl[t < nb ? t : 0]];
     const uint32_t idt = key_id(krow);
@@ -698,7 +752,7 @@ __device__ __forceinline__ int filter_pool_mfma(const PruneArgs& a, const uint64
     }
     if (qn) flush();
     else __syncthreads();
-    ph.ev += pclock(a) - e0;
+    padd(ph, ph.ev, pclock(ph) - e0);
     // ---- evaluations and the survivors, in order (in place: a chunk is read before any of
     // its entries is written, and writes land at or below it)
     int live = 0;
@@ -750,7 +804,7 @@ __device__ __forceinline__ void count_add(unsigned long long* c, int idx, uint32
 constexpr int RING_P = 512;
 
 struct FwdLayout {
-  int W, NS, L, HB, offB, offF, bytes;
+  int W, NS, L, offB, offF, bytes;
 };
 __host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD,
                                                          bool mfma) {
@@ -758,12 +812,9 @@ __host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD,
   l.W = (K <= 64 && TOPM <= 64) ? 1 : 2;
   l.NS = 64 * l.W;
   l.L = K + RING;
-  // the beam's id set holds at most TOPM + K ids: 256 slots up to 192 of them (three
-  // quarters full at most), else 512
-  l.HB = TOPM + K <= 192 ? 8 : 9;
   l.offB = RING_P * 8;
   l.offF = ((l.L > RING_P ? l.L : RING_P) * 8 + 15) / 16 * 16;
-  const int beam = l.offB + l.NS * 8 + (4 << l.HB) + l.NS * 2;
+  const int beam = l.offB + l.NS * 8 + HS_WORDS * 4 + l.NS * 2;
   // the filter's selection, live list, killer masks and re-score queue
   const int filt = l.offF + (FD + 1) * 8 + (l.L + 17) * 4 + (mfma ? FQ_CAP * 2 : 0);
   l.bytes = ((beam > filt ? beam : filt) + 15) / 16 * 16;
@@ -771,7 +822,8 @@ __host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD,
 }
 
 // mfma: filter_pool_mfma on the 16-bit copy (u8 rows always take it).
-template <int MC, class T, int KIND, int W, bool MF>
+// Ph: PhaseOn in profiling runs.
+template <int MC, class T, int KIND, int W, bool MF, class Ph>
 // Waves per SIMD: six (80 VGPRs) for u8 rows up to 128 elements, fewer where the rows' registers
 // would spill.
 __global__ __launch_bounds__(64)
@@ -788,7 +840,7 @@ void k_forward(PruneArgs a) {
   uint64_t* P = R;  // after the pool is formed
   uint64_t* S = reinterpret_cast<uint64_t*>(dsm + ly.offB);
   uint32_t* tab = reinterpret_cast<uint32_t*>(S + ly.NS);
-  uint16_t* clb = reinterpret_cast<uint16_t*>(tab + (1 << ly.HB));
+  uint16_t* clb = reinterpret_cast<uint16_t*>(tab + HS_WORDS);
   uint64_t* sel = reinterpret_cast<uint64_t*>(dsm + ly.offF);  // after the beam
   uint16_t* cl = reinterpret_cast<uint16_t*>(sel + a.FD + 1);
   uint16_t* km = cl + ((ly.L + 17) & ~1);
@@ -800,12 +852,12 @@ void k_forward(PruneArgs a) {
     R[i] = i < RING ? mk_key(__uint_as_float(0x7F800000u), TG_INV) : TG_KEY_INF;
   __syncthreads();
   uint32_t n_col = 0, n_adj = 0, n_flt = 0;
-  PhaseAcc ph;
-  const long long c0 = pclock(a);
+  Ph ph;
+  const long long c0 = pclock(ph);
   if (KIND == 0) {
     uint32_t ring_c = 0;
     const uint32_t ep = a.ep[a.seg_of ? a.seg_of[u] : 0];
-    beam_search<MC, T, W>(a, xu, ep, 10, S, tab, ly.HB, clb, R, nullptr, ring_c, n_col,
+    beam_search<MC, T, W>(a, xu, ep, 10, S, tab, clb, R, nullptr, ring_c, n_col,
                           n_adj, ph);
   } else {
     // two-hop ids y_i = G[G[u][i/K]][i%K], i < 480
@@ -820,7 +872,7 @@ void k_forward(PruneArgs a) {
     n_adj = (RING + K - 1) / K;
   }
   __syncthreads();
-  const long long c1 = pclock(a);
+  const long long c1 = pclock(ph);
   // pool = merge(own list, sorted ring), in registers; the own list is a kNN row, sorted by
   // (distance, id) already (builds keep them so, tg_set_knn rejects others)
   uint64_t pv[16];
@@ -842,7 +894,7 @@ void k_forward(PruneArgs a) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) pv[8 + q] = rr[q];
   }
-  const long long c1s = pclock(a);
+  const long long c1s = pclock(ph);
   reg_bitonic_merge<16>(pv);
   __syncthreads();
 #pragma unroll
@@ -862,13 +914,13 @@ void k_forward(PruneArgs a) {
   for (int q = 0; q < PQ; ++q)
     if (dup[q]) P[q * TG_WAVE + lane] = key_with_id(P[q * TG_WAVE + lane], TG_INV);
   __syncthreads();
-  const long long c2 = pclock(a);
+  const long long c2 = pclock(ph);
   int deg;
   if constexpr (MF) deg = filter_pool_mfma<MC, T>(a, P, L, u, a.fwd_rule, sel, cl, km, fq, n_flt, ph);
   else deg = filter_pool<MC, T>(a, P, L, u, a.fwd_rule, sel, cl, n_flt, ph);
   __syncthreads();
-  if (a.phase_clock && lane == 0 && a.counters) {
-    const long long c3 = clock64();
+  if (Ph::on && lane == 0 && a.counters) {
+    const long long c3 = pclock(ph);
     atomicAdd(&cnt_slot(a.counters)[6], (unsigned long long)(c1 - c0));
     atomicAdd(&cnt_slot(a.counters)[7], (unsigned long long)(c3 - c2));
     atomicAdd(&cnt_slot(a.counters)[8], (unsigned long long)(c2 - c1));
@@ -914,7 +966,7 @@ __global__ __launch_bounds__(64) void k_reverse(PruneArgs a) {
     else if (n == 128) merge_pool<2>(a, u, deg, buf, nr, P);
     else merge_pool<4>(a, u, deg, buf, nr, P);
     mark_dups(P, n);
-    PhaseAcc ph;  // not reported for the reverse pass
+    PhaseOff ph;  // not reported for the reverse pass
     int nd;
     if constexpr (MF) nd = filter_pool_mfma<MC, T>(a, P, L, u, a.rev_rule, sel, cl, km, fq, n_flt, ph);
     else nd = filter_pool<MC, T>(a, P, L, u, a.rev_rule, sel, cl, n_flt, ph);
@@ -1200,18 +1252,18 @@ __global__ __launch_bounds__(64) void k_rank_reverse(PruneArgs a) {
 template <int MC, class T>
 __global__ __launch_bounds__(64) void k_cal_ep(PruneArgs a, const float* centroid, uint32_t* ep) {
   __shared__ uint64_t M0[128], S[128];
-  __shared__ uint32_t tab[HSET];
+  __shared__ __attribute__((aligned(16))) uint32_t tab[HS_WORDS];
   __shared__ uint16_t cl[128];
   const uint32_t seg = blockIdx.x;
   const uint32_t start = a.seg_lo ? a.seg_lo[seg] : 0u;
   Row16<MC> c;
   load_row16<MC>(c, centroid + size_t(seg) * a.D, a.D, threadIdx.x & 15);
   uint32_t rc = 0, ne = 0, na = 0;
-  PhaseAcc ph;  // not reported for the entry point
+  PhaseOff ph;  // not reported for the entry point
   if (a.K <= 64 && a.TOPM <= 64)
-    beam_search<MC, T, 1>(a, c, start, 30, S, tab, 9, cl, nullptr, M0, rc, ne, na, ph);
+    beam_search<MC, T, 1>(a, c, start, 30, S, tab, cl, nullptr, M0, rc, ne, na, ph);
   else
-    beam_search<MC, T, 2>(a, c, start, 30, S, tab, 9, cl, nullptr, M0, rc, ne, na, ph);
+    beam_search<MC, T, 2>(a, c, start, 30, S, tab, cl, nullptr, M0, rc, ne, na, ph);
   if (threadIdx.x == 0) ep[seg] = key_id(M0[0]);
   count_add(a.counters, 4, ne);
 }
@@ -1259,14 +1311,20 @@ template <int MC, class T, bool MF>
 static void launch_filter_mc(const PruneArgs& a, int phase, hipStream_t s) {
   const dim3 grid(grid_rows(a.perm, a.N)), block(64);
   const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD, MF && !std::is_same<T, uint8_t>::value);
+#define FWD(KIND, W)                                                                            \
+  do {                                                                                         \
+    if (a.phase_clock) k_forward<MC, T, KIND, W, MF, PhaseOn><<<grid, block, f.bytes, s>>>(a); \
+    else k_forward<MC, T, KIND, W, MF, PhaseOff><<<grid, block, f.bytes, s>>>(a);              \
+  } while (0)
   switch (phase) {
     case PH_FWD_PATH:
-      if (f.W == 1) k_forward<MC, T, 0, 1, MF><<<grid, block, f.bytes, s>>>(a);
-      else k_forward<MC, T, 0, 2, MF><<<grid, block, f.bytes, s>>>(a);
+      if (f.W == 1) FWD(0, 1);
+      else FWD(0, 2);
       break;
-    case PH_FWD_2HOP: k_forward<MC, T, 1, 1, MF><<<grid, block, f.bytes, s>>>(a); break;
+    case PH_FWD_2HOP: FWD(1, 1); break;
     default: k_reverse<MC, T, MF><<<grid, block, 0, s>>>(a); break;
   }
+#undef FWD
 }
 
 template <class T>

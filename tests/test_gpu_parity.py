@@ -502,6 +502,27 @@ def test_block_filter_edges(name, D):
         _compare(X, G, GD, kind, fr, rr, FD, 64, th)
 
 
+@pytest.mark.parametrize("K,TOPM", [(24, 20), (64, 64), (65, 64), (128, 128)])
+def test_path_collect_id_set(K, TOPM):
+    """Path Collect's id set with every list's ids in one bucket, in two neighbours at the
+    table's end, and spread: rows, evaluation counts and entry points equal to the oracle."""
+    rng = np.random.default_rng(K)
+    N = 20000
+    X = rng.integers(0, 200, (N, 8)).astype(np.float32)
+    bucket = (np.arange(N, dtype=np.uint32) * np.uint32(0x9E3779)) >> np.uint32(25)
+    for which in ([5], [126, 127, 0], range(128)):
+        members = np.flatnonzero(np.isin(bucket, which))
+        ids = np.empty((N, K), np.uint32)
+        d = np.empty((N, K), np.float32)
+        for u in range(N):
+            c = rng.choice(members, K + 1, replace=False, shuffle=False)
+            c = c[c != u][:K]
+            dist = ((X[c] - X[u]) ** 2).sum(1)
+            o = np.lexsort((c, dist))
+            ids[u], d[u] = c[o], dist[o]
+        _compare(X, ids, d, 0, 0, 0, 16, TOPM, 1.2)
+
+
 @pytest.mark.parametrize("N,D,K", [(34, 32, 33), (48, 32, 40), (70, 64, 64), (130, 32, 100),
                                    (32768, 32, 8), (32769, 32, 8), (50000, 32, 6)])
 def test_overflow_areas_and_grouping(N, D, K):
