@@ -1063,7 +1063,7 @@ int tg_mlp_eval(int device, uint32_t D, uint32_t B, uint32_t P, const float* X, 
   HIPX(hipMemcpyAsync(w.L.mu, mu, size_t(D) * 4, hipMemcpyHostToDevice, w.st));
   HIPX(hipMemcpyAsync(w.L.scal, &scale, 4, hipMemcpyHostToDevice, w.st));
   HIPX(mlp_set_params(w.L, params, w.st));
-  mlp_forward_backward(w.L, w.X, nullptr, B, P, margin, w.st);
+  mlp_forward_backward(w.L, w.X, B, P, margin, w.st);
   LearnConfig c;
   launch_mlp_adam(w.L, 1, 0, c, w.g, w.st);
   if (int rc = check_launch("encoder check")) return rc;

@@ -23,6 +23,7 @@ namespace {
 
 constexpr int GT = 64;  // GEMM tile edge
 constexpr int GK = 32;  // GEMM k step
+constexpr int GS = 4;   // k steps staged together
 constexpr int GPAD = 8;
 // Grouping chunk: at least 1024 vectors and at most about 1024 chunks, so the stable scatter
 // (one wave per chunk, serial within it) has about four waves per CU and the per-chunk
@@ -41,11 +42,13 @@ struct GemmArgs {
   const uint16_t* B;
   uint32_t M, Nc, Kd, lda, ldb;
   float* Cf;            // EPI_Z: [M x ldc]; EPI_PART: partial z at Cf + z * zstride
+  float* CfT;           // EPI_Z: optional transpose of rows < nT, [Nc x ldct] (ldct % 4 == 0)
+  uint32_t nT;
   uint32_t ldc;
   size_t zstride;
   uint16_t* Cb;         // EPI_H row-major BF16 output
   uint32_t ldcb;
-  uint16_t* CT;         // EPI_H / EPI_DH transposed BF16 output [Nc x ldct]
+  uint16_t* CT;         // EPI_H / EPI_DH transposed BF16 output [Nc x ldct] (M, ldct % 4 == 0)
   uint32_t ldct;
   const float* bias;    // bias of output column j at bias[j * bias_stride]
   uint32_t bias_stride;
@@ -53,10 +56,16 @@ struct GemmArgs {
   uint32_t ldm;
 };
 
+// The products of a training step have few tiles (80 to 640 workgroups) and few k steps, so each
+// is bound by the latency of its chain of loads: GS k steps are staged together behind one
+// barrier, the next group's loads are issued before this group's products, the relu mask is
+// requested before the products, and transposed outputs leave as four rows per store.  The
+// products run in the order of the k steps.  (10240 x 96 batch, one step at a time / this: H 15.8 /
+// 9.0 us, Z 7.7 / 5.8, dH 10.6 / 7.5, weight gradients 10.6 / 7.6.)
 template <int EPI>
 __global__ __launch_bounds__(256) void k_gemm_nt(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[GT][GK + GPAD];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[GT][GK + GPAD];
+  __shared__ __attribute__((aligned(16))) uint16_t As[GT][GS * GK + GPAD];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[GT][GS * GK + GPAD];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const uint32_t row0 = blockIdx.x * GT, col0 = blockIdx.y * GT;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
@@ -68,27 +77,62 @@ __global__ __launch_bounds__(256) void k_gemm_nt(GemmArgs g) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int lr = tid >> 2, lk = (tid & 3) * 8;
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const uint32_t kk = uint32_t(kb) * GK + lk;
-    uint4 va = make_uint4(0, 0, 0, 0), vb = make_uint4(0, 0, 0, 0);
-    if (row0 + lr < g.M) va = *reinterpret_cast<const uint4*>(g.A + size_t(row0 + lr) * g.lda + kk);
-    if (col0 + lr < g.Nc) vb = *reinterpret_cast<const uint4*>(g.B + size_t(col0 + lr) * g.ldb + kk);
-    *reinterpret_cast<uint4*>(&As[lr][lk]) = va;
-    *reinterpret_cast<uint4*>(&Bs[lr][lk]) = vb;
-    __syncthreads();
-    bf16x8 fa[2], fb[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      fa[i] = *reinterpret_cast<const bf16x8*>(&As[wr + 16 * i + (lane & 15)][8 * (lane >> 4)]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      fb[j] = *reinterpret_cast<const bf16x8*>(&Bs[wc + 16 * j + (lane & 15)][8 * (lane >> 4)]);
+  uint16_t hm[2][2][4];
+  if (EPI == EPI_DH) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t col = col0 + wc + 16 * j + (lane & 15);
+          const uint32_t row = row0 + wr + 16 * i + 4 * (lane >> 4) + r;
+          hm[i][j][r] = row < g.M && col < g.Nc ? g.mask[size_t(row) * g.ldm + col] : uint16_t(0);
+        }
+  }
+  const int lr = tid >> 2, lk = (tid & 3) * 8;
+  const bool ina = row0 + lr < g.M, inb = col0 + lr < g.Nc;
+  const uint16_t* Ar = g.A + size_t(ina ? row0 + lr : 0) * g.lda + lk;
+  const uint16_t* Br = g.B + size_t(inb ? col0 + lr : 0) * g.ldb + lk;
+  uint4 va[GS], vb[GS];
+  auto fetch = [&](int kb) {
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      va[q] = vb[q] = make_uint4(0, 0, 0, 0);
+      if (kb + q < kb1) {
+        if (ina) va[q] = *reinterpret_cast<const uint4*>(Ar + size_t(kb + q) * GK);
+        if (inb) vb[q] = *reinterpret_cast<const uint4*>(Br + size_t(kb + q) * GK);
+      }
+    }
+  };
+  fetch(kb0);
+  for (int kb = kb0; kb < kb1; kb += GS) {
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      if (kb + q >= kb1) break;
+      *reinterpret_cast<uint4*>(&As[lr][q * GK + lk]) = va[q];
+      *reinterpret_cast<uint4*>(&Bs[lr][q * GK + lk]) = vb[q];
+    }
+    __syncthreads();
+    if (kb + GS < kb1) fetch(kb + GS);
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      if (kb + q >= kb1) break;
+      bf16x8 fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        fa[i] = *reinterpret_cast<const bf16x8*>(
+            &As[wr + 16 * i + (lane & 15)][q * GK + 8 * (lane >> 4)]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        fb[j] = *reinterpret_cast<const bf16x8*>(
+            &Bs[wc + 16 * j + (lane & 15)][q * GK + 8 * (lane >> 4)]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
     __syncthreads();
   }
   // lane holds C[4 * (lane / 16) + r][lane % 16] of each 16 x 16 tile
@@ -97,27 +141,31 @@ __global__ __launch_bounds__(256) void k_gemm_nt(GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint32_t col = col0 + wc + 16 * j + (lane & 15);
-      if (col >= g.Nc) continue;
       const uint32_t rb = row0 + wr + 16 * i + 4 * (lane >> 4);
+      if (col >= g.Nc || rb >= g.M) continue;
+      float v[4];
+      uint32_t h[4];
+      const float bias =
+          EPI == EPI_H || EPI == EPI_Z ? g.bias[size_t(col) * g.bias_stride] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const uint32_t row = rb + r;
-        if (row >= g.M) continue;
-        float v = acc[i][j][r];
-        if (EPI == EPI_H) {
-          v = fmaxf(v + g.bias[size_t(col) * g.bias_stride], 0.f);
-          const uint16_t b = f2bf(v);
-          g.Cb[size_t(row) * g.ldcb + col] = b;
-          if (g.CT) g.CT[size_t(col) * g.ldct + row] = b;
-        } else if (EPI == EPI_Z) {
-          g.Cf[size_t(row) * g.ldc + col] = v + g.bias[size_t(col) * g.bias_stride];
-        } else if (EPI == EPI_DH) {
-          const float h = bf2f(g.mask[size_t(row) * g.ldm + col]);
-          g.CT[size_t(col) * g.ldct + row] = f2bf(h > 0.f ? v : 0.f);
-        } else {
-          g.Cf[blockIdx.z * g.zstride + size_t(row) * g.ldc + col] = v;
-        }
+        v[r] = acc[i][j][r];
+        if (EPI == EPI_H) v[r] = fmaxf(v[r] + bias, 0.f);
+        if (EPI == EPI_Z) v[r] = v[r] + bias;
+        if (EPI == EPI_DH) v[r] = bf2f(hm[i][j][r]) > 0.f ? v[r] : 0.f;
+        h[r] = EPI == EPI_H || EPI == EPI_DH ? f2bf(v[r]) : 0;
+        if (rb + r >= g.M) continue;
+        if (EPI == EPI_H) g.Cb[size_t(rb + r) * g.ldcb + col] = uint16_t(h[r]);
+        if (EPI == EPI_Z) g.Cf[size_t(rb + r) * g.ldc + col] = v[r];
+        if (EPI == EPI_PART)
+          g.Cf[blockIdx.z * g.zstride + size_t(rb + r) * g.ldc + col] = v[r];
       }
+      if (EPI == EPI_DH || (EPI == EPI_H && g.CT))
+        *reinterpret_cast<uint2*>(g.CT + size_t(col) * g.ldct + rb) =
+            make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+      if (EPI == EPI_Z && g.CfT && rb < g.nT)
+        *reinterpret_cast<float4*>(g.CfT + size_t(col) * g.ldct + rb) =
+            make_float4(v[0], v[1], v[2], v[3]);
     }
 }
 
@@ -127,33 +175,72 @@ void gemm(const GemmArgs& g, uint32_t splits, hipStream_t st) {
   k_gemm_nt<EPI><<<grid, 256, 0, st>>>(g);
 }
 
-// xn = bf16((x - mu) * s) for rows X[rows[m]] (or X[first + m]); Xn [M x D], XnT [D x ldt]
+// A training batch's rows: anchors i < B are samp[j_i], j_i = (pa (step B + i) + pc) mod S, then P
+// positives per anchor, samp[subG[j_i][0..P)]
+struct BatchRows {
+  const uint32_t *samp, *subG;  // samp == nullptr: rows first + m instead
+  uint32_t Ks, S, B, P, step;
+  uint64_t pa, pc;
+};
+
+// xn = bf16((x - mu) * s) for the batch's rows (or X[first + m]); Xn [M x D], XnT [D x ldt].
+// D is a multiple of 32; with XnT, M is one of 4.  Each workgroup works out its own 64 rows (one
+// launch less per step) and every thread's loads are issued together.
+// (10240 x 96 floats: 14.0 -> 5.8 us, and 4.7 us for the rows' own launch.)
 __global__ __launch_bounds__(256) void k_mlp_gather(const float* __restrict__ X, uint32_t D,
-                                                    const uint32_t* __restrict__ rows,
-                                                    uint32_t first, uint32_t M,
+                                                    BatchRows br, uint32_t first, uint32_t M,
                                                     const float* __restrict__ mu,
                                                     const float* __restrict__ scal, uint16_t* Xn,
                                                     uint16_t* XnT, uint32_t ldt) {
-  __shared__ uint16_t tile[64][65];
+  __shared__ uint16_t tile[64][66];
+  __shared__ uint32_t node[64];
   const int tid = threadIdx.x;
   const uint32_t m0 = blockIdx.x * 64, d0 = blockIdx.y * 64;
+  if (tid < 64 && m0 + tid < M) {
+    const uint32_t m = m0 + tid;
+    if (br.samp) {
+      const uint32_t i = m < br.B ? m : (m - br.B) / br.P;
+      const uint32_t j = uint32_t((br.pa * (uint64_t(br.step) * br.B + i) + br.pc) % br.S);
+      node[tid] = br.samp[m < br.B ? j : br.subG[size_t(j) * br.Ks + (m - br.B - i * br.P)]];
+    } else {
+      node[tid] = first + m;
+    }
+  }
+  __syncthreads();
   const float s = scal[0];
-  for (int e = tid; e < 64 * 64; e += 256) {
-    const int r = e >> 6, c = e & 63;
-    const uint32_t m = m0 + r, d = d0 + c;
-    if (m < M && d < D) {
-      const uint32_t node = rows ? rows[m] : first + m;
-      const uint16_t b = f2bf((X[size_t(node) * D + d] - mu[d]) * s);
-      Xn[size_t(m) * D + d] = b;
-      tile[r][c] = b;
+  const int c = (tid & 15) * 4;
+  const uint32_t d = d0 + c;
+  if (d < D) {
+    const float4 mv = *reinterpret_cast<const float4*>(mu + d);
+    float4 x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = q * 16 + (tid >> 4);
+      x[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (m0 + r < M) x[q] = *reinterpret_cast<const float4*>(X + size_t(node[r]) * D + d);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = q * 16 + (tid >> 4);
+      const uint32_t h0 = f2bf((x[q].x - mv.x) * s), h1 = f2bf((x[q].y - mv.y) * s);
+      const uint32_t h2 = f2bf((x[q].z - mv.z) * s), h3 = f2bf((x[q].w - mv.w) * s);
+      const uint2 w = make_uint2(h0 | h1 << 16, h2 | h3 << 16);
+      if (m0 + r < M) *reinterpret_cast<uint2*>(Xn + size_t(m0 + r) * D + d) = w;
+      if (XnT) {
+        *reinterpret_cast<uint32_t*>(&tile[r][c]) = w.x;
+        *reinterpret_cast<uint32_t*>(&tile[r][c + 2]) = w.y;
+      }
     }
   }
   if (!XnT) return;
   __syncthreads();
-  for (int e = tid; e < 64 * 64; e += 256) {
-    const int c = e >> 6, r = e & 63;
-    const uint32_t m = m0 + r, d = d0 + c;
-    if (m < M && d < D) XnT[size_t(d) * ldt + m] = tile[r][c];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int col = q * 16 + (tid >> 4), r = (tid & 15) * 4;
+    if (d0 + col >= D || m0 + r >= M) continue;
+    *reinterpret_cast<uint2*>(XnT + size_t(d0 + col) * ldt + m0 + r) =
+        make_uint2(uint32_t(tile[r][col]) | uint32_t(tile[r + 1][col]) << 16,
+                   uint32_t(tile[r + 2][col]) | uint32_t(tile[r + 3][col]) << 16);
   }
 }
 
@@ -163,24 +250,57 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Sums of 32 values over the 64 lanes, lane l receiving the sum of value l / 2.  Each stage halves
+// the values a lane holds, so 31 exchanges do what 32 butterflies do with 192, and every sum is
+// the butterfly's own tree (partners at distance 32, 16, 8, 4, 2, 1; either order of the two).
+__device__ __forceinline__ float wave_sum32(const float (&v)[32]) {
+  float w[16], x[8], y[4], z[2];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {  // lanes 32..63 go on with values 16..31
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]),
+                                                    __float_as_uint(v[k + 16]), false, false);
+    w[k] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {  // odd rows of 16 lanes with values 8..15
+    const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(w[k]),
+                                                    __float_as_uint(w[k + 8]), false, false);
+    x[k] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  }
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float keep = lane & 8 ? x[k + 4] : x[k], give = lane & 8 ? x[k] : x[k + 4];
+    y[k] = keep + __shfl_xor(give, 8, TG_WAVE);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const float keep = lane & 4 ? y[k + 2] : y[k], give = lane & 4 ? y[k] : y[k + 2];
+    z[k] = keep + __shfl_xor(give, 4, TG_WAVE);
+  }
+  const float keep = lane & 2 ? z[1] : z[0], give = lane & 2 ? z[0] : z[1];
+  const float u = keep + __shfl_xor(give, 2, TG_WAVE);
+  return u + __shfl_xor(u, 1, TG_WAVE);
+}
+
 // Contrastive loss and its gradient with respect to the codes: one workgroup of four waves
 // per pair of anchors (B is even), so each negative's code is read once for both; thread tid
 // takes the negatives c = tid, tid + 256, ... for each anchor in that order, the wave
 // partials are added in wave order, and wave a finishes anchor b0 + a (deterministic, and
-// the same sums as one anchor per workgroup).
+// the same sums as one anchor per workgroup).  The negatives are read from the anchors' transpose
+// ZT [CODE x B] (a wave reads 64 consecutive floats; by rows, each of its loads touched 64
+// lines), the two anchors stay in scalar registers, and the sums go through wave_sum32.  What is
+// left is arithmetic: 64 operations per pair of codes and 32 per active one, about 10 us of the
+// vector units for B = 2048.  (62.3 -> 21.5 us.)
 constexpr int LOSS_AP = 2;
-__global__ __launch_bounds__(256) void k_mlp_loss(const float* __restrict__ Z, uint32_t B,
+__global__ __launch_bounds__(256) void k_mlp_loss(const float* __restrict__ Z,
+                                                  const float* __restrict__ ZT, uint32_t B,
                                                   uint32_t P, float margin, uint32_t M,
                                                   uint16_t* dZb, uint16_t* dZT, float* lossp) {
   __shared__ float red[LOSS_AP][4][MLP_CODE + 2];
-  __shared__ float zas[LOSS_AP][MLP_CODE];
-  const uint32_t b0 = blockIdx.x * LOSS_AP;
+  const uint32_t b0 = blockIdx.x * LOSS_AP;  // B is even
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (tid < LOSS_AP * int(MLP_CODE)) {
-    const uint32_t b = b0 + uint32_t(tid) / MLP_CODE;
-    zas[tid / MLP_CODE][tid % MLP_CODE] = b < B ? Z[size_t(b) * MLP_CODE + tid % MLP_CODE] : 0.f;
-  }
-  __syncthreads();
+  const float* za = Z + size_t(b0) * MLP_CODE;
   float acc[LOSS_AP][MLP_CODE];
   float nact[LOSS_AP], lneg[LOSS_AP];
 #pragma unroll
@@ -190,18 +310,17 @@ __global__ __launch_bounds__(256) void k_mlp_loss(const float* __restrict__ Z, u
     for (int k = 0; k < int(MLP_CODE); ++k) acc[q][k] = 0.f;
   }
   for (uint32_t c = tid; c < B; c += 256) {
-    const float* zc = Z + size_t(c) * MLP_CODE;
     float zv[MLP_CODE];
 #pragma unroll
-    for (int k = 0; k < int(MLP_CODE); ++k) zv[k] = zc[k];
+    for (int k = 0; k < int(MLP_CODE); ++k) zv[k] = ZT[size_t(k) * B + c];
 #pragma unroll
     for (int q = 0; q < LOSS_AP; ++q) {
       const uint32_t b = b0 + uint32_t(q);
-      if (c == b || b >= B) continue;
+      if (c == b) continue;
       float d2 = 0.f;
 #pragma unroll
       for (int k = 0; k < int(MLP_CODE); ++k) {
-        const float e = zas[q][k] - zv[k];
+        const float e = za[q * int(MLP_CODE) + k] - zv[k];
         d2 = fmaf(e, e, d2);
       }
       if (d2 < margin) {
@@ -215,11 +334,8 @@ __global__ __launch_bounds__(256) void k_mlp_loss(const float* __restrict__ Z, u
 #pragma unroll
   for (int q = 0; q < LOSS_AP; ++q) {
     const float n = wave_sum(nact[q]), l = wave_sum(lneg[q]);
-#pragma unroll
-    for (int k = 0; k < int(MLP_CODE); ++k) {
-      const float v = wave_sum(acc[q][k]);
-      if (lane == k) red[q][wave][2 + k] = v;
-    }
+    const float v = wave_sum32(acc[q]);
+    if (!(lane & 1)) red[q][wave][2 + (lane >> 1)] = v;
     if (lane == 0) {
       red[q][wave][0] = n;
       red[q][wave][1] = l;
@@ -229,14 +345,13 @@ __global__ __launch_bounds__(256) void k_mlp_loss(const float* __restrict__ Z, u
   if (wave >= LOSS_AP) return;
   const int qa = wave;
   const uint32_t b = b0 + uint32_t(qa);
-  if (b >= B) return;
   const int k = lane & 31;
   const float na = ((red[qa][0][0] + red[qa][1][0]) + red[qa][2][0]) + red[qa][3][0];
   const float ln = ((red[qa][0][1] + red[qa][1][1]) + red[qa][2][1]) + red[qa][3][1];
   const float accs =
       ((red[qa][0][2 + k] + red[qa][1][2 + k]) + red[qa][2][2 + k]) + red[qa][3][2 + k];
   const float cpos = 2.f / float(B * P), cneg = 4.f / (float(B) * float(B - 1));
-  const float zak = zas[qa][k];
+  const float zak = za[qa * int(MLP_CODE) + k];
   float sp = 0.f, lpos = 0.f;
   for (uint32_t j = 0; j < P; ++j) {
     const uint32_t row = B + b * P + j;
@@ -272,11 +387,16 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float* prm, float* mom, float*
   float p = prm[idx];
   if (mode >= 1) {
     float g = 0.f;
-    if (idx < n1) {
-      for (uint32_t z = 0; z < splits; ++z) g += gpart[size_t(z) * n1 + idx];
-    } else {
-      const uint32_t r = idx - n1;
-      for (uint32_t z = 0; z < splits; ++z) g += gpart[size_t(splits) * n1 + size_t(z) * n2 + r];
+    // the partials, eight requested at a time, added in order (7.4 -> 3.9 us)
+    const float* gp = idx < n1 ? gpart + idx : gpart + size_t(splits) * n1 + (idx - n1);
+    const uint32_t stride = idx < n1 ? n1 : n2;
+    for (uint32_t z = 0; z < splits; z += 8) {
+      float t[8];
+#pragma unroll
+      for (uint32_t q = 0; q < 8; ++q) t[q] = z + q < splits ? gp[size_t(z + q) * stride] : 0.f;
+#pragma unroll
+      for (uint32_t q = 0; q < 8; ++q)
+        if (z + q < splits) g += t[q];
     }
     if (mode == 1) {
       grad_out[idx] = g;
@@ -329,17 +449,6 @@ __global__ void k_scale_final(const double* part, uint32_t nb, uint32_t N, uint3
   for (uint32_t b = 0; b < nb; ++b) t += part[b];
   const double var = t / (double(N) * D);
   scal[0] = var > 0.0 ? float(1.0 / sqrt(var)) : 1.0f;
-}
-
-// batch rows: anchors = samp[perm(step * B + i)], positives = samp[subG[anchor][0..P)]
-__global__ void k_mlp_rows(uint32_t* rows, const uint32_t* __restrict__ samp,
-                           const uint32_t* __restrict__ subG, uint32_t Ks, uint32_t S,
-                           uint32_t B, uint32_t P, uint64_t pa, uint64_t pc, uint32_t step) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= B) return;
-  const uint32_t j = uint32_t((pa * (uint64_t(step) * B + i) + pc) % S);
-  rows[i] = samp[j];
-  for (uint32_t p = 0; p < P; ++p) rows[B + i * P + p] = samp[subG[size_t(j) * Ks + p]];
 }
 
 // ------------------------------------------------------------------ k-means in code space
@@ -681,12 +790,20 @@ __global__ __launch_bounds__(64) void k_seed_lists(const uint32_t* __restrict__ 
   for (int j = lane; j < int(K); j += TG_WAVE) G[size_t(u) * K + j] = acc[j];
 }
 
-// loss of the batch: fixed-order sum of the per-anchor partials (one thread)
-__global__ void k_loss_sum(const float* lossp, uint32_t B, float* out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// loss of the batch: the per-anchor partials added in order by one thread, from LDS (as loads, one
+// at a time: 87 us for 2048)
+__global__ __launch_bounds__(256) void k_loss_sum(const float* __restrict__ lossp, uint32_t B,
+                                                  float* out) {
+  __shared__ float v[256];
   double s = 0.0;
-  for (uint32_t b = 0; b < B; ++b) s += lossp[b];
-  *out = float(s);
+  for (uint32_t b0 = 0; b0 < B; b0 += 256) {
+    if (b0 + threadIdx.x < B) v[threadIdx.x] = lossp[b0 + threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (uint32_t b = 0; b < min(256u, B - b0); ++b) s += v[b];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = float(s);
 }
 
 __global__ void k_fill_u16(uint16_t* p, uint16_t v, size_t n) {
@@ -779,7 +896,6 @@ hipError_t learner_reserve(Learner& L, uint32_t D, uint32_t M, uint32_t N, uint3
   }
   const uint32_t Mb = std::max(M, std::min(N, ENC_CHUNK));
   if (L.Mcap < Mb) {
-    LX(rmalloc(&L.rows, Mb));
     LX(rmalloc(&L.Xn, size_t(Mb) * D));
     LX(rmalloc(&L.XnT, size_t(D + 1) * Mb));
     LX(rmalloc(&L.Hb, size_t(Mb) * MLP_HID));
@@ -788,6 +904,7 @@ hipError_t learner_reserve(Learner& L, uint32_t D, uint32_t M, uint32_t N, uint3
     LX(rmalloc(&L.dZT, size_t(MLP_CODE) * Mb));
     LX(rmalloc(&L.dHT, size_t(MLP_HID) * Mb));
     LX(rmalloc(&L.Z, size_t(Mb) * MLP_CODE));
+    LX(rmalloc(&L.ZT, size_t(Mb) * MLP_CODE));
     LX(rmalloc(&L.lossp, Mb));
     L.Mcap = Mb;
     L.ones_M = 0;
@@ -831,7 +948,6 @@ void learner_release(Learner& L) {
   rfree(L.mu);
   rfree(L.scal);
   rfree(L.dpart);
-  rfree(L.rows);
   rfree(L.Xn);
   rfree(L.XnT);
   rfree(L.Hb);
@@ -840,6 +956,7 @@ void learner_release(Learner& L) {
   rfree(L.dZT);
   rfree(L.dHT);
   rfree(L.Z);
+  rfree(L.ZT);
   rfree(L.lossp);
   rfree(L.codes);
   rfree(L.cent);
@@ -883,8 +1000,10 @@ void launch_mlp_adam(Learner& L, int mode, uint32_t t, const LearnConfig& c, flo
                                               L.W2b, L.W2Tb, grad_out);
 }
 
-void mlp_forward_backward(Learner& L, const float* X, const uint32_t* rows, uint32_t B,
-                          uint32_t P, float margin, hipStream_t st) {
+namespace {
+// one batch: rows `br`, or (without samp) X's first B (1 + P) rows; B is a multiple of 32
+void forward_backward(Learner& L, const float* X, const BatchRows& br, uint32_t B, uint32_t P,
+                      float margin, hipStream_t st) {
   const uint32_t D = L.D, M = B * (1 + P);
   // row of ones closing Xn^T and H^T (bias gradients); unchanged while M is
   if (L.ones_M != M) {
@@ -892,7 +1011,7 @@ void mlp_forward_backward(Learner& L, const float* X, const uint32_t* rows, uint
     k_fill_u16<<<(M + 255) / 256, 256, 0, st>>>(L.HT + size_t(MLP_HID) * M, 0x3F80, M);
     L.ones_M = M;
   }
-  k_mlp_gather<<<dim3((M + 63) / 64, (D + 63) / 64), 256, 0, st>>>(X, D, rows, 0, M, L.mu, L.scal,
+  k_mlp_gather<<<dim3((M + 63) / 64, (D + 63) / 64), 256, 0, st>>>(X, D, br, 0, M, L.mu, L.scal,
                                                                    L.Xn, L.XnT, M);
   GemmArgs g{};
   // H = relu(Xn W1^T + b1)
@@ -903,10 +1022,9 @@ void mlp_forward_backward(Learner& L, const float* X, const uint32_t* rows, uint
   g = GemmArgs{};
   g.A = L.Hb; g.lda = MLP_HID; g.B = L.W2b; g.ldb = MLP_HID; g.M = M; g.Nc = MLP_CODE;
   g.Kd = MLP_HID; g.Cf = L.Z; g.ldc = MLP_CODE; g.bias = L.prm + mlp_n1(D) + MLP_HID;
-  g.bias_stride = MLP_HID + 1;
+  g.bias_stride = MLP_HID + 1; g.CfT = L.ZT; g.ldct = B; g.nT = B;
   gemm<EPI_Z>(g, 1, st);
-  k_mlp_loss<<<(B + LOSS_AP - 1) / LOSS_AP, 256, 0, st>>>(L.Z, B, P, margin, M, L.dZb, L.dZT,
-                                                         L.lossp);
+  k_mlp_loss<<<B / LOSS_AP, 256, 0, st>>>(L.Z, L.ZT, B, P, margin, M, L.dZb, L.dZT, L.lossp);
   const uint32_t kt = M / GK;
   const uint32_t splits = std::min(L.splits, std::max(1u, kt));
   // unused split slots must read as zero in the reduction
@@ -929,6 +1047,12 @@ void mlp_forward_backward(Learner& L, const float* X, const uint32_t* rows, uint
   g.Cf = L.gpart; g.ldc = D + 1; g.zstride = mlp_n1(D);
   gemm<EPI_PART>(g, splits, st);
 }
+}  // namespace
+
+void mlp_forward_backward(Learner& L, const float* X, uint32_t B, uint32_t P, float margin,
+                          hipStream_t st) {
+  forward_backward(L, X, BatchRows{}, B, P, margin, st);
+}
 
 void mlp_encode(Learner& L, const float* X, uint32_t first, uint32_t n, float* out,
                 hipStream_t st) {
@@ -936,7 +1060,7 @@ void mlp_encode(Learner& L, const float* X, uint32_t first, uint32_t n, float* o
   for (uint32_t c0 = 0; c0 < n; c0 += L.Mcap) {
     const uint32_t m = std::min(L.Mcap, n - c0);
     k_mlp_gather<<<dim3((m + 63) / 64, (D + 63) / 64), 256, 0, st>>>(
-        X, D, nullptr, first + c0, m, L.mu, L.scal, L.Xn, nullptr, 0);
+        X, D, BatchRows{}, first + c0, m, L.mu, L.scal, L.Xn, nullptr, 0);
     GemmArgs g{};
     g.A = L.Xn; g.lda = D; g.B = L.W1b; g.ldb = D; g.M = m; g.Nc = MLP_HID; g.Kd = D;
     g.Cb = L.Hb; g.ldcb = MLP_HID; g.CT = nullptr; g.bias = L.prm + D; g.bias_stride = D + 1;
@@ -996,11 +1120,10 @@ hipError_t learned_seed(Learner& L, const float* X, uint32_t N, uint32_t D, uint
     uint32_t t = 0;
     for (uint32_t ep = 0; ep < c.epochs; ++ep) {
       for (uint32_t sidx = 0; sidx < steps; ++sidx) {
-        k_mlp_rows<<<(B + 255) / 256, 256, 0, st>>>(L.rows, samp, subG, Ks, S, B, P,
-                                                   perm_a[ep], perm_c[ep], sidx);
-        mlp_forward_backward(L, X, L.rows, B, P, c.margin, st);
+        const BatchRows br{samp, subG, Ks, S, B, P, sidx, perm_a[ep], perm_c[ep]};
+        forward_backward(L, X, br, B, P, c.margin, st);
         if (sidx + 1 == steps && (ep == 0 || ep + 1 == c.epochs))
-          k_loss_sum<<<1, 64, 0, st>>>(L.lossp, B, L.loss_hist + (ep == 0 ? 0 : 1));
+          k_loss_sum<<<1, 256, 0, st>>>(L.lossp, B, L.loss_hist + (ep == 0 ? 0 : 1));
         launch_mlp_adam(L, 2, ++t, c, nullptr, st);
       }
     }
@@ -1014,7 +1137,8 @@ hipError_t learned_seed(Learner& L, const float* X, uint32_t N, uint32_t D, uint
     mix(uint64_t(reinterpret_cast<uintptr_t>(X)));
     mix(uint64_t(reinterpret_cast<uintptr_t>(samp)));
     mix(uint64_t(reinterpret_cast<uintptr_t>(subG)));
-    mix(uint64_t(reinterpret_cast<uintptr_t>(L.rows)));
+    mix(uint64_t(reinterpret_cast<uintptr_t>(L.Xn)));
+    mix(uint64_t(reinterpret_cast<uintptr_t>(L.ZT)));
     mix(uint64_t(reinterpret_cast<uintptr_t>(L.prm)));
     mix(uint64_t(reinterpret_cast<uintptr_t>(L.gpart)));
     mix(N); mix(D); mix(S); mix(Ks); mix(B); mix(P); mix(c.epochs); mix(seed);

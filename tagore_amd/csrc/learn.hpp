@@ -35,10 +35,10 @@ struct Learner {
   double* dpart = nullptr;  // [ceil(rows/1024) * max(D,1)] column / scale partials
   uint32_t dpart_rows = 0;
   // batch (M rows: B anchors, then B*P positives)
-  uint32_t* rows = nullptr;
   uint16_t *Xn = nullptr, *XnT = nullptr, *Hb = nullptr, *HT = nullptr;
   uint16_t *dZb = nullptr, *dZT = nullptr, *dHT = nullptr;
   float *Z = nullptr, *lossp = nullptr;
+  float* ZT = nullptr;      // the anchors' codes transposed, [CODE x B]
   uint32_t ones_M = 0;  // batch size whose rows of ones are in place in XnT / HT
   // codes and buckets
   float* codes = nullptr;  // [N * CODE]
@@ -85,11 +85,11 @@ void launch_mlp_stats(Learner& L, const float* Xs, uint32_t S, uint32_t D, hipSt
 // Initialise the parameters from host values (flat block) and clear the Adam moments.
 hipError_t mlp_set_params(Learner& L, const float* host_prm, hipStream_t st);
 
-// One forward/backward over a batch whose rows are X[rows[i]] (rows == null: X[i]); rows
-// [0,B) are anchors, rows B + b*P + j the positives of anchor b.  Leaves the split-K gradient
-// partials in L.gpart and per-anchor losses in L.lossp.
-void mlp_forward_backward(Learner& L, const float* X, const uint32_t* rows, uint32_t B,
-                          uint32_t P, float margin, hipStream_t st);
+// One forward/backward over the batch X[0 .. B (1 + P)) (B a multiple of 32): rows [0,B) are
+// anchors, rows B + b*P + j the positives of anchor b.  Leaves the split-K gradient partials in
+// L.gpart and per-anchor losses in L.lossp.
+void mlp_forward_backward(Learner& L, const float* X, uint32_t B, uint32_t P, float margin,
+                          hipStream_t st);
 // mode 0: refresh the BF16 weight copies; 1: reduce the gradient into grad_out only;
 // 2: Adam step (t >= 1) then refresh the copies.
 void launch_mlp_adam(Learner& L, int mode, uint32_t t, const LearnConfig& c, float* grad_out,

@@ -32,6 +32,12 @@ def _params(D, seed):
     return p
 
 
+@pytest.mark.parametrize("D,B,P", [(32, 32, 16), (160, 96, 3), (96, 2048, 4), (1024, 64, 1)])
+def test_encoder_tile_remainders(D, B, P):
+    """One k step and many, half tiles, rows beyond the last full tile, the default batch."""
+    test_encoder_matches_oracle(D, B, P)
+
+
 @pytest.mark.parametrize("D,B,P", [(128, 64, 4), (96, 32, 2), (64, 128, 1)])
 def test_encoder_matches_oracle(D, B, P):
     _say(f"encoder D={D} B={B} P={P}")
