@@ -1144,7 +1144,9 @@ int learned_init(tg_state* s, const tg_knn_params* p, uint64_t* evals) {
   sp.K = Ks;
   sp.iters = 4;
   sp.seed = p->seed ^ 0x5A3D1E5Bull;
-  sp.precision = TG_PREC_EXACT;
+  // the caller's kind of screen (same lists and counts as EXACT; 50000 x 96 unit rows 2.80 / 1.93 /
+  // 1.81 ms with EXACT / FP32 / BF16, x 960 13.4 / 12.2 / 10.5, x 128 u8 rows 2.84 / 1.40 / 1.39)
+  sp.precision = p->precision == TG_PREC_FP8 ? uint32_t(TG_PREC_BF16) : p->precision;
   sp.init = TG_INIT_RANDOM;
   sp.flags = TG_FLAG_GRAPH_ITERS;  // short kernels: later builds replay the captured sequence
   if (int rc = tg_knn_build(s->sub, &sp)) return rc;
