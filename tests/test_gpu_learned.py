@@ -157,3 +157,30 @@ def test_training_graph_replays_match_eager():
             assert np.array_equal(G_g, G_e) and np.array_equal(GD_g, GD_e), f"lists, replay {rep}"
             assert s.stats()["learn_loss"] == loss_e
             s.knn_build(32, 2, 1 + rep, "bf16")  # unrelated device work between replays
+
+
+@pytest.mark.parametrize("N,D,S", [(64, 32, 64), (4096, 32, 4096), (4097, 64, 4097), (9000, 96, 5003)])
+def test_learned_sample_remainders(N, D, S):
+    """One bucket and several, label tiles of exactly 4096 and one more, a sample that half
+    duplicates: canonical lists, and the iterations from them equal to the oracle with every
+    screen that the sample's own graph can take."""
+    rng = np.random.default_rng(N)
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    X[N // 2:] = X[rng.integers(0, N // 2, N - N // 2)] + np.float32(1e-3)
+    K, seed = 12, 0x99
+    lists = []
+    for prec in ("exact", "fp32", "bf16"):
+        _say(f"learned N={N} D={D} S={S} {prec}")
+        with State(N, D) as s:
+            s.set_data(X)
+            s.knn_build(K, 0, seed, prec, init="learned", sample=S)
+            G0, GD0 = s.get_knn()
+            _check_lists(X, G0, GD0)
+            lists.append((G0, GD0, s.codes()))
+            s.knn_build(K, 4, seed, prec, init="learned", sample=S)
+            G4, GD4 = s.get_knn()
+        ref, refd, _ = oracle.gnn_descent(X, K, 4, seed, init=(G0, GD0))
+        assert np.array_equal(G4, ref) and np.array_equal(GD4, refd)
+    for other in lists[1:]:
+        for x, y in zip(lists[0], other):
+            assert np.array_equal(x, y)
