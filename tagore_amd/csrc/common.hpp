@@ -623,10 +623,9 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 // overflow array is split into OV_AREAS areas with a counter each, a workgroup starting at its
 // own and going on to the next when one is full: with a single counter the waves of a graph
 // with hubs queued for it (sampling of 500k x 96, K = 64: 4.7 -> 0.9 ms; the u8 local join of
-// 1M x 128, K = 96: 11.0 -> 8.7 ms).  Overflow beyond ov_cap sets
-// *err.
+// 1M x 128, K = 96: 11.0 -> 8.7 ms, both with 64 areas).  Overflow beyond ov_cap sets *err.
 // ---------------------------------------------------------------------------------------
-constexpr uint32_t OV_AREAS = 64;
+constexpr uint32_t OV_AREAS = 256;
 constexpr uint32_t OV_STRIDE = 32;  // words between the areas' counters (a cache line each)
 struct PushBuf {
   uint32_t* cnt;       // [N] pushes per destination

@@ -116,8 +116,11 @@ struct GroupArgs {
 
 // whether any overflow entry was taken (a wave-uniform answer, in every wave)
 __device__ __forceinline__ bool pb_overflowed(const PushBuf& pb) {
-  static_assert(OV_AREAS == TG_WAVE, "one counter per lane");
-  return __ballot(pb.ov_used[lane_id() * OV_STRIDE] != 0) != 0;
+  static_assert(OV_AREAS % TG_WAVE == 0, "whole rounds of lanes");
+  uint32_t used = 0;
+#pragma unroll
+  for (uint32_t a = 0; a < OV_AREAS; a += TG_WAVE) used |= pb.ov_used[(a + lane_id()) * OV_STRIDE];
+  return __ballot(used != 0) != 0;
 }
 
 struct ResetArgs {
