@@ -681,55 +681,67 @@ __device__ __forceinline__ uint64_t pb_get(const PushBuf& pb, uint32_t v, uint32
   return o < pb.ov_cap ? pb.ov_sorted[o] : TG_KEY_INF;
 }
 
-// Keeps the R smallest keys pushed to v that pass `pred` (and, if uniq, merges identical
-// keys), sorted ascending into buf[0..R); returns how many there are (<= R <= 128).
-// buf must hold 256 u64 (LDS).  Optional seed keys (sorted, unique, <= R, all passing pred)
-// start the running selection.
+// pb_top for at most 64 NPL keys: they go to registers straight from memory, are sorted there
+// and leave through LDS once, compacted.  (Through LDS before and after the sort, the count read
+// after the row: k_merge 784 -> 719 us, k_rev_reduce 543 -> 425, k_rupdate 301 -> 232 for
+// 1M x 128, K = 96; 143 -> 109 and 86 -> 57 for k_merge and k_rupdate of 160k x 96, K = 64.)
+template <int NPL, class Pred>
+__device__ __forceinline__ int pb_top_reg(const PushBuf& pb, uint32_t v, uint32_t n, int R,
+                                          bool uniq, Pred pred, uint64_t* buf,
+                                          const uint64_t* seed, int nseed) {
+  const int lane = threadIdx.x, tot = nseed + int(n);
+  uint64_t k[NPL];
+#pragma unroll
+  for (int r = 0; r < NPL; ++r) {
+    const int i = r * TG_WAVE + lane;
+    k[r] = TG_KEY_INF;
+    if (i < nseed) k[r] = seed[i];
+    else if (i < tot) k[r] = pb_get(pb, v, uint32_t(i - nseed));
+  }
+#pragma unroll
+  for (int r = 0; r < NPL; ++r)
+    if (r * TG_WAVE + lane >= nseed && !pred(k[r])) k[r] = TG_KEY_INF;
+  if constexpr (NPL == 1) {
+    if (tot <= 16) reg_bitonic_upto<16>(k[0]);
+    else if (tot <= 32) reg_bitonic_upto<32>(k[0]);
+    else reg_bitonic_upto<64>(k[0]);
+  } else {
+    reg_bitonic<NPL>(k);
+  }
+  int pos = 0;
+  uint64_t last = TG_KEY_INF;  // the previous slot's last key (no key equals it)
+#pragma unroll
+  for (int r = 0; r < NPL; ++r) {
+    bool keep = k[r] != TG_KEY_INF;
+    if (uniq) {
+      const uint64_t up = uint64_t(__shfl_up(long(k[r]), 1, TG_WAVE));
+      keep = keep && k[r] != (lane == 0 ? last : up);
+      last = readlane64(k[r], TG_WAVE - 1);
+    }
+    const uint64_t m = ballot(keep);
+    const int p = pos + mask_rank(m);
+    if (keep && p < R) buf[p] = k[r];
+    pos += int(__popcll(m));
+  }
+  __syncthreads();
+  return pos < R ? pos : R;
+}
+
+// Keeps the R smallest of the n = pb_count keys pushed to v that pass `pred` (and, if uniq,
+// merges identical keys), sorted ascending into buf[0..R); returns how many there are (<= R <=
+// 128).  buf must hold 256 u64 (LDS).  Optional seed keys (sorted, unique, <= R, all passing
+// pred) start the running selection.
 template <class Pred>
-__device__ int pb_top(const PushBuf& pb, uint32_t v, int R, bool uniq, Pred pred, uint64_t* buf,
-                      const uint64_t* seed = nullptr, int nseed = 0) {
+__device__ int pb_top(const PushBuf& pb, uint32_t v, uint32_t n, int R, bool uniq, Pred pred,
+                      uint64_t* buf, const uint64_t* seed = nullptr, int nseed = 0) {
   const int lane = threadIdx.x;
-  const uint32_t n = pb_count(pb, v);
-  if (uint32_t(nseed) + n <= 256) {
-    // seed and pushes fit buf together (most nodes): one sort of the next power of two
-    // above their count, then the first R (unique if requested) -- what the chunked path
-    // selects
-    const int tot = nseed + int(n);
-    const int m = pow2_at_least(max(tot, 1));
-    for (int i = lane; i < m; i += TG_WAVE) {
-      uint64_t k = TG_KEY_INF;
-      if (i < nseed) {
-        k = seed[i];
-      } else if (i < tot) {
-        k = pb_get(pb, v, uint32_t(i - nseed));
-        if (!pred(k)) k = TG_KEY_INF;
-      }
-      buf[i] = k;
-    }
-    __syncthreads();
-    wave_sort<256>(buf, m);
-    uint64_t kk[4];
-    bool kp[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {  // every read before any write
-      const int i = r * TG_WAVE + lane;
-      kk[r] = i < m ? buf[i] : TG_KEY_INF;
-      kp[r] = kk[r] != TG_KEY_INF && (!uniq || i == 0 || buf[i - 1] != kk[r]);
-    }
-    __syncthreads();
-    int pos = 0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint64_t bm = ballot(kp[r]);
-      const int p = pos + mask_rank(bm);
-      if (kp[r] && p < R) buf[p] = kk[r];
-      pos += int(__popcll(bm));
-    }
-    const int nb = pos < R ? pos : R;
-    __syncthreads();
-    for (int i = nb + lane; i < 256; i += TG_WAVE) buf[i] = TG_KEY_INF;
-    __syncthreads();
-    return nb;
+  // seed and pushes fit registers together (most nodes): one sort of the next power of two above
+  // their number, then the first R (unique if requested) -- what the chunked path selects
+  const uint32_t tot = uint32_t(nseed) + n;
+  if (n <= 256 && tot <= 256) {
+    if (tot <= 64) return pb_top_reg<1>(pb, v, n, R, uniq, pred, buf, seed, nseed);
+    if (tot <= 128) return pb_top_reg<2>(pb, v, n, R, uniq, pred, buf, seed, nseed);
+    return pb_top_reg<4>(pb, v, n, R, uniq, pred, buf, seed, nseed);
   }
   int nbest = nseed;
   for (int i = lane; i < 128; i += TG_WAVE) buf[i] = i < nseed ? seed[i] : TG_KEY_INF;

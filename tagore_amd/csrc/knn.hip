@@ -187,7 +187,7 @@ __global__ __launch_bounds__(64) void k_rsample(KnnArgs a) {
       else reg_bitonic_upto<64>(key[kind]);
       r = min(int(n[kind]), S);
     } else {
-      r = pb_top(pb, v, S, false, [](uint64_t) { return true; }, buf);
+      r = pb_top(pb, v, n[kind], S, false, [](uint64_t) { return true; }, buf);
       key[kind] = lane < r ? buf[lane] : TG_KEY_INF;
       __syncthreads();
     }
@@ -353,9 +353,10 @@ __global__ __launch_bounds__(64) void k_merge(KnnArgs a) {
   // before any row changes) and entered only below its worst distance and when not listed;
   // a build's distances are canonical (its lists start from the initial sort), so a listed
   // id would have arrived with its listed key.  No id search is needed here.
+  const uint32_t n = pb_count(a.pc, v);
   load_row_lds(a, a.G, a.GD, v, row);
   const float worst = key_d(row.gk[K - 1]);
-  const int nc = pb_top(a.pc, v, K, true,
+  const int nc = pb_top(a.pc, v, n, K, true,
                         [&](uint64_t k) { return key_id(k) != v && key_d(k) < worst; }, buf);
   if (nc > 0)
     merge_row(K, row.gk, row.vf, buf, nc, a.G + size_t(v) * K, a.GD + size_t(v) * K,
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(64) void k_rev_reduce(KnnArgs a) {
   const uint32_t v = blockIdx.x;
   if (v >= a.N) return;
   const int K = a.K;
-  const int n = pb_top(a.pr, v, K, true, [](uint64_t) { return true; }, buf);
+  const int n = pb_top(a.pr, v, pb_count(a.pr, v), K, true, [](uint64_t) { return true; }, buf);
   for (int i = threadIdx.x; i < K; i += TG_WAVE) {
     a.R0[size_t(v) * K + i] = i < n ? buf[i] : TG_KEY_INF;
     a.V[size_t(v) * K + i] = 0;
@@ -989,9 +990,10 @@ __global__ __launch_bounds__(64) void k_rupdate(KnnArgs a) {
   if (w >= a.N) return;
   const int K = a.K;
   const int n0 = a.Rn0[w];
-  for (int i = threadIdx.x; i < n0; i += TG_WAVE) seed[i] = a.R0[size_t(w) * K + i];
+  const uint32_t np = pb_count(a.pr, w);
+  for (int i = threadIdx.x; i < K; i += TG_WAVE) seed[i] = a.R0[size_t(w) * K + i];
   __syncthreads();
-  const int n = pb_top(a.pr, w, K, true, [](uint64_t) { return true; }, buf, seed, n0);
+  const int n = pb_top(a.pr, w, np, K, true, [](uint64_t) { return true; }, buf, seed, n0);
   for (int i = threadIdx.x; i < K; i += TG_WAVE)
     a.R1[size_t(w) * K + i] = i < n ? buf[i] : TG_KEY_INF;
   if (threadIdx.x == 0) a.Rn1[w] = n;

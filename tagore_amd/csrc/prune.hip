@@ -955,7 +955,7 @@ __global__ __launch_bounds__(64) void k_reverse(PruneArgs a) {
   if (u >= a.N) return;
   const int lane = threadIdx.x;
   const int K = a.K, FD = a.FD;
-  const int nr = pb_top(a.rev, u, K, false, [](uint64_t) { return true; }, buf);
+  const int nr = pb_top(a.rev, u, pb_count(a.rev, u), K, false, [](uint64_t) { return true; }, buf);
   const int deg = a.fwd_deg[u];
   const int L = deg + nr;
   uint32_t* row = a.out_ids + size_t(u) * FD;
@@ -1199,10 +1199,11 @@ __global__ __launch_bounds__(64) void k_rank_reverse(PruneArgs a) {
   if (u >= a.N) return;
   const int lane = threadIdx.x;
   const int d = a.FD, h = d / 2;
+  const uint32_t np = pb_count(a.rev, u);
   for (int i = lane; i < 128; i += TG_WAVE)
     T[i] = i < d ? a.fwd_ids[size_t(u) * d + i] : TG_INV;
   // R1[u]: the d smallest (detour, src) pushes, already sorted by (detour, id)
-  const int r = pb_top(a.rev, u, d, false, [](uint64_t) { return true; }, buf);
+  const int r = pb_top(a.rev, u, np, d, false, [](uint64_t) { return true; }, buf);
   uint32_t* row = a.out_ids + size_t(u) * d;
   // Later copies of a source get detour INV and go last, by id.  Sources repeat only where a
   // given kNN row lists an id twice.
