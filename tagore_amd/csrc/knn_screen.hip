@@ -269,11 +269,17 @@ __device__ __forceinline__ uint64_t key_min_row16(float d, uint32_t id) {
 }
 
 // Membership of Q keys in kNN rows (rows sorted by (distance, id), canonical distances):
-// found[q] = key[q] is an entry of row v[q], for the searches with on[q].  The binary searches
-// run on the distances alone -- one load per step; the ids are read where a distance is equal
-// -- and in lockstep, so the dependent loads of one step are in flight together.  (Every lane
-// searches a row of its own, so each load is an L2 request of its own: their number sets the
-// push phase's time.)
+// found[q] = key[q] is an entry of row v[q], for the searches with on[q], whose keys lie below
+// the row's last distance.  Every lane searches a row of its own, so each load is an L2 request of
+// its own, and their number and round trips set the push phase's time.  A search runs on
+// blocks of four distances: by the blocks' last ones, then one load for the block (any 4-byte
+// alignment); the ids are read where a distance is equal.  The searches go in lockstep, so the
+// loads of one step are in flight together.  (By single distances, two or three requests and as
+// many round trips more: local join 2290 -> 2151 us for 1M x 128 u8 rows, K = 96; 1590 -> 1493 for
+// 160k x 96 clusters, K = 64.)
+struct __attribute__((packed, aligned(4))) Dist4 {
+  float x[4];
+};
 template <int Q>
 __device__ __forceinline__ void rows_have_keys(const uint32_t* G, const float* GD, int K,
                                                const uint32_t (&v)[Q], const uint64_t (&key)[Q],
@@ -283,11 +289,11 @@ __device__ __forceinline__ void rows_have_keys(const uint32_t* G, const float* G
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     lo[q] = 0;
-    hi[q] = on[q] ? K : 0;
+    hi[q] = on[q] ? (K + 3) / 4 - 1 : 0;
     row[q] = GD + size_t(v[q]) * K;
     found[q] = false;
   }
-  // lower bound of the distance
+  // the first block whose last distance is not below the key's (the last block at the latest)
   for (;;) {
     bool any = false;
 #pragma unroll
@@ -298,7 +304,7 @@ __device__ __forceinline__ void rows_have_keys(const uint32_t* G, const float* G
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       mid[q] = (lo[q] + hi[q]) >> 1;
-      x[q] = lo[q] < hi[q] ? row[q][mid[q]] : 0.f;
+      x[q] = lo[q] < hi[q] ? row[q][4 * mid[q] + 3] : 0.f;
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -308,15 +314,31 @@ __device__ __forceinline__ void rows_have_keys(const uint32_t* G, const float* G
       }
     }
   }
-  // the entries of that distance
+  // its first entry of that distance, and that entry's id
+  int at[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
+    at[q] = -1;
     if (!on[q]) continue;
-    for (int p = lo[q]; p < K && row[q][p] == key_d(key[q]); ++p)
-      if (G[size_t(v[q]) * K + p] == key_id(key[q])) {
-        found[q] = true;
-        break;
-      }
+    const float d = key_d(key[q]);
+    if (K >= 4) {
+      const int s = min(4 * lo[q], K - 4);  // the entries before the block's are below d
+      const Dist4 y = *reinterpret_cast<const Dist4*>(row[q] + s);
+#pragma unroll
+      for (int k = 3; k >= 0; --k) at[q] = y.x[k] == d ? s + k : at[q];
+    } else {
+      for (int k = K - 1; k >= 0; --k) at[q] = row[q][k] == d ? k : at[q];
+    }
+  }
+  uint32_t id[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) id[q] = at[q] >= 0 ? G[size_t(v[q]) * K + at[q]] : TG_INV;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (at[q] < 0) continue;
+    found[q] = id[q] == key_id(key[q]);
+    for (int p = at[q] + 1; !found[q] && p < K && row[q][p] == key_d(key[q]); ++p)
+      found[q] = G[size_t(v[q]) * K + p] == key_id(key[q]);
   }
 }
 
