@@ -544,6 +544,27 @@ def test_overflow_areas_and_grouping(N, D, K):
     _compare(X, Gr, GDr, 0, 0, 0, min(K, 24), 32, 1.2)
 
 
+@pytest.mark.parametrize("n", [16, 17, 32, 33, 64, 65, 128, 129, 256, 257])
+def test_push_list_sizes(n):
+    """A hub with n pushers, around the sizes where the lists' register sorts change.  Graphs and
+    the NSG prune equal to the oracle."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n + 1, 32)).astype(np.float32)
+    X[n // 2] = 0.01 * X[n // 2]  # nearest to everything
+    K = min(n - 1, 12)
+    _say(f"hub of {n}")
+    Gr, GDr, ev = oracle.gnn_descent(X, K, 6, 5)
+    assert np.count_nonzero(Gr == n // 2) == n
+    for prec in ("exact", "bf16"):
+        with State(n + 1, 32) as s:
+            s.set_data(X)
+            s.knn_build(K, 6, 5, prec)
+            G, GD = s.get_knn()
+            assert s.stats()["knn_evals"] == ev
+        assert np.array_equal(G, Gr) and np.array_equal(GD, GDr)
+    _compare(X, Gr, GDr, 0, 0, 0, K, 32, 1.2)
+
+
 @pytest.mark.parametrize("lo,hi", [(0, 255), (-200, 200)])
 @pytest.mark.parametrize("D,K", [(4, 3), (20, 17), (64, 16), (100, 33), (128, 64), (136, 40),
                                  (256, 20), (264, 12)])
