@@ -594,7 +594,7 @@ void k_localjoin_exact_screen(KnnArgs a) {
 // every queued pair is offered to both jobs.  The queue is worked by all 16 lane groups:
 //   * rows up to 256 elements (MC <= 4): straight from global memory, where the block's rows
 //     have just been read (L2);
-//   * wider rows: 64 elements of every queued row at a time through LDS, 16 pairs per group
+//   * wider rows: 64 elements of every queued row at a time through LDS, 12 pairs per group
 //     with their partial sums in registers -- a row is read once more, not once per pair.
 // Two iterations of 500k x 96 (K = 64, learned lists, 150 re-scores per node): 48.5 -> 13.0 ms;
 // eight of 160k x 96 clusters from random lists 46 -> 12.8 ms; two of 100k x 960 (170 re-scores
@@ -777,8 +777,11 @@ void k_localjoin_screen(KnnArgs a) {
         if (t < NB && e0 + gg + 16 * t < n) offer(t == 0 ? ent[0] : ent[1], t == 0 ? dd[0] : d1);
       }
     } else {
-      // 64 elements of every row at a time; pass p0 holds pairs p0 + gg + 16 k in group gg
-      constexpr int PK = 16;
+      // 64 elements of every row at a time; pass p0 holds pairs p0 + gg + 16 k in group gg.  PK:
+      // what three waves per SIMD keep in registers; a second pass for nodes with more than 192
+      // pairs costs less than spills (learned build of 100k x 960, PK 8 / 10 / 12 / 16 / 20:
+      // 32.7 / 32.2 / 32.2 / 33.5 / 44.0 ms; 60k x 288 from random lists, 12 / 16: 16.3 / 19.4)
+      constexpr int PK = 12;
       constexpr int PPR = 64 * int(sizeof(T)) / 16, NP = 128 * PPR / 256;
       unsigned char* stage = smem + KEYS + QBYTES;
       for (int p0 = 0; p0 < n; p0 += 16 * PK) {
