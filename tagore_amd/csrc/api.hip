@@ -168,6 +168,7 @@ struct tg_state {
   bool cert_int = false;           // integer data whose screen distances are exact
   bool cert_u8 = false;            // and every value in [0, 255]: X8 holds the u8 copy
   uint8_t* X8 = nullptr;
+  uint32_t* x8_ok = nullptr;       // device word: X8 matches X (SearchArgs)
   float* n2s = nullptr;            // [N] |x - 128|^2 of the u8 rows
   uint32_t* fill = nullptr;
   uint32_t* scan_tmp = nullptr;
@@ -403,6 +404,7 @@ int ensure_prep(tg_state* s) {
     if (!s->n2s && dalloc(&s->n2s, N)) return TG_ERR_HIP;
     launch_make_u8(s->X, N * s->D, s->X8, s->stream);
     if (s->D <= 256) launch_u8_shift_norms(s->X8, s->N, s->D, s->n2s, s->stream);
+    fill_u32(s->x8_ok, 1, 1, s->stream);
   }
   s->prep_valid = true;
   return TG_OK;
@@ -571,7 +573,7 @@ int tg_create(uint32_t N, uint32_t D, int device, tg_state** out) {
     return fail(TG_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
   if (dalloc(&s->X, size_t(N) * D) || dalloc(&s->misc, 64) || dalloc(&s->centroid, D) ||
-      dalloc(&s->ep_dev, 1)) {
+      dalloc(&s->ep_dev, 1) || dalloc(&s->x8_ok, 1)) {
     std::string m = g_err;
     tg_free(s);
     return fail(TG_ERR_HIP, m);
@@ -627,6 +629,7 @@ int tg_free(tg_state* s) {
   dfree(s->nrm2);
   dfree(s->cert_flags);
   dfree(s->X8);
+  dfree(s->x8_ok);
   dfree(s->n2s);
   dfree(s->fill);
   dfree(s->scan_tmp);
@@ -655,6 +658,7 @@ int tg_free(tg_state* s) {
 int tg_set_data(tg_state* s, const float* rows) {
   if (!s || !rows) return fail(TG_ERR_ARG, "null argument");
   HIPX(hipSetDevice(s->device));
+  fill_u32(s->x8_ok, 0, 1, s->stream);
   HIPX(hipMemcpyAsync(s->X, rows, size_t(s->N) * s->D * 4, hipMemcpyHostToDevice, s->stream));
   HIPX(hipStreamSynchronize(s->stream));
   s->has_knn = false;
@@ -674,6 +678,7 @@ int tg_gen_data(tg_state* s, int32_t kind, uint32_t ncomp, uint64_t seed, float 
     if (dalloc(&s->centres, size_t(ncomp) * s->D)) return TG_ERR_HIP;
     s->ncomp_alloc = ncomp;
   }
+  fill_u32(s->x8_ok, 0, 1, s->stream);
   launch_gen_data(kind, s->N, s->D, ncomp, seed, sigma, s->centres, s->X, s->misc, s->stream);
   if (int rc = check_launch("gen_data")) return rc;
   HIPX(hipStreamSynchronize(s->stream));
@@ -1888,6 +1893,7 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
   SearchArgs a{};
   a.X = s->X;
   a.X8 = s->prep_valid && s->cert_u8 && D <= 256 ? s->X8 : nullptr;
+  a.x8_ok = s->x8_ok;
   a.N = N;
   a.D = D;
   a.deg = s->out_deg;
@@ -2009,6 +2015,7 @@ int tg_search_noalloc(tg_state* s, uint32_t nq, const float* queries_dev,
   SearchArgs a{};
   a.X = s->X;
   a.X8 = s->prep_valid && s->cert_u8 && s->D <= 256 ? s->X8 : nullptr;
+  a.x8_ok = s->x8_ok;
   a.N = N;
   a.D = s->D;
   a.deg = s->out_deg;

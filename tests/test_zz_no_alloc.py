@@ -12,6 +12,7 @@ import ctypes
 import numpy as np
 import pytest
 
+import oracle
 import tagore_amd
 from tagore_amd import SearchParams, SearchStats, State
 
@@ -119,3 +120,73 @@ def test_search_noalloc_rejects_bad_arguments():
         bad = SearchParams(16, 4, 1, N)
         assert L.tg_search_noalloc(s._h, 4, ptr, ctypes.byref(bad), ptr, ptr, None,
                                    None) == tagore_amd.TG_ERR_ARG
+
+
+@pytest.mark.parametrize("second", ["fractional", "integer", "signed"])
+def test_captured_search_reads_the_current_vectors(second):
+    """A captured search replayed after tg_set_data brought other vectors (and the index was
+    installed again): every replay answers from the vectors the handle holds then, with eager
+    work and synchronisation between the replays.  The first vectors are u8 and prepared."""
+    hip = _hip()
+    vp = ctypes.c_void_p
+    hip.hipStreamBeginCapture.argtypes = [vp, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [vp, ctypes.POINTER(vp)]
+    hip.hipGraphInstantiate.argtypes = [ctypes.POINTER(vp), vp, vp, vp, ctypes.c_size_t]
+    hip.hipGraphLaunch.argtypes = [vp, vp]
+    hip.hipGraphExecDestroy.argtypes = [vp]
+    hip.hipGraphDestroy.argtypes = [vp]
+    rng = np.random.default_rng(17)
+    N, D, nq, k, L, FD = 3000, 64, 50, 10, 32, 16
+    X1 = rng.integers(0, 256, (N, D)).astype(np.float32)
+    X2 = rng.integers(0, 256, (N, D)).astype(np.float32)
+    if second == "fractional":
+        X2 += 0.5
+    if second == "signed":
+        X2 -= 128
+    Q = rng.integers(0, 256, (nq, D)).astype(np.float32)
+    graph_ids = rng.integers(0, N, (N, FD)).astype(np.uint32)
+    deg = np.full(N, FD, np.uint32)
+    ref = [oracle.search(X, deg, graph_ids, 7, Q, L, k, 0x33) for X in (X1, X2)]
+    assert not np.array_equal(ref[0][0], ref[1][0])
+    side, graph, run = vp(), vp(), vp()
+    assert hip.hipStreamCreate(ctypes.byref(side)) == 0
+    ids, d = np.empty((nq, k), np.uint32), np.empty((nq, k), np.float32)
+    with State(N, D) as s, _Dev(hip, Q.nbytes) as q_dev, _Dev(hip, ids.nbytes) as i_dev, \
+            _Dev(hip, d.nbytes) as d_dev:
+        def install(X, prepare):
+            s.set_data(X)
+            if prepare:
+                s.knn_build(8, 2, 1, "bf16")
+            s.set_pruned(deg, graph_ids, 7)
+
+        def replay(what, expect):
+            _say(f"captured search, {second}: {what}")
+            assert hip.hipGraphLaunch(run, side) == 0
+            assert hip.hipStreamSynchronize(side) == 0
+            assert hip.hipMemcpy(ids.ctypes.data, i_dev.p, ids.nbytes, D2H) == 0
+            assert hip.hipMemcpy(d.ctypes.data, d_dev.p, d.nbytes, D2H) == 0
+            assert np.array_equal(ids, expect[0]) and np.array_equal(d, expect[1]), what
+
+        install(X1, True)
+        assert hip.hipMemcpy(q_dev.p, Q.ctypes.data, Q.nbytes, H2D) == 0
+        p = SearchParams(L, k, 0x33, 0xFFFFFFFF)
+        assert hip.hipStreamBeginCapture(side, 0) == 0
+        rc = tagore_amd.lib().tg_search_noalloc(s._h, nq, q_dev.p, ctypes.byref(p), i_dev.p,
+                                                d_dev.p, side, None)
+        assert hip.hipStreamEndCapture(side, ctypes.byref(graph)) == 0
+        assert rc == 0, tagore_amd.lib().tg_last_error()
+        assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+        replay("captured vectors", ref[0])
+        install(X2, False)
+        replay("new vectors", ref[1])
+        gi, gd, _ = s.search(Q, k=k, L=L, seed=0x33)
+        assert np.array_equal(gi, ref[1][0]) and np.array_equal(gd, ref[1][1])
+        replay("new vectors again", ref[1])
+        install(X2, True)
+        replay("new vectors, prepared", ref[1])
+        install(X1, False)
+        replay("first vectors back", ref[0])
+        install(X1, True)
+        replay("first vectors, prepared", ref[0])
+        assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(side) == 0
