@@ -229,7 +229,9 @@ int tg_knn_dist_check(tg_state* s, uint32_t nq, uint64_t seed, double* max_rel_e
 
 /* Device buffers in the reference's capsule order (pybind.cu:132-141):
  * 0 graph u32[N*K], 1 reverse graph, 2 data f32[N*D], 3 distances f32[N*K],
- * 4 reverse distances, 5 reverse counts, 6 centroid f32[D], 7 sample lists u32[N*128]. */
+ * 4 reverse distances, 5 reverse counts, 6 centroid f32[D], 7 sample lists u32[N*128].
+ * A caller may write to the data (2) between calls; once it was asked for, the narrow copies
+ * of the vectors are made anew by each build and prune, and searches read the FP32 rows. */
 int tg_buffer(tg_state* s, int32_t idx, void** dev_ptr, size_t* bytes);
 
 /* Timing of the last tg_knn_build / tg_prune (device window, HIP events, ms) and the

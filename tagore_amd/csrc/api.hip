@@ -138,6 +138,7 @@ struct tg_state {
   hipStream_t stream = nullptr;
   uint32_t N = 0, D = 0;
   float* X = nullptr;
+  bool x_lent = false;       // tg_buffer gave X away: no copy of it outlives a call
   float* centres = nullptr;  // synthetic-data centres
   uint32_t ncomp_alloc = 0;
   uint32_t* misc = nullptr;  // [64] small scratch
@@ -350,7 +351,7 @@ int ensure_knn_scratch(tg_state* s, uint32_t K) {
 // Norms, data-set certificates and the 16-bit copy of the current vectors (computed once per
 // data set, like the reference's host-side FP16 copy, pybind.cu:58-61).
 int ensure_prep(tg_state* s) {
-  if (s->prep_valid) return TG_OK;
+  if (s->prep_valid && !s->x_lent) return TG_OK;
   const size_t N = s->N;
   if (!s->nrm2) {
     if (dalloc(&s->nrm2, N) || dalloc(&s->cert_flags, 7) || dalloc(&s->Xb, N * s->D))
@@ -404,7 +405,7 @@ int ensure_prep(tg_state* s) {
     if (!s->n2s && dalloc(&s->n2s, N)) return TG_ERR_HIP;
     launch_make_u8(s->X, N * s->D, s->X8, s->stream);
     if (s->D <= 256) launch_u8_shift_norms(s->X8, s->N, s->D, s->n2s, s->stream);
-    fill_u32(s->x8_ok, 1, 1, s->stream);
+    fill_u32(s->x8_ok, s->x_lent ? 0 : 1, 1, s->stream);
   }
   s->prep_valid = true;
   return TG_OK;
@@ -412,7 +413,7 @@ int ensure_prep(tg_state* s) {
 
 // FP8 copy with per-vector scales and its norms (once per data set)
 int ensure_prep8(tg_state* s) {
-  if (s->prep8_valid) return TG_OK;
+  if (s->prep8_valid && !s->x_lent) return TG_OK;
   const size_t N = s->N;
   if (!s->Xq8) {
     if (dalloc(&s->Xq8, N * s->D) || dalloc(&s->sc8, N) || dalloc(&s->nq8, N) ||
@@ -1844,6 +1845,10 @@ namespace {
 constexpr uint32_t SEARCH_GRID = 256 * 12;  // workgroups: 12 queries in flight per CU
 constexpr uint32_t SEARCH_VCAP = 8192;      // listed visited ids per query
 constexpr size_t SEARCH_HEAD = 64;          // bytes of the counters before the results
+// the u8 rows a search may read: a search prepares nothing, so only those of an earlier call
+const uint8_t* search_rows8(const tg_state* s) {
+  return s->prep_valid && s->cert_u8 && s->D <= 256 && !s->x_lent ? s->X8 : nullptr;
+}
 }  // namespace
 
 int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_params* p,
@@ -1892,7 +1897,7 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
   fill_u32(reinterpret_cast<uint32_t*>(scnt), 0, 4, st);
   SearchArgs a{};
   a.X = s->X;
-  a.X8 = s->prep_valid && s->cert_u8 && D <= 256 ? s->X8 : nullptr;
+  a.X8 = search_rows8(s);
   a.x8_ok = s->x8_ok;
   a.N = N;
   a.D = D;
@@ -2014,7 +2019,7 @@ int tg_search_noalloc(tg_state* s, uint32_t nq, const float* queries_dev,
   fill_u32(bitmap, 0, size_t(grid) * words, st);
   SearchArgs a{};
   a.X = s->X;
-  a.X8 = s->prep_valid && s->cert_u8 && s->D <= 256 ? s->X8 : nullptr;
+  a.X8 = search_rows8(s);
   a.x8_ok = s->x8_ok;
   a.N = N;
   a.D = s->D;
@@ -2185,7 +2190,17 @@ int tg_buffer(tg_state* s, int32_t idx, void** dev_ptr, size_t* bytes) {
   switch (idx) {
     case 0: *dev_ptr = s->G; *bytes = N * K * 4; break;
     case 1: *dev_ptr = s->R0; *bytes = s->R0 ? N * K * 8 : 0; break;
-    case 2: *dev_ptr = s->X; *bytes = N * s->D * 4; break;
+    case 2:
+      // the caller may write to X from here on
+      if (!s->x_lent && s->prep_valid && s->cert_u8) {
+        HIPX(hipSetDevice(s->device));
+        fill_u32(s->x8_ok, 0, 1, s->stream);
+        HIPX(hipStreamSynchronize(s->stream));
+      }
+      s->x_lent = true;
+      *dev_ptr = s->X;
+      *bytes = N * s->D * 4;
+      break;
     case 3: *dev_ptr = s->GD; *bytes = N * K * 4; break;
     case 4: *dev_ptr = s->R1; *bytes = s->R1 ? N * K * 8 : 0; break;
     case 5: *dev_ptr = s->Rn0; *bytes = s->Rn0 ? N * 4 : 0; break;
