@@ -238,6 +238,10 @@ int copy_out(tg_state* s, void* dst, const void* src, size_t n) {
     HIPX(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
     return TG_OK;
   }
+  // The chunks run on the handle's stream, which no other stream orders itself with.  A plain
+  // copy waits for the default stream and the streams that it waits for: a caller's own work on
+  // a lent buffer, enqueued there, has to be in the result here too
+  HIPX(hipStreamSynchronize(nullptr));
   const size_t nc = (n + COPY_CHUNK - 1) / COPY_CHUNK;
   std::atomic<int> err{int(hipSuccess)};
   // lane l: chunks l, l + COPY_LANES, ..; the next one is on its way (all on the handle's

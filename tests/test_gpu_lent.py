@@ -62,3 +62,46 @@ def test_vectors_written_through_the_lent_buffer(first, second):
         oi, od, oc = oracle.search(X1, deg, ids, ep, Q, 32, 10, 0x44)
         gi, gd, st = s.search(Q, k=10, L=32, seed=0x44)
         assert np.array_equal(gi, oi) and np.array_equal(gd, od)
+
+
+@pytest.mark.parametrize("own_stream", [False, True])
+@pytest.mark.parametrize("N", [1000, 1 << 19])
+def test_results_follow_the_callers_work_on_lent_lists(N, own_stream):
+    """New distances written into the lent lists by the caller's asynchronous copies on the
+    default stream, or on a stream that the default one waits for, with other work before
+    them: the copy to the host (plain, and by chunks) comes after them."""
+    hip = _hip()
+    vp = ctypes.c_void_p
+    hip.hipMalloc.argtypes = [ctypes.POINTER(vp), ctypes.c_size_t]
+    hip.hipFree.argtypes = [vp]
+    hip.hipMemcpyAsync.argtypes = [vp, vp, ctypes.c_size_t, ctypes.c_int, vp]
+    hip.hipStreamCreate.argtypes = [ctypes.POINTER(vp)]
+    hip.hipStreamDestroy.argtypes = [vp]
+    hip.hipStreamSynchronize.argtypes = [vp]
+    K, big, D2D = 4, 256 << 20, 3
+    rng = np.random.default_rng(N)
+    ids = rng.integers(0, N, (N, K)).astype(np.uint32)
+    d1 = (np.arange(K) + 0.5 * rng.random((N, K))).astype(np.float32)
+    d2 = (np.arange(K) + 0.5 * rng.random((N, K))).astype(np.float32)
+    src, a, b, stream = vp(), vp(), vp(), vp()
+    assert hip.hipMalloc(ctypes.byref(src), d2.nbytes) == 0
+    assert hip.hipMalloc(ctypes.byref(a), big) == 0 and hip.hipMalloc(ctypes.byref(b), big) == 0
+    if own_stream:
+        assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    with State(N, 4) as s:
+        s.set_knn(ids, d1)
+        s.get_knn()
+        ptr, nbytes = s.buffer(3)
+        assert nbytes == d2.nbytes
+        assert hip.hipMemcpy(src, d2.ctypes.data, d2.nbytes, H2D) == 0
+        print(f"lent lists N={N} own stream {own_stream}", flush=True)
+        for _ in range(100):  # some 10 ms before the lists change
+            assert hip.hipMemcpyAsync(a, b, big, D2D, stream) == 0
+        assert hip.hipMemcpyAsync(ptr, src, d2.nbytes, D2D, stream) == 0
+        G, GD = s.get_knn()
+        assert np.array_equal(G, ids) and np.array_equal(GD, d2)
+        assert hip.hipStreamSynchronize(stream) == 0
+    for p in (src, a, b):
+        assert hip.hipFree(p) == 0
+    if own_stream:
+        assert hip.hipStreamDestroy(stream) == 0
