@@ -211,7 +211,8 @@ struct tg_state {
   std::vector<hipEvent_t> ev_pool;
   hipEvent_t win[2] = {};      // window events of a build, prune or search
   CopyOut out;
-  // search: queries on the device, and [counters | ids | dists] of the results, grown on demand
+  // search: queries on the device, and [counters | ids | dists] of the results, grown on demand up to
+  // SEARCH_KEEP
   float* sq = nullptr;
   size_t sq_cap = 0;
   unsigned char* sres = nullptr;
@@ -1849,6 +1850,21 @@ namespace {
 constexpr uint32_t SEARCH_GRID = 256 * 12;  // workgroups: 12 queries in flight per CU
 constexpr uint32_t SEARCH_VCAP = 8192;      // listed visited ids per query
 constexpr size_t SEARCH_HEAD = 64;          // bytes of the counters before the results
+constexpr size_t SEARCH_KEEP = size_t(64) << 20;  // larger buffers go back after the call
+// the handle's query and result buffers, given back at the end of a call that made them large
+struct SearchBuffers {
+  tg_state* s;
+  ~SearchBuffers() {
+    if (s->sq_cap * 4 > SEARCH_KEEP) {
+      dfree(s->sq);
+      s->sq_cap = 0;
+    }
+    if (s->sres_cap > SEARCH_KEEP) {
+      dfree(s->sres);
+      s->sres_cap = 0;
+    }
+  }
+};
 // the u8 rows a search may read: a search prepares nothing, so only those of an earlier call
 const uint8_t* search_rows8(const tg_state* s) {
   return s->prep_valid && s->cert_u8 && s->D <= 256 && !s->x_lent ? s->X8 : nullptr;
@@ -1874,7 +1890,8 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
       return TG_ERR_HIP;
     fill_u32(s->sbm, 0, size_t(SEARCH_GRID) * words, s->stream);
   }
-  // device buffers of the handle, grown to the largest call so far
+  // device buffers of the handle, grown on demand
+  SearchBuffers give_back{s};
   const size_t nr = size_t(nq) * p->k * 4;          // bytes of the ids, and of the distances
   const size_t need = SEARCH_HEAD + 2 * nr;
   if (s->sq_cap < size_t(nq) * D) {

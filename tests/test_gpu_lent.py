@@ -105,3 +105,33 @@ def test_results_follow_the_callers_work_on_lent_lists(N, own_stream):
         assert hip.hipFree(p) == 0
     if own_stream:
         assert hip.hipStreamDestroy(stream) == 0
+
+
+def test_search_gives_large_buffers_back():
+    """A search over many queries leaves no more than its bound of device memory with the
+    handle (2 x 64 MiB); small and large calls in turn answer alike."""
+    hip = _hip()
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]
+
+    def free_bytes():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    rng = np.random.default_rng(3)
+    N, D, nq = 500, 256, 400_000  # queries of 410 MB, results of 160 MB at k = 50
+    X = rng.integers(0, 256, (N, D)).astype(np.float32)
+    Q = X[rng.integers(0, N, nq)]
+    ids = rng.integers(0, N, (N, 4)).astype(np.uint32)
+    with State(N, D) as s:
+        s.set_data(X)
+        s.set_pruned(np.full(N, 4, np.uint32), ids, 0)
+        small = s.search(Q[:20], k=50, L=50, seed=1)
+        before = free_bytes()
+        for rep in range(2):
+            print(f"large search {rep}", flush=True)
+            large = s.search(Q, k=50, L=50, seed=1)
+            assert before - free_bytes() <= 128 << 20
+            assert np.array_equal(large[0][:20], small[0]) and np.array_equal(large[1][:20], small[1])
+            again = s.search(Q[:20], k=50, L=50, seed=1)
+            assert np.array_equal(again[0], small[0]) and np.array_equal(again[1], small[1])
