@@ -164,6 +164,7 @@ struct tg_state {
   uint32_t* cert_flags = nullptr;  // [7], see k_screen_prep and k_screen_copy
   bool copy16 = false;             // Xb can serve as the screen copy
   float kap16 = 0.f, pscale16 = 2.f;  // its bound and product scale (KnnArgs)
+  float kap16_dpg = 0.f;              // the bound of k_dpg_screen's products
   bool prep_valid = false;         // Xb / norms / certificates match the current X
   bool cert_bf16 = false;          // every value of X is exactly representable in BF16
   bool cert_int = false;           // integer data whose screen distances are exact
@@ -398,7 +399,8 @@ int ensure_prep(tg_state* s) {
       s->pscale16 = std::ldexp(2.f, 2 * (ex - 15));
     }
   }
-  s->kap16 = screen_kappa16(rho, s->D);
+  s->kap16 = screen_kappa16(rho, s->D, s->D);
+  s->kap16_dpg = screen_kappa16(rho, s->D, DPG_CHAIN);
   // every MFMA partial sum, |a|^2+|b|^2 and |a-b|^2 stay integers below 2^24
   const double lim = 16777216.0;
   s->cert_int = f[1] == 0 && (f[2] == 0 ? 2.0 * qmax < lim : 4.0 * qmax < lim);
@@ -1572,7 +1574,7 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
         q.nrm2 = s->nrm2;
         q.nq = s->nq8;
         q.ne = s->ne8;
-        q.kap = s->kap16;
+        q.kap = s->kap16_dpg;
         q.pscale = s->pscale16;
         q.sc8 = s->sc8;
         q.Xb = s->Xb;

@@ -69,6 +69,7 @@ struct DpgScreen {
   float eta;            // FP8: relative slack of the bound
   float kap, pscale;    // 16-bit rows (see KnnArgs)
 };
+constexpr uint32_t DPG_CHAIN = 128;  // elements of a product's chain (screen_kappa16), 16-bit rows
 // precision: KP_BF16 (the 16-bit copy) or KP_FP8; K <= 64
 void launch_dpg_screen(const PruneArgs& a, const DpgScreen& q, int precision, hipStream_t s);
 

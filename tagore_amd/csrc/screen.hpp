@@ -10,23 +10,12 @@
 #include <stdint.h>
 
 #include "common.hpp"
+#include "rules.hpp"
 
 namespace tg {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-// kappa, host side.  rho bounds |x' - x| / |x| over the rows (0 for exact copies): the product
-// is off by at most (2 rho + rho^2) |a||b| and |a||b| <= (|a|^2 + |b|^2) / 2.  Accumulation of
-// 16-bit rows: an MFMA step of 32 products adds at most 32 + D / 32 roundings of 2^-23 to any
-// product, whatever its internal order; FP32 products (16x16x4) D / 4 + 5; the canonical fold
-// D / 64 + 14 of 2^-24 to d <= 2 (|a|^2 + |b|^2), the norms and s itself a few.  Together below
-// D / 4 + 128 (FP32: D / 2 + 128) in units of 2^-23.
-inline float screen_kappa16(double rho, uint32_t D) {
-  const double q = (2.0 * rho + rho * rho) * (1.0 + rho) * (1.0 + rho);
-  return float((q + (0.25 * D + 128.0) / 8388608.0) * (1.0 + 1e-5));
-}
-inline float screen_kappa32(uint32_t D) { return float((0.5 * D + 128.0) / 8388608.0); }
 
 // Staging of R rows (ids in LDS) through LDS, DC elements at a time, by a 256-thread
 // workgroup.  PREC 1: FP32 rows; 2: 16-bit rows; 3: FP8 rows.
