@@ -307,7 +307,9 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
  * (64 MiB - 256) / ((8192 + ceil(N/32)) * 4) workgroups run at once (TG_ERR_CAPACITY when
  * not even one fits, i.e. N above about 5.3e8).  stream: a hipStream_t, or NULL for the
  * handle's stream.  stats == NULL: the call only enqueues work and returns; otherwise it
- * waits for the search and fills stats (evals, expansions; ms is not measured, 0).  Every
+ * waits for the search and fills stats (evals, expansions; ms is not measured, 0).  Replays of
+ * a captured call answer from the handle's vectors at that time (a captured call reads the
+ * FP32 rows; others take the u8 copy of integer data that an earlier call made).  Every
  * call on one GPU shares that GPU's array: calls that overlap in time on one GPU (other
  * streams, other host threads, other handles) race and must be serialised by the caller. */
 int tg_search_noalloc(tg_state* s, uint32_t nq, const float* queries_dev,

@@ -170,7 +170,6 @@ struct tg_state {
   bool cert_int = false;           // integer data whose screen distances are exact
   bool cert_u8 = false;            // and every value in [0, 255]: X8 holds the u8 copy
   uint8_t* X8 = nullptr;
-  uint32_t* x8_ok = nullptr;       // device word: X8 matches X (SearchArgs)
   float* n2s = nullptr;            // [N] |x - 128|^2 of the u8 rows
   uint32_t* fill = nullptr;
   uint32_t* scan_tmp = nullptr;
@@ -412,7 +411,6 @@ int ensure_prep(tg_state* s) {
     if (!s->n2s && dalloc(&s->n2s, N)) return TG_ERR_HIP;
     launch_make_u8(s->X, N * s->D, s->X8, s->stream);
     if (s->D <= 256) launch_u8_shift_norms(s->X8, s->N, s->D, s->n2s, s->stream);
-    fill_u32(s->x8_ok, s->x_lent ? 0 : 1, 1, s->stream);
   }
   s->prep_valid = true;
   return TG_OK;
@@ -581,7 +579,7 @@ int tg_create(uint32_t N, uint32_t D, int device, tg_state** out) {
     return fail(TG_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
   if (dalloc(&s->X, size_t(N) * D) || dalloc(&s->misc, 64) || dalloc(&s->centroid, D) ||
-      dalloc(&s->ep_dev, 1) || dalloc(&s->x8_ok, 1)) {
+      dalloc(&s->ep_dev, 1)) {
     std::string m = g_err;
     tg_free(s);
     return fail(TG_ERR_HIP, m);
@@ -637,7 +635,6 @@ int tg_free(tg_state* s) {
   dfree(s->nrm2);
   dfree(s->cert_flags);
   dfree(s->X8);
-  dfree(s->x8_ok);
   dfree(s->n2s);
   dfree(s->fill);
   dfree(s->scan_tmp);
@@ -666,7 +663,6 @@ int tg_free(tg_state* s) {
 int tg_set_data(tg_state* s, const float* rows) {
   if (!s || !rows) return fail(TG_ERR_ARG, "null argument");
   HIPX(hipSetDevice(s->device));
-  fill_u32(s->x8_ok, 0, 1, s->stream);
   HIPX(hipMemcpyAsync(s->X, rows, size_t(s->N) * s->D * 4, hipMemcpyHostToDevice, s->stream));
   HIPX(hipStreamSynchronize(s->stream));
   s->has_knn = false;
@@ -686,7 +682,6 @@ int tg_gen_data(tg_state* s, int32_t kind, uint32_t ncomp, uint64_t seed, float 
     if (dalloc(&s->centres, size_t(ncomp) * s->D)) return TG_ERR_HIP;
     s->ncomp_alloc = ncomp;
   }
-  fill_u32(s->x8_ok, 0, 1, s->stream);
   launch_gen_data(kind, s->N, s->D, ncomp, seed, sigma, s->centres, s->X, s->misc, s->stream);
   if (int rc = check_launch("gen_data")) return rc;
   HIPX(hipStreamSynchronize(s->stream));
@@ -1921,7 +1916,6 @@ int tg_search(tg_state* s, uint32_t nq, const float* queries, const tg_search_pa
   SearchArgs a{};
   a.X = s->X;
   a.X8 = search_rows8(s);
-  a.x8_ok = s->x8_ok;
   a.N = N;
   a.D = D;
   a.deg = s->out_deg;
@@ -2042,8 +2036,11 @@ int tg_search_noalloc(tg_state* s, uint32_t nq, const float* queries_dev,
   fill_u32(bitmap, 0, size_t(grid) * words, st);
   SearchArgs a{};
   a.X = s->X;
-  a.X8 = search_rows8(s);
-  a.x8_ok = s->x8_ok;
+  // A captured launch may be replayed on vectors that replaced these: it reads the FP32 rows,
+  // which are where they were, not a copy that no replay renews
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPX(hipStreamIsCapturing(st, &cap));
+  a.X8 = cap == hipStreamCaptureStatusNone ? search_rows8(s) : nullptr;
   a.N = N;
   a.D = s->D;
   a.deg = s->out_deg;
@@ -2214,13 +2211,7 @@ int tg_buffer(tg_state* s, int32_t idx, void** dev_ptr, size_t* bytes) {
     case 0: *dev_ptr = s->G; *bytes = N * K * 4; break;
     case 1: *dev_ptr = s->R0; *bytes = s->R0 ? N * K * 8 : 0; break;
     case 2:
-      // the caller may write to X from here on
-      if (!s->x_lent && s->prep_valid && s->cert_u8) {
-        HIPX(hipSetDevice(s->device));
-        fill_u32(s->x8_ok, 0, 1, s->stream);
-        HIPX(hipStreamSynchronize(s->stream));
-      }
-      s->x_lent = true;
+      s->x_lent = true;  // the caller may write to X from here on
       *dev_ptr = s->X;
       *bytes = N * s->D * 4;
       break;

@@ -186,8 +186,6 @@ void fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 struct SearchArgs {
   const float* X;
   const uint8_t* X8;  // u8 copy (KnnArgs::X8) or null
-  const uint32_t* x8_ok;  // 1 while X8 matches X: read by the kernel, since a captured launch
-                          // can be replayed on vectors that replaced the captured ones
   uint32_t N, D;
   const uint32_t* deg;
   const uint32_t* ids;

@@ -132,7 +132,7 @@ __device__ __forceinline__ void eval_f32(const float* X, int D, const Row16<MC>&
   }
 }
 
-// U8: a.X8 holds the u8 copy of the data (used while *a.x8_ok).
+// U8: a.X8 holds the u8 copy of the data.
 template <int MC, int NPL, bool U8>
 __global__ __launch_bounds__(64) void k_search(SearchArgs a) {
   extern __shared__ uint32_t vtab[];  // visited hash, 2^hbits ids
@@ -146,14 +146,13 @@ __global__ __launch_bounds__(64) void k_search(SearchArgs a) {
   const uint32_t hcap = (3u << hb) >> 2;
   uint32_t* bm = a.bitmap + size_t(blockIdx.x) * a.words;
   uint32_t* vl = a.vlist + size_t(blockIdx.x) * a.vcap;
-  const bool fresh8 = U8 && *a.x8_ok != 0;
   unsigned long long n_eval = 0, n_exp = 0;
   for (uint32_t q = blockIdx.x; q < a.nq; q += gridDim.x) {
     const float* qrow = a.Q + size_t(q) * D;
     Row16<MC> xq, x8;
     load_row16<MC>(xq, qrow, int(D), t);
     bool q8 = false;
-    if constexpr (U8) q8 = query_u8<MC>(x8, qrow, int(D)) && fresh8;
+    if constexpr (U8) q8 = query_u8<MC>(x8, qrow, int(D));
     auto eval = [&](int n) {
       if constexpr (U8) {
         if (q8) {
