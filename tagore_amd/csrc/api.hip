@@ -159,10 +159,10 @@ struct tg_state {
   uint8_t* Xq8 = nullptr;  // FP8 e4m3 copy of X with per-vector scales (screen)
   float *sc8 = nullptr, *nq8 = nullptr, *ne8 = nullptr;
   bool prep8_valid = false;
-  uint16_t* Xb = nullptr;  // 16-bit copy of X (screen): BF16 when exact, else scaled FP16
+  uint16_t* Xb = nullptr;  // 16-bit copy of X (screen): BF16 when exact, scaled FP16, or rounded BF16
   float* nrm2 = nullptr;
   uint32_t* cert_flags = nullptr;  // [7], see k_screen_prep and k_screen_copy
-  bool copy16 = false;             // Xb can serve as the screen copy
+  bool copy_bf16 = false;             // Xb holds BF16 (exact or rounded), else scaled FP16
   float kap16 = 0.f, pscale16 = 2.f;  // its bound and product scale (KnnArgs)
   float kap16_dpg = 0.f;              // the bound of k_dpg_screen's products
   bool prep_valid = false;         // Xb / norms / certificates match the current X
@@ -371,31 +371,43 @@ int ensure_prep(tg_state* s) {
   float qmax, vmax;
   std::memcpy(&qmax, &f[3], 4);
   std::memcpy(&vmax, &f[5], 4);
-  // the 16-bit copy: exact BF16, or FP16 with the largest value scaled below 2^15.  A row
-  // error above 2^-9 (rows far smaller than the largest value) or values beyond the scales
-  // that keep the products in FP32's range: no 16-bit screen, the FP32 one serves
-  s->copy16 = true;
-  s->pscale16 = 2.f;
+  // The 16-bit copy: BF16 where that is exact, else FP16 with the largest value scaled below
+  // 2^15.  FP16 cannot hold rows far below the largest value, and its products would leave
+  // FP32's range for data beyond these scales; a row error above 2^-9, which is BF16's, shows
+  // the former.  Such data takes rounded BF16: one small row among 40k x 960 and DPG had no
+  // screen at all (48.1 ms a call against XXX, YYY with none), the build took FP32 products
+  // (19.0 against ZZZ)
   double rho = 0.0;
+  auto row_error = [&](float& r) -> int {
+    HIPX(hipMemcpyAsync(f, s->cert_flags, sizeof(f), hipMemcpyDeviceToHost, s->stream));
+    HIPX(hipStreamSynchronize(s->stream));
+    std::memcpy(&r, &f[6], 4);
+    return TG_OK;
+  };
+  s->copy_bf16 = true;
+  s->pscale16 = 2.f;
   if (s->cert_bf16) {
-    launch_screen_copy(s->X, s->N, s->D, false, 1.f, s->Xb, s->cert_flags, s->stream);
+    launch_screen_copy(s->X, s->N, s->D, COPY_EXACT, 1.f, s->Xb, s->cert_flags, s->stream);
   } else {
     int ex = 0;
-    s->copy16 = std::isfinite(vmax);
-    if (s->copy16) {
-      (void)std::frexp(vmax, &ex);  // vmax < 2^ex
-      s->copy16 = ex >= -30 && ex <= 55;
-    }
-    if (s->copy16) {
-      launch_screen_copy(s->X, s->N, s->D, true, std::ldexp(1.f, 15 - ex), s->Xb, s->cert_flags,
-                         s->stream);
-      HIPX(hipMemcpyAsync(f, s->cert_flags, sizeof(f), hipMemcpyDeviceToHost, s->stream));
-      HIPX(hipStreamSynchronize(s->stream));
+    if (std::isfinite(vmax)) (void)std::frexp(vmax, &ex);  // vmax < 2^ex
+    if (std::isfinite(vmax) && ex >= -30 && ex <= 55) {
+      launch_screen_copy(s->X, s->N, s->D, COPY_FP16, std::ldexp(1.f, 15 - ex), s->Xb,
+                         s->cert_flags, s->stream);
       float r;
-      std::memcpy(&r, &f[6], 4);
-      s->copy16 = r <= 0x1p-9f;
+      if (int rc = row_error(r)) return rc;
+      if (r <= 0x1p-9f) {
+        rho = r;
+        s->copy_bf16 = false;
+        s->pscale16 = std::ldexp(2.f, 2 * (ex - 15));
+      }
+    }
+    if (s->copy_bf16) {
+      fill_u32(s->cert_flags + 6, 0, 1, s->stream);
+      launch_screen_copy(s->X, s->N, s->D, COPY_BF16, 1.f, s->Xb, s->cert_flags, s->stream);
+      float r;
+      if (int rc = row_error(r)) return rc;
       rho = r;
-      s->pscale16 = std::ldexp(2.f, 2 * (ex - 15));
     }
   }
   s->kap16 = screen_kappa16(rho, s->D, s->D);
@@ -1237,8 +1249,6 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
   sec.next = 0;
   clear_status(s);
   HIPX(hipEventRecord(w0, st));
-  // data that no 16-bit copy screens well takes the FP32 screen instead (same graph)
-  const int prec = p->precision == TG_PREC_BF16 && !s->copy16 ? int(TG_PREC_FP32) : p->precision;
   // precision-dependent parts of the argument block (re-applied after every swap)
   // integer data makes the FP32 / BF16 screens exact; FP8 rounds integers above 16
   const bool exact_screen =
@@ -1257,8 +1267,9 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       k.seg_key = s->seg_key;
     }
     k.exact_screen = exact_screen ? 1 : 0;
-    k.kap = prec == TG_PREC_BF16 ? s->kap16 : screen_kappa32(s->D);
-    k.pscale = prec == TG_PREC_BF16 ? s->pscale16 : 2.f;
+    k.kap = p->precision == TG_PREC_BF16 ? s->kap16 : screen_kappa32(s->D);
+    k.pscale = p->precision == TG_PREC_BF16 ? s->pscale16 : 2.f;
+    k.copy_bf16 = s->copy_bf16 ? 1 : 0;
     k.Xr16 = rows16;
     k.X8 = (p->precision != TG_PREC_EXACT && s->cert_u8 && s->D <= 256) ? s->X8 : nullptr;
     k.n2s = k.X8 ? s->n2s : nullptr;
@@ -1311,7 +1322,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       launch_knn_rsample(a, st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(3)) return TG_ERR_HIP;
-      launch_knn_localjoin(a, prec, int(p->tile), st);
+      launch_knn_localjoin(a, p->precision, int(p->tile), st);
       if (sc.stop()) return TG_ERR_HIP;
       if (sc.start(4)) return TG_ERR_HIP;
       pb_group_overflow({&a.pc}, N, s->fill, s->scan_tmp, st);
@@ -1330,7 +1341,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
     for (uint32_t it = 0; it < it2; ++it) {
       if (sc.start(6)) return TG_ERR_HIP;
       pb_reset({&a.pr}, N, st);
-      launch_knn_phase2(a, prec, st);
+      launch_knn_phase2(a, p->precision, st);
       pb_group_overflow({&a.pr}, N, s->fill, s->scan_tmp, st);
       launch_knn_rupdate(a, st);
       if (sc.stop()) return TG_ERR_HIP;
@@ -1351,7 +1362,7 @@ static int knn_build_impl(tg_state* s, const tg_knn_params* p) {
       key.insert(key.end(), b, b + n);
     };
     put(&a, sizeof(a));
-    const uint64_t extra[] = {it1, it2, uint64_t(prec), p->tile,
+    const uint64_t extra[] = {it1, it2, uint64_t(p->precision), p->tile,
                               uint64_t(reinterpret_cast<uintptr_t>(s->fill)),
                               uint64_t(reinterpret_cast<uintptr_t>(s->scan_tmp)),
                               uint64_t(reinterpret_cast<uintptr_t>(s->rv_hist)),
@@ -1523,16 +1534,16 @@ static int prune_impl(tg_state* s, const tg_prune_params* p) {
     a.rows_bf16 = 1;
   }
   a.rows8 = s->cert_u8 ? s->X8 : nullptr;
-  if (s->copy16 && s->D % 8 == 0) {
+  if (s->D % 8 == 0) {
     a.Xb = s->Xb;
     a.nrm2 = s->nrm2;
     a.kap = s->kap16;
     a.pscale = s->pscale16;
-    a.h_bf16 = s->cert_bf16 ? 1 : 0;
+    a.h_bf16 = s->copy_bf16 ? 1 : 0;
   }
   // DPG's pair distances on an MFMA Gram (K <= 64) with exact re-scores near the threshold
   const bool dpg_screen = p->kind == TG_KIND_DPG && K <= 64 &&
-                          ((p->precision == TG_PREC_BF16 && s->D % 8 == 0 && s->copy16) ||
+                          ((p->precision == TG_PREC_BF16 && s->D % 8 == 0) ||
                            (p->precision == TG_PREC_FP8 && s->D % 16 == 0));
   if (dpg_screen && p->precision == TG_PREC_FP8)
     if (int rc = ensure_prep8(s)) return rc;

@@ -49,7 +49,7 @@ struct PruneArgs {
   const uint16_t* Xb;
   const float* nrm2;
   float kap, pscale;
-  int h_bf16;            // the copy is BF16 (every value exact), else scaled FP16
+  int h_bf16;            // the copy is BF16 (exact or rounded), else scaled FP16
   // segments: rows [seg_lo[c], seg_lo[c+1]) form independent data sets (null: one segment)
   const uint32_t* seg_of;  // [N] segment of each row
   const uint32_t* seg_lo;  // [nseg + 1]
@@ -107,7 +107,8 @@ struct KnnArgs {
   // the screen copies a', b' with the rigorous bound |s - dist(a,b)| <= kap (|a|^2 + |b|^2)
   // (screen.hpp); only candidates whose bound interval can change a decision are re-scored
   // with the canonical distance.
-  const uint16_t* Xb;  // [N*D] 16-bit rows: BF16 when exact (then Xr16), else scaled FP16
+  const uint16_t* Xb;  // [N*D] 16-bit rows: BF16 when exact (then Xr16), else scaled FP16 or
+  int copy_bf16;       // (copy_bf16) rounded BF16
   const float* nrm2;   // [N] |x|^2 (FP64 sum rounded once)
   float kap;
   float pscale;        // 2 / scale^2 of the 16-bit copy (2 for BF16 and FP32 rows)
@@ -142,11 +143,12 @@ void launch_make_u8(const float* X, size_t n, uint8_t* X8, hipStream_t s);
 // |x - 128|^2 of every u8 row (the norms of the rows shifted into int8)
 void launch_u8_shift_norms(const uint8_t* X8, uint32_t N, uint32_t D, float* n2s, hipStream_t s);
 // screen-mode preparation: norms and the data-set certificates in flags[0..5], then the
-// 16-bit copy (half: scaled FP16, its largest relative row error in flags[6]; else BF16
-// bits); flags zeroed by the caller
+// 16-bit copy, the largest relative row error of one that rounds in flags[6]; flags zeroed by
+// the caller
+enum { COPY_EXACT = 0, COPY_FP16, COPY_BF16 };  // BF16 bits; scaled FP16; BF16 rounded
 void launch_screen_prep(const float* X, uint32_t N, uint32_t D, float* nrm2, uint32_t* flags,
                         hipStream_t s);
-void launch_screen_copy(const float* X, uint32_t N, uint32_t D, bool half, float scale,
+void launch_screen_copy(const float* X, uint32_t N, uint32_t D, int kind, float scale,
                         uint16_t* Xb, uint32_t* flags, hipStream_t s);
 
 void launch_knn_init(const KnnArgs& a, hipStream_t s);

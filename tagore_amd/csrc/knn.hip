@@ -766,7 +766,8 @@ __device__ __forceinline__ float screen_bound8(float na, float qa, float ea, flo
   return 2.0f * (ea * qb + qa * eb + ea * eb) + eta * (na + nb + 2.0f * qa * qb);
 }
 
-template <int MC, int PREC, class T>
+// BF: the 16-bit copy is BF16, else scaled FP16.
+template <int MC, int PREC, class T, bool BF>
 __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
   __shared__ RowLds row;
   __shared__ uint32_t ids[512];  // gathered ids, then the candidates compacted in place
@@ -856,7 +857,7 @@ __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
   constexpr int MB = (MC + 1) / 2;
   constexpr int MF = (MC + 3) / 4;
   constexpr bool SCREEN = PREC == KP_BF16 || PREC == KP_FP8;
-  constexpr bool HALF = PREC == KP_BF16 && std::is_same<T, float>::value;  // FP16 copy
+  constexpr bool HALF = PREC == KP_BF16 && !BF;  // FP16 copy
   RowBf<PREC == KP_BF16 && !HALF ? MB : 1> ub;
   RowH<HALF ? MB : 1> uh;
   RowF8<PREC == KP_FP8 ? MF : 1> uf;
@@ -934,7 +935,8 @@ __global__ __launch_bounds__(64) void k_phase2(KnnArgs a) {
           const float E = PREC == KP_FP8
                               ? screen_bound8(nu, qu, eu, nb[b], a.nq[y[b]], a.ne[y[b]], a.eta)
                               : a.kap * nsum;
-          if (t == 0) keep[q] = (s - E < worst) ? 1 : 0;
+          // (not a number where |x|^2 is beyond FP32: kept)
+          if (t == 0) keep[q] = (s - E >= worst) ? 0 : 1;
         }
       }
     }
@@ -1099,17 +1101,21 @@ int launch_knn_rev_build(const KnnArgs& a, uint32_t* hist, uint32_t* scan_tmp, h
 void launch_knn_rev_reduce(const KnnArgs& a, hipStream_t s) { k_rev_reduce<<<a.N, 64, 0, s>>>(a); }
 void launch_knn_phase2(const KnnArgs& a, int precision, hipStream_t s) {
   const int mc = (int(a.D) + 63) / 64;
-#define P2(M, P, T) k_phase2<M, P, T><<<grid_rows(a.perm, a.N), 64, 0, s>>>(a)
-#define P2_MC(P, T)                                                  \
+#define P2(M, P, T, BF) k_phase2<M, P, T, BF><<<grid_rows(a.perm, a.N), 64, 0, s>>>(a)
+#define P2_MC(P, T, BF)                                              \
   do {                                                               \
-    if (mc <= 2) P2(2, P, T); else if (mc <= 4) P2(4, P, T); else P2(16, P, T); \
+    if (mc <= 2) P2(2, P, T, BF);                                    \
+    else if (mc <= 4) P2(4, P, T, BF);                               \
+    else P2(16, P, T, BF);                                           \
   } while (0)
   if (precision == KP_FP8) {
-    if (a.Xr16) P2_MC(KP_FP8, uint16_t); else P2_MC(KP_FP8, float);
+    if (a.Xr16) P2_MC(KP_FP8, uint16_t, false); else P2_MC(KP_FP8, float, false);
   } else if (precision == KP_BF16) {
-    if (a.Xr16) P2_MC(KP_BF16, uint16_t); else P2_MC(KP_BF16, float);
+    if (a.Xr16) P2_MC(KP_BF16, uint16_t, true);
+    else if (a.copy_bf16) P2_MC(KP_BF16, float, true);
+    else P2_MC(KP_BF16, float, false);
   } else {
-    if (a.Xr16) P2_MC(KP_EXACT, uint16_t); else P2_MC(KP_EXACT, float);
+    if (a.Xr16) P2_MC(KP_EXACT, uint16_t, false); else P2_MC(KP_EXACT, float, false);
   }
 #undef P2_MC
 #undef P2

@@ -81,11 +81,14 @@ __global__ __launch_bounds__(256) void k_screen_prep(const float* X, uint32_t N,
   }
 }
 
-// 16-bit copy of the rows: BF16 bits (HALF false; every value exact), or FP16 of x * scale
-// (a power of two that puts the largest value below 2^15; results below the smallest normal
-// FP16 value become 0).  HALF: flags[6] = max over the rows of |x' / scale - x| / |x|, rounded
-// up (FP32 bits).
-template <bool HALF>
+// 16-bit copy of the rows: BF16 bits (COPY_EXACT: every value exact), FP16 of x * scale (a power
+// of two that puts the largest value below 2^15), or BF16 to nearest (scale 1); results below
+// the smallest normal value become 0.  The last two: flags[6] = max over the rows of
+// |x' / scale - x| / |x|, rounded up (FP32 bits).  Rows whose |x|^2 is no finite FP32 value are
+// left out (their screen distances decide nothing), as are rows with |x| below 2^-100: lost
+// altogether, one moves s by 2 |a| |b| at most, which the other row's share of the bound covers
+// (kappa is above 2^-16; both rows that small: s = d = 0).
+template <int KIND>
 __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N, uint32_t D,
                                                      float scale, uint16_t* Xb, uint32_t* flags) {
   __shared__ uint32_t sh[4];
@@ -102,11 +105,19 @@ __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N,
       uint32_t h[4];
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        if (HALF) {
-          _Float16 f = _Float16(v[b] * scale);
-          if (fabsf(float(f)) < 0x1p-14f) f = _Float16(0.f);
-          h[b] = __builtin_bit_cast(uint16_t, f);
-          const double w = double(float(f)) * inv;
+        if (KIND != COPY_EXACT) {
+          float x16;
+          if (KIND == COPY_FP16) {
+            _Float16 f = _Float16(v[b] * scale);
+            if (fabsf(float(f)) < 0x1p-14f) f = _Float16(0.f);
+            h[b] = __builtin_bit_cast(uint16_t, f);
+            x16 = float(f);
+          } else {
+            h[b] = f2bf(v[b]);
+            if (fabsf(bf2f(h[b])) < 0x1p-126f) h[b] = 0;
+            x16 = bf2f(h[b]);
+          }
+          const double w = double(x16) * inv;
           s2 += double(v[b]) * double(v[b]);
           e2 += (w - double(v[b])) * (w - double(v[b]));
         } else {
@@ -115,17 +126,18 @@ __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N,
       }
       *reinterpret_cast<uint2*>(Xb + row * D + j) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
     }
-    if (HALF) {
+    if (KIND != COPY_EXACT) {
 #pragma unroll
       for (int o = 8; o >= 1; o >>= 1) {
         s2 += __shfl_xor(s2, o, 16);
         e2 += __shfl_xor(e2, o, 16);
       }
-      const float r = e2 > 0.0 ? float(sqrt(e2 / s2) * (1.0 + 1e-6)) : 0.f;
+      const bool in = KIND == COPY_FP16 ? e2 > 0.0 : s2 >= 0x1p-200 && s2 <= 3.4028234e38;
+      const float r = in ? float(sqrt(e2 / s2) * (1.0 + 1e-6)) : 0.f;
       worst = op_max(worst, __float_as_uint(r));
     }
   }
-  if (HALF) {
+  if (KIND != COPY_EXACT) {
     worst = wg_reduce(worst, sh, op_max);
     if (threadIdx.x == 0) atomicMax(&flags[6], worst);
   }
@@ -218,10 +230,13 @@ void launch_screen_prep(const float* X, uint32_t N, uint32_t D, float* nrm2, uin
                         hipStream_t s) {
   k_screen_prep<<<prep_grid(N), 256, 0, s>>>(X, N, D, nrm2, flags);
 }
-void launch_screen_copy(const float* X, uint32_t N, uint32_t D, bool half, float scale,
+void launch_screen_copy(const float* X, uint32_t N, uint32_t D, int kind, float scale,
                         uint16_t* Xb, uint32_t* flags, hipStream_t s) {
-  if (half) k_screen_copy<true><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags);
-  else k_screen_copy<false><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags);
+#define SC(KIND) k_screen_copy<KIND><<<prep_grid(N), 256, 0, s>>>(X, N, D, scale, Xb, flags)
+  if (kind == COPY_EXACT) SC(COPY_EXACT);
+  else if (kind == COPY_FP16) SC(COPY_FP16);
+  else SC(COPY_BF16);
+#undef SC
 }
 
 // Local join when the screen distances are the canonical distances (integer data): each job's
@@ -582,8 +597,8 @@ void k_localjoin_exact_screen(KnnArgs a) {
 }
 
 // -------------------------------------------------------------------------------------
-// Screened local join of real-valued data.  PREC 1: FP32 MFMA, 2: 16-bit MFMA (FP16 copy, or
-// BF16 when T = uint16_t: rows that BF16 holds exactly), 3: FP8 MFMA.  The jobs are those of
+// Screened local join of real-valued data.  PREC 1: FP32 MFMA, 2: 16-bit MFMA (BF: BF16 copy,
+// else FP16), 3: FP8 MFMA.  T = uint16_t: rows that BF16 holds exactly.  The jobs are those of
 // k_localjoin_exact_screen: a row's minimum over a 16-wide tile, for rows of A over the tiles
 // of B and of A, and of B over the tiles of A.  Every 16 x 16 block of pairs holds whole jobs
 // of its rows and of its columns (A x A is symmetric: blocks on and above the diagonal only),
@@ -603,11 +618,10 @@ void k_localjoin_exact_screen(KnnArgs a) {
 // of the narrow kernel's cycles issue VALU work, the rest waits on the list, row and push
 // round trips; the wide one streams each sampled row twice.
 // -------------------------------------------------------------------------------------
-template <int PREC, int MC, class T, int DC>
+template <int PREC, int MC, class T, int DC, bool BF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MC <= 4 ? 6 : 3)))
 void k_localjoin_screen(KnnArgs a) {
   using St = ScreenStage<PREC, DC, 128>;
-  constexpr bool BF = std::is_same<T, uint16_t>::value;
   constexpr int QCAP = 1024;  // pairs queued per pass (one pass, but for degenerate data)
   constexpr bool WIDE = MC > 4;
   constexpr int KEYS = 3 * 256 * 8, QBYTES = QCAP * 2;
@@ -727,8 +741,9 @@ void k_localjoin_screen(KnnArgs a) {
     if (q < w) first += int(wsum[q]);
     total += int(wsum[q]);
   }
-  const T* X = reinterpret_cast<const T*>(BF ? static_cast<const void*>(a.Xr16)
-                                             : static_cast<const void*>(a.X));
+  const T* X = reinterpret_cast<const T*>(std::is_same<T, uint16_t>::value
+                                              ? static_cast<const void*>(a.Xr16)
+                                              : static_cast<const void*>(a.X));
   // offers pair (i, x)'s distance to its two jobs
   auto offer = [&](uint32_t e, float d) {
     const int i = int(e >> 7), x = int(e & 127u);
@@ -868,24 +883,28 @@ void launch_knn_localjoin_screen(const KnnArgs& a, int precision, int tile, hipS
     return;
   }
   const int mc = (int(a.D) + 63) / 64;
-#define LJS(P, M, T, DC) \
-  k_localjoin_screen<P, M, T, DC><<<grid_rows(a.perm, a.N), 256, 0, s>>>(a)
-#define LJS_DC(P, M, T)                                                      \
+#define LJS(P, M, T, DC, BF) \
+  k_localjoin_screen<P, M, T, DC, BF><<<grid_rows(a.perm, a.N), 256, 0, s>>>(a)
+#define LJS_DC(P, M, T, BF)                                                  \
   do {                                                                       \
     constexpr int near_ = (P == 3 ? 64 : P == 2 ? 32 : 16);                  \
-    if ((tile == 1) == (M > 4)) LJS(P, M, T, near_);                         \
-    else LJS(P, M, T, 2 * near_);                                            \
+    if ((tile == 1) == (M > 4)) LJS(P, M, T, near_, BF);                     \
+    else LJS(P, M, T, 2 * near_, BF);                                        \
   } while (0)
-#define LJS_MC(P, T)                                                       \
+#define LJS_MC(P, T, BF)                                                   \
   do {                                                                     \
-    if (mc <= 2) LJS_DC(P, 2, T); else if (mc <= 4) LJS_DC(P, 4, T); else LJS_DC(P, 16, T); \
+    if (mc <= 2) LJS_DC(P, 2, T, BF);                                      \
+    else if (mc <= 4) LJS_DC(P, 4, T, BF);                                 \
+    else LJS_DC(P, 16, T, BF);                                             \
   } while (0)
   if (precision == KP_FP8) {
-    if (a.Xr16) LJS_MC(3, uint16_t); else LJS_MC(3, float);
+    if (a.Xr16) LJS_MC(3, uint16_t, false); else LJS_MC(3, float, false);
   } else if (precision == KP_BF16) {
-    if (a.Xr16) LJS_MC(2, uint16_t); else LJS_MC(2, float);
+    if (a.Xr16) LJS_MC(2, uint16_t, true);
+    else if (a.copy_bf16) LJS_MC(2, float, true);
+    else LJS_MC(2, float, false);
   } else {
-    if (a.Xr16) LJS_MC(1, uint16_t); else LJS_MC(1, float);
+    if (a.Xr16) LJS_MC(1, uint16_t, false); else LJS_MC(1, float, false);
   }
 #undef LJS_MC
 #undef LJS_DC

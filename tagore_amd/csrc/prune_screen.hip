@@ -24,17 +24,16 @@ __device__ __forceinline__ float dpg_bound(float na, float qa, float ea, float n
   return 2.0f * (ea * qb + qa * eb + ea * eb) + eta * (na + nb + 2.0f * qa * qb);
 }
 
-// PREC 2: 16-bit rows (q.Xb; BF16 when T = uint16_t, else scaled FP16), PREC 3: FP8 rows
+// PREC 2: 16-bit rows (q.Xb; BF: BF16, else scaled FP16), PREC 3: FP8 rows
 // (q.Xq8, scales q.sc8).  256 threads; wave w owns rows 16w..16w+15 of the 64 x 64 Gram,
 // against the column blocks at or after its own (pairs r < j only).
 // 100k x 960, K = 64: 15.5 -> 5.5 ms (the FP16 copy leaves 55 of the 2,016 pairs undecided;
 // one BF16 product with its eight times wider bound left several times as many, and each reads
 // two 3.8 KB rows).
-template <int PREC, int MC, class T>
+template <int PREC, int MC, class T, bool BF>
 __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
   constexpr int DC = PREC == 3 ? 256 : 128;  // elements staged per round (256 bytes per row)
   static_assert(PREC == 3 || DC == int(DPG_CHAIN), "a chain per round");
-  constexpr bool BF = std::is_same<T, uint16_t>::value;
   using St = ScreenStage<PREC, DC, 64>;
   constexpr int MROW = 65;
   constexpr int SMEM = St::BYTES > 64 * MROW * 4 ? St::BYTES : 64 * MROW * 4;
@@ -166,15 +165,19 @@ __global__ __launch_bounds__(256) void k_dpg_screen(PruneArgs a, DpgScreen q) {
 
 void launch_dpg_screen(const PruneArgs& a, const DpgScreen& q, int precision, hipStream_t s) {
   const int mc = (int(a.D) + 63) / 64;
-#define DS(P, M, T) k_dpg_screen<P, M, T><<<grid_rows(a.perm, a.N), 256, 0, s>>>(a, q)
-#define DS_MC(P, T)                                                    \
+#define DS(P, M, T, BF) k_dpg_screen<P, M, T, BF><<<grid_rows(a.perm, a.N), 256, 0, s>>>(a, q)
+#define DS_MC(P, T, BF)                                                \
   do {                                                                 \
-    if (mc <= 2) DS(P, 2, T); else if (mc <= 4) DS(P, 4, T); else DS(P, 16, T); \
+    if (mc <= 2) DS(P, 2, T, BF);                                      \
+    else if (mc <= 4) DS(P, 4, T, BF);                                 \
+    else DS(P, 16, T, BF);                                             \
   } while (0)
   if (precision == KP_FP8) {
-    if (a.rows_bf16) DS_MC(3, uint16_t); else DS_MC(3, float);
+    if (a.rows_bf16) DS_MC(3, uint16_t, false); else DS_MC(3, float, false);
   } else {
-    if (a.rows_bf16) DS_MC(2, uint16_t); else DS_MC(2, float);
+    if (a.rows_bf16) DS_MC(2, uint16_t, true);
+    else if (a.h_bf16) DS_MC(2, float, true);
+    else DS_MC(2, float, false);
   }
 #undef DS_MC
 #undef DS

@@ -602,3 +602,57 @@ def test_large_copies_round_trip(N, K):
             s.set_knn(i, x)
             G, GD = s.get_knn()
             assert np.array_equal(G, i) and np.array_equal(GD, x)
+
+
+def _uneven(name, X):
+    X = X.copy()
+    n = X.shape[0]
+    if name == "small row":
+        X[n // 3] *= np.float32(1e-8)
+    elif name == "large value":
+        X[n // 3, 1] = 3e7
+    elif name == "rows of every size":
+        X *= np.float32(10.0) ** np.linspace(-12, 6, n).astype(np.float32)[:, None]
+    elif name == "tiny and zero rows":
+        X[::7] *= np.float32(1e-33)
+        X[::11] = 0
+    elif name == "norms beyond FP32":  # whose distances to others are not finite
+        X[5] *= np.float32(1e25)
+        X[n // 2:n // 2 + 9] = X[n // 2] + np.float32(1e-3) * X[n // 2:n // 2 + 9]
+        X[n // 2:n // 2 + 9] *= np.float32(6e18) / np.abs(X[n // 2]).max()
+    return X
+
+
+@pytest.mark.parametrize("name", ["small row", "large value", "rows of every size",
+                                  "tiny and zero rows", "norms beyond FP32"])
+@pytest.mark.parametrize("D,K", [(24, 22), (96, 33), (200, 24), (264, 24), (960, 40)])
+def test_uneven_rows_keep_the_16_bit_screen(name, D, K):
+    """Data that one FP16 scale does not fit: builds under BF16 equal the exact ones, most of
+    DPG's pairs are still decided by the screen, and the Filter's and DPG's rows equal the
+    oracle's."""
+    X = _uneven(name, gmm_unit(700, D, 6, D + K))
+    _say(f"uneven rows: {name} D={D} K={K}")
+    with State(*X.shape) as s:
+        s.set_data(X)
+        s.knn_build(K, 4, 3, "exact")
+        Ge, GDe = s.get_knn()
+        ev = s.stats()["knn_evals"]
+        for tile in (0, 1):
+            s.knn_build(K, 4, 3, "bf16", tile=tile)
+            G, GD = s.get_knn()
+            assert np.array_equal(G, Ge) and np.array_equal(GD, GDe)
+            assert s.stats()["knn_evals"] == ev
+        s.prune("dpg", "dist", "rank", 12, 32, 0.0, "fp32")
+        want = s.get_pruned()
+        s.prune("dpg", "dist", "rank", 12, 32, 0.0, "bf16")
+        got = s.get_pruned()
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        left = s.stats()["prune_counters"]["rescored"]
+        pairs = X.shape[0] * K * (K - 1) // 2
+        print(f"  undecided {left} of {pairs}", flush=True)
+        assert 0 < left < pairs // 2, "every pair took a canonical distance"
+    if name != "norms beyond FP32":
+        G, GD = oracle.knn_bruteforce(X, K)
+        for args in [(0, 0, 0, 12, 32, 1.2), (1, 1, 1, 12, 32, 0.5)]:
+            _compare(X, G, GD, *args)
+        _compare(X, G, GD, 3, 0, 2, 12, 32, 0.0, "bf16")
