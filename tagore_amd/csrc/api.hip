@@ -374,9 +374,9 @@ int ensure_prep(tg_state* s) {
   // The 16-bit copy: BF16 where that is exact, else FP16 with the largest value scaled below
   // 2^15.  FP16 cannot hold rows far below the largest value, and its products would leave
   // FP32's range for data beyond these scales; a row error above 2^-9, which is BF16's, shows
-  // the former.  Such data takes rounded BF16: one small row among 40k x 960 and DPG had no
-  // screen at all (48.1 ms a call against XXX, YYY with none), the build took FP32 products
-  // (19.0 against ZZZ)
+  // the former.  Such data takes rounded BF16: with one small row among 40k x 960, DPG takes
+  // 5.9 ms a call (2.3 without that row, 48.2 with no screen) and the build 16.8 (13.8; 19.0 with
+  // FP32 products)
   double rho = 0.0;
   auto row_error = [&](float& r) -> int {
     HIPX(hipMemcpyAsync(f, s->cert_flags, sizeof(f), hipMemcpyDeviceToHost, s->stream));
