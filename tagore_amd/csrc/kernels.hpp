@@ -108,7 +108,7 @@ struct KnnArgs {
   // (screen.hpp); only candidates whose bound interval can change a decision are re-scored
   // with the canonical distance.
   const uint16_t* Xb;  // [N*D] 16-bit rows: BF16 when exact (then Xr16), else scaled FP16 or
-  int copy_bf16;       // (copy_bf16) rounded BF16
+                       // rounded BF16 (copy_bf16)
   const float* nrm2;   // [N] |x|^2 (FP64 sum rounded once)
   float kap;
   float pscale;        // 2 / scale^2 of the 16-bit copy (2 for BF16 and FP32 rows)
@@ -120,6 +120,7 @@ struct KnnArgs {
   // an integer below 2^24): the MFMA screen distance IS the canonical distance, no bound
   // and no re-score are needed.
   int exact_screen;
+  int copy_bf16;       // Xb is BF16
   // rows used for canonical re-scores: BF16 copy when the data set is BF16-exact, else X
   const uint16_t* Xr16;
   const uint8_t* X8;     // u8 copy of X (integers in [0, 255] as x - 128, D <= 256) or null
