@@ -29,6 +29,7 @@
 // 1M x 128: 2.26 -> 0.93 ms.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "rules.hpp"
 
 namespace tg {
 
@@ -139,6 +140,7 @@ __global__ __launch_bounds__(64) void k_search(SearchArgs a) {
   __shared__ uint64_t S[256];     // candidate keys
   __shared__ uint32_t nbr[256];   // initial ids, then the fresh neighbours of a round
   __shared__ uint32_t firstocc[64];
+  static_assert(sizeof(S) + sizeof(nbr) + sizeof(firstocc) == SEARCH_LDS, "search_hash_bits");
   const int lane = threadIdx.x, t = lane & 15;
   const uint32_t N = a.N, D = a.D, FD = a.FD;
   const int L = int(a.L), hb = int(a.hbits);
@@ -385,19 +387,25 @@ __global__ __launch_bounds__(64) void k_search(SearchArgs a) {
   }
 }
 
+template <int MC, int NPL, bool U8>
+void launch_search_t(SearchArgs a, uint32_t grid, hipStream_t s) {
+  // workgroups a CU has to hold: those launched, up to what the registers allow (asked for only
+  // where it can matter)
+  uint32_t per_cu = (grid + 255) / 256;
+  int fit = 0;
+  if (per_cu > 4 && hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k_search<MC, NPL, U8>, 64, 0) ==
+                        hipSuccess && fit > 0)
+    per_cu = std::min(per_cu, uint32_t(fit));
+  a.hbits = search_hash_bits(a.L, a.FD, per_cu);
+  k_search<MC, NPL, U8><<<grid, 64, size_t(4) << a.hbits, s>>>(a);
+}
+
 }  // namespace
 
-// Slots of the visited hash: two thirds filled at the usual L * FD / 2 + L visited ids, 2^10 to
-// 2^13 (the largest leaves five workgroups per CU; longer searches go on in the bitmap).
-void launch_search(const SearchArgs& args, uint32_t grid, hipStream_t s) {
-  SearchArgs a = args;
-  const uint32_t usual = a.L * a.FD / 2 + a.L + 128;
-  a.hbits = 10;
-  while (a.hbits < 13 && (2u << a.hbits) < 3 * usual) ++a.hbits;
-  const size_t lds = size_t(4) << a.hbits;
+void launch_search(const SearchArgs& a, uint32_t grid, hipStream_t s) {
   const int mc = (int(a.D) + 63) / 64;
   const int npl = a.L <= 64 ? 1 : (a.L <= 128 ? 2 : 4);
-#define SR(M, P, U) k_search<M, P, U><<<grid, 64, lds, s>>>(a)
+#define SR(M, P, U) launch_search_t<M, P, U>(a, grid, s)
 #define SR_P(M, U)                                \
   do {                                            \
     if (npl == 1) SR(M, 1, U);                    \

@@ -206,3 +206,27 @@ def test_search_visited_set_and_rows(D, FD, L):
             if step == 0 and D % 8 == 0:
                 s.knn_build(4, 2, 1, "bf16")  # prepares the data
                 s.set_pruned(deg, ids, 5)
+
+
+@pytest.mark.parametrize("D,FD,L,nq", [(32, 96, 200, 3200), (160, 48, 256, 2100), (264, 64, 128, 1300),
+                                       (64, 128, 64, 1025)])
+def test_search_batches_with_small_hashes(D, FD, L, nq):
+    """Batches whose workgroups share a CU's LDS, so that their visited hashes are smaller than
+    the searches need and most ids are in the bitmap; integer and fractional queries."""
+    rng = np.random.default_rng(D + nq)
+    N = 12000
+    X = rng.integers(0, 256, (N, D)).astype(np.float32)
+    Q = rng.integers(0, 256, (nq, D)).astype(np.float32)
+    Q[1::2] += 0.25
+    ids = rng.integers(0, N, (N, FD)).astype(np.uint32)
+    deg = np.full(N, FD, np.uint32)
+    _say(f"batch search D={D} FD={FD} L={L} nq={nq}")
+    oi, od, oc = oracle.search(X, deg, ids, 5, Q, L, 10, 0x77)
+    with State(N, D) as s:
+        s.set_data(X)
+        s.knn_build(4, 2, 1, "fp32")  # prepares the u8 rows
+        s.set_pruned(deg, ids, 5)
+        for rep in range(2):
+            gi, gd, st = s.search(Q, k=10, L=L, seed=0x77)
+            assert np.array_equal(gi, oi) and np.array_equal(gd, od)
+            assert st["evals"] == oc["evals"] and st["expansions"] == oc["expansions"]

@@ -14,6 +14,10 @@ SRC = """
 extern "C" float kappa16(double rho, uint32_t D, uint32_t chain) {
   return tg::screen_kappa16(rho, D, chain);
 }
+extern "C" uint32_t hash_bits(uint32_t L, uint32_t FD, uint32_t per_cu) {
+  return tg::search_hash_bits(L, FD, per_cu);
+}
+extern "C" uint32_t search_lds() { return tg::SEARCH_LDS; }
 extern "C" float kappa32(uint32_t D) { return tg::screen_kappa32(D); }
 """
 
@@ -73,3 +77,19 @@ def test_screen_slack_covers_any_accumulation(rules, D, step, chain, how):
         s = (na + nb) - 2.0 * float(dot)
         kap = rules.kappa16(0.0, D, chain) if step == 32 else rules.kappa32(D)
         assert abs(s - d) <= kap * (na + nb), (at, abs(s - d) / (na + nb) * 2**23, kap * 2**23)
+
+
+@pytest.mark.parametrize("L", [1, 10, 64, 65, 128, 256])
+@pytest.mark.parametrize("FD", [1, 16, 32, 48, 96, 128])
+def test_search_hash_leaves_room_for_the_workgroups(rules, L, FD):
+    """A CU's 160 KB hold as many workgroups as are to run there, up to 21 (the smallest hash);
+    up to four, the hash has the size that the number of visited ids asks for; the initial ids
+    always fit."""
+    usual = L * FD // 2 + L + 128
+    want = next((b for b in range(10, 13) if 2 << b >= 3 * usual), 13)
+    for per_cu in range(1, 22):
+        bits = rules.hash_bits(L, FD, per_cu)
+        lds = -(-((4 << bits) + rules.search_lds()) // 1280) * 1280
+        assert per_cu * lds <= 160 * 1024, (per_cu, bits)
+        assert bits == want if per_cu <= 4 else 10 <= bits <= want
+        assert (3 << bits) // 4 >= 256 + 128
