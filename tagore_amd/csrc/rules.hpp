@@ -31,10 +31,10 @@ inline float screen_kappa32(uint32_t D) { return float((1.25 * D + 128.0) / 8388
 // L * FD / 2 + L visited ids, 2^10 to 2^13, but no more than leaves room for `per_cu` workgroups
 // in a CU's 160 KB (allocated in units of 1,280 bytes; SEARCH_LDS besides the hash).  A search
 // that fills its hash goes on in a bitmap in device memory, which costs less than waves that do
-// not run.  10,000 queries, 12 or (u8 rows above 128, all rows above 256 elements) 8 workgroups
+// not run.  10,000 queries, 12 or (all rows above 256 elements, u8 rows above 128) 8 workgroups
 // per CU, at the largest size / at this one: 200k x 96 FP32 rows, FD 32, L 256 10.9 / 5.5 ms, FD
-// 48, L 128 5.7 / 3.2; 300k x 128 u8 rows, FD 32, L 256 8.2 / 4.3; 100k x 256 u8 rows, FD 32, L
-// 256 8.0 / 5.4; 50k x 960, FD 48, L 128 8.9 / 6.9.  1,000 queries (4 per CU), 300k x 128, FD
+// 48, L 128 5.7 / 3.2; 300k x 128 u8 rows, FD 32, L 256 8.2 / 4.3; 100k x 256 u8 rows, FD 48, L
+// 128 4.3 / 2.9; 50k x 960, FD 48, L 128 8.9 / 6.9.  1,000 queries (4 per CU), 300k x 128, FD
 // 48, L 128: 0.64 ms at 2^13, 0.80 at 2^11.
 constexpr uint32_t SEARCH_LDS = 256 * 8 + 256 * 4 + 64 * 4;
 inline uint32_t search_hash_bits(uint32_t L, uint32_t FD, uint32_t per_cu) {

@@ -134,8 +134,9 @@ __device__ __forceinline__ void eval_f32(const float* X, int D, const Row16<MC>&
 }
 
 // U8: a.X8 holds the u8 copy of the data.
-template <int MC, int NPL, bool U8>
-__global__ __launch_bounds__(64) void k_search(SearchArgs a) {
+// WV: waves per SIMD that the registers leave at least.
+template <int MC, int NPL, bool U8, int WV>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WV))) void k_search(SearchArgs a) {
   extern __shared__ uint32_t vtab[];  // visited hash, 2^hbits ids
   __shared__ uint64_t S[256];     // candidate keys
   __shared__ uint32_t nbr[256];   // initial ids, then the fresh neighbours of a round
@@ -387,17 +388,27 @@ __global__ __launch_bounds__(64) void k_search(SearchArgs a) {
   }
 }
 
-template <int MC, int NPL, bool U8>
-void launch_search_t(SearchArgs a, uint32_t grid, hipStream_t s) {
+template <int MC, int NPL, bool U8, int WV>
+void launch_search_w(SearchArgs a, uint32_t grid, uint32_t per_cu, hipStream_t s) {
   // workgroups a CU has to hold: those launched, up to what the registers allow (asked for only
   // where it can matter)
-  uint32_t per_cu = (grid + 255) / 256;
   int fit = 0;
-  if (per_cu > 4 && hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k_search<MC, NPL, U8>, 64, 0) ==
-                        hipSuccess && fit > 0)
+  if (per_cu > 4 && hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k_search<MC, NPL, U8, WV>, 64,
+                                                                 0) == hipSuccess && fit > 0)
     per_cu = std::min(per_cu, uint32_t(fit));
   a.hbits = search_hash_bits(a.L, a.FD, per_cu);
-  k_search<MC, NPL, U8><<<grid, 64, size_t(4) << a.hbits, s>>>(a);
+  k_search<MC, NPL, U8, WV><<<grid, 64, size_t(4) << a.hbits, s>>>(a);
+}
+template <int MC, int NPL, bool U8>
+void launch_search_t(const SearchArgs& a, uint32_t grid, hipStream_t s) {
+  const uint32_t per_cu = (grid + 255) / 256;
+  // u8 rows above 128 elements, pool above 128: two waves per SIMD by themselves, three with 20
+  // spilled registers.  More than eight queries per CU need the third (10,000 over 100k x 256, L
+  // 256, FD 16 / 32 / 48: 5.5 / 5.4 / 5.3 ms with two, 4.5 / 4.3 / 4.2 with three); one does not
+  // (554 us, 576)
+  if constexpr (MC == 4 && U8 && NPL == 4)
+    if (per_cu > 8) return launch_search_w<MC, NPL, U8, 3>(a, grid, per_cu, s);
+  launch_search_w<MC, NPL, U8, 1>(a, grid, per_cu, s);
 }
 
 }  // namespace

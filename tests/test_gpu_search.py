@@ -209,7 +209,7 @@ def test_search_visited_set_and_rows(D, FD, L):
 
 
 @pytest.mark.parametrize("D,FD,L,nq", [(32, 96, 200, 3200), (160, 48, 256, 2100), (264, 64, 128, 1300),
-                                       (64, 128, 64, 1025)])
+                                       (64, 128, 64, 1025), (160, 32, 130, 2305)])
 def test_search_batches_with_small_hashes(D, FD, L, nq):
     """Batches whose workgroups share a CU's LDS, so that their visited hashes are smaller than
     the searches need and most ids are in the bitmap; integer and fractional queries."""
