@@ -43,60 +43,68 @@ __device__ __forceinline__ void padd(Ph&, long long& sum, long long dt) {
 }
 constexpr int POOL_MAX = 1024;  // K + 480 <= 608, padded to a power of two
 
-// Id set in LDS: HS_BUCKETS buckets of four ids (INV: empty), each with a 16-bit count, in
-// HS_WORDS words.  An insert takes a place by adding to its bucket's count and moves on to the
+// Id set in LDS: 2^bits buckets of four ids (INV: empty), each with a 16-bit count, in
+// hs_words(bits) words.  An insert takes a place by adding to its bucket's count and moves on to the
 // next bucket when this one is full; a look-up reads one bucket and moves on only past a full
-// one.  The beam's set holds at most TOPM + K <= 256 members, half of the places, so both end
-// whatever the ids are.  Against open addressing over single slots there is no chain of
+// one.  The beam's set holds at most TOPM + K members, less than its places (hs_bits), so both
+// end whatever the ids are.  Against open addressing over single slots there is no chain of
 // compare-and-swaps, as long as the longest of the wave's 64: the inserts of one round overlap.
 // (Path Collect over 1M x 128 u8 rows, K 96, TOPM 64, profiled cycles per node: look-ups and
 // compaction 106k with 256 single slots, 43k with 512, 36k with the buckets; inserts 62k / 58k
 // with 512 / the buckets.)
 // -------------------------------------------------------------------------------------
-constexpr int HS_BUCKETS = 128, HS_WORDS = HS_BUCKETS * 4 + HS_BUCKETS / 2;
+__host__ __device__ constexpr int hs_words(int bits) { return (4 << bits) + ((1 << bits) >> 1); }
+// 64 buckets up to 128 members (W = 1), half of the places, 128 up to 256.  Where the pool's
+// filter needs little LDS itself, 64 up to 192 members (three quarters) too: more buckets
+// would leave 21 workgroups per CU instead of 24.  (FP32 rows without a 16-bit copy, 100k x 36,
+// forward pass with 128 buckets / this: NSG over K = 48 4.15 / 3.86 ms, Vamana 10.9 / 9.9, over K =
+// 96 5.66 / 5.56 and 12.5 / 11.9.)
+__host__ __device__ constexpr int hs_bits(int W, int members, bool mf) {
+  return W == 1 ? 6 : mf ? 7 : members <= 192 ? 6 : 7;
+}
 // (the 24-bit product is a full-rate instruction, the 32-bit one a quarter; ids that share
 // their low 24 bits share a bucket)
-__device__ __forceinline__ uint32_t hbucket(uint32_t id) {
-  return ((id & 0xFFFFFFu) * 0x9E3779u) >> (32 - 7);
+__device__ __forceinline__ uint32_t hbucket(uint32_t id, int bits) {
+  return ((id & 0xFFFFFFu) * 0x9E3779u) >> (32 - bits);
 }
-__device__ __forceinline__ void hset_clear(uint32_t* tab) {  // tab 16-byte aligned
-  for (int i = 4 * threadIdx.x; i < HS_BUCKETS * 4; i += 4 * TG_WAVE)
+__device__ __forceinline__ void hset_clear(uint32_t* tab, int bits) {  // tab 16-byte aligned
+  for (int i = 4 * threadIdx.x; i < (4 << bits); i += 4 * TG_WAVE)
     *reinterpret_cast<uint4*>(tab + i) = make_uint4(TG_INV, TG_INV, TG_INV, TG_INV);
-  tab[HS_BUCKETS * 4 + threadIdx.x] = 0;
+  if (int(threadIdx.x) < (1 << bits) / 2) tab[(4 << bits) + threadIdx.x] = 0;
 }
 // inserts one id per lane and list entry (INV: none)
 template <int C>
-__device__ __forceinline__ void hset_insert(uint32_t* tab, const uint32_t (&id)[C]) {
+__device__ __forceinline__ void hset_insert(uint32_t* tab, const uint32_t (&id)[C], int bits) {
   uint32_t h[C], old[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    h[c] = hbucket(id[c]);
+    h[c] = hbucket(id[c], bits);
     old[c] = 0;
     if (id[c] != TG_INV)
-      old[c] = atomicAdd(&tab[HS_BUCKETS * 4 + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
+      old[c] = atomicAdd(&tab[(4 << bits) + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
   }
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     if (id[c] == TG_INV) continue;
     uint32_t at = (old[c] >> ((h[c] & 1) * 16)) & 0xFFFFu;
     while (at >= 4) {
-      h[c] = (h[c] + 1) & (HS_BUCKETS - 1);
-      const uint32_t o = atomicAdd(&tab[HS_BUCKETS * 4 + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
+      h[c] = (h[c] + 1) & ((1 << bits) - 1);
+      const uint32_t o = atomicAdd(&tab[(4 << bits) + (h[c] >> 1)], 1u << ((h[c] & 1) * 16));
       at = (o >> ((h[c] & 1) * 16)) & 0xFFFFu;
     }
     tab[h[c] * 4 + at] = id[c];
   }
 }
-__device__ __forceinline__ bool hset_has(const uint32_t* tab, uint32_t id) {
-  uint32_t h = hbucket(id);
+__device__ __forceinline__ bool hset_has(const uint32_t* tab, uint32_t id, int bits) {
+  uint32_t h = hbucket(id, bits);
   for (;;) {
     const uint4 v = *reinterpret_cast<const uint4*>(tab + h * 4);
     if (v.x == id || v.y == id || v.z == id || v.w == id) return true;
     if (v.w == TG_INV) return false;
-    h = (h + 1) & (HS_BUCKETS - 1);
+    h = (h + 1) & ((1 << bits) - 1);
   }
 }
-static_assert(HS_BUCKETS / 2 == TG_WAVE, "one lane clears one word of counts");
+static_assert((1 << 7) / 2 <= TG_WAVE, "one lane clears one word of counts");
 
 // -------------------------------------------------------------------------------------
 // Beam search shared by cal_ep and path Collect (spec in the oracle's beam_search).
@@ -118,7 +126,7 @@ static_assert(HS_BUCKETS / 2 == TG_WAVE, "one lane clears one word of counts");
 template <int MC, class T, int W, class Ph>
 __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>& tgt,
                                             uint32_t start,
-                                            int max_exp, uint64_t* S, uint32_t* tab,
+                                            int max_exp, uint64_t* S, uint32_t* tab, int bits,
                                             uint16_t* cl, uint64_t* ring, uint64_t* out, uint32_t& ring_c,
                                             uint32_t& n_eval, uint32_t& n_adj, Ph& ph) {
   const int lane = threadIdx.x;
@@ -144,7 +152,7 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
   n_eval += K;
   n_adj += 1;
   ring_c = K;
-  hset_clear(tab);
+  hset_clear(tab, bits);
   __syncthreads();
   uint64_t v[W], bk[W];
   {
@@ -154,7 +162,7 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
       v[r] = S[r * 64 + lane];
       ids[r] = key_id(v[r]);
     }
-    hset_insert(tab, ids);
+    hset_insert(tab, ids, bits);
   }
   reg_bitonic<W>(v);
 #pragma unroll
@@ -193,7 +201,7 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
       const int j = q * TG_WAVE + lane;
       bool fresh = false;
       if (j < K) {
-        fresh = !hset_has(tab, y[q]);
+        fresh = !hset_has(tab, y[q], bits);
         S[j] = INFKEY | y[q];
       } else {
         S[j] = TG_KEY_INF;
@@ -274,7 +282,7 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
     }
     if (next != TG_KEY_INF) load_adj(key_id(next), y);
     // next dedup set: ids of this round's beam and candidates
-    hset_clear(tab);
+    hset_clear(tab, bits);
     __syncthreads();
     {
       uint32_t ids[2 * W];
@@ -283,7 +291,7 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
         ids[2 * q] = key_id(bk[q]);
         ids[2 * q + 1] = key_id(v[q]);
       }
-      hset_insert(tab, ids);
+      hset_insert(tab, ids, bits);
     }
     const long long s3 = pclock(ph);
     padd(ph, ph.sub[3], s3 - s2);
@@ -793,8 +801,8 @@ __device__ __forceinline__ void count_add(unsigned long long* c, int idx, uint32
 // Forward pass (Collect + Filter + Store reverse pushes).  kind 0: path, 1: two-hop.
 //
 // LDS (dynamic, sized from K, TOPM and FD so that more workgroups fit a CU):
-//   during the beam: the 480-slot ring (padded to 512 for its sort), then S | tab | beam
-//       compaction indices;
+//   during the beam: the 480-slot ring (its sort pads it to 512 in registers), then S | tab |
+//       beam compaction indices;
 //   afterwards: the pool (K + 480 keys, over the ring and the dead start of the beam's
 //       scratch), then the selected list and the filter's lists.
 // The pool is the merge of the sorted own list and the sorted ring, formed in registers as
@@ -804,20 +812,23 @@ __device__ __forceinline__ void count_add(unsigned long long* c, int idx, uint32
 constexpr int RING_P = 512;
 
 struct FwdLayout {
-  int W, NS, L, offB, offF, bytes;
+  int W, NS, L, HB, offB, offF, bytes;
 };
-__host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD,
-                                                         bool mfma) {
+// mf: filter_pool_mfma; queue: its re-score queue (16-bit copy); beam: the path's Collect
+__host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD, bool mf, bool queue,
+                                                bool beam) {
   FwdLayout l;
   l.W = (K <= 64 && TOPM <= 64) ? 1 : 2;
   l.NS = 64 * l.W;
   l.L = K + RING;
-  l.offB = RING_P * 8;
+  l.HB = hs_bits(l.W, TOPM + K, mf);
+  l.offB = RING * 8;
   l.offF = ((l.L > RING_P ? l.L : RING_P) * 8 + 15) / 16 * 16;
-  const int beam = l.offB + l.NS * 8 + HS_WORDS * 4 + l.NS * 2;
+  const int coll = beam ? l.offB + l.NS * 8 + hs_words(l.HB) * 4 + l.NS * 2 : l.offB;
   // the filter's selection, live list, killer masks and re-score queue
-  const int filt = l.offF + (FD + 1) * 8 + (l.L + 17) * 4 + (mfma ? FQ_CAP * 2 : 0);
-  l.bytes = ((beam > filt ? beam : filt) + 15) / 16 * 16;
+  const int lists = (l.L + 17) * 2;
+  const int filt = l.offF + (FD + 1) * 8 + (mf ? 2 * lists : lists) + (queue ? FQ_CAP * 2 : 0);
+  l.bytes = ((coll > filt ? coll : filt) + 15) / 16 * 16;
   return l;
 }
 
@@ -835,12 +846,14 @@ void k_forward(PruneArgs a) {
   if (u >= a.N) return;
   const int lane = threadIdx.x, t = lane & 15;
   const int K = a.K, D = a.D;
-  const FwdLayout ly = fwd_layout(K, int(a.TOPM), int(a.FD), MF && !std::is_same<T, uint8_t>::value);
+  const FwdLayout ly = fwd_layout(K, int(a.TOPM), int(a.FD), MF,
+                                  MF && !std::is_same<T, uint8_t>::value, KIND == 0);
   uint64_t* R = reinterpret_cast<uint64_t*>(dsm);
   uint64_t* P = R;  // after the pool is formed
   uint64_t* S = reinterpret_cast<uint64_t*>(dsm + ly.offB);
   uint32_t* tab = reinterpret_cast<uint32_t*>(S + ly.NS);
-  uint16_t* clb = reinterpret_cast<uint16_t*>(tab + HS_WORDS);
+  const int hb = hs_bits(W, K + int(a.TOPM), MF);  // ly.HB, a constant in most kernels
+  uint16_t* clb = reinterpret_cast<uint16_t*>(tab + hs_words(hb));
   uint64_t* sel = reinterpret_cast<uint64_t*>(dsm + ly.offF);  // after the beam
   uint16_t* cl = reinterpret_cast<uint16_t*>(sel + a.FD + 1);
   uint16_t* km = cl + ((ly.L + 17) & ~1);
@@ -848,8 +861,7 @@ void k_forward(PruneArgs a) {
   const int L = ly.L;
   Row16<MC> xu;
   load_row16<MC>(xu, reinterpret_cast<const T*>(a.rows) + size_t(u) * D, D, t);
-  for (int i = lane; i < RING_P; i += TG_WAVE)
-    R[i] = i < RING ? mk_key(__uint_as_float(0x7F800000u), TG_INV) : TG_KEY_INF;
+  for (int i = lane; i < RING; i += TG_WAVE) R[i] = mk_key(__uint_as_float(0x7F800000u), TG_INV);
   __syncthreads();
   uint32_t n_col = 0, n_adj = 0, n_flt = 0;
   Ph ph;
@@ -857,7 +869,7 @@ void k_forward(PruneArgs a) {
   if (KIND == 0) {
     uint32_t ring_c = 0;
     const uint32_t ep = a.ep[a.seg_of ? a.seg_of[u] : 0];
-    beam_search<MC, T, W>(a, xu, ep, 10, S, tab, clb, R, nullptr, ring_c, n_col,
+    beam_search<MC, T, W>(a, xu, ep, 10, S, tab, hb, clb, R, nullptr, ring_c, n_col,
                           n_adj, ph);
   } else {
     // two-hop ids y_i = G[G[u][i/K]][i%K], i < 480
@@ -885,7 +897,8 @@ void k_forward(PruneArgs a) {
     }
     uint64_t rr[RING_P / 64];
 #pragma unroll
-    for (int q = 0; q < RING_P / 64; ++q) rr[q] = R[q * 64 + lane];
+    for (int q = 0; q < RING_P / 64; ++q)
+      rr[q] = q * 64 + lane < RING ? R[q * 64 + lane] : TG_KEY_INF;
     reg_bitonic<RING_P / 64, uint64_t, true>(rr);
     pv[0] = o[0];
     pv[1] = o[1];
@@ -1253,7 +1266,7 @@ __global__ __launch_bounds__(64) void k_rank_reverse(PruneArgs a) {
 template <int MC, class T>
 __global__ __launch_bounds__(64) void k_cal_ep(PruneArgs a, const float* centroid, uint32_t* ep) {
   __shared__ uint64_t M0[128], S[128];
-  __shared__ __attribute__((aligned(16))) uint32_t tab[HS_WORDS];
+  __shared__ __attribute__((aligned(16))) uint32_t tab[hs_words(7)];
   __shared__ uint16_t cl[128];
   const uint32_t seg = blockIdx.x;
   const uint32_t start = a.seg_lo ? a.seg_lo[seg] : 0u;
@@ -1262,9 +1275,9 @@ __global__ __launch_bounds__(64) void k_cal_ep(PruneArgs a, const float* centroi
   uint32_t rc = 0, ne = 0, na = 0;
   PhaseOff ph;  // not reported for the entry point
   if (a.K <= 64 && a.TOPM <= 64)
-    beam_search<MC, T, 1>(a, c, start, 30, S, tab, cl, nullptr, M0, rc, ne, na, ph);
+    beam_search<MC, T, 1>(a, c, start, 30, S, tab, 7, cl, nullptr, M0, rc, ne, na, ph);
   else
-    beam_search<MC, T, 2>(a, c, start, 30, S, tab, cl, nullptr, M0, rc, ne, na, ph);
+    beam_search<MC, T, 2>(a, c, start, 30, S, tab, 7, cl, nullptr, M0, rc, ne, na, ph);
   if (threadIdx.x == 0) ep[seg] = key_id(M0[0]);
   count_add(a.counters, 4, ne);
 }
@@ -1311,7 +1324,8 @@ __global__ void k_centroid_final(const double* part, uint32_t nch, uint32_t N, u
 template <int MC, class T, bool MF>
 static void launch_filter_mc(const PruneArgs& a, int phase, hipStream_t s) {
   const dim3 grid(grid_rows(a.perm, a.N)), block(64);
-  const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD, MF && !std::is_same<T, uint8_t>::value);
+  const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD, MF, MF && !std::is_same<T, uint8_t>::value,
+                                 phase == PH_FWD_PATH);
 #define FWD(KIND, W)                                                                            \
   do {                                                                                         \
     if (a.phase_clock) k_forward<MC, T, KIND, W, MF, PhaseOn><<<grid, block, f.bytes, s>>>(a); \

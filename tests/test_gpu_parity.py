@@ -656,3 +656,25 @@ def test_uneven_rows_keep_the_16_bit_screen(name, D, K):
         for args in [(0, 0, 0, 12, 32, 1.2), (1, 1, 1, 12, 32, 0.5)]:
             _compare(X, G, GD, *args)
         _compare(X, G, GD, 3, 0, 2, 12, 32, 0.0, "bf16")
+
+
+@pytest.mark.parametrize("K,TOPM", [(30, 24), (64, 64), (65, 20), (96, 64), (100, 92), (100, 93)])
+def test_path_collect_id_set_without_a_copy(K, TOPM):
+    """Path Collect over FP32 rows without a 16-bit copy (D % 8 != 0), whose id set has 64 buckets
+    up to 192 members: lists whose ids share the buckets at the table's end, and spread.  Rows,
+    evaluation counts and entry points equal to the oracle."""
+    rng = np.random.default_rng(K + TOPM)
+    N = 3000
+    X = rng.standard_normal((N, 12)).astype(np.float32)
+    bucket = (np.arange(N, dtype=np.uint32) * np.uint32(0x9E3779)) >> np.uint32(26)
+    for which in ([62, 63, 0], range(64)):
+        members = np.flatnonzero(np.isin(bucket, which))
+        ids = np.empty((N, K), np.uint32)
+        d = np.empty((N, K), np.float32)
+        for u in range(N):
+            c = rng.choice(members, K + 1, replace=False, shuffle=False)
+            c = c[c != u][:K]
+            dist = oracle.dist_pairs(X, np.full(K, u, np.uint32), c.astype(np.uint32))
+            o = np.lexsort((c, dist))
+            ids[u], d[u] = c[o], dist[o]
+        _compare(X, ids, d, 0, 0, 0, 16, TOPM, 1.2)
