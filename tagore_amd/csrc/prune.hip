@@ -55,12 +55,14 @@ constexpr int POOL_MAX = 1024;  // K + 480 <= 608, padded to a power of two
 // -------------------------------------------------------------------------------------
 __host__ __device__ constexpr int hs_words(int bits) { return (4 << bits) + ((1 << bits) >> 1); }
 // 64 buckets up to 128 members (W = 1), half of the places, 128 up to 256.  Where the pool's
-// filter needs little LDS itself, 64 up to 192 members (three quarters) too: more buckets
-// would leave 21 workgroups per CU instead of 24.  (FP32 rows without a 16-bit copy, 100k x 36,
-// forward pass with 128 buckets / this: NSG over K = 48 4.15 / 3.86 ms, Vamana 10.9 / 9.9, over K =
-// 96 5.66 / 5.56 and 12.5 / 11.9.)
-__host__ __device__ constexpr int hs_bits(int W, int members, bool mf) {
-  return W == 1 ? 6 : mf ? 7 : members <= 192 ? 6 : 7;
+// filter needs little LDS itself (no matrix filter), 128 leave 21 workgroups per CU instead of
+// 24, so many nodes take 64 up to 176 members too; their longer chains cost few nodes more than
+// the workgroups give (FP32 rows without a 16-bit copy, TOPM 64, forward pass with 128 / 64
+// buckets: 40k x 36, K = 72 NSG 1.96 / 1.87 ms, Vamana 4.54 / 4.18; 120k x 100, K = 112 8.82 /
+// 8.67 and 29.0 / 27.9; 10k x 36, K = 112 NSG 0.58 / 0.62; 600 x 4, K = 100 0.12 / 0.22.  W = 1,
+// 100k x 36, K = 48: NSG 4.15 / 3.86, Vamana 10.9 / 9.9).
+__host__ __device__ constexpr int hs_bits(int W, uint32_t nodes, int members, bool mf) {
+  return W == 1 ? 6 : (mf || nodes < 32768 || members > 176) ? 7 : 6;
 }
 // (the 24-bit product is a full-rate instruction, the 32-bit one a quarter; ids that share
 // their low 24 bits share a bucket)
@@ -815,13 +817,13 @@ struct FwdLayout {
   int W, NS, L, HB, offB, offF, bytes;
 };
 // mf: filter_pool_mfma; queue: its re-score queue (16-bit copy); beam: the path's Collect
-__host__ __device__ inline FwdLayout fwd_layout(int K, int TOPM, int FD, bool mf, bool queue,
-                                                bool beam) {
+__host__ __device__ inline FwdLayout fwd_layout(uint32_t N, int K, int TOPM, int FD, bool mf,
+                                                bool queue, bool beam) {
   FwdLayout l;
   l.W = (K <= 64 && TOPM <= 64) ? 1 : 2;
   l.NS = 64 * l.W;
   l.L = K + RING;
-  l.HB = hs_bits(l.W, TOPM + K, mf);
+  l.HB = hs_bits(l.W, N, TOPM + K, mf);
   l.offB = RING * 8;
   l.offF = ((l.L > RING_P ? l.L : RING_P) * 8 + 15) / 16 * 16;
   const int coll = beam ? l.offB + l.NS * 8 + hs_words(l.HB) * 4 + l.NS * 2 : l.offB;
@@ -846,13 +848,13 @@ void k_forward(PruneArgs a) {
   if (u >= a.N) return;
   const int lane = threadIdx.x, t = lane & 15;
   const int K = a.K, D = a.D;
-  const FwdLayout ly = fwd_layout(K, int(a.TOPM), int(a.FD), MF,
+  const FwdLayout ly = fwd_layout(a.N, K, int(a.TOPM), int(a.FD), MF,
                                   MF && !std::is_same<T, uint8_t>::value, KIND == 0);
   uint64_t* R = reinterpret_cast<uint64_t*>(dsm);
   uint64_t* P = R;  // after the pool is formed
   uint64_t* S = reinterpret_cast<uint64_t*>(dsm + ly.offB);
   uint32_t* tab = reinterpret_cast<uint32_t*>(S + ly.NS);
-  const int hb = hs_bits(W, K + int(a.TOPM), MF);  // ly.HB, a constant in most kernels
+  const int hb = hs_bits(W, a.N, K + int(a.TOPM), MF);  // ly.HB, a constant in most kernels
   uint16_t* clb = reinterpret_cast<uint16_t*>(tab + hs_words(hb));
   uint64_t* sel = reinterpret_cast<uint64_t*>(dsm + ly.offF);  // after the beam
   uint16_t* cl = reinterpret_cast<uint16_t*>(sel + a.FD + 1);
@@ -1324,7 +1326,7 @@ __global__ void k_centroid_final(const double* part, uint32_t nch, uint32_t N, u
 template <int MC, class T, bool MF>
 static void launch_filter_mc(const PruneArgs& a, int phase, hipStream_t s) {
   const dim3 grid(grid_rows(a.perm, a.N)), block(64);
-  const FwdLayout f = fwd_layout(a.K, a.TOPM, a.FD, MF, MF && !std::is_same<T, uint8_t>::value,
+  const FwdLayout f = fwd_layout(a.N, a.K, a.TOPM, a.FD, MF, MF && !std::is_same<T, uint8_t>::value,
                                  phase == PH_FWD_PATH);
 #define FWD(KIND, W)                                                                            \
   do {                                                                                         \

@@ -658,21 +658,26 @@ def test_uneven_rows_keep_the_16_bit_screen(name, D, K):
         _compare(X, G, GD, 3, 0, 2, 12, 32, 0.0, "bf16")
 
 
-@pytest.mark.parametrize("K,TOPM", [(30, 24), (64, 64), (65, 20), (96, 64), (100, 92), (100, 93)])
-def test_path_collect_id_set_without_a_copy(K, TOPM):
+@pytest.mark.parametrize("N,K,TOPM", [(3000, 30, 24), (3000, 64, 64), (3000, 100, 92),
+                                      (32767, 65, 20), (32768, 65, 20), (32768, 112, 64),
+                                      (32768, 113, 64)])
+def test_path_collect_id_set_without_a_copy(N, K, TOPM):
     """Path Collect over FP32 rows without a 16-bit copy (D % 8 != 0), whose id set has 64 buckets
-    up to 192 members: lists whose ids share the buckets at the table's end, and spread.  Rows,
-    evaluation counts and entry points equal to the oracle."""
+    for short lists and, from 32768 nodes on, up to 176 members: lists whose ids share the
+    buckets at the table's end, and spread.  Rows, evaluation counts and entry points equal to
+    the oracle."""
     rng = np.random.default_rng(K + TOPM)
-    N = 3000
     X = rng.standard_normal((N, 12)).astype(np.float32)
     bucket = (np.arange(N, dtype=np.uint32) * np.uint32(0x9E3779)) >> np.uint32(26)
     for which in ([62, 63, 0], range(64)):
         members = np.flatnonzero(np.isin(bucket, which))
         ids = np.empty((N, K), np.uint32)
         d = np.empty((N, K), np.float32)
+        # a node's list: K members at equal steps from a start of its own
+        step = max(1, members.size // (K + 1))
+        at = (rng.integers(0, members.size, N)[:, None] + step * np.arange(K + 1)) % members.size
         for u in range(N):
-            c = rng.choice(members, K + 1, replace=False, shuffle=False)
+            c = members[at[u]]
             c = c[c != u][:K]
             dist = oracle.dist_pairs(X, np.full(K, u, np.uint32), c.astype(np.uint32))
             o = np.lexsort((c, dist))
