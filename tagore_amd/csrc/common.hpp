@@ -327,26 +327,6 @@ __device__ __forceinline__ void dist16_pairs(const T* const (&a)[NB], const T* c
   for (int k = 0; k < NB; ++k) out[k] = tree16(p[k][0], p[k][1], p[k][2], p[k][3]);
 }
 
-template <int MC, class T>
-__device__ __forceinline__ float dist16(const Row16<MC>& a, const T* __restrict__ b, int D,
-                                        int t) {
-  float p0 = 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f;
-#pragma unroll
-  for (int m = 0; m < MC; ++m) {
-    const int i = m * 64 + 4 * t;
-    if (i < D) {
-      const float4 y = load4(b + i);
-      const float e0 = a.v[m].x - y.x, e1 = a.v[m].y - y.y, e2 = a.v[m].z - y.z,
-                  e3 = a.v[m].w - y.w;
-      p0 = __builtin_fmaf(e0, e0, p0);
-      p1 = __builtin_fmaf(e1, e1, p1);
-      p2 = __builtin_fmaf(e2, e2, p2);
-      p3 = __builtin_fmaf(e3, e3, p3);
-    }
-  }
-  return tree16(p0, p1, p2, p3);
-}
-
 // both rows from memory
 template <int MC, class T>
 __device__ __forceinline__ float dist16_mm(const T* __restrict__ a, const T* __restrict__ b,
@@ -811,22 +791,6 @@ __device__ __forceinline__ bool row_has_key(const uint32_t* G, const float* GD, 
   for (; lo < K && gd[lo] == key_d(key); ++lo)
     if (G[size_t(v) * K + lo] == key_id(key)) return true;
   return false;
-}
-
-template <class T>
-__device__ __forceinline__ int upper_bound_lds(const T* a, int n, T x) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (!(x < a[mid])) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-// dst[0..na+nb) = stable merge of the sorted arrays A[0..na) and B[0..nb) (A first on ties)
-__device__ void merge_lds(const uint64_t* A, int na, const uint64_t* B, int nb, uint64_t* dst) {
-  for (int i = threadIdx.x; i < na; i += TG_WAVE) dst[i + lower_bound_lds(B, nb, A[i])] = A[i];
-  for (int j = threadIdx.x; j < nb; j += TG_WAVE) dst[j + upper_bound_lds(A, na, B[j])] = B[j];
 }
 
 // Loads of the u8 row at r in the quad layout (MC chunks; zero past D).
