@@ -71,6 +71,7 @@ void dfree(T*& p) {
 constexpr int COPY_LANES = 4;
 constexpr size_t COPY_CHUNK = size_t(1) << 20;
 constexpr size_t COPY_DIRECT = size_t(4) << 20;  // below: one plain copy
+static_assert(COPY_DIRECT >= COPY_LANES * COPY_CHUNK, "every thread of a chunked copy has a chunk");
 struct CopyOut {
   unsigned char* pin = nullptr;
   hipEvent_t ev[2 * COPY_LANES] = {};
@@ -259,7 +260,7 @@ int copy_out(tg_state* s, void* dst, const void* src, size_t n) {
       return f == hipSuccess ? hipEventRecord(ev[half], s->stream) : f;
     };
     int half = 0;
-    if (e == hipSuccess && size_t(l) < nc) e = fetch(l, 0);
+    if (e == hipSuccess) e = fetch(l, 0);
     for (size_t c = l; c < nc && e == hipSuccess; c += COPY_LANES, half ^= 1) {
       e = hipEventSynchronize(ev[half]);
       if (e == hipSuccess && c + COPY_LANES < nc) e = fetch(c + COPY_LANES, half ^ 1);
