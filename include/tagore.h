@@ -88,7 +88,10 @@ typedef struct {
   float thre;        /* threshold: alpha for dist, cos(angle) for angle */
   int32_t precision; /* TG_PREC_BF16: read rows from the BF16 copy when every value of the
                         data set is exactly representable in BF16 (bit-identical result);
-                        otherwise FP32 rows.  DPG with K <= 64 under TG_PREC_BF16 / FP8:
+                        otherwise FP32 rows.  Whatever it says, the Filter of the path and
+                        two-hop kinds screens pairs of rows up to 256 elements on the u8 or
+                        the 16-bit copy (D % 8 == 0) and evaluates those that its bound leaves
+                        open in FP32 (bit-identical result).  DPG with K <= 64 under TG_PREC_BF16 / FP8:
                         pair distances screened on an MFMA Gram, exact re-score near the
                         threshold (bit-identical result) */
 } tg_prune_params;

@@ -616,7 +616,9 @@ void k_localjoin_exact_screen(KnnArgs a) {
 // per node) 48 -> 16.1 ms.  Before, one BF16 product left a bound eight times wider, one of the
 // four waves formed the masks, and each re-score read both rows from L2.  What is left: half
 // of the narrow kernel's cycles issue VALU work, the rest waits on the list, row and push
-// round trips; the wide one streams each sampled row twice.
+// round trips; the wide one streams each sampled row twice.  Waves per SIMD were chosen at 96 and
+// 960 elements; at 129 to 256 six spill 44 to 49 vector registers (two iterations of
+// 100k x 160: 5.99 ms, 4.03 with four waves and no spills).
 // -------------------------------------------------------------------------------------
 template <int PREC, int MC, class T, int DC, bool BF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MC <= 4 ? 6 : 3)))

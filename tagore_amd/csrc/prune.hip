@@ -837,8 +837,10 @@ __host__ __device__ inline FwdLayout fwd_layout(uint32_t N, int K, int TOPM, int
 // mfma: filter_pool_mfma on the 16-bit copy (u8 rows always take it).
 // Ph: PhaseOn in profiling runs.
 template <int MC, class T, int KIND, int W, bool MF, class Ph>
-// Waves per SIMD: six (80 VGPRs) for u8 rows up to 128 elements, fewer where the rows' registers
-// would spill.
+// Waves per SIMD, chosen at 96 and 128 elements: six (80 VGPRs; 0 to 6 spilled) for u8 rows, five
+// for 16-bit rows (11 to 15 spilled).  Rows of 129 to 256 elements took the next step down
+// unmeasured: three for 16-bit rows spill nothing, five for u8 rows spill 40 to 55 registers in
+// the path's kernels (four: 2 at most, Vamana over 100k x 160 6.09 -> 4.82 ms).
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(MC == 2 ? (std::is_same<T, uint8_t>::value || !MF ? 6 : 5)
                                            : (MC == 4 ? (std::is_same<T, uint8_t>::value ? 5 : 3) : 2))))
