@@ -109,7 +109,7 @@ struct KnnArgs {
   // with the canonical distance.
   const uint16_t* Xb;  // [N*D] 16-bit rows: BF16 when exact (then Xr16), else scaled FP16 or
                        // rounded BF16 (copy_bf16)
-  const float* nrm2;   // [N] |x|^2 (FP64 sum rounded once)
+  const float* nrm2;   // [N] |x|^2 (FP64 sum rounded once; NaN above 0 and below 2^-96)
   float kap;
   float pscale;        // 2 / scale^2 of the 16-bit copy (2 for BF16 and FP32 rows)
   // FP8: s +- 2 (ea qb + qa eb + ea eb) + eta (|a|^2 + |b|^2 + 2 qa qb)

@@ -34,7 +34,8 @@ __device__ __forceinline__ uint32_t wg_reduce(uint32_t v, uint32_t* sh, Op op) {
 __device__ __forceinline__ uint32_t op_max(uint32_t a, uint32_t b) { return a > b ? a : b; }
 __device__ __forceinline__ uint32_t op_or(uint32_t a, uint32_t b) { return a | b; }
 
-// |x|^2 of every row (FP64 sums, rounded once) and the data-set certificates:
+// |x|^2 of every row (FP64 sums, rounded once; NaN above 0 and below 2^-96) and the data-set
+// certificates:
 // flags[0] |= some value is not exactly representable in BF16,
 // flags[1] |= some value is not an integer in [-256, 256], flags[2] |= some value is
 // negative, flags[3] = max |x|^2 (FP32 bits; exact for integer data below 2^24),
@@ -66,7 +67,9 @@ __global__ __launch_bounds__(256) void k_screen_prep(const float* X, uint32_t N,
 #pragma unroll
     for (int o = 8; o >= 1; o >>= 1) s2 += __shfl_xor(s2, o, 16);
     top = op_max(top, __float_as_uint(float(s2)));
-    if (t == 0) nrm2[row] = float(s2);
+    // products of rows this small are not normal FP32 numbers, which no bound covers: not a
+    // number, so that no screen decides a pair of such a row
+    if (t == 0) nrm2[row] = s2 > 0.0 && s2 < 0x1p-96 ? __uint_as_float(0x7FC00000u) : float(s2);
   }
   bits = wg_reduce(bits, sh, op_or);
   top = wg_reduce(top, sh, op_max);
@@ -84,10 +87,8 @@ __global__ __launch_bounds__(256) void k_screen_prep(const float* X, uint32_t N,
 // 16-bit copy of the rows: BF16 bits (COPY_EXACT: every value exact), FP16 of x * scale (a power
 // of two that puts the largest value below 2^15), or BF16 to nearest (scale 1); results below
 // the smallest normal value become 0.  The last two: flags[6] = max over the rows of
-// |x' / scale - x| / |x|, rounded up (FP32 bits).  Rows whose |x|^2 is no finite FP32 value are
-// left out (their screen distances decide nothing), as are rows with |x| below 2^-100: lost
-// altogether, one moves s by 2 |a| |b| at most, which the other row's share of the bound covers
-// (kappa is above 2^-16; both rows that small: s = d = 0).
+// |x' / scale - x| / |x|, rounded up (FP32 bits).  Rows whose |x|^2 is no finite FP32 value or
+// below 2^-96 are left out: no screen decides a pair of such a row (k_screen_prep).
 template <int KIND>
 __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N, uint32_t D,
                                                      float scale, uint16_t* Xb, uint32_t* flags) {
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(256) void k_screen_copy(const float* X, uint32_t N,
         s2 += __shfl_xor(s2, o, 16);
         e2 += __shfl_xor(e2, o, 16);
       }
-      const bool in = KIND == COPY_FP16 ? e2 > 0.0 : s2 >= 0x1p-200 && s2 <= 3.4028234e38;
+      const bool in = s2 >= 0x1p-96 && s2 <= 3.4028234e38;
       const float r = in ? float(sqrt(e2 / s2) * (1.0 + 1e-6)) : 0.f;
       worst = op_max(worst, __float_as_uint(r));
     }

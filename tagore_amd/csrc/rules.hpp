@@ -15,8 +15,9 @@ namespace tg {
 // chains on the vector unit add fewer.)  A kernel that sums chains of `chain` elements by FP32
 // additions is off by 33 chain / 32 + D / chain.  The canonical fold costs D / 64 + 14 units of
 // 2^-24 of d <= 2 (|a|^2 + |b|^2), the norms, s and the two ends of the interval a few more:
-// below 128 units of 2^-23 for D <= 1024.  Rows whose |x|^2 is below 2^-96 are outside this
-// (their products are not normal FP32 numbers).
+// below 128 units of 2^-23 for D <= 1024.  Products below the smallest normal FP32 number may
+// count as 0, 2^-115 together, which is in the slack of rows with |x|^2 >= 2^-96; smaller rows
+// have no norm (k_screen_prep), and every comparison with their s leaves the pair undecided.
 //
 // 16-bit rows: rho bounds |x' - x| / |x| over the rows (0 for exact copies), which puts the
 // product off by at most (2 rho + rho^2) |a| |b|.

@@ -683,3 +683,33 @@ def test_path_collect_id_set_without_a_copy(N, K, TOPM):
             o = np.lexsort((c, dist))
             ids[u], d[u] = c[o], dist[o]
         _compare(X, ids, d, 0, 0, 0, 16, TOPM, 1.2)
+
+
+@pytest.mark.parametrize("scale", [1e-14, 1e-16, 1e-18, 1e-20, 1e-22])
+@pytest.mark.parametrize("part", [1.0, 0.4])
+@pytest.mark.parametrize("D,K", [(16, 9), (96, 33), (272, 24)])
+def test_rows_below_the_screens_range(scale, part, D, K):
+    """Rows whose squares are at and below FP32's smallest normal numbers, all of them or among
+    others: every precision's build and DPG's screened prune equal the exact ones, real-valued
+    and with values that BF16 holds."""
+    rng = np.random.default_rng(D)
+    X = gmm_unit(600, D, 6, D + K) * np.float32(4)
+    X[rng.random(600) < part] *= np.float32(scale)
+    for bf in (False, True):
+        Y = (X.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32) if bf else X
+        _say(f"small rows: scale={scale} part={part} D={D} K={K} bf16={bf}")
+        with State(*Y.shape) as s:
+            s.set_data(Y)
+            s.knn_build(K, 4, 3, "exact")
+            Ge, GDe = s.get_knn()
+            want = None
+            for prec in ("fp32", "bf16", "fp8"):
+                s.knn_build(K, 4, 3, prec)
+                G, GD = s.get_knn()
+                assert np.array_equal(G, Ge) and np.array_equal(GD, GDe), prec
+                if want is None:
+                    s.prune("dpg", "dist", "rank", 8, 32, 0.0, "fp32")
+                    want = s.get_pruned()
+                s.prune("dpg", "dist", "rank", 8, 32, 0.0, prec)
+                got = s.get_pruned()
+                assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), prec
