@@ -713,3 +713,11 @@ def test_rows_below_the_screens_range(scale, part, D, K):
                 s.prune("dpg", "dist", "rank", 8, 32, 0.0, prec)
                 got = s.get_pruned()
                 assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), prec
+
+
+@pytest.mark.parametrize("name", ["u8", "bf16", "real", "scales"])
+@pytest.mark.parametrize("D", [8, 16, 32, 40])
+def test_block_filter_edges_of_narrow_rows(name, D):
+    """The Filter's blocks on rows of less than one and of one 64-byte step, with every kind of
+    copy: rows and evaluation counts equal to the oracle."""
+    test_block_filter_edges(name, D)
