@@ -56,13 +56,15 @@ constexpr int POOL_MAX = 1024;  // K + 480 <= 608, padded to a power of two
 __host__ __device__ constexpr int hs_words(int bits) { return (4 << bits) + ((1 << bits) >> 1); }
 // 64 buckets up to 128 members (W = 1), half of the places, 128 up to 256.  Where the pool's
 // filter needs little LDS itself (no matrix filter), 128 leave 21 workgroups per CU instead of
-// 24, so many nodes take 64 up to 176 members too; their longer chains cost few nodes more than
-// the workgroups give (FP32 rows without a 16-bit copy, TOPM 64, forward pass with 128 / 64
-// buckets: 40k x 36, K = 72 NSG 1.96 / 1.87 ms, Vamana 4.54 / 4.18; 120k x 100, K = 112 8.82 /
-// 8.67 and 29.0 / 27.9; 10k x 36, K = 112 NSG 0.58 / 0.62; 600 x 4, K = 100 0.12 / 0.22.  W = 1,
-// 100k x 36, K = 48: NSG 4.15 / 3.86, Vamana 10.9 / 9.9).
+// 24, so more nodes than then run at once take 64 up to 176 members too; fewer nodes only wait
+// for the longer chains.  (FP32 rows without a 16-bit copy, forward pass with 128 / 64 buckets:
+// 6k x 100, K = 64, TOPM 88 NSG 0.290 / 0.282 ms, Vamana 0.765 / 0.688; 40k x 36, K = 72, TOPM 64
+// 1.96 / 1.87 and 4.54 / 4.18; 120k x 100, K = 112 8.82 / 8.67 and 29.0 / 27.9; 2k x 100, K = 96
+// 0.222 / 0.243 and 0.610 / 0.624; 600 x 4, K = 100 0.12 / 0.22.  W = 1, 100k x 36, K = 48: NSG 4.15 /
+// 3.86, Vamana 10.9 / 9.9).
+constexpr uint32_t HS_AT_ONCE = 21 * 256;
 __host__ __device__ constexpr int hs_bits(int W, uint32_t nodes, int members, bool mf) {
-  return W == 1 ? 6 : (mf || nodes < 32768 || members > 176) ? 7 : 6;
+  return W == 1 ? 6 : (mf || nodes <= HS_AT_ONCE || members > 176) ? 7 : 6;
 }
 // (the 24-bit product is a full-rate instruction, the 32-bit one a quarter; ids that share
 // their low 24 bits share a bucket)

@@ -659,11 +659,11 @@ def test_uneven_rows_keep_the_16_bit_screen(name, D, K):
 
 
 @pytest.mark.parametrize("N,K,TOPM", [(3000, 30, 24), (3000, 64, 64), (3000, 100, 92),
-                                      (32767, 65, 20), (32768, 65, 20), (32768, 112, 64),
-                                      (32768, 113, 64)])
+                                      (5376, 65, 20), (5377, 65, 20), (5377, 112, 64),
+                                      (5377, 113, 64)])
 def test_path_collect_id_set_without_a_copy(N, K, TOPM):
     """Path Collect over FP32 rows without a 16-bit copy (D % 8 != 0), whose id set has 64 buckets
-    for short lists and, from 32768 nodes on, up to 176 members: lists whose ids share the
+    for short lists and, above 5376 nodes, up to 176 members: lists whose ids share the
     buckets at the table's end, and spread.  Rows, evaluation counts and entry points equal to
     the oracle."""
     rng = np.random.default_rng(K + TOPM)
