@@ -91,9 +91,9 @@ typedef struct {
                         otherwise FP32 rows.  Whatever it says, the Filter of the path and
                         two-hop kinds screens pairs of rows up to 256 elements on the u8 or
                         the 16-bit copy (D % 8 == 0) and evaluates those that its bound leaves
-                        open in FP32 (bit-identical result).  DPG with K <= 64 under TG_PREC_BF16 / FP8:
-                        pair distances screened on an MFMA Gram, exact re-score near the
-                        threshold (bit-identical result) */
+                        open in FP32 (bit-identical result).  DPG with K <= 64 under
+                        TG_PREC_BF16 / FP8: pair distances screened on an MFMA Gram, exact
+                        re-score near the threshold (bit-identical result) */
 } tg_prune_params;
 
 /* Last error message of the calling thread (never NULL). */

@@ -212,8 +212,8 @@ struct tg_state {
   std::vector<hipEvent_t> ev_pool;
   hipEvent_t win[2] = {};      // window events of a build, prune or search
   CopyOut out;
-  // search: queries on the device, and [counters | ids | dists] of the results, grown on demand up to
-  // SEARCH_KEEP
+  // search: queries on the device, and [counters | ids | dists] of the results, grown on demand,
+  // kept up to SEARCH_KEEP each
   float* sq = nullptr;
   size_t sq_cap = 0;
   unsigned char* sres = nullptr;
@@ -358,6 +358,7 @@ int ensure_knn_scratch(tg_state* s, uint32_t K) {
 // data set, like the reference's host-side FP16 copy, pybind.cu:58-61).
 int ensure_prep(tg_state* s) {
   if (s->prep_valid && !s->x_lent) return TG_OK;
+  s->prep_valid = false;
   const size_t N = s->N;
   if (!s->nrm2) {
     if (dalloc(&s->nrm2, N) || dalloc(&s->cert_flags, 7) || dalloc(&s->Xb, N * s->D))

@@ -238,8 +238,8 @@ __device__ __forceinline__ void beam_search(const PruneArgs& a, const Row16<MC>&
     // the beam nor the previous candidates, so no key ties one in the beam).  With TOPM <= 64
     // and at most 64 such candidates, they are compacted and merged with one-slot sorts; none
     // leaves the beam as it is.  (One slot per lane: only once the beam is full of finite keys;
-    // until then the merge also keeps keys without a distance, which count as seen.)  Either way the beam becomes the TOPM smallest keys of beam and
-    // candidates.
+    // until then the merge also keeps keys without a distance, which count as seen.)  Either way
+    // the beam becomes the TOPM smallest keys of beam and candidates.
     uint64_t worst = TG_KEY_INF;
 #pragma unroll
     for (int b = 0; b < W; ++b)
